@@ -161,6 +161,19 @@ int tt_conv2d_fwd_f32(const float* x, const float* w, const float* bias, float* 
                       int N, int C, int H, int W, int K, int R, int S,
                       int sh, int sw, int ph, int pw, int dh, int dw, int groups);
 
+/* The convolution with what follows it in evaluation mode, in one pass over y:
+ *   v = conv(x, w) (+ bias);  v = (v - mean) / sqrt(var + eps) * gamma + beta;  v = v + residual;
+ *   y = relu ? maximum(v, 0) : v
+ * mean / var (both or neither; [K], with optional gamma, beta) stand for BatchNorm with given
+ * statistics (autograd/grad_nn.py:931-959), residual ([N,K,P,Q] or NULL) for the residual Add
+ * (autograd/grad_fcn.py:177-203), relu for Relu (:56).  Every step rounds as the separate entry
+ * points (tt_conv2d_fwd_f32, tt_bn_fwd_eval_f32, tt_add_f32, tt_relu_fwd_f32) do: same bits. */
+int tt_conv2d_norm_act_fwd_f32(const float* x, const float* w, const float* bias, float* y,
+                               const float* mean, const float* var, const float* gamma, const float* beta,
+                               double eps, const float* residual, int relu,
+                               int N, int C, int H, int W, int K, int R, int S,
+                               int sh, int sw, int ph, int pw, int dh, int dw, int groups);
+
 /* dx[N,C,Hx,Wx] = sum over k,r,s of dy[N,K,P,Q] * w[K,C/groups,R,S] (+ bias[C] if not NULL):
  * the input gradient of the convolution above, and -- with x as `dy`, the [C_in,C_out/g,R,S]
  * transposed-convolution weight as `w`, K = C_in, C = C_out -- the forward pass of
@@ -297,6 +310,11 @@ int tt_bn_fwd_train_noalloc_f32(const float* x, const float* gamma, const float*
 /* Normalisation with given statistics (eval mode), autograd/grad_nn.py:931-959:
  * save_* are written from mean[C]/var[C] exactly as in training so that backward can follow. */
 int tt_bn_fwd_eval_f32(const float* x, const float* gamma, const float* beta, float* y,
+                       const float* mean, const float* var,
+                       float* save_mean, float* save_var_eps, float* save_sd,
+                       double eps, int N, int C, int HW);
+/* tt_bn_fwd_eval_f32 followed by a ReLU in the same pass: y = maximum(bn(x), 0), NaN kept. */
+int tt_bn_relu_fwd_eval_f32(const float* x, const float* gamma, const float* beta, float* y,
                        const float* mean, const float* var,
                        float* save_mean, float* save_var_eps, float* save_sd,
                        double eps, int N, int C, int HW);

@@ -39,6 +39,7 @@ PROTOTYPES = {
     'tt_probe_mfma_f32': [_I, POINTER(c_double), POINTER(c_double), POINTER(c_double)],
     'tt_probe_hbm_f32': [c_size_t, POINTER(c_double), POINTER(c_double)],
     'tt_conv2d_fwd_f32': [_P, _P, _P, _P] + [_I] * 14,
+    'tt_conv2d_norm_act_fwd_f32': [_P] * 8 + [c_double, _P, _I] + [_I] * 14,
     'tt_conv2d_dgrad_f32': [_P, _P, _P, _P] + [_I] * 16,
     'tt_conv2d_wgrad_f32': [_P, _P, _P] + [_I] * 16,
     'tt_conv2d_fwd_bf16': [_P, _P, _P, _P] + [_I] * 14,
@@ -69,6 +70,7 @@ PROTOTYPES = {
     'tt_bn_relu_fwd_train_f32': [_P] * 12 + [c_double, c_double, _I, _I, _I],
     'tt_bn_relu_bwd_f32': [_P] * 10 + [_I, _I, _I],
     'tt_bn_fwd_eval_f32': [_P] * 9 + [c_double, _I, _I, _I],
+    'tt_bn_relu_fwd_eval_f32': [_P] * 9 + [c_double, _I, _I, _I],
     'tt_bn_bwd_f32': [_P] * 9 + [_I, _I, _I],
     'tt_relu_fwd_f32': [_P, _P, c_size_t],
     'tt_relu_bwd_f32': [_P, _P, _P, c_size_t],
@@ -267,6 +269,10 @@ def set_conv_math(mode):
     tolerances as 'f32')."""
     if mode not in CONV_MATH:
         raise ValueError(f"conv math must be one of {sorted(CONV_MATH)}, got {mode!r}")
+    if mode != get_conv_math():
+        # a convolution output that is still to be produced on demand belongs to the mode it was asked for in
+        from .xparray import fill_all
+        fill_all()
     call('tt_set_conv_math', CONV_MATH[mode])
 
 

@@ -7,9 +7,10 @@ from math import prod
 
 import numpy as np
 
-from .. import ops
+from .. import _hip, ops
 from ..xparray import hiparray, nparray
 from .function import Function
+from .grad_mode import is_grad_enabled
 from .helper import build_links
 
 
@@ -69,7 +70,17 @@ class Add(Function):
         if a.__class__ is not hiparray:
             y = np.add(a, b)
         elif a.shape == b.shape:
-            y = ops.add_deferred(a, b)      # parked: a ReLU that comes next absorbs it
+            conv = None
+            if not (ctx.requires_grad and is_grad_enabled()):
+                # one operand is a convolution's output that has not been launched yet: add the other to it
+                # on its way to memory
+                conv = _hip.take_pending_if(lambda op: op.__class__ is ops.DeferredConv and op.residual is None
+                                            and (op.out._buf is a._buf) != (op.out._buf is b._buf)
+                                            and op.out.shape == a.shape)
+            if conv is not None:
+                y = conv.absorb_add(b if conv.out._buf is a._buf else a)
+            else:
+                y = ops.add_deferred(a, b)      # parked: a ReLU that comes next absorbs it
         elif b.size < a.size and _trailing(b.shape, a.shape):
             y = ops.add_rowvec(a, b)
         elif a.size < b.size and _trailing(a.shape, b.shape):

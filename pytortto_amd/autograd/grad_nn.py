@@ -15,6 +15,7 @@ import numpy as np
 from .. import _hip, ops
 from ..xparray import hiparray
 from .function import Function
+from .grad_mode import is_grad_enabled
 from .helper import build_links, inplace_precheck, inplace_update
 
 
@@ -47,7 +48,10 @@ class Convolution(Function):
                                f'expected input{xd0.shape} to have {groups * xd1.shape[-3]} channels, '
                                f'but got {xd0.shape[-3]} channels instead')
         _device_only('Convolution', xd0)
-        yd0 = ops.conv2d_fwd(xd0, xd1, xd2, stride, padding, dilation, groups)
+        # without a gradient to keep anything for, the launch is parked: the normalisation, residual add
+        # and ReLU of an evaluation pass join it
+        conv = ops.conv2d_fwd if ctx.requires_grad and is_grad_enabled() else ops.conv2d_fwd_deferred
+        yd0 = conv(xd0, xd1, xd2, stride, padding, dilation, groups)
         yt0 = build_links(yd0, grad_fn=ctx)
         # the reference also keeps a zero-padded copy of the input for the weight gradient
         # (grad_nn.py:714); the kernels address padding implicitly, so the input itself suffices
@@ -148,7 +152,17 @@ class BatchNorm(Function):
                 running_mean.data = new_rm
                 running_var.data = new_rv
         elif have_running:
-            yd0, mean, var_eps, sd = ops.bn_fwd_eval(xd0, gamma, beta, running_mean.data, running_var.data, eps)
+            no_gradient = not (ctx.requires_grad and is_grad_enabled())
+            if no_gradient:
+                conv = _hip.take_pending_if(lambda op: op.__class__ is ops.DeferredConv and op.takes_norm()
+                                            and op.out._buf is xd0._buf and op.out.shape == xd0.shape)
+                if conv is not None:
+                    # x is a convolution's output that has not been launched yet: normalise it on its way
+                    # to memory (nothing is saved: no gradient will flow)
+                    return build_links(conv.absorb_norm(running_mean.data, running_var.data, gamma, beta, eps),
+                                       grad_fn=ctx)
+            yd0, mean, var_eps, sd = ops.bn_fwd_eval(xd0, gamma, beta, running_mean.data, running_var.data, eps,
+                                                       deferred=no_gradient)
         elif xd0.size == xd0.shape[1]:
             # eval mode without buffers and one value per channel: the batch statistics are the value
             # itself and zero (grad_nn.py:935-937); only training refuses this shape (:921-922)
@@ -177,6 +191,10 @@ class BatchNorm(Function):
         return grad0, grad1, grad2
 
 
+# parked operations that a ReLU behind them joins
+_TAKES_RELU = (ops.DeferredBatchNorm, ops.DeferredAdd, ops.DeferredConv, ops.DeferredBatchNormEval)
+
+
 class Relu(Function):
     @staticmethod
     def forward(ctx, *inputs, **params):
@@ -186,11 +204,10 @@ class Relu(Function):
         # only a device input can be the output of a parked device operation (a host array has no buffer)
         parked = None
         if xd0.__class__ is hiparray:
-            parked = _hip.take_pending_if(lambda op: (op.__class__ is ops.DeferredBatchNorm and op.y._buf is xd0._buf)
-                                          or (op.__class__ is ops.DeferredAdd and op.out._buf is xd0._buf))
+            parked = _hip.take_pending_if(lambda op: op.__class__ in _TAKES_RELU and op.out._buf is xd0._buf)
         if parked is not None:
-            # the input is a BatchNorm output, or a residual sum, that has not been launched yet: one
-            # kernel writes maximum(bn(x), 0) (grad_nn.py:942-959 and :56 in one pass) or maximum(a + b, 0)
+            # the input is a BatchNorm output, a residual sum, or a convolution's, that has not been launched
+            # yet: one kernel writes maximum(bn(x), 0) (grad_nn.py:942-959 and :56 in one pass), maximum(a + b, 0) ...
             if inplace:
                 try:
                     inplace_precheck(xt0)

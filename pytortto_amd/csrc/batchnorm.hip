@@ -876,14 +876,13 @@ int tt_bn_fwd_train_noalloc_f32(const float* x, const float* gamma, const float*
                       eps, N, C, HW, g_scratch_ptr[dev], (size_t)kScratchPartials);
 }
 
-int tt_bn_fwd_eval_f32(const float* x, const float* gamma, const float* beta, float* y, const float* mean,
-                       const float* var, float* save_mean, float* save_var_eps, float* save_sd, double eps, int N,
-                       int C, int HW) {
+static int bn_fwd_eval(const char* fn, const float* x, const float* gamma, const float* beta, float* y, const float* mean,
+                       const float* var, float* save_mean, float* save_var_eps, float* save_sd, double eps, int N, int C,
+                       int HW, bool relu) {
   TT_REQUIRE_INIT();
-  if (check_shape("tt_bn_fwd_eval_f32", N, C, HW)) return -1;
-  TT_REQUIRE(x && y && mean && var && save_mean && save_var_eps && save_sd,
-             "tt_bn_fwd_eval_f32: null tensor pointer");
-  TT_REQUIRE_ALIGNED("tt_bn_fwd_eval_f32", x, y);
+  if (check_shape(fn, N, C, HW)) return -1;
+  TT_REQUIRE(x && y && mean && var && save_mean && save_var_eps && save_sd, "%s: null tensor pointer", fn);
+  TT_REQUIRE_ALIGNED(fn, x, y);
   Geometry g;
   int mode;
   plan(N, C, HW, &g, &mode);
@@ -896,12 +895,32 @@ int tt_bn_fwd_eval_f32(const float* x, const float* gamma, const float* beta, fl
   hipStream_t st = tt::stream();
   {
     tt::ProfScope prof(TT_PROF_BN_FWD_APPLY);
-    if (mode == 0) bn_fwd_apply<0><<<grid, kThreads, 0, st>>>(a, g);
-    if (mode == 1) bn_fwd_apply<1><<<grid, kThreads, 0, st>>>(a, g);
-    if (mode == 2) bn_fwd_apply<2><<<grid, kThreads, 0, st>>>(a, g);
+    if (relu) {
+      if (mode == 0) bn_fwd_apply<0, true><<<grid, kThreads, 0, st>>>(a, g);
+      if (mode == 1) bn_fwd_apply<1, true><<<grid, kThreads, 0, st>>>(a, g);
+      if (mode == 2) bn_fwd_apply<2, true><<<grid, kThreads, 0, st>>>(a, g);
+    } else {
+      if (mode == 0) bn_fwd_apply<0><<<grid, kThreads, 0, st>>>(a, g);
+      if (mode == 1) bn_fwd_apply<1><<<grid, kThreads, 0, st>>>(a, g);
+      if (mode == 2) bn_fwd_apply<2><<<grid, kThreads, 0, st>>>(a, g);
+    }
   }
   TT_LAUNCH_CHECK();
   return 0;
+}
+
+int tt_bn_fwd_eval_f32(const float* x, const float* gamma, const float* beta, float* y, const float* mean,
+                       const float* var, float* save_mean, float* save_var_eps, float* save_sd, double eps, int N,
+                       int C, int HW) {
+  return bn_fwd_eval("tt_bn_fwd_eval_f32", x, gamma, beta, y, mean, var, save_mean, save_var_eps, save_sd, eps, N, C, HW,
+                     false);
+}
+
+int tt_bn_relu_fwd_eval_f32(const float* x, const float* gamma, const float* beta, float* y, const float* mean,
+                            const float* var, float* save_mean, float* save_var_eps, float* save_sd, double eps, int N,
+                            int C, int HW) {
+  return bn_fwd_eval("tt_bn_relu_fwd_eval_f32", x, gamma, beta, y, mean, var, save_mean, save_var_eps, save_sd, eps, N, C,
+                     HW, true);
 }
 
 // Backward behind tt_bn_bwd_f32 (ry == nullptr) and tt_bn_relu_bwd_f32 (ry = the fused ReLU's output).

@@ -800,18 +800,18 @@ int tt_conv2d_selftest_raise_async_error(void) {
 // device is touched, tensor pointers are not looked at).
 static int conv2d_fwd(const float* x, const float* w, const float* bias, float* y, int N, int C, int H, int W, int K,
                       int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups, size_t* size_only,
-                      bool check_only = false) {
-  const char* fn = "tt_conv2d_fwd_f32";
+                      bool check_only = false, const Epilogue* epi = nullptr) {
+  const char* fn = epi ? "tt_conv2d_norm_act_fwd_f32" : "tt_conv2d_fwd_f32";
   TT_API_LOCK();
   if (!check_only) {
     TT_REQUIRE_INIT();
-    TT_REQUIRE(x && w && y, "tt_conv2d_fwd_f32: null tensor pointer");
-    TT_REQUIRE_ALIGNED("tt_conv2d_fwd_f32", x, w, y);
+    TT_REQUIRE(x && w && y, "%s: null tensor pointer", fn);
+    TT_REQUIRE_ALIGNED(fn, x, w, y);
   }
   const int P = (H + 2 * ph - dh * (R - 1) - 1) / sh + 1;
   const int Q = (W + 2 * pw - dw * (S - 1) - 1) / sw + 1;
   TT_REQUIRE(H + 2 * ph - dh * (R - 1) - 1 >= 0 && W + 2 * pw - dw * (S - 1) - 1 >= 0,
-             "tt_conv2d_fwd_f32: kernel (%d x %d, dilation %d x %d) larger than padded input (%d x %d)", R, S, dh, dw,
+             "%s: kernel (%d x %d, dilation %d x %d) larger than padded input (%d x %d)", fn, R, S, dh, dw,
              H + 2 * ph, W + 2 * pw);
   if (check_common(fn, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, P, Q)) return -1;
   const int Cg = C / groups, Kg = K / groups;
@@ -835,6 +835,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
 
   Igemm p{};
   p.src = x; p.wp = wp; p.bias = bias; p.out = y;
+  if (epi) p.epi = *epi;
   if (in_place) {
     p.wraw = w;
     p.wRowStride = Kred;
@@ -1170,21 +1171,42 @@ static int images_per_call(int N, long long image_a, long long image_b) {
 }
 static long long out_size(long long in, int k, int s, int p, int d) { return (in + 2LL * p - (long long)d * (k - 1) - 1) / s + 1; }
 
-int tt_conv2d_fwd_f32(const float* x, const float* w, const float* bias, float* y, int N, int C, int H, int W, int K,
-                      int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups) {
+static int conv2d_fwd_runs(const char* fn, const float* x, const float* w, const float* bias, float* y, int N, int C, int H,
+                           int W, int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups,
+                           const Epilogue* epi) {
   const long long xi = (long long)C * H * W;
   const long long yi = sh > 0 && sw > 0 ? (long long)K * out_size(H, R, sh, ph, dh) * out_size(W, S, sw, pw, dw) : 0;
   const int per = images_per_call(N, xi, yi);
-  TT_REQUIRE(per > 0, "tt_conv2d_fwd_f32: a batch of 2^31 elements or more is cut into runs of images, and images of "
-                      "%lld and %lld elements leave no run 16-byte aligned", xi, yi);
-  if (per >= N) return conv2d_fwd(x, w, bias, y, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, nullptr);
+  TT_REQUIRE(per > 0, "%s: a batch of 2^31 elements or more is cut into runs of images, and images of "
+                      "%lld and %lld elements leave no run 16-byte aligned", fn, xi, yi);
+  if (per >= N) return conv2d_fwd(x, w, bias, y, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, nullptr, false, epi);
   for (int n0 = 0; n0 < N; n0 += per) {
     const int n = N - n0 < per ? N - n0 : per;
+    Epilogue run{};
+    if (epi) {
+      run = *epi;
+      if (run.res) run.res += (size_t)n0 * yi;
+    }
     if (int rc = conv2d_fwd(x + (size_t)n0 * xi, w, bias, y + (size_t)n0 * yi, n, C, H, W, K, R, S, sh, sw, ph, pw, dh,
-                            dw, groups, nullptr))
+                            dw, groups, nullptr, false, epi ? &run : nullptr))
       return rc;
   }
   return 0;
+}
+
+int tt_conv2d_fwd_f32(const float* x, const float* w, const float* bias, float* y, int N, int C, int H, int W, int K,
+                      int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups) {
+  return conv2d_fwd_runs("tt_conv2d_fwd_f32", x, w, bias, y, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, nullptr);
+}
+
+int tt_conv2d_norm_act_fwd_f32(const float* x, const float* w, const float* bias, float* y, const float* mean,
+                               const float* var, const float* gamma, const float* beta, double eps, const float* residual,
+                               int relu, int N, int C, int H, int W, int K, int R, int S, int sh, int sw, int ph, int pw,
+                               int dh, int dw, int groups) {
+  TT_REQUIRE((mean == nullptr) == (var == nullptr), "tt_conv2d_norm_act_fwd_f32: mean and var come together");
+  TT_REQUIRE_ALIGNED("tt_conv2d_norm_act_fwd_f32", residual);
+  const Epilogue epi{mean, var, gamma, beta, residual, (float)eps, mean != nullptr, relu != 0, 1};
+  return conv2d_fwd_runs("tt_conv2d_norm_act_fwd_f32", x, w, bias, y, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, &epi);
 }
 
 int tt_conv2d_dgrad_f32(const float* dy, const float* w, const float* bias, float* dx, int N, int C, int Hx, int Wx,

@@ -58,6 +58,7 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
   constexpr int ALINE = line_units(BM), BLINE = line_units(BN);
   __shared__ uintx4 As[2][kK8][ALINE];
   __shared__ uintx4 Bs[2][kK8][BLINE];
+  __shared__ __align__(16) float epi_lds[3 * BM];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -225,6 +226,7 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
   };
 
   const int chunks = p.Kred / kBK;
+  if (p.epi.on) epilogue_constants<BM>(p.epi, g * p.I, i0, p.I, tid, epi_lds);   // published by the barrier below
   fetch(0);
   stage(0);
   __syncthreads();
@@ -249,6 +251,10 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
     const uint32_t u = tt::fd_div(rem, p.divV);
     const uint32_t v = rem - u * p.divV.d;
     obase[y] = (uint32_t)((int)n * p.outStrideN + g * p.outStrideG + ((int)u * p.ou + p.ouh) * p.outRow + (int)v * p.ov + p.ovw);
+  }
+  if (p.epi.on) {
+    store_through_epilogue<BM, MT, NT>(p, acc, obase, mok, g, i0, wm * MT * 32, h, epi_lds);
+    return;
   }
   if (p.bias == nullptr && (p.I & 7) == 0) {
     // rows in whole groups of eight: one scalar test per group, a row's address is a scalar base plus

@@ -23,6 +23,21 @@ struct KEntry {
 typedef int intx2 __attribute__((ext_vector_type(2)));
 typedef const intx2 __attribute__((address_space(4))) * ConstKTab;   // constant address space: scalar (s_load) access
 
+// What a launch does to a value between its accumulator and memory, beside the bias:
+//   v = acc + bias;  v = (v - mean) * (gamma / sd) + beta  (norm);  v = v + res[same element];
+//   v = maximum(v, 0), NaN kept  (relu)
+// -- the evaluation-mode BatchNorm, residual add and ReLU behind a convolution, in the order and with
+// the roundings of the kernels they stand in for.  `on` == 0: none of it.  Bound by memory: the three
+// separate launches read and wrote y up to seven times over (a ResNet-50 evaluation pass at batch 64
+// in bf16 arithmetic spent half its time in them: 5.50 ms, 3.48 ms with this; 184 launches become 60,
+// which at batch 2 takes 3.37 ms to 2.66).
+struct Epilogue {
+  const float *mean, *var, *gamma, *beta;   // [G*I] each; gamma / beta may be null
+  const float* res;                         // laid out as `out`, or null
+  float eps;
+  int norm, relu, on;
+};
+
 struct Igemm {
   const float* src;
   const floatx4* wp;     // [G][KQ][Ipad] x 4 floats
@@ -77,6 +92,7 @@ struct Igemm {
   unsigned* skFlags;         // [block] = skEpoch once the block's partial is in memory
   unsigned skEpoch;          // differs from launch to launch, so the flags never need clearing
   unsigned* skError;         // one word in pinned host memory: set when a wait for a flag ran out
+  Epilogue epi;
 };
 
 
@@ -95,6 +111,85 @@ constexpr int kSrdFlags = 0x00020000;        // raw buffer, 32-bit data format
 constexpr int kSrdRecords = 0x7fffffff;      // offsets with bit 31 set are out of range and read 0
 
 __device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
+
+// Per-row constants of the epilogue's normalisation for the BM rows of a tile, {mean, gamma / sd, beta}
+// each an array of BM in LDS: one thread computes a row's once (a square root and a division) while
+// the tile's first loads are in flight, instead of every lane for each of its rows at the end.  The
+// caller's next barrier publishes them.  Without a normalisation the constants leave a value as it
+// is: (v - 0) * 1 + -0.
+template <int BM>
+__device__ __forceinline__ void epilogue_constants(const Epilogue& e, int first_channel, int i0, int I, int tid, float* lds) {
+  if (tid < BM) {
+    float m = 0.f, k1 = 1.f, k0 = -0.f;
+    if (e.norm) {
+      const int c = first_channel + min(i0 + tid, I - 1);
+      const float sd = __fsqrt_rn(__fadd_rn(e.var[c], e.eps));
+      m = e.mean[c];
+      k1 = __fdiv_rn(e.gamma ? e.gamma[c] : 1.0f, sd);
+      k0 = e.beta ? e.beta[c] : 0.0f;
+    }
+    lds[tid] = m;
+    lds[BM + tid] = k1;
+    lds[2 * BM + tid] = k0;
+  }
+}
+
+// Stores one wave's MT x NT accumulators through the epilogue.  `row0` is the wave's first row inside
+// the tile; accumulator register r of a 32x32 tile holds row 8*(r/4) + 4*h + r%4.  A 32-row strip's
+// residual values are all fetched before its first store (loads and stores share one in-order counter).
+template <int BM, int MT, int NT>
+__device__ __forceinline__ void store_through_epilogue(const Igemm& p, const floatx16 (&acc)[MT][NT], const uint32_t (&obase)[NT],
+                                                       const bool (&mok)[NT], int g, int i0, int row0, int h, const float* lds) {
+  const float floor_ = p.epi.relu ? 0.f : -__builtin_huge_valf();
+#pragma unroll
+  for (int x = 0; x < MT; ++x) {
+    const int r0 = row0 + 32 * x + 4 * h;   // + 8*q + j inside the tile
+    float rs[NT][16], bz[16];
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      bz[r] = 0.f;
+#pragma unroll
+      for (int y = 0; y < NT; ++y) rs[y][r] = -0.f;   // v + -0 is v
+    }
+    if (p.bias) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) bz[r] = p.bias[g * p.I + min(i0 + r0 + 8 * (r >> 2) + (r & 3), p.I - 1)];
+    }
+    if (p.epi.res) {
+#pragma unroll
+      for (int y = 0; y < NT; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int i = i0 + r0 + 8 * (r >> 2) + (r & 3);
+          if (mok[y] && i < p.I) rs[y][r] = p.epi.res[obase[y] + (uint32_t)(i * p.outStrideI)];
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const floatx4 m4 = *reinterpret_cast<const floatx4*>(lds + r0 + 8 * q);
+      const floatx4 s4 = *reinterpret_cast<const floatx4*>(lds + BM + r0 + 8 * q);
+      const floatx4 b4 = *reinterpret_cast<const floatx4*>(lds + 2 * BM + r0 + 8 * q);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + r0 + 8 * q + j;
+        if (i < p.I) {
+          const uint32_t ioff = (uint32_t)(i * p.outStrideI);
+#pragma unroll
+          for (int y = 0; y < NT; ++y) {
+            float v = acc[x][y][4 * q + j];
+            if (p.bias) v += bz[4 * q + j];
+            v = fmaf(v - m4[j], s4[j], b4[j]) + rs[y][4 * q + j];
+            v = (v > floor_ || v != v) ? v : floor_;
+            if (mok[y]) p.out[obase[y] + ioff] = v;
+          }
+        }
+      }
+    }
+  }
+}
 
 // The bf16-first kernels (conv_igemm_bf16.hip).  `supported` tells whether they take launch `p`
 // (tile rows `bm` as planned by the caller); `launch` enqueues it on the library stream.

@@ -89,6 +89,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   static_assert(B_ITEMS >= 1 && kThreads % BM == 0 && kThreads % BN == 0, "tile shape");
   __shared__ floatx4 As[2][kBKQ][BM];
   __shared__ floatx4 Bs[2][kBKQ][BN];
+  __shared__ __align__(16) float epi_lds[3 * BM];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -464,6 +465,10 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
       obase[y] = (uint32_t)((int)n * p.outStrideN + g * p.outStrideG + ((int)u * p.ou + p.ouh) * p.outRow +
                             (int)v * p.ov + p.ovw);
     }
+    if (p.epi.on) {
+      store_through_epilogue<BM, MT, NT>(p, acc, obase, mok, g, i0, wm * MT * 32, h, epi_lds);
+      return;
+    }
     if (p.rowtab == nullptr && p.bias == nullptr && (p.I & 7) == 0) {
       // The common case, without bias and with rows in whole groups of eight: a group is inside the
       // matrix or not for the whole wave (scalar test), a row's address is a scalar base plus the
@@ -590,8 +595,16 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   };
 
   const int chunks = p.KQ / kBKQ;
+  // (published by the barriers of the reduction that follows; the epilogue of the tile before has
+  // ended with one)
+  auto epi_constants = [&]() __attribute__((always_inline)) {
+    if (!p.epi.on) return;
+    epilogue_constants<BM>(p.epi, g * p.I, i0, p.I, tid, epi_lds);
+    if (chunks == 0) __syncthreads();
+  };
   if constexpr (!SK) {
     set_tile(xcd_remap(block_x, p.tiles));
+    epi_constants();
     run_segment(0, chunks);
     epilogue();
   } else {
@@ -649,6 +662,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
       }
       for (int tile = b; tile < p.skDpTiles; tile += (int)gridDim.x) {
         set_tile(tile);
+        epi_constants();
         run_segment(0, chunks);
         epilogue();
         __syncthreads();
@@ -657,12 +671,14 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
         const bool whole = (t > t_first || c0f == 0) && (t < t_last || endc == chunks);
         if (!whole) continue;
         set_tile(p.skDpTiles + t);
+        epi_constants();
         run_segment(0, chunks);
         epilogue();
         __syncthreads();
       }
       if (has_closing) {
         set_tile(p.skDpTiles + t_first);
+        epi_constants();
         run_segment(c0f, chunks);
         // blocks that hold the earlier steps of this tile: the one containing its first step ... b - 1
         const long long t0 = (long long)t_first * chunks;

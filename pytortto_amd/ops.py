@@ -30,8 +30,8 @@ def conv_out_size(size, k, stride, pad, dil):
 
 # ---- convolution -------------------------------------------------------------------------------
 
-def conv2d_fwd(x, w, bias, stride, padding, dilation, groups):
-    """y = conv(x, w) + bias  (autograd/grad_nn.py:595-643, :709-711)."""
+def _conv2d_geometry(x, w, bias, stride, padding, dilation, groups):
+    """(shape of y, the C entry points' integer arguments); raises for an empty output."""
     _f32(x, w, bias)
     n, c, h, wd = x.shape
     k, _, r, s = w.shape
@@ -40,10 +40,95 @@ def conv2d_fwd(x, w, bias, stride, padding, dilation, groups):
     if p <= 0 or q <= 0:
         raise RuntimeError(f'Calculated output size ({k} x {p} x {q}) is too small for input {x.shape} '
                            f'and kernel {(r, s)}')
-    y = hiparray.empty((n, k, p, q))
-    _hip.call('tt_conv2d_fwd_f32', x.ptr, w.ptr, _ptr(bias), y.ptr, n, c, h, wd, k, r, s,
-              stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1], groups)
+    return (n, k, p, q), (n, c, h, wd, k, r, s, stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1],
+                          groups)
+
+
+def conv2d_fwd(x, w, bias, stride, padding, dilation, groups):
+    """y = conv(x, w) + bias  (autograd/grad_nn.py:595-643, :709-711)."""
+    shape, dims = _conv2d_geometry(x, w, bias, stride, padding, dilation, groups)
+    y = hiparray.empty(shape)
+    _hip.call('tt_conv2d_fwd_f32', x.ptr, w.ptr, _ptr(bias), y.ptr, *dims)
     return y
+
+
+class DeferredConv:
+    """A convolution whose result needs no gradient, not launched yet (see ``_hip.defer``).  What
+    follows it in an evaluation pass -- a BatchNorm with given statistics, a residual add, a ReLU --
+    joins the launch and is applied to the accumulators before they are stored (``absorb_norm``,
+    ``absorb_add``, ``run_with_relu``); anything else finds it launched with what has joined so far.
+    The values in between are never stored: their arrays are produced on demand by the launch up to
+    that point, should anybody ask, and at the latest just before an operand is written in place."""
+
+    def __init__(self, x, w, bias, shape, dims):
+        self.x, self.w, self.bias, self.dims = x, w, bias, dims
+        self.norm = self.residual = None
+        self.out = hiparray.lazy(shape)
+
+    def _operands(self):
+        return (self.x, self.w, self.bias, *(self.norm[:4] if self.norm else ()), self.residual)
+
+    def _launcher(self, relu):
+        """The launch of what has joined so far, as a function of the array to fill."""
+        x, w, bias, dims, norm, residual = self.x, self.w, self.bias, self.dims, self.norm, self.residual
+        if norm is None and residual is None and not relu:
+            return lambda out: _hip.call('tt_conv2d_fwd_f32', x.ptr, w.ptr, _ptr(bias), out.ptr, *dims)
+        mean, var, gamma, beta, eps = norm or (None, None, None, None, 0.0)
+        return lambda out: _hip.call('tt_conv2d_norm_act_fwd_f32', x.ptr, w.ptr, _ptr(bias), out.ptr, _ptr(mean),
+                                     _ptr(var), _ptr(gamma), _ptr(beta), eps, _ptr(residual), int(relu), *dims)
+
+    def _on_demand(self):
+        """The output so far is about to be absorbed: leave it to be produced on demand."""
+        self.out._buf.fill_on_demand(self._launcher(False), self._operands())
+
+    def takes_norm(self):
+        return self.norm is None and self.residual is None
+
+    def absorb_norm(self, mean, var, gamma, beta, eps):
+        _f32(mean, var, gamma, beta)
+        self._on_demand()
+        self.norm = (mean, var, gamma, beta, float(eps))
+        self.out = hiparray.lazy(self.out.shape)
+        _hip.defer(self)
+        return self.out
+
+    def absorb_add(self, residual):
+        _f32(residual)
+        self._on_demand()
+        self.residual = residual
+        self.out = hiparray.lazy(self.out.shape)
+        _hip.defer(self)
+        return self.out
+
+    def run(self):
+        self._launcher(False)(self.out)
+
+    def run_with_relu(self, out=None):
+        launch = self._launcher(True)
+        if out is None:
+            out = self.out
+        else:
+            self._on_demand()
+        launch(out)
+        return out
+
+    def poison(self, exc):
+        poison([self.out], exc)
+
+
+# beyond these the C entry point may refuse a geometry or cut the batch into runs: launched at once,
+# so that an error is raised where it belongs
+_DEFER_EXTENT, _DEFER_ELEMENTS = 8192, 1 << 31
+
+
+def conv2d_fwd_deferred(x, w, bias, stride, padding, dilation, groups):
+    """``conv2d_fwd`` with the launch parked for the operations behind it to join."""
+    shape, dims = _conv2d_geometry(x, w, bias, stride, padding, dilation, groups)
+    if max(x.shape[2:]) >= _DEFER_EXTENT or max(x.size, prod(shape)) >= _DEFER_ELEMENTS or 0 in x.shape:
+        return conv2d_fwd(x, w, bias, stride, padding, dilation, groups)
+    op = DeferredConv(x, w, bias, shape, dims)
+    _hip.defer(op)
+    return op.out
 
 
 def conv2d_dgrad(dy, w, bias, out_hw, stride, padding, dilation, groups):
@@ -156,6 +241,10 @@ class DeferredBatchNorm:
         self.y._buf.fill_on_demand(recompute, (x, gamma, beta))
         return out
 
+    @property
+    def out(self):
+        return self.y
+
     def poison(self, exc):
         poison([self.y, *self.stats, self.new_rm, self.new_rv], exc)
 
@@ -203,15 +292,47 @@ def bn_relu_bwd(x, dy, relu_y, gamma, mean, var_eps, sd, need=(True, True, True)
     return dx, dgamma, dbeta
 
 
-def bn_fwd_eval(x, gamma, beta, mean_in, var_in, eps):
-    """Normalisation with given statistics (autograd/grad_nn.py:931-959)."""
+class DeferredBatchNormEval:
+    """Normalisation with given statistics (autograd/grad_nn.py:931-959), not launched yet: a ReLU that
+    comes next is applied in the same pass, as ``DeferredBatchNorm`` has it for training."""
+
+    def __init__(self, x, gamma, beta, mean_in, var_in, eps):
+        self.operands = (x, gamma, beta, mean_in, var_in)
+        self.eps, self.dims = float(eps), _nchw(x)
+        self.out = hiparray.lazy(x.shape)
+        self.stats = [hiparray.empty((self.dims[1],)) for _ in range(3)]     # mean, var + eps, sd
+
+    def _launch(self, entry, out, stats):
+        x, gamma, beta, mean_in, var_in = self.operands
+        _hip.call(entry, x.ptr, _ptr(gamma), _ptr(beta), out.ptr, mean_in.ptr, var_in.ptr, stats[0].ptr, stats[1].ptr,
+                  stats[2].ptr, self.eps, *self.dims)
+
+    def run(self):
+        self._launch('tt_bn_fwd_eval_f32', self.out, self.stats)
+
+    def run_with_relu(self, out=None):
+        if out is None:
+            out = self.out
+        else:
+            def recompute(buf):
+                self._launch('tt_bn_fwd_eval_f32', buf, [hiparray.empty((self.dims[1],)) for _ in range(3)])
+            self.out._buf.fill_on_demand(recompute, self.operands)
+        self._launch('tt_bn_relu_fwd_eval_f32', out, self.stats)
+        return out
+
+    def poison(self, exc):
+        poison([self.out, *self.stats], exc)
+
+
+def bn_fwd_eval(x, gamma, beta, mean_in, var_in, eps, deferred=False):
+    """(y, mean, var + eps, sd); with ``deferred`` the launch is parked for a ReLU to join."""
     _f32(x, gamma, beta, mean_in, var_in)
-    n, c, hw = _nchw(x)
-    y = hiparray.empty(x.shape)
-    mean, var_eps, sd = hiparray.empty((c,)), hiparray.empty((c,)), hiparray.empty((c,))
-    _hip.call('tt_bn_fwd_eval_f32', x.ptr, _ptr(gamma), _ptr(beta), y.ptr, mean_in.ptr, var_in.ptr,
-              mean.ptr, var_eps.ptr, sd.ptr, float(eps), n, c, hw)
-    return y, mean, var_eps, sd
+    op = DeferredBatchNormEval(x, gamma, beta, mean_in, var_in, eps)
+    if deferred:
+        _hip.defer(op)
+    else:
+        op.run()
+    return (op.out, *op.stats)
 
 
 def bn_bwd(x, dy, gamma, mean, var_eps, sd, need=(True, True, True)):

@@ -127,6 +127,13 @@ def before_write(buf):
                 lazy.ptr
 
 
+def fill_all():
+    """Fill every on-demand buffer now."""
+    with _hip._lock:
+        for lazy in list(_unfilled):
+            lazy.ptr
+
+
 def poison(arrays, exc):
     """Make every later use of ``arrays`` raise ``exc``: the operation that was to fill them failed."""
     def fail(buf):
