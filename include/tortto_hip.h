@@ -185,6 +185,14 @@ int tt_conv2d_dgrad_f32(const float* dy, const float* w, const float* bias, floa
                         int sh, int sw, int ph, int pw, int dh, int dw, int groups,
                         int P, int Q);
 
+/* tt_conv2d_dgrad_f32 at stride 1 x 1, with dx_add ([N,C,Hx,Wx] or NULL) -- what other consumers of x
+ * have sent back already -- added to the result, and that multiplied by (relu_y > 0) if relu_y
+ * ([N,C,Hx,Wx], the output x of a ReLU) is not NULL: the gradient accumulation of
+ * tensor.py:568-613 and the ReLU backward of autograd/grad_nn.py:67 without launches of their own, with their roundings (same bits). */
+int tt_conv2d_dgrad_acc_f32(const float* dy, const float* w, float* dx, const float* dx_add, const float* relu_y,
+                            int N, int C, int Hx, int Wx, int K, int R, int S,
+                            int sh, int sw, int ph, int pw, int dh, int dw, int groups, int P, int Q);
+
 /* dw[K,C/groups,R,S] = sum over n,p,q of x~[n,c,p*sh+r*dh-ph,q*sw+s*dw-pw] * dy[n,k,p,q]
  * (x~ = x zero-padded).  Deterministic: fixed split of the reduction, partial sums combined
  * in float64.  Replaces _conv2d_backward_w: autograd/grad_nn.py:646-656 (called from :731
@@ -339,6 +347,21 @@ int tt_bn_relu_fwd_train_f32(const float* x, const float* gamma, const float* be
                              const float* running_mean_in, const float* running_var_in,
                              float* running_mean_out, float* running_var_out, float* num_batches_tracked,
                              double momentum, double eps, int N, int C, int HW);
+/* The same pair with everything a residual block puts around a BatchNorm, in the rounding of the
+ * separate entry points (same bits):
+ * tt_bn_act_fwd_train_f32: y = bn(x), + residual if not NULL, then maximum(., 0) if relu; save_coef
+ * (NULL or [2][C]) receives the two constants of bn(x) = (x - mean) * coef[0][c] + coef[1][c].
+ * tt_bn_act_bwd_f32: tt_bn_bwd_f32 on dy, or, with coef (from the forward call), on
+ * dy * (bn(x) > 0) -- the mask of a ReLU right behind the BatchNorm, from x instead of from the
+ * ReLU's output -- and with dx_add ([N,C,HW] or NULL) added to dx. */
+int tt_bn_act_fwd_train_f32(const float* x, const float* gamma, const float* beta, const float* residual, float* y,
+                            float* save_mean, float* save_var_eps, float* save_sd, float* save_coef,
+                            const float* running_mean_in, const float* running_var_in,
+                            float* running_mean_out, float* running_var_out, float* num_batches_tracked,
+                            double momentum, double eps, int relu, int N, int C, int HW);
+int tt_bn_act_bwd_f32(const float* x, const float* dy, const float* coef, const float* gamma,
+                      const float* save_mean, const float* save_var_eps, const float* save_sd,
+                      float* dx, const float* dx_add, float* dgamma, float* dbeta, int N, int C, int HW);
 int tt_bn_relu_bwd_f32(const float* x, const float* dy, const float* relu_y, const float* gamma,
                        const float* save_mean, const float* save_var_eps, const float* save_sd,
                        float* dx, float* dgamma, float* dbeta, int N, int C, int HW);

@@ -41,6 +41,7 @@ PROTOTYPES = {
     'tt_conv2d_fwd_f32': [_P, _P, _P, _P] + [_I] * 14,
     'tt_conv2d_norm_act_fwd_f32': [_P] * 8 + [c_double, _P, _I] + [_I] * 14,
     'tt_conv2d_dgrad_f32': [_P, _P, _P, _P] + [_I] * 16,
+    'tt_conv2d_dgrad_acc_f32': [_P] * 5 + [_I] * 16,
     'tt_conv2d_wgrad_f32': [_P, _P, _P] + [_I] * 16,
     'tt_conv2d_fwd_bf16': [_P, _P, _P, _P] + [_I] * 14,
     'tt_conv2d_dgrad_bf16': [_P, _P, _P, _P] + [_I] * 16,
@@ -69,6 +70,8 @@ PROTOTYPES = {
     'tt_bn_fwd_train_noalloc_f32': [_P] * 12 + [c_double, c_double, _I, _I, _I],
     'tt_bn_relu_fwd_train_f32': [_P] * 12 + [c_double, c_double, _I, _I, _I],
     'tt_bn_relu_bwd_f32': [_P] * 10 + [_I, _I, _I],
+    'tt_bn_act_fwd_train_f32': [_P] * 14 + [c_double, c_double] + [_I] * 4,
+    'tt_bn_act_bwd_f32': [_P] * 11 + [_I, _I, _I],
     'tt_bn_fwd_eval_f32': [_P] * 9 + [c_double, _I, _I, _I],
     'tt_bn_relu_fwd_eval_f32': [_P] * 9 + [c_double, _I, _I, _I],
     'tt_bn_bwd_f32': [_P] * 9 + [_I, _I, _I],

@@ -70,15 +70,16 @@ class Add(Function):
         if a.__class__ is not hiparray:
             y = np.add(a, b)
         elif a.shape == b.shape:
-            conv = None
+            # one operand is the output of a BatchNorm, or (without gradients) of a convolution, that has not
+            # been launched yet: add the other to it on its way to memory
+            takes = (ops.DeferredBatchNorm,)
             if not (ctx.requires_grad and is_grad_enabled()):
-                # one operand is a convolution's output that has not been launched yet: add the other to it
-                # on its way to memory
-                conv = _hip.take_pending_if(lambda op: op.__class__ is ops.DeferredConv and op.residual is None
-                                            and (op.out._buf is a._buf) != (op.out._buf is b._buf)
-                                            and op.out.shape == a.shape)
-            if conv is not None:
-                y = conv.absorb_add(b if conv.out._buf is a._buf else a)
+                takes = (ops.DeferredBatchNorm, ops.DeferredConv)
+            parked = _hip.take_pending_if(lambda op: op.__class__ in takes and op.residual is None
+                                          and (op.out._buf is a._buf) != (op.out._buf is b._buf)
+                                          and op.out.shape == a.shape)
+            if parked is not None:
+                y = parked.absorb_add(b if parked.out._buf is a._buf else a)
             else:
                 y = ops.add_deferred(a, b)      # parked: a ReLU that comes next absorbs it
         elif b.size < a.size and _trailing(b.shape, a.shape):

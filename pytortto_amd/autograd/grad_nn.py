@@ -16,7 +16,7 @@ from .. import _hip, ops
 from ..xparray import hiparray
 from .function import Function
 from .grad_mode import is_grad_enabled
-from .helper import build_links, inplace_precheck, inplace_update
+from .helper import build_links, inplace_precheck, inplace_update, take_arrived
 
 
 def _device_only(name, data):
@@ -24,6 +24,19 @@ def _device_only(name, data):
         raise RuntimeError(f'{name}: pytortto_amd implements the device (HIP) path only and got a host '
                            f'{data.__class__.__name__}; move the tensors with .cuda() first '
                            f'(host tensors belong to tortto\'s NumPy path)')
+
+
+def _relu_waiting_for(ctx, i, like):
+    """(node, output) of the ReLU that made input ``i`` when this node's gradient is the last one it waits
+    for; (None, None) otherwise, and when the backward of a BatchNorm in front of it will apply its mask."""
+    fn = ctx.next_functions[i][0]
+    if fn is None or getattr(fn, '_forward_cls', None) is not Relu or fn.prev_function_counts != 1 \
+            or fn.to_save is None or fn.params.get('bn_coef') is not None:
+        return None, None
+    y, version = fn.to_save[0]
+    if y._version != version or y.data.__class__ is not hiparray or y.shape != like.shape:
+        return None, None
+    return fn, y.data
 
 
 class Convolution(Function):
@@ -70,7 +83,15 @@ class Convolution(Function):
         if ctx.needs_input_grad[1]:
             grad1 = ops.conv2d_wgrad(xd0, gd0, xd1.shape, stride, padding, dilation, groups)
         if ctx.needs_input_grad[0]:
-            grad0 = ops.conv2d_dgrad(gd0, xd1, None, xd0.shape[-2:], stride, padding, dilation, groups)
+            # at stride 1 one launch writes every element of dx once: it adds what other consumers of x have
+            # already sent, and, when nothing more is to come, applies the backward of the ReLU that made x
+            add = relu_y = relu = None
+            if stride[0] == 1 and stride[1] == 1:
+                add = take_arrived(ctx, 0, xd0)
+                relu, relu_y = _relu_waiting_for(ctx, 0, xd0)
+            grad0 = ops.conv2d_dgrad(gd0, xd1, None, xd0.shape[-2:], stride, padding, dilation, groups, add, relu_y)
+            if relu is not None:
+                relu.params['masked'] = grad0
         return grad0, grad1, grad2
 
 
@@ -181,14 +202,14 @@ class BatchNorm(Function):
         gd0, = grad_outputs
         xd0, xd1 = ctx.saved_tensors
         p = ctx.params
+        coef = None
         parked = _hip.take_pending_if(lambda op: op.__class__ is ops.DeferredReluBackward and op.out._buf is gd0._buf)
         if parked is not None:
-            # the gradient comes straight from a ReLU whose mask has not been applied yet: apply it
-            # while reading dy (grad_nn.py:67 folded into :977-988)
-            return ops.bn_relu_bwd(xd0, parked.dy, parked.y, xd1, p['mean'], p['var'], p['sd'],
-                                   need=ctx.needs_input_grad)
-        grad0, grad1, grad2 = ops.bn_bwd(xd0, gd0, xd1, p['mean'], p['var'], p['sd'], need=ctx.needs_input_grad)
-        return grad0, grad1, grad2
+            # the gradient comes straight from the ReLU fused with this forward, its mask not applied
+            # yet: apply it while reading dy (grad_nn.py:67 folded into :977-988)
+            gd0, coef = parked.dy, parked.coef
+        add = take_arrived(ctx, 0, xd0) if ctx.needs_input_grad[0] else None
+        return ops.bn_bwd(xd0, gd0, xd1, p['mean'], p['var'], p['sd'], need=ctx.needs_input_grad, coef=coef, add=add)
 
 
 # parked operations that a ReLU behind them joins
@@ -214,12 +235,13 @@ class Relu(Function):
                 except RuntimeError:
                     parked.run()
                     raise
-                parked.run_with_relu()
-                yt0 = inplace_update(xt0, ctx)
-            else:
-                yt0 = build_links(parked.run_with_relu(hiparray.empty(xd0.shape)), grad_fn=ctx)
+            out = None if inplace else hiparray.empty(xd0.shape)
             if parked.__class__ is ops.DeferredBatchNorm:
-                ctx.params['after_batch_norm'] = True
+                out = parked.run_with_relu(out, keep_coef=ctx.requires_grad and is_grad_enabled())
+                ctx.params['bn_coef'] = parked.coef
+            else:
+                out = parked.run_with_relu(out)
+            yt0 = inplace_update(xt0, ctx) if inplace else build_links(out, grad_fn=ctx)
         elif xd0.__class__ is hiparray:
             if inplace:
                 inplace_precheck(xt0)
@@ -241,9 +263,12 @@ class Relu(Function):
         gd0, = grad_outputs
         yd0, = ctx.saved_tensors
         if yd0.__class__ is hiparray:
-            if ctx.params.get('after_batch_norm') and gd0.__class__ is hiparray:
+            if gd0 is not None and gd0 is ctx.params.get('masked'):
+                return gd0                              # the kernel that wrote this gradient has applied the mask
+            coef = ctx.params.get('bn_coef')
+            if coef is not None and gd0.__class__ is hiparray:
                 # the BatchNorm backward that follows can apply the mask itself; parked until then
-                return ops.relu_bwd_deferred(gd0, yd0)
+                return ops.relu_bwd_deferred(gd0, yd0, coef)
             return ops.relu_bwd(gd0, yd0)
         return gd0 * (yd0 > 0)
 

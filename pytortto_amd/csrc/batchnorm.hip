@@ -111,6 +111,33 @@ __device__ __forceinline__ float4 mask4(float4 g, float4 y) {
   return make_float4(mask1(g.x, y.x), mask1(g.y, y.y), mask1(g.z, y.z), mask1(g.w, y.w));
 }
 
+__device__ __forceinline__ float4 add4(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+
+// How a backward pass behind a fused ReLU learns where the ReLU was open:
+//   kMaskY   : from the ReLU's output, read along with dy
+//   kMaskCoef: from x and the forward's two constants of the channel, which the forward call stored:
+//              bn(x) = fma(x - mean, gamma / sd, beta) again, the same operation on the same values
+//              and so the same sign as the forward saw.  x is read anyway, so the ReLU's output stays
+//              out of both sweeps: 8 of 10 tensor passes of a training pass are left (256 channels of
+//              64 x 56 x 56, forward and backward: 398 us, 330 now).
+constexpr int kNoMask = 0, kMaskY = 1, kMaskCoef = 2;
+struct MaskCoef {
+  float k1, k0;   // gamma / sd and beta of the forward
+};
+template <int kMask>
+__device__ __forceinline__ MaskCoef mask_coef(const float* __restrict__ coef, int c, int C) {
+  MaskCoef k{0.f, 0.f};
+  if constexpr (kMask == kMaskCoef) {
+    k.k1 = coef[c];
+    k.k0 = coef[C + c];
+  }
+  return k;
+}
+__device__ __forceinline__ float bn1(float v, float mean, const MaskCoef k) { return fmaf(v - mean, k.k1, k.k0); }
+__device__ __forceinline__ float4 bn4(float4 v, float mean, const MaskCoef k) {
+  return make_float4(bn1(v.x, mean, k), bn1(v.y, mean, k), bn1(v.z, mean, k), bn1(v.w, mean, k));
+}
+
 constexpr int kStreamU = 8;   // float4 loads in flight per thread in the stream reduce kernel
 
 struct Geometry {
@@ -185,12 +212,12 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_planes(const float* __rest
 // vectors (flattened over planes, so no batch is cut short at a plane end) and issues kU loads
 // per tensor and thread before it consumes the first: enough bytes in flight per block that the
 // reduction tails of other blocks do not leave the memory system idle.
-template <int kKind, bool kRelu = false>
+template <int kKind, int kMask = kNoMask>
 __global__ __launch_bounds__(kThreads) void bn_reduce_stream(const float* __restrict__ x,
                                                              const float* __restrict__ dy,
                                                              const float* __restrict__ mean,
                                                              double2* __restrict__ partial, Geometry g,
-                                                             const float* __restrict__ ry = nullptr) {
+                                                             const float* __restrict__ mk = nullptr) {
   __shared__ double lds[2 * kWaves];
   const int c = blockIdx.y, split = blockIdx.x;
   constexpr bool kBwd = kKind == 1;
@@ -200,6 +227,7 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_stream(const float* __rest
   const float ref = kKind == 1 ? mean[c] : (kKind == 0 ? x[(size_t)c * g.HW] : 0.f);
   const uint32_t e0 = (uint32_t)split * (uint32_t)g.per_block;
   const uint32_t e1 = min(total, e0 + (uint32_t)g.per_block);
+  const MaskCoef mc = mask_coef<kMask>(mk, c, g.C);
   const float4 fill = make_float4(ref, ref, ref, ref);
   const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
   double sa = 0.0, sb = 0.0;
@@ -218,7 +246,8 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_stream(const float* __rest
         // dy is streamed in both backward sweeps: x is read four times per training pass, dy twice,
         // and at these sizes the memory-side cache cannot hold both
         float4 q = load_stream(reinterpret_cast<const float4*>(dy + off));
-        if constexpr (kRelu) q = mask4(q, load_stream(reinterpret_cast<const float4*>(ry + off)));
+        if constexpr (kMask == kMaskY) q = mask4(q, load_stream(reinterpret_cast<const float4*>(mk + off)));
+        if constexpr (kMask == kMaskCoef) q = mask4(q, bn4(t, ref, mc));
         gq[u] = ok ? q : zero;
       }
     }
@@ -247,12 +276,12 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_stream(const float* __rest
 }
 
 // Flat kernel: any HW.  Vector index e over the channel's N*HW/VEC vectors, n = e / (HW/VEC).
-template <int kKind, int VEC, bool kRelu = false>
+template <int kKind, int VEC, int kMask = kNoMask>
 __global__ __launch_bounds__(kThreads) void bn_reduce_flat(const float* __restrict__ x,
                                                            const float* __restrict__ dy,
                                                            const float* __restrict__ mean,
                                                            double2* __restrict__ partial, Geometry g,
-                                                           const float* __restrict__ ry = nullptr) {
+                                                           const float* __restrict__ mk = nullptr) {
   __shared__ double lds[2 * kWaves];
   const int c = blockIdx.y, split = blockIdx.x;
   const uint32_t hwv = (uint32_t)g.HW / VEC;
@@ -261,6 +290,7 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_flat(const float* __restri
   const float ref = kKind == 1 ? mean[c] : (kKind == 0 ? x[(size_t)c * g.HW] : 0.f);
   const uint32_t e0 = (uint32_t)split * (uint32_t)g.per_block;
   const uint32_t e1 = min(total, e0 + (uint32_t)g.per_block);
+  const MaskCoef mc = mask_coef<kMask>(mk, c, g.C);
   double sa = 0.0, sb = 0.0;
   for (uint32_t e = e0 + threadIdx.x; e < e1; e += kThreads) {
     const uint32_t n = tt::fd_div(e, g.hwv_div);
@@ -272,12 +302,17 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_flat(const float* __restri
       v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
       if constexpr (kBwd) {
         float4 u = *reinterpret_cast<const float4*>(dy + off);
-        if constexpr (kRelu) u = mask4(u, *reinterpret_cast<const float4*>(ry + off));
+        if constexpr (kMask == kMaskY) u = mask4(u, *reinterpret_cast<const float4*>(mk + off));
+        if constexpr (kMask == kMaskCoef) u = mask4(u, bn4(t, ref, mc));
         gq[0] = u.x; gq[1] = u.y; gq[2] = u.z; gq[3] = u.w;
       }
     } else {
       v[0] = x[off];
-      if constexpr (kBwd) gq[0] = kRelu ? mask1(dy[off], ry[off]) : dy[off];
+      if constexpr (kBwd) {
+        gq[0] = dy[off];
+        if constexpr (kMask == kMaskY) gq[0] = mask1(gq[0], mk[off]);
+        if constexpr (kMask == kMaskCoef) gq[0] = mask1(gq[0], bn1(v[0], ref, mc));
+      }
     }
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
@@ -297,6 +332,11 @@ __global__ __launch_bounds__(kThreads) void bn_reduce_flat(const float* __restri
 
 // ---- sweep 2: y = (x - m) * k1 + k0      (forward)
 //               dx = dy * k1 + (x - m) * k2 + k0   (backward)
+// Fused around it, bound by memory like the sweep itself, so that what counts is tensor passes (a residual
+// block's forward read and wrote the normalised values once more for the add, 5 passes, 3 now; an
+// accumulation behind the backward took 3, 1 now), each with the rounding of the launch it stands in for: forward, a residual added
+// (kAdd) and a ReLU behind that (kAct != 0); backward, the ReLU's mask on dy (kAct: a kMask* value) and
+// the gradient that had already arrived for x added to dx (kAdd).
 struct Coef {
   float m, k0, k1, k2;
 };
@@ -318,10 +358,11 @@ __device__ __forceinline__ float4 apply4(const float4 v, const float4 gq, const 
   return o;
 }
 
-template <bool kBwd, bool kRelu>
+template <bool kBwd, int kAct, bool kAdd>
 __device__ __forceinline__ void sweep2_planes(const float* __restrict__ x, const float* __restrict__ dy,
                                               float* __restrict__ out, const Geometry& g, int c, int split,
-                                              const Coef k, const float* __restrict__ ry) {
+                                              const Coef k, const float* __restrict__ ry, const MaskCoef mc,
+                                              const float* __restrict__ addend) {
   const int hw4 = g.HW >> 2;
   const int n0 = split * g.per_block;
   const int n1 = min(g.N, n0 + g.per_block);
@@ -331,33 +372,38 @@ __device__ __forceinline__ void sweep2_planes(const float* __restrict__ x, const
     const float4* __restrict__ px = reinterpret_cast<const float4*>(x + off);
     const float4* __restrict__ pg = reinterpret_cast<const float4*>(dy + (kBwd ? off : 0));
     float4* __restrict__ po = reinterpret_cast<float4*>(out + off);
-    const float4* __restrict__ pr = reinterpret_cast<const float4*>(ry + (kBwd && kRelu ? off : 0));
+    const float4* __restrict__ pr = reinterpret_cast<const float4*>(ry + (kBwd && kAct == kMaskY ? off : 0));
+    const float4* __restrict__ pa = reinterpret_cast<const float4*>(addend + (kAdd ? off : 0));
     for (int i0 = threadIdx.x; i0 < hw4; i0 += kThreads * kU) {
-      float4 v[kU], gq[kU];
+      float4 v[kU], gq[kU], ad[kU];
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
         const int i = min(i0 + kThreads * u, hw4 - 1);   // clamped: out-of-range threads re-read, never store
         // backward: the last use of x and dy in the pass; forward: x is read again by the backward
         v[u] = kBwd ? load_stream(px + i) : px[i];
         gq[u] = kBwd ? load_stream(pg + i) : v[u];
-        if constexpr (kBwd && kRelu) gq[u] = mask4(gq[u], load_stream(pr + i));
+        if constexpr (kAdd) ad[u] = load_stream(pa + i);
+        if constexpr (kBwd && kAct == kMaskY) gq[u] = mask4(gq[u], load_stream(pr + i));
+        if constexpr (kBwd && kAct == kMaskCoef) gq[u] = mask4(gq[u], bn4(v[u], k.m, mc));
       }
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
         const int i = i0 + kThreads * u;
         if (i < hw4) {
-          const float4 o = apply4<kBwd>(v[u], gq[u], k);
-          store_stream(po + i, (!kBwd && kRelu) ? relu4(o) : o);
+          float4 o = apply4<kBwd>(v[u], gq[u], k);
+          if constexpr (kAdd) o = add4(o, ad[u]);
+          store_stream(po + i, (!kBwd && kAct) ? relu4(o) : o);
         }
       }
     }
   }
 }
 
-template <bool kBwd, int VEC, bool kRelu>
+template <bool kBwd, int VEC, int kAct, bool kAdd>
 __device__ __forceinline__ void sweep2_flat(const float* __restrict__ x, const float* __restrict__ dy,
                                             float* __restrict__ out, const Geometry& g, int c, int split,
-                                            const Coef k, const float* __restrict__ ry) {
+                                            const Coef k, const float* __restrict__ ry, const MaskCoef mc,
+                                            const float* __restrict__ addend) {
   const uint32_t hwv = (uint32_t)g.HW / VEC;
   const uint32_t total = (uint32_t)g.N * hwv;
   const uint32_t e0 = (uint32_t)split * (uint32_t)g.per_block;
@@ -371,20 +417,24 @@ __device__ __forceinline__ void sweep2_flat(const float* __restrict__ x, const f
       const float4 v = kBwd ? load_stream(px) : *px;
       float4 gq = v;
       if (kBwd) gq = load_stream(reinterpret_cast<const float4*>(dy + off));
-      if constexpr (kBwd && kRelu) gq = mask4(gq, load_stream(reinterpret_cast<const float4*>(ry + off)));
-      const float4 o = apply4<kBwd>(v, gq, k);
-      store_stream(reinterpret_cast<float4*>(out + off), (!kBwd && kRelu) ? relu4(o) : o);
+      if constexpr (kBwd && kAct == kMaskY) gq = mask4(gq, load_stream(reinterpret_cast<const float4*>(ry + off)));
+      if constexpr (kBwd && kAct == kMaskCoef) gq = mask4(gq, bn4(v, k.m, mc));
+      float4 o = apply4<kBwd>(v, gq, k);
+      if constexpr (kAdd) o = add4(o, load_stream(reinterpret_cast<const float4*>(addend + off)));
+      store_stream(reinterpret_cast<float4*>(out + off), (!kBwd && kAct) ? relu4(o) : o);
     } else {
       const float v = kBwd ? __builtin_nontemporal_load(x + off) : x[off];
       float o;
       if (kBwd) {
         float gv = __builtin_nontemporal_load(dy + off);
-        if constexpr (kRelu) gv = mask1(gv, __builtin_nontemporal_load(ry + off));
+        if constexpr (kAct == kMaskY) gv = mask1(gv, __builtin_nontemporal_load(ry + off));
+        if constexpr (kAct == kMaskCoef) gv = mask1(gv, bn1(v, k.m, mc));
         o = fmaf(gv, k.k1, fmaf(v - k.m, k.k2, k.k0));
       } else {
         o = fmaf(v - k.m, k.k1, k.k0);
-        if constexpr (kRelu) o = relu1(o);
       }
+      if constexpr (kAdd) o += __builtin_nontemporal_load(addend + off);
+      if constexpr (!kBwd && kAct) o = relu1(o);
       __builtin_nontemporal_store(o, out + off);
     }
   }
@@ -408,10 +458,12 @@ struct FwdArgs {
   int partial_splits;       // partials per channel written by the first sweep
   float one_minus_mom, mom, unbias, eps;
   float* nbt;               // training: the module's batch counter, incremented by one (may be null)
+  const float* res;         // kAdd: laid out as x, added to the normalised values
+  float* coef;              // [2][C], may be null: gamma / sd and beta as applied, for the backward's mask
 };
 
 // kMode: 0 planes, 1 flat VEC=4, 2 flat VEC=1
-template <int kMode, bool kRelu = false>
+template <int kMode, bool kRelu, bool kAdd>
 __global__ __launch_bounds__(kThreads) void bn_fwd_apply(FwdArgs a, Geometry g) {
   __shared__ Coef sk;
   const int c = g.C - 1 - (int)blockIdx.y;
@@ -443,6 +495,10 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_apply(FwdArgs a, Geometry g) 
         a.save_mean[c] = mean;
         a.save_var_eps[c] = var_eps;
         a.save_sd[c] = sd;
+        if (a.coef) {
+          a.coef[c] = sk.k1;
+          a.coef[g.C + c] = bet;
+        }
         if (a.rm_in && !a.given_mean) {
           // separate roundings, as NumPy evaluates (1-m)*rm + m*mean on float32 arrays
           a.rm_out[c] = __fadd_rn(__fmul_rn(a.one_minus_mom, a.rm_in[c]), __fmul_rn(a.mom, mean));
@@ -455,9 +511,10 @@ __global__ __launch_bounds__(kThreads) void bn_fwd_apply(FwdArgs a, Geometry g) 
   }
   __syncthreads();
   const Coef k = sk;
-  if (kMode == 0) sweep2_planes<false, kRelu>(a.x, a.x, a.y, g, c, split, k, a.x);
-  if (kMode == 1) sweep2_flat<false, 4, kRelu>(a.x, a.x, a.y, g, c, split, k, a.x);
-  if (kMode == 2) sweep2_flat<false, 1, kRelu>(a.x, a.x, a.y, g, c, split, k, a.x);
+  const MaskCoef none{0.f, 0.f};
+  if (kMode == 0) sweep2_planes<false, kRelu, kAdd>(a.x, a.x, a.y, g, c, split, k, a.x, none, a.res);
+  if (kMode == 1) sweep2_flat<false, 4, kRelu, kAdd>(a.x, a.x, a.y, g, c, split, k, a.x, none, a.res);
+  if (kMode == 2) sweep2_flat<false, 1, kRelu, kAdd>(a.x, a.x, a.y, g, c, split, k, a.x, none, a.res);
 }
 
 struct BwdArgs {
@@ -472,10 +529,11 @@ struct BwdArgs {
   float* dbeta;
   const double2* partial;
   int partial_splits;
-  const float* ry;   // fused ReLU backward: the ReLU's output; dy is masked by (ry > 0) on the fly
+  const float* mk;   // kMaskY: the ReLU's output; kMaskCoef: the forward's [2][C] constants
+  const float* add;  // kAdd: laid out as x, added to dx
 };
 
-template <int kMode, bool kRelu = false>
+template <int kMode, int kMask, bool kAdd>
 __global__ __launch_bounds__(kThreads) void bn_bwd_apply(BwdArgs a, Geometry g) {
   __shared__ Coef sk;
   const int c = g.C - 1 - (int)blockIdx.y;
@@ -501,9 +559,10 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_apply(BwdArgs a, Geometry g) 
   if (a.dx == nullptr) return;
   __syncthreads();
   const Coef k = sk;
-  if (kMode == 0) sweep2_planes<true, kRelu>(a.x, a.dy, a.dx, g, c, split, k, a.ry);
-  if (kMode == 1) sweep2_flat<true, 4, kRelu>(a.x, a.dy, a.dx, g, c, split, k, a.ry);
-  if (kMode == 2) sweep2_flat<true, 1, kRelu>(a.x, a.dy, a.dx, g, c, split, k, a.ry);
+  const MaskCoef mc = mask_coef<kMask>(a.mk, c, g.C);
+  if (kMode == 0) sweep2_planes<true, kMask, kAdd>(a.x, a.dy, a.dx, g, c, split, k, a.mk, mc, a.add);
+  if (kMode == 1) sweep2_flat<true, 4, kMask, kAdd>(a.x, a.dy, a.dx, g, c, split, k, a.mk, mc, a.add);
+  if (kMode == 2) sweep2_flat<true, 1, kMask, kAdd>(a.x, a.dy, a.dx, g, c, split, k, a.mk, mc, a.add);
 }
 
 // ---- small channels: one kernel per pass ---------------------------------------------------------
@@ -531,7 +590,7 @@ __device__ __forceinline__ void for_channel_elements(const Geometry& g, F&& f) {
   }
 }
 
-template <int EMAX, int BT, bool kRelu = false>
+template <int EMAX, int BT, bool kRelu, bool kAdd>
 __global__ __launch_bounds__(BT) void bn_fwd_small(FwdArgs a, Geometry g) {
   __shared__ double red[2 * BT / tt::kWave];
   __shared__ Coef sk;
@@ -564,21 +623,31 @@ __global__ __launch_bounds__(BT) void bn_fwd_small(FwdArgs a, Geometry g) {
     a.save_mean[c] = mean;
     a.save_var_eps[c] = var_eps;
     a.save_sd[c] = sd;
+    if (a.coef) {
+      a.coef[c] = sk.k1;
+      a.coef[g.C + c] = sk.k0;
+    }
     if (a.rm_in) {   // separate roundings, as NumPy evaluates (1-m)*rm + m*mean on float32 arrays
       a.rm_out[c] = __fadd_rn(__fmul_rn(a.one_minus_mom, a.rm_in[c]), __fmul_rn(a.mom, mean));
       a.rv_out[c] = __fadd_rn(__fmul_rn(a.one_minus_mom, a.rv_in[c]), __fmul_rn(a.mom, __fmul_rn(var, a.unbias)));
     }
     if (a.nbt && c == 0) *a.nbt = __fadd_rn(*a.nbt, 1.0f);
   }
+  float ad[EMAX];   // fetched together, behind the registers that the statistics have given back
+  if constexpr (kAdd)
+    for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
+      ad[kk] = __builtin_nontemporal_load(a.res + (size_t)c * g.HW + off);
+    });
   __syncthreads();
   const Coef k = sk;
   for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
-    const float o = fmaf(v[kk] - k.m, k.k1, k.k0);
+    float o = fmaf(v[kk] - k.m, k.k1, k.k0);
+    if constexpr (kAdd) o += ad[kk];
     __builtin_nontemporal_store(kRelu ? relu1(o) : o, yc + off);
   });
 }
 
-template <int EMAX, int BT, bool kRelu = false>
+template <int EMAX, int BT, int kMask, bool kAdd>
 __global__ __launch_bounds__(BT) void bn_bwd_small(BwdArgs a, Geometry g) {
   __shared__ double red[2 * BT / tt::kWave];
   __shared__ Coef sk;
@@ -592,8 +661,12 @@ __global__ __launch_bounds__(BT) void bn_bwd_small(BwdArgs a, Geometry g) {
   for_channel_elements<EMAX, BT>(g, [&](int k, size_t off) {
     v[k] = __builtin_nontemporal_load(xc + off);
     gq[k] = __builtin_nontemporal_load(dyc + off);
-    if constexpr (kRelu) gq[k] = mask1(gq[k], __builtin_nontemporal_load(a.ry + (size_t)c * g.HW + off));
+    if constexpr (kMask == kMaskY) gq[k] = mask1(gq[k], __builtin_nontemporal_load(a.mk + (size_t)c * g.HW + off));
   });
+  if constexpr (kMask == kMaskCoef) {
+    const MaskCoef mc = mask_coef<kMask>(a.mk, c, g.C);
+    for_channel_elements<EMAX, BT>(g, [&](int k, size_t) { gq[k] = mask1(gq[k], bn1(v[k], mean, mc)); });
+  }
   double s_dy = 0.0, s_dyxmu = 0.0;
   for_channel_elements<EMAX, BT>(g, [&](int k, size_t) {
     s_dy += (double)gq[k];
@@ -613,11 +686,18 @@ __global__ __launch_bounds__(BT) void bn_bwd_small(BwdArgs a, Geometry g) {
     if (a.dgamma) a.dgamma[c] = (float)(s_dyxmu / sd);
   }
   if (a.dx == nullptr) return;
+  float ad[EMAX];
+  if constexpr (kAdd)
+    for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
+      ad[kk] = __builtin_nontemporal_load(a.add + (size_t)c * g.HW + off);
+    });
   __syncthreads();
   const Coef k = sk;
   float* __restrict__ dxc = a.dx + (size_t)c * g.HW;
   for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
-    __builtin_nontemporal_store(fmaf(gq[kk], k.k1, fmaf(v[kk] - k.m, k.k2, k.k0)), dxc + off);
+    float o = fmaf(gq[kk], k.k1, fmaf(v[kk] - k.m, k.k2, k.k0));
+    if constexpr (kAdd) o += ad[kk];
+    __builtin_nontemporal_store(o, dxc + off);
   });
 }
 
@@ -684,22 +764,54 @@ int check_shape(const char* fn, int N, int C, int HW) {
   return 0;
 }
 
-template <int kKind>
+template <int kKind, int kMask = kNoMask>
 void launch_reduce(int mode, dim3 grid, const float* x, const float* dy, const float* mean, double2* partial,
-                   const Geometry& g, const float* ry = nullptr) {
+                   const Geometry& g, const float* mk = nullptr) {
   hipStream_t st = tt::stream();
-  if constexpr (kKind == 1) {
-    if (ry) {   // backward behind a fused ReLU: dy is masked by (ry > 0) as it is read
-      if (mode == 3) bn_reduce_stream<1, true><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g, ry);
-      if (mode == 1) bn_reduce_flat<1, 4, true><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g, ry);
-      if (mode == 2) bn_reduce_flat<1, 1, true><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g, ry);
-      return;
-    }
+  if constexpr (kMask == kNoMask) {
+    if (mode == 0) bn_reduce_planes<kKind><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g);
   }
-  if (mode == 0) bn_reduce_planes<kKind><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g);
-  if (mode == 3) bn_reduce_stream<kKind><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g);
-  if (mode == 1) bn_reduce_flat<kKind, 4><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g);
-  if (mode == 2) bn_reduce_flat<kKind, 1><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g);
+  if (mode == 3) bn_reduce_stream<kKind, kMask><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g, mk);
+  if (mode == 1) bn_reduce_flat<kKind, 4, kMask><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g, mk);
+  if (mode == 2) bn_reduce_flat<kKind, 1, kMask><<<grid, kThreads, 0, st>>>(x, dy, mean, partial, g, mk);
+}
+
+// The second sweeps and the single-kernel passes, by what is fused into them.
+template <bool kRelu, bool kAdd>
+void launch_fwd_apply(int mode, dim3 grid, const FwdArgs& a, const Geometry& g) {
+  hipStream_t st = tt::stream();
+  if (mode == 0) bn_fwd_apply<0, kRelu, kAdd><<<grid, kThreads, 0, st>>>(a, g);
+  if (mode == 1) bn_fwd_apply<1, kRelu, kAdd><<<grid, kThreads, 0, st>>>(a, g);
+  if (mode == 2) bn_fwd_apply<2, kRelu, kAdd><<<grid, kThreads, 0, st>>>(a, g);
+}
+void launch_fwd_apply(bool relu, int mode, dim3 grid, const FwdArgs& a, const Geometry& g) {
+  if (relu) a.res ? launch_fwd_apply<true, true>(mode, grid, a, g) : launch_fwd_apply<true, false>(mode, grid, a, g);
+  else a.res ? launch_fwd_apply<false, true>(mode, grid, a, g) : launch_fwd_apply<false, false>(mode, grid, a, g);
+}
+template <bool kRelu, bool kAdd>
+void launch_fwd_small(int cfg, const FwdArgs& a, const Geometry& g) {
+  hipStream_t st = tt::stream();
+  if (cfg == 1) bn_fwd_small<kSmallValues, kThreads, kRelu, kAdd><<<g.C, kThreads, 0, st>>>(a, g);
+  else if (cfg == 2) bn_fwd_small<kSmallValuesMax, kThreads, kRelu, kAdd><<<g.C, kThreads, 0, st>>>(a, g);
+  else bn_fwd_small<kSmallValues, kSmallThreads, kRelu, kAdd><<<g.C, kSmallThreads, 0, st>>>(a, g);
+}
+void launch_fwd_small(bool relu, int cfg, const FwdArgs& a, const Geometry& g) {
+  if (relu) a.res ? launch_fwd_small<true, true>(cfg, a, g) : launch_fwd_small<true, false>(cfg, a, g);
+  else a.res ? launch_fwd_small<false, true>(cfg, a, g) : launch_fwd_small<false, false>(cfg, a, g);
+}
+template <int kMask, bool kAdd>
+void launch_bwd_apply(int mode, dim3 grid, const BwdArgs& a, const Geometry& g) {
+  hipStream_t st = tt::stream();
+  if (mode == 0) bn_bwd_apply<0, kMask, kAdd><<<grid, kThreads, 0, st>>>(a, g);
+  if (mode == 1) bn_bwd_apply<1, kMask, kAdd><<<grid, kThreads, 0, st>>>(a, g);
+  if (mode == 2) bn_bwd_apply<2, kMask, kAdd><<<grid, kThreads, 0, st>>>(a, g);
+}
+template <int kMask, bool kAdd>
+void launch_bwd_small(int cfg, const BwdArgs& a, const Geometry& g) {
+  hipStream_t st = tt::stream();
+  if (cfg == 1) bn_bwd_small<kSmallValues, kThreads, kMask, kAdd><<<g.C, kThreads, 0, st>>>(a, g);
+  else if (cfg == 2) bn_bwd_small<kSmallValuesMax, kThreads, kMask, kAdd><<<g.C, kThreads, 0, st>>>(a, g);
+  else bn_bwd_small<kSmallValues, kSmallThreads, kMask, kAdd><<<g.C, kSmallThreads, 0, st>>>(a, g);
 }
 
 // Geometry of the first sweep: the stream kernel when planes are float4-aligned, else as plan().
@@ -766,11 +878,12 @@ static int bn_fwd_train(const char* fn, const float* x, const float* gamma, cons
                         float* save_mean, float* save_var_eps, float* save_sd, const float* running_mean_in,
                         const float* running_var_in, float* running_mean_out, float* running_var_out,
                         float* num_batches_tracked, double momentum, double eps, int N, int C, int HW,
-                        double2* fixed_partials, size_t fixed_capacity, bool relu = false) {
+                        double2* fixed_partials, size_t fixed_capacity, bool relu = false,
+                        const float* residual = nullptr, float* save_coef = nullptr) {
   TT_REQUIRE_INIT();
   if (check_shape(fn, N, C, HW)) return -1;
   TT_REQUIRE(x && y && save_mean && save_var_eps && save_sd, "%s: null tensor pointer", fn);
-  TT_REQUIRE_ALIGNED(fn, x, y);
+  TT_REQUIRE_ALIGNED(fn, x, y, residual);
   const long long m = (long long)N * HW;
   TT_REQUIRE(m > 1, "Expected more than 1 value per channel when training, got input size [%d, %d, %d]", N, C, HW);
   const bool track = running_mean_in && running_var_in;
@@ -784,23 +897,15 @@ static int bn_fwd_train(const char* fn, const float* x, const float* gamma, cons
   a.rm_out = running_mean_out; a.rv_out = running_var_out;
   a.given_mean = nullptr; a.given_var = nullptr;
   a.nbt = num_batches_tracked;
+  a.res = residual;
+  a.coef = save_coef;
   a.one_minus_mom = (float)(1.0 - momentum);
   a.mom = (float)momentum;
   a.unbias = (float)((double)m / (double)(m - 1));
   a.eps = (float)eps;
-  hipStream_t st = tt::stream();
   if (const int cfg = small_channel_config(N, C, HW)) {
     tt::ProfScope prof(timed ? TT_PROF_BN_FWD_APPLY : -1);
-    const Geometry gs = small_geometry(N, C, HW);
-    if (relu) {
-      if (cfg == 1) bn_fwd_small<kSmallValues, kThreads, true><<<C, kThreads, 0, st>>>(a, gs);
-      else if (cfg == 2) bn_fwd_small<kSmallValuesMax, kThreads, true><<<C, kThreads, 0, st>>>(a, gs);
-      else bn_fwd_small<kSmallValues, kSmallThreads, true><<<C, kSmallThreads, 0, st>>>(a, gs);
-    } else {
-      if (cfg == 1) bn_fwd_small<kSmallValues, kThreads><<<C, kThreads, 0, st>>>(a, gs);
-      else if (cfg == 2) bn_fwd_small<kSmallValuesMax, kThreads><<<C, kThreads, 0, st>>>(a, gs);
-      else bn_fwd_small<kSmallValues, kSmallThreads><<<C, kSmallThreads, 0, st>>>(a, gs);
-    }
+    launch_fwd_small(relu, cfg, a, small_geometry(N, C, HW));
     TT_LAUNCH_CHECK();
     return 0;
   }
@@ -830,15 +935,7 @@ static int bn_fwd_train(const char* fn, const float* x, const float* gamma, cons
   a.partial_splits = gr.splits;
   {
     tt::ProfScope prof(timed ? TT_PROF_BN_FWD_APPLY : -1);
-    if (relu) {
-      if (mode == 0) bn_fwd_apply<0, true><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 1) bn_fwd_apply<1, true><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 2) bn_fwd_apply<2, true><<<grid, kThreads, 0, st>>>(a, g);
-    } else {
-      if (mode == 0) bn_fwd_apply<0><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 1) bn_fwd_apply<1><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 2) bn_fwd_apply<2><<<grid, kThreads, 0, st>>>(a, g);
-    }
+    launch_fwd_apply(relu, mode, grid, a, g);
   }
   TT_LAUNCH_CHECK();
   return 0;
@@ -860,6 +957,16 @@ int tt_bn_relu_fwd_train_f32(const float* x, const float* gamma, const float* be
   return bn_fwd_train("tt_bn_relu_fwd_train_f32", x, gamma, beta, y, save_mean, save_var_eps, save_sd, running_mean_in,
                       running_var_in, running_mean_out, running_var_out, num_batches_tracked, momentum, eps, N, C, HW,
                       nullptr, 0, true);
+}
+
+int tt_bn_act_fwd_train_f32(const float* x, const float* gamma, const float* beta, const float* residual, float* y,
+                            float* save_mean, float* save_var_eps, float* save_sd, float* save_coef,
+                            const float* running_mean_in, const float* running_var_in, float* running_mean_out,
+                            float* running_var_out, float* num_batches_tracked, double momentum, double eps, int relu,
+                            int N, int C, int HW) {
+  return bn_fwd_train("tt_bn_act_fwd_train_f32", x, gamma, beta, y, save_mean, save_var_eps, save_sd, running_mean_in,
+                      running_var_in, running_mean_out, running_var_out, num_batches_tracked, momentum, eps, N, C, HW,
+                      nullptr, 0, relu != 0, residual, save_coef);
 }
 
 int tt_bn_fwd_train_noalloc_f32(const float* x, const float* gamma, const float* beta, float* y, float* save_mean,
@@ -892,18 +999,9 @@ static int bn_fwd_eval(const char* fn, const float* x, const float* gamma, const
   a.save_mean = save_mean; a.save_var_eps = save_var_eps; a.save_sd = save_sd;
   a.given_mean = mean; a.given_var = var;
   a.eps = (float)eps;
-  hipStream_t st = tt::stream();
   {
     tt::ProfScope prof(TT_PROF_BN_FWD_APPLY);
-    if (relu) {
-      if (mode == 0) bn_fwd_apply<0, true><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 1) bn_fwd_apply<1, true><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 2) bn_fwd_apply<2, true><<<grid, kThreads, 0, st>>>(a, g);
-    } else {
-      if (mode == 0) bn_fwd_apply<0><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 1) bn_fwd_apply<1><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 2) bn_fwd_apply<2><<<grid, kThreads, 0, st>>>(a, g);
-    }
+    launch_fwd_apply(relu, mode, grid, a, g);
   }
   TT_LAUNCH_CHECK();
   return 0;
@@ -923,29 +1021,24 @@ int tt_bn_relu_fwd_eval_f32(const float* x, const float* gamma, const float* bet
                      HW, true);
 }
 
-// Backward behind tt_bn_bwd_f32 (ry == nullptr) and tt_bn_relu_bwd_f32 (ry = the fused ReLU's output).
-static int bn_bwd(const char* fn, const float* x, const float* dy, const float* ry, const float* gamma,
-                  const float* save_mean, const float* save_var_eps, const float* save_sd, float* dx, float* dgamma,
-                  float* dbeta, int N, int C, int HW) {
+}  // extern "C"
+
+// Backward behind the three entry points: kMask says what `mk` is, `add` (may be null) is added to dx.
+template <int kMask>
+static int bn_bwd(const char* fn, const float* x, const float* dy, const float* mk, const float* gamma,
+                  const float* save_mean, const float* save_var_eps, const float* save_sd, float* dx, const float* add,
+                  float* dgamma, float* dbeta, int N, int C, int HW) {
   TT_REQUIRE_INIT();
   if (check_shape(fn, N, C, HW)) return -1;
   TT_REQUIRE(x && dy && save_mean && save_var_eps && save_sd, "%s: null tensor pointer", fn);
-  TT_REQUIRE_ALIGNED(fn, x, dy, dx, ry);
+  TT_REQUIRE_ALIGNED(fn, x, dy, dx, add);
+  if (kMask == kMaskY) TT_REQUIRE_ALIGNED(fn, mk);
   if (!dx && !dgamma && !dbeta) return 0;
+  BwdArgs a{x, dy, gamma, save_mean, save_var_eps, save_sd, dx, dgamma, dbeta, nullptr, 0, mk, add};
   if (const int cfg = small_channel_config(N, C, HW)) {
     tt::ProfScope prof(TT_PROF_BN_BWD_APPLY);
     const Geometry gs = small_geometry(N, C, HW);
-    BwdArgs b{x, dy, gamma, save_mean, save_var_eps, save_sd, dx, dgamma, dbeta, nullptr, 0, ry};
-    hipStream_t st = tt::stream();
-    if (ry) {
-      if (cfg == 1) bn_bwd_small<kSmallValues, kThreads, true><<<C, kThreads, 0, st>>>(b, gs);
-      else if (cfg == 2) bn_bwd_small<kSmallValuesMax, kThreads, true><<<C, kThreads, 0, st>>>(b, gs);
-      else bn_bwd_small<kSmallValues, kSmallThreads, true><<<C, kSmallThreads, 0, st>>>(b, gs);
-    } else {
-      if (cfg == 1) bn_bwd_small<kSmallValues, kThreads><<<C, kThreads, 0, st>>>(b, gs);
-      else if (cfg == 2) bn_bwd_small<kSmallValuesMax, kThreads><<<C, kThreads, 0, st>>>(b, gs);
-      else bn_bwd_small<kSmallValues, kSmallThreads><<<C, kSmallThreads, 0, st>>>(b, gs);
-    }
+    add ? launch_bwd_small<kMask, true>(cfg, a, gs) : launch_bwd_small<kMask, false>(cfg, a, gs);
     TT_LAUNCH_CHECK();
     return 0;
   }
@@ -958,39 +1051,44 @@ static int bn_bwd(const char* fn, const float* x, const float* dy, const float* 
   dim3 grid(g.splits, C);
   {
     tt::ProfScope prof(TT_PROF_BN_BWD_REDUCE);
-    launch_reduce<1>(rmode, dim3(gr.splits, C), x, dy, save_mean, (double2*)ws, gr, ry);
+    launch_reduce<1, kMask>(rmode, dim3(gr.splits, C), x, dy, save_mean, (double2*)ws, gr, mk);
   }
   TT_LAUNCH_CHECK();
-  BwdArgs a{x, dy, gamma, save_mean, save_var_eps, save_sd, dx, dgamma, dbeta, (const double2*)ws, gr.splits, ry};
-  hipStream_t st = tt::stream();
+  a.partial = (const double2*)ws;
+  a.partial_splits = gr.splits;
   {
     tt::ProfScope prof(TT_PROF_BN_BWD_APPLY);
-    if (ry) {
-      if (mode == 0) bn_bwd_apply<0, true><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 1) bn_bwd_apply<1, true><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 2) bn_bwd_apply<2, true><<<grid, kThreads, 0, st>>>(a, g);
-    } else {
-      if (mode == 0) bn_bwd_apply<0><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 1) bn_bwd_apply<1><<<grid, kThreads, 0, st>>>(a, g);
-      if (mode == 2) bn_bwd_apply<2><<<grid, kThreads, 0, st>>>(a, g);
-    }
+    add ? launch_bwd_apply<kMask, true>(mode, grid, a, g) : launch_bwd_apply<kMask, false>(mode, grid, a, g);
   }
   TT_LAUNCH_CHECK();
   return 0;
 }
 
+extern "C" {
+
 int tt_bn_bwd_f32(const float* x, const float* dy, const float* gamma, const float* save_mean,
                   const float* save_var_eps, const float* save_sd, float* dx, float* dgamma, float* dbeta, int N,
                   int C, int HW) {
-  return bn_bwd("tt_bn_bwd_f32", x, dy, nullptr, gamma, save_mean, save_var_eps, save_sd, dx, dgamma, dbeta, N, C, HW);
+  return bn_bwd<kNoMask>("tt_bn_bwd_f32", x, dy, nullptr, gamma, save_mean, save_var_eps, save_sd, dx, nullptr, dgamma,
+                         dbeta, N, C, HW);
 }
 
 int tt_bn_relu_bwd_f32(const float* x, const float* dy, const float* relu_y, const float* gamma, const float* save_mean,
                        const float* save_var_eps, const float* save_sd, float* dx, float* dgamma, float* dbeta, int N,
                        int C, int HW) {
   TT_REQUIRE(relu_y != nullptr, "tt_bn_relu_bwd_f32: null ReLU output");
-  return bn_bwd("tt_bn_relu_bwd_f32", x, dy, relu_y, gamma, save_mean, save_var_eps, save_sd, dx, dgamma, dbeta, N, C,
-                HW);
+  return bn_bwd<kMaskY>("tt_bn_relu_bwd_f32", x, dy, relu_y, gamma, save_mean, save_var_eps, save_sd, dx, nullptr, dgamma,
+                        dbeta, N, C, HW);
+}
+
+int tt_bn_act_bwd_f32(const float* x, const float* dy, const float* coef, const float* gamma, const float* save_mean,
+                      const float* save_var_eps, const float* save_sd, float* dx, const float* dx_add, float* dgamma,
+                      float* dbeta, int N, int C, int HW) {
+  if (coef)
+    return bn_bwd<kMaskCoef>("tt_bn_act_bwd_f32", x, dy, coef, gamma, save_mean, save_var_eps, save_sd, dx, dx_add, dgamma,
+                             dbeta, N, C, HW);
+  return bn_bwd<kNoMask>("tt_bn_act_bwd_f32", x, dy, nullptr, gamma, save_mean, save_var_eps, save_sd, dx, dx_add, dgamma,
+                         dbeta, N, C, HW);
 }
 
 int tt_channel_sum_f32(const float* t, float* out, int N, int K, int HW) {

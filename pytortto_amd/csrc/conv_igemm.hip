@@ -1,7 +1,7 @@
 // Implicit-GEMM convolution on fp32 MFMA for gfx950: Conv2d forward, and the gather-form input
 // gradient that also serves as ConvTranspose2d forward.  NCHW float32, no im2col buffer in HBM.
-// (This file: launch planning, index tables, weight repacks and the float32 / bf16 instantiations; the
-// kernel body itself is conv_igemm_kernel.h, shared with conv_igemm_x3.hip.)
+// (This file: launch planning, index tables and weight repacks.  The kernel body is conv_igemm_kernel.h,
+// instantiated once per arithmetic by conv_igemm_f32.hip, conv_igemm_rounded.hip and conv_igemm_x3.hip.)
 //
 // Per group the kernel computes   D[i, m] = sum_k  Wp[i, k] * G[k, m]   (+ bias[i])
 //   forward: i = output channel, m = (n, p, q) output pixel, k = (c, r, s),
@@ -156,37 +156,6 @@ __global__ void pack_w_dgrad_dense(const float* __restrict__ w, floatx4* __restr
   wp[(size_t)kq * a.Ipad + i] = floatx4{v[0], v[1], v[2], v[3]};
 }
 
-}  // namespace
-
-#include "conv_igemm_kernel.h"
-
-namespace {
-
-using namespace ttc;
-
-template <int WM, int WN, int MT, int NT, bool SK, int MODE, bool AT>
-__global__ __launch_bounds__(kThreads, 2) void igemm_f32(const Igemm p) {
-  igemm_body<WM, WN, MT, NT, SK, MODE, AT, 0>(p, (int)blockIdx.x);
-}
-// The same launch on bf16 matrix instructions (tt_set_conv_math); three blocks per CU.
-template <int WM, int WN, int MT, int NT, bool SK, int MODE, bool AT>
-__global__ __launch_bounds__(kThreads, 3) void igemm_bf16(const Igemm p) {
-  igemm_body<WM, WN, MT, NT, SK, MODE, AT, 1>(p, (int)blockIdx.x);
-}
-
-template <int WM, int WN, int MT, int NT, int MODE>
-__global__ __launch_bounds__(kThreads, 2) void igemm_multi_f32(const IgemmMulti m) {
-  int ci = 0;
-  while (ci + 1 < m.n && (int)blockIdx.x >= m.first[ci + 1]) ++ci;
-  igemm_body<WM, WN, MT, NT, false, MODE, false, 0>(m.c[ci], (int)blockIdx.x - m.first[ci]);
-}
-template <int WM, int WN, int MT, int NT, int MODE>
-__global__ __launch_bounds__(kThreads, 3) void igemm_multi_bf16(const IgemmMulti m) {
-  int ci = 0;
-  while (ci + 1 < m.n && (int)blockIdx.x >= m.first[ci + 1]) ++ci;
-  igemm_body<WM, WN, MT, NT, false, MODE, false, 1>(m.c[ci], (int)blockIdx.x - m.first[ci]);
-}
-
 // ---- host side -------------------------------------------------------------------------------------
 
 int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
@@ -221,6 +190,10 @@ bool bf16_math() { return tt::conv_math() == TT_CONV_MATH_BF16; }
 bool split_math() { return tt::conv_math() == TT_CONV_MATH_BF16X3; }
 // bf16 terms per operand element of the matrix instructions in use (0: float32 instructions)
 int math_terms() { return bf16_math() ? 1 : split_math() ? 3 : 0; }
+const IgemmUnit& unit(int terms, bool epilogue) {
+  if (epilogue) return terms == 3 ? igemm_epi_bf16x3_unit() : terms == 1 ? igemm_epi_bf16_unit() : igemm_epi_f32_unit();
+  return terms == 3 ? igemm_bf16x3_unit() : terms == 1 ? igemm_bf16_unit() : igemm_f32_unit();
+}
 
 // Blocks of a persistent launch: the bf16 kernels hide their loads with a third block per CU
 // (measured: 3 % faster than two, four do not fit the register file).
@@ -253,79 +226,7 @@ TileChoice choose_tile(int I, int M, int groups, int chunks, bool allow_stream_k
 // bytes of stream-K partial accumulators for the largest tile: one slot per block
 size_t sk_workspace_bytes() { return (size_t)sk_launch_blocks() * 128 * 128 * sizeof(float); }
 
-// The stream-K wait is safe only while every block of the persistent grid is resident at once
-// (sk_launch_blocks() = 2 per CU, 3 for the bf16 kernels).  What the device can hold of one
-// instantiation is asked once (registers and LDS of the compiled kernel decide it); an
-// instantiation that cannot hold that many is launched data-parallel instead, one tile per block:
-// a register-count regression then costs speed, never a stalled launch.
-template <int WM, int WN, int MT, int NT, int MODE, bool AT, int BFK>
-int sk_resident_blocks_per_cu() {
-  static int cached = -1;
-  if (cached < 0) {
-    int n = 0;
-    hipError_t e;
-    if constexpr (BFK == 1) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, igemm_bf16<WM, WN, MT, NT, true, MODE, AT>, kThreads, 0);
-    else e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, igemm_f32<WM, WN, MT, NT, true, MODE, AT>, kThreads, 0);
-    if (e != hipSuccess) {
-      (void)hipGetLastError();
-      n = 0;
-    }
-    cached = n;
-  }
-  return cached;
-}
 int g_sk_forced_occupancy = -1;   // >= 0: pretend every instantiation holds this many blocks per CU (tests of the fallback)
-
-// Returns whether the persistent (stream-K) grid was launched.
-template <int WM, int WN, int MT, int NT, int MODE, bool AT>
-bool launch_mode(const Igemm& p, int groups, int sk_blocks, hipStream_t st) {
-  const bool bf = tt::conv_math() == TT_CONV_MATH_BF16;
-  if (sk_blocks > 0) {
-    int held = bf ? sk_resident_blocks_per_cu<WM, WN, MT, NT, MODE, AT, 1>() : sk_resident_blocks_per_cu<WM, WN, MT, NT, MODE, AT, 0>();
-    if (g_sk_forced_occupancy >= 0) held = g_sk_forced_occupancy;
-    if ((long long)held * cus() < sk_blocks) sk_blocks = 0;   // the data-parallel launch ignores the stream-K fields
-  }
-  if (sk_blocks > 0) {
-    if (bf) igemm_bf16<WM, WN, MT, NT, true, MODE, AT><<<dim3(sk_blocks, 1), kThreads, 0, st>>>(p);
-    else igemm_f32<WM, WN, MT, NT, true, MODE, AT><<<dim3(sk_blocks, 1), kThreads, 0, st>>>(p);
-  } else if (bf) {
-    igemm_bf16<WM, WN, MT, NT, false, MODE, AT><<<dim3(p.tiles, groups), kThreads, 0, st>>>(p);
-  } else {
-    igemm_f32<WM, WN, MT, NT, false, MODE, AT><<<dim3(p.tiles, groups), kThreads, 0, st>>>(p);
-  }
-  return sk_blocks > 0;
-}
-// smallest number of resident blocks per CU over every stream-K instantiation of one tile shape
-template <int WM, int WN, int MT, int NT, int BFK>
-int sk_min_resident() {
-  const int all[] = {sk_resident_blocks_per_cu<WM, WN, MT, NT, kModeGemm, true, BFK>(),
-                     sk_resident_blocks_per_cu<WM, WN, MT, NT, kModeGemm, false, BFK>(),
-                     sk_resident_blocks_per_cu<WM, WN, MT, NT, kModeTapMask, true, BFK>(),
-                     sk_resident_blocks_per_cu<WM, WN, MT, NT, kModeTapMask, false, BFK>(),
-                     sk_resident_blocks_per_cu<WM, WN, MT, NT, kModeTapMask64, false, BFK>(),
-                     sk_resident_blocks_per_cu<WM, WN, MT, NT, kModeCompare, false, BFK>()};
-  int lo = all[0];
-  for (int v : all) lo = v < lo ? v : lo;
-  return lo;
-}
-template <int BFK>
-int sk_min_resident_all() {
-  const int all[] = {sk_min_resident<2, 2, 2, 2, BFK>(), sk_min_resident<1, 4, 2, 2, BFK>(),
-                     sk_min_resident<1, 4, 1, 2, BFK>(), sk_min_resident<2, 2, 1, 1, BFK>()};
-  int lo = all[0];
-  for (int v : all) lo = v < lo ? v : lo;
-  return lo;
-}
-template <int WM, int WN, int MT, int NT>
-bool launch_config(const Igemm& p, int groups, int sk_blocks, hipStream_t st) {
-  const bool at = p.wTransStride > 0;
-  if (p.mode == kModeGemm && at) return launch_mode<WM, WN, MT, NT, kModeGemm, true>(p, groups, sk_blocks, st);
-  if (p.mode == kModeGemm) return launch_mode<WM, WN, MT, NT, kModeGemm, false>(p, groups, sk_blocks, st);
-  if (p.mode == kModeTapMask && at) return launch_mode<WM, WN, MT, NT, kModeTapMask, true>(p, groups, sk_blocks, st);
-  if (p.mode == kModeTapMask) return launch_mode<WM, WN, MT, NT, kModeTapMask, false>(p, groups, sk_blocks, st);
-  if (p.mode == kModeTapMask64) return launch_mode<WM, WN, MT, NT, kModeTapMask64, false>(p, groups, sk_blocks, st);
-  return launch_mode<WM, WN, MT, NT, kModeCompare, false>(p, groups, sk_blocks, st);
-}
 
 // Picks how the kernel addresses the gathered operand (see Igemm::mode) and completes the table
 // arguments accordingly.  Needs the source geometry fields of `p`; `pixels` = U*V pixels per
@@ -448,17 +349,7 @@ int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_pa
   const int plan[8] = {t.bm, t.bn, p.tiles, p.tilesI, t.sk_blocks, t.sk_blocks > 0 ? p.skDpTiles : p.tiles,
                        t.sk_blocks > 0 ? p.skBlocks : 0, p.mode | math_terms() << 8};
   std::copy(plan, plan + 8, g_last_launch);
-  bool persistent;
-  if (split_math())
-    persistent = x3_launch(p, groups, t.sk_blocks, t.bm, t.bn, g_sk_forced_occupancy, st);
-  else if (t.bm == 128 && t.bn == 128)
-    persistent = launch_config<2, 2, 2, 2>(p, groups, t.sk_blocks, st);
-  else if (t.bm == 64 && t.bn == 256)
-    persistent = launch_config<1, 4, 2, 2>(p, groups, t.sk_blocks, st);
-  else if (t.bm == 32 && t.bn == 256)
-    persistent = launch_config<1, 4, 1, 2>(p, groups, t.sk_blocks, st);
-  else
-    persistent = launch_config<2, 2, 1, 1>(p, groups, t.sk_blocks, st);
+  const bool persistent = unit(math_terms(), p.epi.on).launch(p, groups, t.sk_blocks, t.bm, t.bn, g_sk_forced_occupancy, st);
   if (!persistent) {   // also when the device could not hold the persistent grid: one tile per block
     g_last_launch[4] = 0;
     g_last_launch[5] = p.tiles;
@@ -468,20 +359,6 @@ int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_pa
   return 0;
 }
 
-// Launches the data-parallel GEMMs in `list` (same tile shape, same addressing mode, no stream-K,
-// no transposed weights) as one grid.
-template <int WM, int WN, int MT, int NT>
-void launch_multi_config(const IgemmMulti& m, int groups, hipStream_t st) {
-  const dim3 grid(m.first[m.n], groups);
-  const bool bf = bf16_math();
-  if (m.c[0].mode == kModeTapMask) {
-    if (bf) igemm_multi_bf16<WM, WN, MT, NT, kModeTapMask><<<grid, kThreads, 0, st>>>(m);
-    else igemm_multi_f32<WM, WN, MT, NT, kModeTapMask><<<grid, kThreads, 0, st>>>(m);
-  } else {
-    if (bf) igemm_multi_bf16<WM, WN, MT, NT, kModeCompare><<<grid, kThreads, 0, st>>>(m);
-    else igemm_multi_f32<WM, WN, MT, NT, kModeCompare><<<grid, kThreads, 0, st>>>(m);
-  }
-}
 int launch_igemm_multi(IgemmMulti& m, int groups, TileChoice t, int prof_id) {
   tt::ProfScope prof(prof_id);
   m.first[0] = 0;
@@ -493,17 +370,7 @@ int launch_igemm_multi(IgemmMulti& m, int groups, TileChoice t, int prof_id) {
   }
   const int plan[8] = {t.bm, t.bn, m.first[m.n], 0, 0, m.first[m.n], 0, m.c[0].mode | math_terms() << 8};   // several launches in one grid
   std::copy(plan, plan + 8, g_last_launch);
-  hipStream_t st = tt::stream();
-  if (split_math())
-    x3_launch_multi(m, groups, t.bm, t.bn, st);
-  else if (t.bm == 128 && t.bn == 128)
-    launch_multi_config<2, 2, 2, 2>(m, groups, st);
-  else if (t.bm == 64 && t.bn == 256)
-    launch_multi_config<1, 4, 2, 2>(m, groups, st);
-  else if (t.bm == 32 && t.bn == 256)
-    launch_multi_config<1, 4, 1, 2>(m, groups, st);
-  else
-    launch_multi_config<2, 2, 1, 1>(m, groups, st);
+  unit(math_terms(), false).launch_multi(m, groups, t.bm, t.bn, tt::stream());
   TT_LAUNCH_CHECK();
   return 0;
 }
@@ -751,7 +618,8 @@ int tt_set_conv_dense_cell_min_tiles(int tiles) {
 int tt_conv2d_stream_k_blocks_per_cu(int bf16, int* blocks) {
   TT_REQUIRE_INIT();
   TT_REQUIRE(blocks != nullptr, "tt_conv2d_stream_k_blocks_per_cu: null result pointer");
-  *blocks = bf16 == 3 ? x3_min_resident_blocks() : bf16 ? sk_min_resident_all<1>() : sk_min_resident_all<0>();
+  const int terms = bf16 == 3 ? 3 : bf16 ? 1 : 0;
+  *blocks = std::min(unit(terms, false).min_resident_blocks(), unit(terms, true).min_resident_blocks());
   return 0;
 }
 
@@ -867,7 +735,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
 
 static int conv2d_dgrad(const float* dy, const float* w, const float* bias, float* dx, int N, int C, int Hx, int Wx,
                         int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups, int P,
-                        int Q, size_t* size_only, bool check_only = false) {
+                        int Q, size_t* size_only, bool check_only = false, const Epilogue* epi = nullptr) {
   const char* fn = "tt_conv2d_dgrad_f32";
   TT_API_LOCK();
   if (!check_only) {
@@ -884,7 +752,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
   if (P == 1 && Q == 1 && R * S > 1 && ph == 0 && pw == 0 && dh == 1 && dw == 1 && Hx == R && Wx == S && groups == 1 &&
       bias == nullptr && tt::fits_i32((long long)C * R * S))
     return conv2d_dgrad(dy, w, nullptr, dx, N, C * R * S, 1, 1, K, 1, 1, 1, 1, 0, 0, 1, 1, 1, 1, 1, size_only,
-                        check_only);
+                        check_only, epi);
   const int Cg = C / groups, Kg = K / groups;
   const int gh = gcd(sh, dh), gw = gcd(sw, dw);
   const int rstep = sh / gh, sstep = sw / gw;   // valid taps of a class: r0, r0+rstep, ...
@@ -1090,6 +958,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
       p.ou = sh; p.ouh = ch; p.ov = sw; p.ovw = cw;
       p.kStride = P * Q;   // 1x1 layers: dx[c][n,hw] = sum_k w[k][c] * dy[n][k][hw]
       p.cellFill = cell_fill;
+      if (epi) p.epi = *epi;   // stride 1: this is the only class, and its launch writes every element of dx
       p.Kred = Kred;
       if (KQ > 0) {
         // h = u*sh + ch reads dy row (h + ph - r0*dh)/sh = u + (ch + ph - r0*dh)/sh  (exact)
@@ -1205,25 +1074,49 @@ int tt_conv2d_norm_act_fwd_f32(const float* x, const float* w, const float* bias
                                int dh, int dw, int groups) {
   TT_REQUIRE((mean == nullptr) == (var == nullptr), "tt_conv2d_norm_act_fwd_f32: mean and var come together");
   TT_REQUIRE_ALIGNED("tt_conv2d_norm_act_fwd_f32", residual);
-  const Epilogue epi{mean, var, gamma, beta, residual, (float)eps, mean != nullptr, relu != 0, 1};
+  const Epilogue epi{mean, var, gamma, beta, residual, nullptr, (float)eps, mean != nullptr, relu != 0, 1};
   return conv2d_fwd_runs("tt_conv2d_norm_act_fwd_f32", x, w, bias, y, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, &epi);
+}
+
+static int conv2d_dgrad_runs(const char* fn, const float* dy, const float* w, const float* bias, float* dx, int N, int C,
+                             int Hx, int Wx, int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw,
+                             int groups, int P, int Q, const Epilogue* epi) {
+  const long long xi = (long long)C * Hx * Wx, yi = (long long)K * P * Q;
+  const int per = images_per_call(N, xi, yi);
+  TT_REQUIRE(per > 0, "%s: a batch of 2^31 elements or more is cut into runs of images, and images of "
+                      "%lld and %lld elements leave no run 16-byte aligned", fn, xi, yi);
+  if (per >= N)
+    return conv2d_dgrad(dy, w, bias, dx, N, C, Hx, Wx, K, R, S, sh, sw, ph, pw, dh, dw, groups, P, Q, nullptr, false, epi);
+  for (int n0 = 0; n0 < N; n0 += per) {
+    const int n = N - n0 < per ? N - n0 : per;
+    Epilogue run{};
+    if (epi) {
+      run = *epi;
+      if (run.res) run.res += (size_t)n0 * xi;
+      if (run.mask) run.mask += (size_t)n0 * xi;
+    }
+    if (int rc = conv2d_dgrad(dy + (size_t)n0 * yi, w, bias, dx + (size_t)n0 * xi, n, C, Hx, Wx, K, R, S, sh, sw, ph, pw,
+                              dh, dw, groups, P, Q, nullptr, false, epi ? &run : nullptr))
+      return rc;
+  }
+  return 0;
 }
 
 int tt_conv2d_dgrad_f32(const float* dy, const float* w, const float* bias, float* dx, int N, int C, int Hx, int Wx,
                         int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups, int P,
                         int Q) {
-  const long long xi = (long long)C * Hx * Wx, yi = (long long)K * P * Q;
-  const int per = images_per_call(N, xi, yi);
-  TT_REQUIRE(per > 0, "tt_conv2d_dgrad_f32: a batch of 2^31 elements or more is cut into runs of images, and images of "
-                      "%lld and %lld elements leave no run 16-byte aligned", xi, yi);
-  if (per >= N) return conv2d_dgrad(dy, w, bias, dx, N, C, Hx, Wx, K, R, S, sh, sw, ph, pw, dh, dw, groups, P, Q, nullptr);
-  for (int n0 = 0; n0 < N; n0 += per) {
-    const int n = N - n0 < per ? N - n0 : per;
-    if (int rc = conv2d_dgrad(dy + (size_t)n0 * yi, w, bias, dx + (size_t)n0 * xi, n, C, Hx, Wx, K, R, S, sh, sw, ph, pw,
-                              dh, dw, groups, P, Q, nullptr))
-      return rc;
-  }
-  return 0;
+  return conv2d_dgrad_runs("tt_conv2d_dgrad_f32", dy, w, bias, dx, N, C, Hx, Wx, K, R, S, sh, sw, ph, pw, dh, dw, groups,
+                           P, Q, nullptr);
+}
+
+int tt_conv2d_dgrad_acc_f32(const float* dy, const float* w, float* dx, const float* dx_add, const float* relu_y, int N,
+                            int C, int Hx, int Wx, int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw,
+                            int groups, int P, int Q) {
+  TT_REQUIRE(sh == 1 && sw == 1, "tt_conv2d_dgrad_acc_f32: stride %d x %d, only 1 x 1 is supported", sh, sw);
+  TT_REQUIRE_ALIGNED("tt_conv2d_dgrad_acc_f32", dx_add, relu_y);
+  const Epilogue epi{nullptr, nullptr, nullptr, nullptr, dx_add, relu_y, 0.f, 0, 0, 1};
+  return conv2d_dgrad_runs("tt_conv2d_dgrad_acc_f32", dy, w, nullptr, dx, N, C, Hx, Wx, K, R, S, sh, sw, ph, pw, dh, dw,
+                           groups, P, Q, &epi);
 }
 
 // Instrumentation (tests, host-only): images per run for a batch of N images of `image_a` and

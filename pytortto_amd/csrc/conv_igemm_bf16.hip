@@ -50,7 +50,7 @@ constexpr int line_units(int n) { return n + n / 16 + 2; }
 //   kQuads: the repacked copy wp[k/4][row][4] of the float32 kernels
 constexpr int kRows = 0, kCols = 1, kQuads = 2;
 
-template <int WM, int WN, int MT, int NT, bool GEMM, int AMODE>
+template <int WM, int WN, int MT, int NT, bool GEMM, int AMODE, bool EPI>
 __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, const int tilesM) {
   static_assert(WM * WN == 4, "four waves per block");
   constexpr int BM = WM * MT * 32, BN = WN * NT * 32;
@@ -58,7 +58,7 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
   constexpr int ALINE = line_units(BM), BLINE = line_units(BN);
   __shared__ uintx4 As[2][kK8][ALINE];
   __shared__ uintx4 Bs[2][kK8][BLINE];
-  __shared__ __align__(16) float epi_lds[3 * BM];
+  __shared__ __align__(16) float epi_lds[EPI ? 4 * BM : 4];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
   };
 
   const int chunks = p.Kred / kBK;
-  if (p.epi.on) epilogue_constants<BM>(p.epi, g * p.I, i0, p.I, tid, epi_lds);   // published by the barrier below
+  if constexpr (EPI) epilogue_constants<BM>(p, g * p.I, i0, tid, epi_lds);   // published by the barrier below
   fetch(0);
   stage(0);
   __syncthreads();
@@ -252,8 +252,8 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
     const uint32_t v = rem - u * p.divV.d;
     obase[y] = (uint32_t)((int)n * p.outStrideN + g * p.outStrideG + ((int)u * p.ou + p.ouh) * p.outRow + (int)v * p.ov + p.ovw);
   }
-  if (p.epi.on) {
-    store_through_epilogue<BM, MT, NT>(p, acc, obase, mok, g, i0, wm * MT * 32, h, epi_lds);
+  if constexpr (EPI) {
+    store_through_epilogue<BM, MT, NT>(p, acc, obase, mok, i0, wm * MT * 32, h, epi_lds);
     return;
   }
   if (p.bias == nullptr && (p.I & 7) == 0) {
@@ -309,16 +309,16 @@ __global__ __launch_bounds__(kThreads, 3) void igemm_bf16_first(const Igemm p, c
   }
 }
 
-template <int WM, int WN, int MT, int NT>
+template <int WM, int WN, int MT, int NT, bool EPI>
 void launch_shape(const Igemm& p, dim3 grid, int tilesM, hipStream_t st) {
   const bool gemm = p.mode == kModeGemm;
   const int amode = p.wTransStride > 0 ? kCols : (p.wRowStride > 0 ? kRows : kQuads);
-  if (gemm && amode == kRows) igemm_bf16_first<WM, WN, MT, NT, true, kRows><<<grid, kThreads, 0, st>>>(p, tilesM);
-  else if (gemm && amode == kCols) igemm_bf16_first<WM, WN, MT, NT, true, kCols><<<grid, kThreads, 0, st>>>(p, tilesM);
-  else if (gemm) igemm_bf16_first<WM, WN, MT, NT, true, kQuads><<<grid, kThreads, 0, st>>>(p, tilesM);
-  else if (amode == kRows) igemm_bf16_first<WM, WN, MT, NT, false, kRows><<<grid, kThreads, 0, st>>>(p, tilesM);
-  else if (amode == kCols) igemm_bf16_first<WM, WN, MT, NT, false, kCols><<<grid, kThreads, 0, st>>>(p, tilesM);
-  else igemm_bf16_first<WM, WN, MT, NT, false, kQuads><<<grid, kThreads, 0, st>>>(p, tilesM);
+  if (gemm && amode == kRows) igemm_bf16_first<WM, WN, MT, NT, true, kRows, EPI><<<grid, kThreads, 0, st>>>(p, tilesM);
+  else if (gemm && amode == kCols) igemm_bf16_first<WM, WN, MT, NT, true, kCols, EPI><<<grid, kThreads, 0, st>>>(p, tilesM);
+  else if (gemm) igemm_bf16_first<WM, WN, MT, NT, true, kQuads, EPI><<<grid, kThreads, 0, st>>>(p, tilesM);
+  else if (amode == kRows) igemm_bf16_first<WM, WN, MT, NT, false, kRows, EPI><<<grid, kThreads, 0, st>>>(p, tilesM);
+  else if (amode == kCols) igemm_bf16_first<WM, WN, MT, NT, false, kCols, EPI><<<grid, kThreads, 0, st>>>(p, tilesM);
+  else igemm_bf16_first<WM, WN, MT, NT, false, kQuads, EPI><<<grid, kThreads, 0, st>>>(p, tilesM);
 }
 
 }  // namespace
@@ -340,8 +340,14 @@ void bf16_first_launch(const Igemm& p, int groups, int bm, hipStream_t st) {
   const int tilesM = (p.M + 127) / 128;
   const int tilesI = p.Ipad / bm;
   const dim3 grid((unsigned)(tilesI * tilesM), (unsigned)groups);
-  if (bm == 128) launch_shape<2, 2, 2, 2>(p, grid, tilesM, st);
-  else launch_shape<1, 4, 2, 1>(p, grid, tilesM, st);
+  if (p.epi.on) {
+    if (bm == 128) launch_shape<2, 2, 2, 2, true>(p, grid, tilesM, st);
+    else launch_shape<1, 4, 2, 1, true>(p, grid, tilesM, st);
+  } else if (bm == 128) {
+    launch_shape<2, 2, 2, 2, false>(p, grid, tilesM, st);
+  } else {
+    launch_shape<1, 4, 2, 1, false>(p, grid, tilesM, st);
+  }
 }
 
 }  // namespace ttc

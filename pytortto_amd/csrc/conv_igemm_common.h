@@ -25,15 +25,21 @@ typedef const intx2 __attribute__((address_space(4))) * ConstKTab;   // constant
 
 // What a launch does to a value between its accumulator and memory, beside the bias:
 //   v = acc + bias;  v = (v - mean) * (gamma / sd) + beta  (norm);  v = v + res[same element];
-//   v = maximum(v, 0), NaN kept  (relu)
-// -- the evaluation-mode BatchNorm, residual add and ReLU behind a convolution, in the order and with
-// the roundings of the kernels they stand in for.  `on` == 0: none of it.  Bound by memory: the three
+//   v = maximum(v, 0), NaN kept  (relu);  v = v * (mask[same element] > 0)
+// -- forward, the evaluation-mode BatchNorm, residual add and ReLU behind a convolution; backward, the
+// gradient that has already arrived for x added to this one (res) and the backward of the ReLU that
+// made x (mask) -- in the order and with the roundings of the kernels they stand in for.  `on` == 0:
+// none of it.  Bound by memory: the three
 // separate launches read and wrote y up to seven times over (a ResNet-50 evaluation pass at batch 64
-// in bf16 arithmetic spent half its time in them: 5.50 ms, 3.48 ms with this; 184 launches become 60,
-// which at batch 2 takes 3.37 ms to 2.66).
+// in bf16 arithmetic spent half its time in them: 5.50 ms, 3.37 ms with this; 184 launches become 60,
+// which at batch 2 takes 3.37 ms to 2.66).  Backward, the accumulation and the mask behind a residual
+// block's input gradient were seven tensor passes and are three: with the residual add and the masks of
+// batchnorm.hip, a ResNet-50 training step at batch 64 takes 20.53 ms for 21.97, at batch 32 in bf16
+// arithmetic 9.64 for 10.27.
 struct Epilogue {
   const float *mean, *var, *gamma, *beta;   // [G*I] each; gamma / beta may be null
   const float* res;                         // laid out as `out`, or null
+  const float* mask;                        // likewise
   float eps;
   int norm, relu, on;
 };
@@ -106,23 +112,30 @@ struct IgemmMulti {
   int n;
 };
 
+// stream-K flags: one word per block.  A wait that runs out (about four seconds of polling: a block
+// that was never scheduled, i.e. a grid that does not fit the device at two blocks per CU next to
+// foreign work) is reported through a word in pinned host memory, which the host reads after its
+// next stream synchronisation without any device operation.
+constexpr int kSkFlagWords = 4096, kSkSpinLimit = 1 << 22;
+
 constexpr int kModeCompare = 0, kModeGemm = 1, kModeTapMask = 2, kModeTapMask64 = 3;
 constexpr int kSrdFlags = 0x00020000;        // raw buffer, 32-bit data format
 constexpr int kSrdRecords = 0x7fffffff;      // offsets with bit 31 set are out of range and read 0
 
 __device__ __forceinline__ float as_float(unsigned v) { return __builtin_bit_cast(float, v); }
 
-// Per-row constants of the epilogue's normalisation for the BM rows of a tile, {mean, gamma / sd, beta}
-// each an array of BM in LDS: one thread computes a row's once (a square root and a division) while
-// the tile's first loads are in flight, instead of every lane for each of its rows at the end.  The
-// caller's next barrier publishes them.  Without a normalisation the constants leave a value as it
-// is: (v - 0) * 1 + -0.
+// Per-row constants of the epilogue for the BM rows of a tile, {mean, gamma / sd, beta, bias} each an
+// array of BM in LDS: one thread computes a row's once (a square root and a division) while the tile's
+// first loads are in flight, instead of every lane for each of its rows at the end.  The caller's next
+// barrier publishes them.  Without a bias or a normalisation the constants leave a value as it is:
+// v + -0, (v - 0) * 1 + -0.
 template <int BM>
-__device__ __forceinline__ void epilogue_constants(const Epilogue& e, int first_channel, int i0, int I, int tid, float* lds) {
+__device__ __forceinline__ void epilogue_constants(const Igemm& p, int first_channel, int i0, int tid, float* lds) {
+  const Epilogue& e = p.epi;
   if (tid < BM) {
+    const int c = first_channel + min(i0 + tid, p.I - 1);
     float m = 0.f, k1 = 1.f, k0 = -0.f;
     if (e.norm) {
-      const int c = first_channel + min(i0 + tid, I - 1);
       const float sd = __fsqrt_rn(__fadd_rn(e.var[c], e.eps));
       m = e.mean[c];
       k1 = __fdiv_rn(e.gamma ? e.gamma[c] : 1.0f, sd);
@@ -131,39 +144,40 @@ __device__ __forceinline__ void epilogue_constants(const Epilogue& e, int first_
     lds[tid] = m;
     lds[BM + tid] = k1;
     lds[2 * BM + tid] = k0;
+    lds[3 * BM + tid] = p.bias ? p.bias[c] : -0.f;
   }
 }
 
 // Stores one wave's MT x NT accumulators through the epilogue.  `row0` is the wave's first row inside
 // the tile; accumulator register r of a 32x32 tile holds row 8*(r/4) + 4*h + r%4.  A 32-row strip's
-// residual values are all fetched before its first store (loads and stores share one in-order counter).
+// residual and mask values are all fetched before its first store (loads and stores share one in-order
+// counter).  Rows and pixels past the end re-read the last row / pixel 0 and are never stored.
 template <int BM, int MT, int NT>
 __device__ __forceinline__ void store_through_epilogue(const Igemm& p, const floatx16 (&acc)[MT][NT], const uint32_t (&obase)[NT],
-                                                       const bool (&mok)[NT], int g, int i0, int row0, int h, const float* lds) {
+                                                       const bool (&mok)[NT], int i0, int row0, int h, const float* lds) {
   const float floor_ = p.epi.relu ? 0.f : -__builtin_huge_valf();
 #pragma unroll
   for (int x = 0; x < MT; ++x) {
     const int r0 = row0 + 32 * x + 4 * h;   // + 8*q + j inside the tile
-    float rs[NT][16], bz[16];
+    float rs[NT][16], ms[NT][16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      bz[r] = 0.f;
 #pragma unroll
-      for (int y = 0; y < NT; ++y) rs[y][r] = -0.f;   // v + -0 is v
+      for (int y = 0; y < NT; ++y) {
+        rs[y][r] = -0.f;   // v + -0 is v
+        ms[y][r] = 1.f;
+      }
     }
-    if (p.bias) {
+    auto fetch = [&](const float* __restrict__ from, float (&to)[NT][16]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) bz[r] = p.bias[g * p.I + min(i0 + r0 + 8 * (r >> 2) + (r & 3), p.I - 1)];
-    }
-    if (p.epi.res) {
+      for (int r = 0; r < 16; ++r) {
+        const uint32_t ioff = (uint32_t)(min(i0 + r0 + 8 * (r >> 2) + (r & 3), p.I - 1) * p.outStrideI);
 #pragma unroll
-      for (int y = 0; y < NT; ++y)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int i = i0 + r0 + 8 * (r >> 2) + (r & 3);
-          if (mok[y] && i < p.I) rs[y][r] = p.epi.res[obase[y] + (uint32_t)(i * p.outStrideI)];
-        }
-    }
+        for (int y = 0; y < NT; ++y) to[y][r] = from[obase[y] + ioff];
+      }
+    };
+    if (p.epi.res) fetch(p.epi.res, rs);
+    if (p.epi.mask) fetch(p.epi.mask, ms);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
     __builtin_amdgcn_sched_barrier(0);
@@ -172,6 +186,7 @@ __device__ __forceinline__ void store_through_epilogue(const Igemm& p, const flo
       const floatx4 m4 = *reinterpret_cast<const floatx4*>(lds + r0 + 8 * q);
       const floatx4 s4 = *reinterpret_cast<const floatx4*>(lds + BM + r0 + 8 * q);
       const floatx4 b4 = *reinterpret_cast<const floatx4*>(lds + 2 * BM + r0 + 8 * q);
+      const floatx4 z4 = *reinterpret_cast<const floatx4*>(lds + 3 * BM + r0 + 8 * q);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int i = i0 + r0 + 8 * q + j;
@@ -179,10 +194,10 @@ __device__ __forceinline__ void store_through_epilogue(const Igemm& p, const flo
           const uint32_t ioff = (uint32_t)(i * p.outStrideI);
 #pragma unroll
           for (int y = 0; y < NT; ++y) {
-            float v = acc[x][y][4 * q + j];
-            if (p.bias) v += bz[4 * q + j];
+            float v = acc[x][y][4 * q + j] + z4[j];
             v = fmaf(v - m4[j], s4[j], b4[j]) + rs[y][4 * q + j];
             v = (v > floor_ || v != v) ? v : floor_;
+            v *= ms[y][4 * q + j] > 0.f ? 1.f : 0.f;
             if (mok[y]) p.out[obase[y] + ioff] = v;
           }
         }
@@ -197,14 +212,21 @@ bool bf16_first_supported(const Igemm& p, int groups, int bm);
 void bf16_first_launch(const Igemm& p, int groups, int bm, hipStream_t st);
 
 
-// Float32 arithmetic in three bf16 terms (conv_igemm_x3.hip: the kernel body of conv_igemm_kernel.h
-// instantiated on six v_mfma_f32_32x32x16_bf16 per product step).  `bm` x `bn` is the tile the caller
-// planned; `sk_blocks` > 0 asks for the persistent (stream-K) grid, which is launched only if the
-// device holds that many blocks at once (`forced_occupancy` >= 0 replaces what the device says:
-// tests); returns whether the persistent grid was launched.
-bool x3_launch(const Igemm& p, int groups, int sk_blocks, int bm, int bn, int forced_occupancy, hipStream_t st);
-void x3_launch_multi(const IgemmMulti& m, int groups, int bm, int bn, hipStream_t st);
-// resident blocks per compute unit of its stream-K kernels, the smallest over every instantiation
-int x3_min_resident_blocks();
+// The kernel body of conv_igemm_kernel.h in one arithmetic (conv_igemm_launch.h).  launch: `bm` x `bn` is
+// the tile the caller planned; `sk_blocks` > 0 asks for the persistent (stream-K) grid, which is launched
+// only if the device holds that many blocks at once (`forced_occupancy` >= 0 replaces what the device
+// says: tests); returns whether it was.  min_resident_blocks: resident blocks per compute unit of its
+// stream-K kernels, the smallest over every instantiation.
+struct IgemmUnit {
+  bool (*launch)(const Igemm& p, int groups, int sk_blocks, int bm, int bn, int forced_occupancy, hipStream_t st);
+  void (*launch_multi)(const IgemmMulti& m, int groups, int bm, int bn, hipStream_t st);
+  int (*min_resident_blocks)();
+};
+const IgemmUnit& igemm_f32_unit();
+const IgemmUnit& igemm_bf16_unit();
+const IgemmUnit& igemm_bf16x3_unit();
+const IgemmUnit& igemm_epi_f32_unit();   // for launches with Igemm::epi.on
+const IgemmUnit& igemm_epi_bf16_unit();
+const IgemmUnit& igemm_epi_bf16x3_unit();
 
 }  // namespace ttc

@@ -1,6 +1,6 @@
 // The implicit-GEMM convolution kernel body for gfx950, shared by the translation units that
-// instantiate it: conv_igemm.hip (float32 and bf16 matrix instructions) and conv_igemm_x3.hip (float32
-// arithmetic in three bf16 terms).  Everything here is device code in an unnamed namespace: each unit
+// instantiate it through conv_igemm_launch.h: conv_igemm_f32.hip, conv_igemm_rounded.hip and
+// conv_igemm_x3.hip.  Everything here is device code in an unnamed namespace: each unit
 // gets its own copy.
 #pragma once
 #include <type_traits>
@@ -36,11 +36,6 @@ __device__ __forceinline__ void wait_loads() {
 // costs.  Ordering is by completion: the writer waits for its stores (vmcnt) before the flag goes
 // up, the reader issues its loads after it has seen the flag.
 constexpr int kSystemScope = 1 | 16;   // sc0, sc1
-// stream-K flags: one word per block.  A wait that runs out (about four seconds of polling: a block
-// that was never scheduled, i.e. a grid that does not fit the device at two blocks per CU next to
-// foreign work) is reported through a word in pinned host memory, which the host reads after its
-// next stream synchronisation without any device operation.
-constexpr int kSkFlagWords = 4096, kSkSpinLimit = 1 << 22;
 __device__ __forceinline__ void store_coherent(__amdgpu_buffer_rsrc_t rsrc, int byte_off, floatx4 v) {
   typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uintx4, v), rsrc, byte_off, 0, kSystemScope);
@@ -78,7 +73,10 @@ __device__ __forceinline__ void three_terms(const floatx4 lo, const floatx4 hi, 
 // be one of several that share a grid, see igemm_multi_f32).
 // BF: 0 = float32 matrix instructions; 1 = operands rounded to bfloat16; 3 = float32 arithmetic on the
 // bf16 matrix instructions (three bf16 terms per operand element, six products per step).
-template <int WM, int WN, int MT, int NT, bool SK, int MODE, bool AT, int BF>
+// EPI: the launch applies Igemm::epi to what it stores.  A parameter because of its registers: in the
+// kernels of launches without it, they took 64 x 64 tiles from seven resident blocks per compute unit to
+// four and 128 x 128 ones from three to two (a grouped layer of short launches: 126 us, 144 with it).
+template <int WM, int WN, int MT, int NT, bool SK, int MODE, bool AT, int BF, bool EPI>
 __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   static_assert(WM * WN == 4, "four waves per block");
   constexpr bool GEMM = MODE == kModeGemm, BUF = MODE != kModeCompare;
@@ -89,7 +87,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   static_assert(B_ITEMS >= 1 && kThreads % BM == 0 && kThreads % BN == 0, "tile shape");
   __shared__ floatx4 As[2][kBKQ][BM];
   __shared__ floatx4 Bs[2][kBKQ][BN];
-  __shared__ __align__(16) float epi_lds[3 * BM];
+  __shared__ __align__(16) float epi_lds[EPI ? 4 * BM : 4];
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -465,8 +463,8 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
       obase[y] = (uint32_t)((int)n * p.outStrideN + g * p.outStrideG + ((int)u * p.ou + p.ouh) * p.outRow +
                             (int)v * p.ov + p.ovw);
     }
-    if (p.epi.on) {
-      store_through_epilogue<BM, MT, NT>(p, acc, obase, mok, g, i0, wm * MT * 32, h, epi_lds);
+    if constexpr (EPI) {
+      store_through_epilogue<BM, MT, NT>(p, acc, obase, mok, i0, wm * MT * 32, h, epi_lds);
       return;
     }
     if (p.rowtab == nullptr && p.bias == nullptr && (p.I & 7) == 0) {
@@ -598,9 +596,10 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   // (published by the barriers of the reduction that follows; the epilogue of the tile before has
   // ended with one)
   auto epi_constants = [&]() __attribute__((always_inline)) {
-    if (!p.epi.on) return;
-    epilogue_constants<BM>(p.epi, g * p.I, i0, p.I, tid, epi_lds);
-    if (chunks == 0) __syncthreads();
+    if constexpr (EPI) {
+      epilogue_constants<BM>(p, g * p.I, i0, tid, epi_lds);
+      if (chunks == 0) __syncthreads();
+    }
   };
   if constexpr (!SK) {
     set_tile(xcd_remap(block_x, p.tiles));

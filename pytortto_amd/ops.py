@@ -131,18 +131,22 @@ def conv2d_fwd_deferred(x, w, bias, stride, padding, dilation, groups):
     return op.out
 
 
-def conv2d_dgrad(dy, w, bias, out_hw, stride, padding, dilation, groups):
+def conv2d_dgrad(dy, w, bias, out_hw, stride, padding, dilation, groups, add=None, relu_y=None):
     """dx = sum_k,r,s dy * w  for a conv weight ``w[K, C/g, R, S]`` (autograd/grad_nn.py:659-682).
     ``out_hw`` is the spatial size of the result; ``bias`` (length C) is added when given
-    (transposed-convolution forward, grad_nn.py:755-757)."""
-    _f32(dy, w, bias)
+    (transposed-convolution forward, grad_nn.py:755-757).  At stride 1 without a bias, ``add`` (what
+    has already arrived for x) is added to dx, and the sum multiplied by ``relu_y > 0``."""
+    _f32(dy, w, bias, add, relu_y)
     n, k, p, q = dy.shape
     _, cg, r, s = w.shape
     c = cg * groups
     hx, wx = out_hw
     dx = hiparray.empty((n, c, hx, wx))
-    _hip.call('tt_conv2d_dgrad_f32', dy.ptr, w.ptr, _ptr(bias), dx.ptr, n, c, hx, wx, k, r, s,
-              stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1], groups, p, q)
+    dims = (n, c, hx, wx, k, r, s, stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1], groups, p, q)
+    if add is None and relu_y is None:
+        _hip.call('tt_conv2d_dgrad_f32', dy.ptr, w.ptr, _ptr(bias), dx.ptr, *dims)
+    else:
+        _hip.call('tt_conv2d_dgrad_acc_f32', dy.ptr, w.ptr, dx.ptr, _ptr(add), _ptr(relu_y), *dims)
     return dx
 
 
@@ -196,57 +200,70 @@ def bn_fwd_train(x, gamma, beta, running_mean, running_var, momentum, eps, num_b
 
 
 class DeferredBatchNorm:
-    """A training forward that has not been launched yet (see ``_hip.defer``).  ``run()`` launches
-    it as it is; ``run_with_relu(out)`` launches the variant whose output is ``maximum(y, 0)`` --
-    into ``out``, or into the normalisation's own array when ``out`` is None (an in-place ReLU).
-    When the ReLU's result went elsewhere, the normalised values themselves were never stored:
-    their array recomputes them (same kernels, same bits, scratch statistics, no running update)
-    should anybody ask for it, and at the latest just before ``x``, ``gamma`` or ``beta`` is written in
-    place: what is read back is always what the reference stored when the operation ran."""
+    """A training forward that has not been launched yet (see ``_hip.defer``).  What follows may join
+    the launch: a residual added to the normalised values (``absorb_add``) and a ReLU
+    (``run_with_relu(out)``: the output is ``maximum(., 0)``, in ``out``, or in the operation's own array
+    when ``out`` is None, an in-place ReLU); ``run()`` launches what has joined so far.
+    The values in between are then never stored: their arrays recompute them (same kernels, same bits,
+    scratch statistics, no running update) should anybody ask, and at the latest just before an operand
+    is written in place: what is read back is always what the reference stored when the operation ran."""
 
     def __init__(self, x, gamma, beta, running_mean, running_var, momentum, eps, num_batches_tracked):
         self.x, self.gamma, self.beta = x, gamma, beta
         self.momentum, self.eps = float(momentum if momentum is not None else 0.0), float(eps)
         self.nbt = num_batches_tracked
         self.dims = n, c, hw = _nchw(x)
-        self.y = hiparray.lazy(x.shape)
+        self.residual = None
+        self.out = self.y = hiparray.lazy(x.shape)
         self.stats = [hiparray.empty((c,)) for _ in range(3)]        # mean, var + eps, sd
         self.track = running_mean is not None and running_var is not None
         self.rm_in, self.rv_in = (running_mean, running_var) if self.track else (None, None)
         self.new_rm = hiparray.empty((c,)) if self.track else None
         self.new_rv = hiparray.empty((c,)) if self.track else None
 
-    def _launch(self, entry, out):
+    def _launch(self, out, relu, coef=None):
         mean, var_eps, sd = self.stats
-        _hip.call(entry, self.x.ptr, _ptr(self.gamma), _ptr(self.beta), out.ptr, mean.ptr, var_eps.ptr, sd.ptr,
-                  _ptr(self.rm_in), _ptr(self.rv_in), _ptr(self.new_rm), _ptr(self.new_rv), _ptr(self.nbt),
-                  self.momentum, self.eps, *self.dims)
+        _hip.call('tt_bn_act_fwd_train_f32', self.x.ptr, _ptr(self.gamma), _ptr(self.beta), _ptr(self.residual), out.ptr,
+                  mean.ptr, var_eps.ptr, sd.ptr, _ptr(coef), _ptr(self.rm_in), _ptr(self.rv_in), _ptr(self.new_rm),
+                  _ptr(self.new_rv), _ptr(self.nbt), self.momentum, self.eps, int(relu), *self.dims)
 
-    def run(self):
-        self._launch('tt_bn_fwd_train_f32', self.y)
-
-    def run_with_relu(self, out=None):
-        if out is None:
-            self._launch('tt_bn_relu_fwd_train_f32', self.y)
-            return self.y
-        self._launch('tt_bn_relu_fwd_train_f32', out)
-        x, gamma, beta, eps, dims = self.x, self.gamma, self.beta, self.eps, self.dims
+    def _on_demand(self):
+        """The output so far is about to be absorbed: leave it to be recomputed on demand."""
+        x, gamma, beta, residual, eps, dims = self.x, self.gamma, self.beta, self.residual, self.eps, self.dims
 
         def recompute(buf):
             scratch = [hiparray.empty((dims[1],)) for _ in range(3)]
-            _hip.call('tt_bn_fwd_train_f32', x.ptr, _ptr(gamma), _ptr(beta), buf.ptr, scratch[0].ptr, scratch[1].ptr,
-                      scratch[2].ptr, None, None, None, None, None, 0.0, eps, *dims)
-        # x, gamma and beta as they are now: should one of them be written in place later (an
-        # optimiser step, ``+=``), the normalised values are produced first
-        self.y._buf.fill_on_demand(recompute, (x, gamma, beta))
+            _hip.call('tt_bn_act_fwd_train_f32', x.ptr, _ptr(gamma), _ptr(beta), _ptr(residual), buf.ptr, scratch[0].ptr,
+                      scratch[1].ptr, scratch[2].ptr, None, None, None, None, None, None, 0.0, eps, 0, *dims)
+        # the operands as they are now: should one of them be written in place later (an optimiser step,
+        # ``+=``), the values are produced first
+        self.out._buf.fill_on_demand(recompute, (x, gamma, beta, residual))
+
+    def run(self):
+        self._launch(self.out, False)
+
+    def absorb_add(self, residual):
+        _f32(residual)
+        self._on_demand()
+        self.residual = residual
+        self.out = hiparray.lazy(self.out.shape)
+        _hip.defer(self)
+        return self.out
+
+    def run_with_relu(self, out=None, keep_coef=False):
+        """With ``keep_coef`` the channels' two constants stay in ``coef``, for the backward to apply the
+        ReLU's mask from x alone (only without a residual in between)."""
+        self.coef = hiparray.empty((2 * self.dims[1],)) if keep_coef and self.residual is None else None
+        if out is None:
+            out = self.out
+            self._launch(out, True, self.coef)
+        else:
+            self._launch(out, True, self.coef)
+            self._on_demand()
         return out
 
-    @property
-    def out(self):
-        return self.y
-
     def poison(self, exc):
-        poison([self.y, *self.stats, self.new_rm, self.new_rv], exc)
+        poison([self.y, self.out, *self.stats, self.new_rm, self.new_rv], exc)
 
 
 def bn_fwd_train_deferred(x, gamma, beta, running_mean, running_var, momentum, eps, num_batches_tracked=None):
@@ -259,11 +276,12 @@ def bn_fwd_train_deferred(x, gamma, beta, running_mean, running_var, momentum, e
 
 
 class DeferredReluBackward:
-    """``dy * (y > 0)`` not launched yet: a BatchNorm backward that comes next forms the product
-    itself while it reads ``dy`` (``bn_relu_bwd``); anything else finds it computed."""
+    """``dy * (y > 0)`` not launched yet: the backward of the BatchNorm the ReLU was fused with forms the
+    product itself while it reads ``dy`` (``bn_bwd`` with ``coef``, the constants that forward kept);
+    anything else finds it computed."""
 
-    def __init__(self, dy, y):
-        self.dy, self.y = dy, y
+    def __init__(self, dy, y, coef):
+        self.dy, self.y, self.coef = dy, y, coef
         self.out = hiparray.lazy(y.shape)
 
     def run(self):
@@ -273,23 +291,11 @@ class DeferredReluBackward:
         poison([self.out], exc)
 
 
-def relu_bwd_deferred(dy, y):
+def relu_bwd_deferred(dy, y, coef):
     _f32(dy, y)
-    op = DeferredReluBackward(dy, y)
+    op = DeferredReluBackward(dy, y, coef)
     _hip.defer(op)
     return op.out
-
-
-def bn_relu_bwd(x, dy, relu_y, gamma, mean, var_eps, sd, need=(True, True, True)):
-    """``bn_bwd`` on the gradient ``dy * (relu_y > 0)``, masked as it is read."""
-    _f32(x, dy, relu_y, gamma)
-    n, c, hw = _nchw(x)
-    dx = hiparray.empty(x.shape) if need[0] else None
-    dgamma = hiparray.empty((c,)) if need[1] else None
-    dbeta = hiparray.empty((c,)) if need[2] else None
-    _hip.call('tt_bn_relu_bwd_f32', x.ptr, dy.ptr, relu_y.ptr, _ptr(gamma), mean.ptr, var_eps.ptr, sd.ptr,
-              _ptr(dx), _ptr(dgamma), _ptr(dbeta), n, c, hw)
-    return dx, dgamma, dbeta
 
 
 class DeferredBatchNormEval:
@@ -335,15 +341,17 @@ def bn_fwd_eval(x, gamma, beta, mean_in, var_in, eps, deferred=False):
     return (op.out, *op.stats)
 
 
-def bn_bwd(x, dy, gamma, mean, var_eps, sd, need=(True, True, True)):
-    """Backward (autograd/grad_nn.py:966-989): returns ``(dx, dgamma, dbeta)``."""
-    _f32(x, dy, gamma)
+def bn_bwd(x, dy, gamma, mean, var_eps, sd, need=(True, True, True), coef=None, add=None):
+    """Backward (autograd/grad_nn.py:966-989): returns ``(dx, dgamma, dbeta)``.  With ``coef`` the gradient
+    is ``dy * (bn(x) > 0)``, masked as it is read (a fused ReLU's backward); ``add`` (what has already
+    arrived for x) is added to dx."""
+    _f32(x, dy, gamma, add)
     n, c, hw = _nchw(x)
     dx = hiparray.empty(x.shape) if need[0] else None
     dgamma = hiparray.empty((c,)) if need[1] else None
     dbeta = hiparray.empty((c,)) if need[2] else None
-    _hip.call('tt_bn_bwd_f32', x.ptr, dy.ptr, _ptr(gamma), mean.ptr, var_eps.ptr, sd.ptr,
-              _ptr(dx), _ptr(dgamma), _ptr(dbeta), n, c, hw)
+    _hip.call('tt_bn_act_bwd_f32', x.ptr, dy.ptr, _ptr(coef), _ptr(gamma), mean.ptr, var_eps.ptr, sd.ptr,
+              _ptr(dx), _ptr(add), _ptr(dgamma), _ptr(dbeta), n, c, hw)
     return dx, dgamma, dbeta
 
 
