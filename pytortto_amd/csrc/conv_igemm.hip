@@ -305,6 +305,9 @@ int g_last_launch[8] = {};
 bool g_bf16_first = true;
 bool g_bf16_first_always = false;   // tests: also where the tile-count rule would keep the other kernels
 
+// Whether the channel-last kernels (conv_hwc.hip) are to be asked; tests switch them with the bf16-first ones.
+bool hwc_math(int groups) { return groups == 1 && bf16_math() && g_bf16_first; }
+
 int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_partial) {
   tt::ProfScope prof(prof_id);
   p.tilesI = p.Ipad / t.bm;
@@ -683,6 +686,16 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
              H + 2 * ph, W + 2 * pw);
   if (check_common(fn, N, C, H, W, K, R, S, sh, sw, ph, pw, dh, dw, groups, P, Q)) return -1;
   const int Cg = C / groups, Kg = K / groups;
+  if (hwc_math(groups) && !check_only) {
+    const HwcConv hc{N, C, H, W, K, P, Q, R, S, sh, sw, ph, pw, dh, dw, false};
+    if (hwc_supported(hc, g_bf16_first_always)) {
+      if (size_only) {
+        *size_only = hwc_workspace(hc);
+        return 0;
+      }
+      return hwc_conv(hc, x, w, bias, y, epi, TT_PROF_CONV_IGEMM_FWD, g_last_launch);
+    }
+  }
   const int Kred = Cg * R * S;
   const int M = N * P * Q;
   const int KQ = ceil_div(Kred, 4 * kBKQ) * kBKQ;
@@ -754,6 +767,17 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
     return conv2d_dgrad(dy, w, nullptr, dx, N, C * R * S, 1, 1, K, 1, 1, 1, 1, 0, 0, 1, 1, 1, 1, 1, size_only,
                         check_only, epi);
   const int Cg = C / groups, Kg = K / groups;
+  if (hwc_math(groups) && !check_only && sh == 1 && sw == 1) {
+    // dx[h] reads dy[h + ph - r*dh]: a convolution of dy with the taps in reverse order
+    const HwcConv hc{N, K, P, Q, C, Hx, Wx, R, S, 1, 1, (R - 1) * dh - ph, (S - 1) * dw - pw, dh, dw, true};
+    if (hwc_supported(hc, g_bf16_first_always)) {
+      if (size_only) {
+        *size_only = hwc_workspace(hc);
+        return 0;
+      }
+      return hwc_conv(hc, dy, w, bias, dx, epi, TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
+    }
+  }
   const int gh = gcd(sh, dh), gw = gcd(sw, dw);
   const int rstep = sh / gh, sstep = sw / gw;   // valid taps of a class: r0, r0+rstep, ...
   const int eh = dh / gh, ew = dw / gw;          // dy row/column step per tap

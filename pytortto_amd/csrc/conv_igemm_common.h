@@ -212,6 +212,20 @@ bool bf16_first_supported(const Igemm& p, int groups, int bm);
 void bf16_first_launch(const Igemm& p, int groups, int bm, hipStream_t st);
 
 
+// The channel-last kernels (conv_hwc.hip): one group, operands rounded to bfloat16.  x is [N][C][H][W], the result [N][I][P][Q]; output pixel (u, v) reads
+// input rows u*sh - ph + r*dh (ph, pw may be negative).  dgrad: w is [C][I][R][S] with its taps reversed
+// instead of [I][C][R][S].
+struct HwcConv {
+  int N, C, H, W, I, P, Q, R, S, sh, sw, ph, pw, dh, dw;
+  bool dgrad;
+};
+// Whether they take it; `always`: also where the size rule prefers the other kernels (small test shapes).
+bool hwc_supported(const HwcConv& c, bool always);
+size_t hwc_workspace(const HwcConv& c);
+// Enqueues the call; `plan8` as tt_conv2d_last_launch reports it.
+int hwc_conv(const HwcConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi, int prof_id,
+             int* plan8);
+
 // The kernel body of conv_igemm_kernel.h in one arithmetic (conv_igemm_launch.h).  launch: `bm` x `bn` is
 // the tile the caller planned; `sk_blocks` > 0 asks for the persistent (stream-K) grid, which is launched
 // only if the device holds that many blocks at once (`forced_occupancy` >= 0 replaces what the device

@@ -1,0 +1,104 @@
+"""The channel-last convolution kernels (bf16 arithmetic) at the sizes where they can go wrong: channels and rows that fill no chunk or tile, images smaller than a tile, split reductions
+of even and ragged share, reversed taps with more padding than the kernel reaches, 2 and 31 taps."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from pytortto_amd import _hip, ops
+from pytortto_amd.xparray import hiparray
+from tests.test_gpu_conv_bf16 import _forward_and_input_gradient
+
+pytestmark = pytest.mark.gpu
+
+# n, c, h, w, k, r, s, stride, pad, dilation, groups
+CASES = [(1, 3, 6, 5, 5, 3, 3, (1, 1), (1, 1), (1, 1), 1),        # one chunk mostly padding, one ragged tile
+         (2, 64, 9, 7, 64, 3, 3, (1, 1), (1, 1), (1, 1), 1),      # whole chunks, 64-row tiles
+         (2, 65, 9, 7, 65, 3, 3, (1, 1), (1, 1), (1, 1), 1),      # one past them
+         (2, 160, 9, 7, 190, 3, 3, (1, 1), (1, 1), (1, 1), 1),    # 64-row tiles where 128 pad more
+         (3, 130, 7, 7, 40, 1, 1, (1, 1), (0, 0), (1, 1), 1),     # one tap, pixels no multiple of four
+         (9, 16, 4, 4, 130, 3, 3, (1, 1), (1, 1), (1, 1), 1),     # eight images in a tile
+         (3, 512, 5, 5, 96, 3, 3, (1, 1), (1, 1), (1, 1), 1),     # split reduction, ragged last share
+         (2, 256, 8, 8, 256, 3, 3, (2, 2), (1, 1), (1, 1), 1),    # stride 2 (forward), split
+         (2, 40, 13, 11, 72, 1, 2, (1, 1), (0, 1), (1, 1), 1),    # two taps
+         (1, 33, 40, 9, 31, 31, 1, (1, 1), (15, 0), (1, 1), 1),   # 31 taps
+         (2, 48, 12, 10, 80, 5, 3, (1, 1), (4, 2), (2, 1), 1),    # dilation
+         (2, 32, 6, 6, 32, 2, 2, (1, 1), (1, 1), (1, 1), 1),      # more rows out than in
+         (2, 32, 8, 8, 48, 3, 3, (1, 3), (0, 0), (1, 1), 1),      # unequal strides
+         (5, 128, 16, 16, 128, 3, 3, (1, 1), (1, 1), (1, 1), 1)]
+
+
+def _plan():
+    plan = (ctypes.c_int * 8)()
+    _hip.call('tt_conv2d_last_launch', plan)
+    return plan
+
+
+@pytest.fixture
+def math():
+    """Every launch the kernels support is sent to them, whatever its size."""
+    _hip.set_conv_math('bf16')
+    _hip.call('tt_conv2d_bf16_first_enable', 2)
+    try:
+        yield
+    finally:
+        _hip.call('tt_conv2d_bf16_first_enable', 1)
+        _hip.set_conv_math('f32')
+
+
+@pytest.mark.parametrize('case', CASES, ids=lambda c: '-'.join(map(str, c[:7])))
+def test_forward_and_input_gradient(case, math):
+    _forward_and_input_gradient(case)
+    n, c, h, w, k, r, s, st, pd, dl, g = case
+    rng = np.random.default_rng(2)
+    x, wt = (hiparray(rng.standard_normal(v).astype(np.float32)) for v in ((n, c, h, w), (k, c, r, s)))
+    y = ops.conv2d_fwd(x, wt, None, st, pd, dl, g)
+    assert _plan()[4] == -1 and _plan()[7] >> 8 == 1
+    # the same product in the kernels that gather in place: another order of summation
+    dx = ops.conv2d_dgrad(y, wt, None, (h, w), st, pd, dl, g)
+    assert (_plan()[4] == -1) == (st == (1, 1))
+    _hip.call('tt_conv2d_bf16_first_enable', 0)
+    for got, other in ((y, ops.conv2d_fwd(x, wt, None, st, pd, dl, g)), (dx, ops.conv2d_dgrad(y, wt, None, (h, w), st, pd, dl, g))):
+        assert _plan()[4] != -1
+        np.testing.assert_allclose(got.get(), other.get(), rtol=1e-4, atol=1e-5 * float(np.abs(other.get()).max()))
+
+
+@pytest.mark.parametrize('split', [False, True])
+def test_values_next_to_the_image_are_not_touched(split, math):
+    """Non-finite values in the images before and after one: nothing of theirs reaches it, and its own reach
+    exactly the outputs whose window covers them."""
+    n, c, h, k = 3, 256 if split else 16, 6, 40
+    rng = np.random.default_rng(4)
+    x = rng.standard_normal((n, c, h, h)).astype(np.float32)
+    wt = hiparray(rng.standard_normal((k, c, 3, 3)).astype(np.float32))
+    clean = ops.conv2d_fwd(hiparray(x), wt, None, (1, 1), (1, 1), (1, 1), 1).get()
+    x[0], x[2] = np.nan, np.inf
+    x[1, 5, 0, 0] = np.nan
+    y = ops.conv2d_fwd(hiparray(x), wt, None, (1, 1), (1, 1), (1, 1), 1).get()
+    hit = np.zeros((h, h), bool)
+    hit[:2, :2] = True
+    assert np.isnan(y[1][:, hit]).all()
+    np.testing.assert_array_equal(y[1][:, ~hit], clean[1][:, ~hit])
+
+
+@pytest.mark.parametrize('dims,taken', [((8, 64, 14, 14, 64, 3, 3), False),        # little work
+                                        ((16, 64, 56, 56, 64, 3, 3), False),       # few channels, tiles enough
+                                        ((64, 128, 28, 28, 128, 3, 3), True),      # the same with more channels
+                                        ((16, 256, 14, 14, 256, 3, 3), True),      # few tiles, long reduction
+                                        ((16, 160, 45, 37, 192, 3, 3), False),     # padded channels
+                                        ((16, 2048, 7, 7, 512, 1, 1), True),       # 1x1 on 49 pixels
+                                        ((16, 512, 8, 8, 2048, 1, 1), False)])     # plain matrix product
+def test_size_rule_and_workspace(dims, taken, math):
+    """Which calls go there by default; the workspace query says what a call asks for."""
+    _hip.call('tt_conv2d_bf16_first_enable', 1)
+    n, c, h, w, k, r, s = dims
+    geometry = (1, 1, r // 2, s // 2, 1, 1, 1)
+    x, wt = hiparray.zeros((n, c, h, w)), hiparray.zeros((k, c, r, s))
+    ops.conv2d_fwd(x, wt, None, (1, 1), (r // 2, s // 2), (1, 1), 1)
+    nbytes = ctypes.c_size_t()
+    _hip.call('tt_workspace_size_conv2d_fwd_f32', ctypes.byref(nbytes), *dims, *geometry)
+    layouts = 2 * (n * c * h * w + k * c * r * s)
+    if taken:
+        assert _plan()[4] == -1 and _plan()[:2] == [128, 128] and nbytes.value >= layouts
+    else:
+        assert nbytes.value != layouts and nbytes.value > 0
