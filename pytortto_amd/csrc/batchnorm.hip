@@ -576,18 +576,38 @@ __global__ __launch_bounds__(kThreads) void bn_bwd_apply(BwdArgs a, Geometry g) 
 // in flight while others reduce or store (measured, 256 channels of 64 x 14 x 14 values: backward
 // 32 -> 15 us, forward 12.5 -> 10 us; 1024 such channels are 10 % slower that way and keep 256 threads).
 
-template <int EMAX, int BT, typename F>
+template <int EMAX, int BT, int FROM = 0, typename F>
 __device__ __forceinline__ void for_channel_elements(const Geometry& g, F&& f) {
   const int total = g.N * g.HW;
   const size_t image = (size_t)g.C * g.HW;
+  // A thread index the compiler cannot connect with the one of the pass before: it otherwise keeps the 64-bit
+  // offsets of all elements from the loads to the stores, two registers each, and half as many waves fit.
+  int t = (int)threadIdx.x;
+  asm volatile("" : "+v"(t));
 #pragma unroll
-  for (int k = 0; k < EMAX; ++k) {
-    const int e = (int)threadIdx.x + k * BT;
+  for (int k = FROM; k < EMAX; ++k) {
+    const int e = t + k * BT;
     if (e < total) {
       const uint32_t n = tt::fd_div((uint32_t)e, g.hwv_div);
       f(k, (size_t)n * image + ((uint32_t)e - n * (uint32_t)g.HW));
     }
   }
+}
+
+// The stores of a single-kernel pass, value(k) plus (kAdd) the addend's element: 16 addends are fetched
+// at a time, so that they take 16 registers next to the channel's values and not as many as those (256
+// threads x 64 values, 1024 channels of 32 x 14 x 14: 50 us with all of them fetched first and the offsets
+// kept, 29 now).
+template <int EMAX, int BT, bool kAdd, int FROM = 0, typename F>
+__device__ __forceinline__ void store_channel(const Geometry& g, const float* __restrict__ addend, float* __restrict__ out, F&& value) {
+  constexpr int kTo = FROM + 16 < EMAX ? FROM + 16 : EMAX;
+  float ad[16];
+  if constexpr (kAdd)
+    for_channel_elements<kTo, BT, FROM>(g, [&](int k, size_t off) { ad[k - FROM] = __builtin_nontemporal_load(addend + off); });
+  for_channel_elements<kTo, BT, FROM>(g, [&](int k, size_t off) {
+    __builtin_nontemporal_store(value(k, kAdd ? ad[k - FROM] : -0.f), out + off);
+  });
+  if constexpr (kTo < EMAX) store_channel<EMAX, BT, kAdd, kTo>(g, addend, out, value);
 }
 
 template <int EMAX, int BT, bool kRelu, bool kAdd>
@@ -633,17 +653,12 @@ __global__ __launch_bounds__(BT) void bn_fwd_small(FwdArgs a, Geometry g) {
     }
     if (a.nbt && c == 0) *a.nbt = __fadd_rn(*a.nbt, 1.0f);
   }
-  float ad[EMAX];   // fetched together, behind the registers that the statistics have given back
-  if constexpr (kAdd)
-    for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
-      ad[kk] = __builtin_nontemporal_load(a.res + (size_t)c * g.HW + off);
-    });
   __syncthreads();
   const Coef k = sk;
-  for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
+  store_channel<EMAX, BT, kAdd>(g, kAdd ? a.res + (size_t)c * g.HW : nullptr, yc, [&](int kk, float add) {
     float o = fmaf(v[kk] - k.m, k.k1, k.k0);
-    if constexpr (kAdd) o += ad[kk];
-    __builtin_nontemporal_store(kRelu ? relu1(o) : o, yc + off);
+    if constexpr (kAdd) o += add;
+    return kRelu ? relu1(o) : o;
   });
 }
 
@@ -686,18 +701,12 @@ __global__ __launch_bounds__(BT) void bn_bwd_small(BwdArgs a, Geometry g) {
     if (a.dgamma) a.dgamma[c] = (float)(s_dyxmu / sd);
   }
   if (a.dx == nullptr) return;
-  float ad[EMAX];
-  if constexpr (kAdd)
-    for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
-      ad[kk] = __builtin_nontemporal_load(a.add + (size_t)c * g.HW + off);
-    });
   __syncthreads();
   const Coef k = sk;
-  float* __restrict__ dxc = a.dx + (size_t)c * g.HW;
-  for_channel_elements<EMAX, BT>(g, [&](int kk, size_t off) {
+  store_channel<EMAX, BT, kAdd>(g, kAdd ? a.add + (size_t)c * g.HW : nullptr, a.dx + (size_t)c * g.HW, [&](int kk, float add) {
     float o = fmaf(gq[kk], k.k1, fmaf(v[kk] - k.m, k.k2, k.k0));
-    if constexpr (kAdd) o += ad[kk];
-    __builtin_nontemporal_store(o, dxc + off);
+    if constexpr (kAdd) o += add;
+    return o;
   });
 }
 
