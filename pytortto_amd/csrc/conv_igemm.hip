@@ -172,11 +172,21 @@ int cus() { return tt::compute_units(); }
 int sk_blocks_f32() { return 2 * cus(); }
 
 // Stream-K pays (partial tiles through memory, a wait at the end) and only helps when the
-// tiles do not spread evenly over the CUs; it needs a reduction long enough to split.
-bool wants_stream_k(long long tiles, int chunks, int groups) {
+// tiles do not spread evenly over the CUs; it needs a reduction long enough to split.  `fewest`: there is
+// no smaller tile that would raise the tile count instead.
+bool wants_stream_k(long long tiles, int chunks, int groups, bool fewest) {
   if (groups != 1 || chunks < 8) return false;
   // many tiles and a short reduction: hardware block scheduling balances better than fixed rounds
   if (tiles >= 3LL * sk_blocks_f32() && chunks < 64) return false;
+  if (tiles <= cus()) {
+    // All tiles run at once, each a chain of `chunks` steps; split, the chain is a block's share (eight
+    // steps at least, see launch_igemm) and the exchange of partial sums, which takes as long as about a
+    // dozen steps (16 channels from 32 over 3x3, 128 tiles of 18 steps: 31.7 us split, 14.5 whole; a
+    // classifier's 2048 to 10, one tile of 128 steps: 81 us whole, 17.5 split).
+    const long long share = std::max(8LL, (tiles * chunks + sk_blocks_f32() - 1) / sk_blocks_f32());
+    if (chunks <= share + 12) return false;
+    if (fewest) return true;
+  }
   if (tiles * chunks < 4LL * sk_blocks_f32()) return false;
   const long long rounds = (tiles + cus() - 1) / cus();
   return (double)tiles / (double)(rounds * cus()) < 0.93;
@@ -199,26 +209,28 @@ const IgemmUnit& unit(int terms, bool epilogue) {
 // (measured: 3 % faster than two, four do not fit the register file).
 int sk_launch_blocks() { return bf16_math() ? 3 * cus() : sk_blocks_f32(); }
 
-// 128x128 by default, 64 rows when a group has no more than 64 of them.  When that leaves
-// CUs idle or unevenly loaded the reduction is split stream-K fashion; if it is too short for
-// that, 64x64 tiles raise the block count instead.  `small` asks for 64x64 tiles outright: many
-// light blocks (four or five resident per CU) balance better and exchange no partial sums where a
+// 128x128 by default, 64 rows when a group has no more than 64 of them, 32 when it has no more than 32
+// and there are tiles enough (the float32 schedules: an empty row costs as much matrix time as a full
+// one; 8 rows per group, 41 us in 64-row tiles, 30 in these).  When that leaves CUs idle or unevenly loaded the reduction is split stream-K fashion; if it is
+// too short for that, 64x64 tiles raise the block count instead.  `small` asks for 64x64 tiles outright:
+// many light blocks (four or five resident per CU) balance better and exchange no partial sums where a
 // tile's reduction is short (plain matrix products with at most 32 chunks) or where several
 // short launches share a grid (the stride-parity classes of an input gradient).
 TileChoice choose_tile(int I, int M, int groups, int chunks, bool allow_stream_k = true, bool small = false) {
   TileChoice t;
   t.bm = I <= 64 ? 64 : 128;
   t.bn = I <= 64 ? 256 : 128;
-  if (small && groups == 1) { t.bm = 64; t.bn = 64; }
+  if (I <= 32 && !bf16_math() && (long long)ceil_div(M, 256) * groups >= cus()) t.bm = 32;
+  else if (small && groups == 1) { t.bm = 64; t.bn = 64; }
   t.sk_blocks = 0;
   const long long tiles = (long long)ceil_div(I, t.bm) * ceil_div(M, t.bn);
-  if (allow_stream_k && wants_stream_k(tiles, chunks, groups)) {
+  if (allow_stream_k && wants_stream_k(tiles, chunks, groups, false)) {
     t.sk_blocks = sk_launch_blocks();
   } else if (tiles * groups < cus()) {
     t.bm = 64;
     t.bn = 64;
     const long long small = (long long)ceil_div(I, 64) * ceil_div(M, 64);
-    if (allow_stream_k && wants_stream_k(small, chunks, groups)) t.sk_blocks = sk_launch_blocks();
+    if (allow_stream_k && wants_stream_k(small, chunks, groups, true)) t.sk_blocks = sk_launch_blocks();
   }
   return t;
 }

@@ -1,0 +1,23 @@
+"""The tile rule of the float32 forward and input gradient at its lines: up to 32 rows with tiles enough for
+the device, and few tiles with a long reduction, which is shared between blocks where that shortens it."""
+import pytest
+
+from tests.test_gpu_conv import _last_launch, _run_conv
+
+pytestmark = pytest.mark.gpu
+
+# n, c, h, w, k, r, s, stride, pad, dilation, groups; tile of the input gradient (rows, pixels, shared between blocks)
+CASES = [((4, 32, 128, 128, 32, 3, 3, (1, 1), (1, 1), (1, 1), 1), (32, 256, False)),     # 256 tiles
+         ((4, 31, 128, 127, 32, 3, 3, (1, 1), (1, 1), (1, 1), 1), (64, 64, False)),      # 254
+         ((4, 33, 128, 128, 8, 1, 1, (1, 1), (0, 0), (1, 1), 1), (64, 64, False)),       # 33 rows, plain product
+         ((2, 6, 182, 182, 10, 3, 2, (1, 1), (1, 1), (1, 1), 2), (32, 256, False)),      # per group
+         ((1, 16, 9, 9, 336, 1, 1, (1, 1), (0, 0), (1, 1), 1), (64, 64, True)),          # 21 chunks: eight and the exchange
+         ((1, 16, 9, 9, 320, 1, 1, (1, 1), (0, 0), (1, 1), 1), (64, 64, False)),         # 20: not shorter
+         ((2, 10, 1, 1, 2048, 1, 1, (1, 1), (0, 0), (1, 1), 1), (64, 64, True))]         # 128
+
+
+@pytest.mark.parametrize('case,tile', CASES, ids=[str(c[:6]) for c, _ in CASES])
+def test_tile_rule(case, tile):
+    _run_conv(case)
+    plan = _last_launch()
+    assert (plan['bm'], plan['bn'], plan['sharing_blocks'] > 0) == tile
