@@ -207,7 +207,9 @@ def call(name, *args):
     A deferred operation runs first."""
     if _pending is not None:
         flush()
-    check(getattr(lib(), name)(*args))
+    status = getattr(_lib if _ready else lib(), name)(*args)
+    if status != 0:
+        check(status)
 
 
 def is_available():
