@@ -21,3 +21,9 @@ def test_tile_rule(case, tile):
     _run_conv(case)
     plan = _last_launch()
     assert (plan['bm'], plan['bn'], plan['sharing_blocks'] > 0) == tile
+
+
+@pytest.mark.parametrize('k,c,r', [(192, 24, 3), (129, 160, 3), (190, 7, 3), (320, 33, 1), (193, 16, 3), (130, 3, 7)])
+def test_weight_gradient_rows_that_fill_no_128(k, c, r):
+    """Rows and columns on either side of the lines between 64- and 128-wide tiles."""
+    _run_conv((3, c, 11, 9, k, r, r, (1, 1), (r // 2, r // 2), (1, 1), 1))
