@@ -397,6 +397,11 @@ int tt_maxpool2d_fwd_f32(const float* x, float* y, int* tap, int NC, int H, int 
  * reference does not sum them.  Pixels no window chose receive 0. */
 int tt_maxpool2d_bwd_f32(const float* dy, const int* tap, float* dx, int NC, int H, int W, int P, int Q,
                          int kh, int kw, int sh, int sw, int ph, int pw, int dh, int dw);
+/* The same pair with a byte per tap index, for windows of at most 256 taps. */
+int tt_maxpool2d_fwd_tap8_f32(const float* x, float* y, unsigned char* tap, int NC, int H, int W, int P, int Q,
+                              int kh, int kw, int sh, int sw, int ph, int pw, int dh, int dw);
+int tt_maxpool2d_bwd_tap8_f32(const float* dy, const unsigned char* tap, float* dx, int NC, int H, int W, int P, int Q,
+                              int kh, int kw, int sh, int sw, int ph, int pw, int dh, int dw);
 
 /* ---- classifier head: spatial mean, Linear, LogSoftmax, NLLLoss ------------------------------- */
 

@@ -81,6 +81,8 @@ PROTOTYPES = {
     'tt_leaky_relu_bwd_f32': [_P, _P, _P, c_float, c_size_t],
     'tt_maxpool2d_fwd_f32': [_P, _P, _P] + [_I] * 13,
     'tt_maxpool2d_bwd_f32': [_P, _P, _P] + [_I] * 13,
+    'tt_maxpool2d_fwd_tap8_f32': [_P, _P, _P] + [_I] * 13,
+    'tt_maxpool2d_bwd_tap8_f32': [_P, _P, _P] + [_I] * 13,
     'tt_mean_rows_f32': [_P, _P, _I, _I],
     'tt_mean_rows_bwd_f32': [_P, _P, _I, _I],
     'tt_transpose2d_f32': [_P, _P, _I, _I],

@@ -174,6 +174,7 @@ int sk_blocks_f32() { return 2 * cus(); }
 // Stream-K pays (partial tiles through memory, a wait at the end) and only helps when the
 // tiles do not spread evenly over the CUs; it needs a reduction long enough to split.  `fewest`: there is
 // no smaller tile that would raise the tile count instead.
+bool bf16_math();
 bool wants_stream_k(long long tiles, int chunks, int groups, bool fewest) {
   if (groups != 1 || chunks < 8) return false;
   // many tiles and a short reduction: hardware block scheduling balances better than fixed rounds
@@ -184,7 +185,7 @@ bool wants_stream_k(long long tiles, int chunks, int groups, bool fewest) {
     // dozen steps (16 channels from 32 over 3x3, 128 tiles of 18 steps: 31.7 us split, 14.5 whole; a
     // classifier's 2048 to 10, one tile of 128 steps: 81 us whole, 17.5 split).
     const long long share = std::max(8LL, (tiles * chunks + sk_blocks_f32() - 1) / sk_blocks_f32());
-    if (chunks <= share + 12) return false;
+    if (chunks <= share + 12 && !bf16_math()) return false;   // (those kernels' steps are too short to count)
     if (fewest) return true;
   }
   if (tiles * chunks < 4LL * sk_blocks_f32()) return false;

@@ -439,13 +439,14 @@ def _pool_dims(x):
 
 def maxpool2d_fwd(x, out_hw, kernel_size, stride, padding, dilation):
     """(y, tap): maxima over the -inf padded windows and, per output, the winning tap as
-    kernel_row * kw + kernel_column (``_max_pool2d``, grad_nn.py:784-808)."""
+    kernel_row * kw + kernel_column (``_max_pool2d``, grad_nn.py:784-808): a byte each where that fits."""
     _f32(x)
     nc, h, w = _pool_dims(x)
     p, q = out_hw
     y = hiparray.empty(x.shape[:-2] + (p, q))
-    tap = hiparray.empty(x.shape[:-2] + (p, q), np.int32)
-    _hip.call('tt_maxpool2d_fwd_f32', x.ptr, y.ptr, tap.ptr, nc, h, w, p, q, *kernel_size, *stride, *padding,
+    byte = kernel_size[0] * kernel_size[1] <= 256
+    tap = hiparray.empty(x.shape[:-2] + (p, q), np.uint8 if byte else np.int32)
+    _hip.call('tt_maxpool2d_fwd_tap8_f32' if byte else 'tt_maxpool2d_fwd_f32', x.ptr, y.ptr, tap.ptr, nc, h, w, p, q, *kernel_size, *stride, *padding,
               *dilation)
     return y, tap
 
@@ -454,12 +455,12 @@ def maxpool2d_bwd(dy, tap, in_hw, kernel_size, stride, padding, dilation):
     """dx: every output gradient assigned to its window's arg-max pixel, the last window in
     (p, q) order winning where several chose the same pixel (``_max_pool2d_backward``, :811-824)."""
     _f32(dy)
-    if tap.dtype != np.int32 or tap.shape != dy.shape:
-        raise ValueError('maxpool2d_bwd: `tap` must be the int32 array the forward returned')
+    if tap.dtype not in (np.uint8, np.int32) or tap.shape != dy.shape:
+        raise ValueError('maxpool2d_bwd: `tap` must be the array the forward returned')
     nc, p, q = _pool_dims(dy)
     h, w = in_hw
     dx = hiparray.empty(dy.shape[:-2] + (h, w))
-    _hip.call('tt_maxpool2d_bwd_f32', dy.ptr, tap.ptr, dx.ptr, nc, h, w, p, q, *kernel_size, *stride, *padding,
+    _hip.call('tt_maxpool2d_bwd_tap8_f32' if tap.dtype == np.uint8 else 'tt_maxpool2d_bwd_f32', dy.ptr, tap.ptr, dx.ptr, nc, h, w, p, q, *kernel_size, *stride, *padding,
               *dilation)
     return dx
 
