@@ -270,6 +270,8 @@ int tt_conv2d_last_launch(int* plan8);
  * launches go to kernels built around the bf16 matrix instruction (operands converted on their way
  * into LDS, 32-deep chunks) when they have at least one tile per compute unit or a reduction of at
  * most 1024 (1, the default) or whenever those kernels support the geometry (2: small test shapes);
+ * and to channel-last kernels where those are faster (1: from 128 channels, or few tiles with a long
+ * reduction; 2: whenever they support the geometry);
  * 0 keeps every launch on the float32 kernels' bf16 instantiations, which also serve the launches
  * the former do not take.  Both compute the same thing: the convolution of
  * the bf16-rounded operands in float32. */

@@ -650,8 +650,8 @@ int tt_conv2d_last_launch(int* plan8) {
   return 0;
 }
 
-// Instrumentation (tests): with bf16 arithmetic selected, route the launches the bf16-first kernels
-// support to them (1, the default) or keep everything on the float32 kernels' bf16 instantiations (0).
+// Instrumentation (tests): with bf16 arithmetic selected, route the launches the bf16-first and the
+// channel-last kernels support to them (1, the default) or keep everything on the float32 kernels' bf16 instantiations (0).
 int tt_conv2d_bf16_first_enable(int on) {
   TT_API_LOCK();
   g_bf16_first = on != 0;
