@@ -157,10 +157,15 @@ _lock = threading.RLock()
 
 
 def defer(op):
-    """Park ``op`` (an object with ``run()``); whatever was parked before runs now."""
+    """Park ``op`` (an object with ``run()``); whatever was parked before runs now.  Should that fail, ``op`` will
+    never run either, and its arrays are marked."""
     global _pending
     with _lock:
-        flush()
+        try:
+            flush()
+        except Exception as exc:
+            _poison(op, exc)
+            raise
         _pending = op
 
 
@@ -188,9 +193,31 @@ def take_pending_if(wanted):
     return op
 
 
+def join_pending(wanted, join):
+    """``join(op)`` for the parked operation, removed from the slot, if ``wanted(op)`` holds for it; otherwise
+    None.  One step: no other thread finds the slot empty and the arrays not filled yet.  ``wanted`` makes sure that
+    ``join`` will not refuse its operands -- an operation that is refused stays parked --, and should ``join`` fail
+    all the same, the arrays that will now never be filled are marked as ``flush`` does it."""
+    with _lock:
+        op = take_pending_if(wanted)
+        if op is None:
+            return None
+        try:
+            return join(op)
+        except Exception as exc:
+            _poison(op, exc)
+            raise
+
+
+def _poison(op, exc):
+    """``op`` will never fill its arrays: any later use of them raises ``exc`` instead of reading memory nobody wrote."""
+    poison = getattr(op, 'poison', None)
+    if poison is not None:
+        poison(exc)
+
+
 def flush():
-    """Run the parked operation, if any.  Should it fail, the arrays it was to fill are marked:
-    any later use of them raises the same error instead of reading memory nobody wrote."""
+    """Run the parked operation, if any.  Should it fail, the arrays it was to fill are marked."""
     with _lock:
         op = take_pending()
         if op is None:
@@ -198,9 +225,7 @@ def flush():
         try:
             op.run()
         except Exception as exc:
-            poison = getattr(op, 'poison', None)
-            if poison is not None:
-                poison(exc)
+            _poison(op, exc)
             raise
 
 

@@ -75,12 +75,10 @@ class Add(Function):
             takes = (ops.DeferredBatchNorm,)
             if not (ctx.requires_grad and is_grad_enabled()):
                 takes = (ops.DeferredBatchNorm, ops.DeferredConv)
-            parked = _hip.take_pending_if(lambda op: op.__class__ in takes and op.residual is None
-                                          and (op.out._buf is a._buf) != (op.out._buf is b._buf)
-                                          and op.out.shape == a.shape)
-            if parked is not None:
-                y = parked.absorb_add(b if parked.out._buf is a._buf else a)
-            else:
+            y = _hip.join_pending(lambda op: op.__class__ in takes and op.residual is None and ops.computes_on(a, b)
+                                  and (op.out._buf is a._buf) != (op.out._buf is b._buf) and op.out.shape == a.shape,
+                                  lambda op: op.absorb_add(b if op.out._buf is a._buf else a))
+            if y is None:
                 y = ops.add_deferred(a, b)      # parked: a ReLU that comes next absorbs it
         elif b.size < a.size and _trailing(b.shape, a.shape):
             y = ops.add_rowvec(a, b)

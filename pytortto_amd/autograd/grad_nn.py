@@ -175,13 +175,14 @@ class BatchNorm(Function):
         elif have_running:
             no_gradient = not (ctx.requires_grad and is_grad_enabled())
             if no_gradient:
-                conv = _hip.take_pending_if(lambda op: op.__class__ is ops.DeferredConv and op.takes_norm()
-                                            and op.out._buf is xd0._buf and op.out.shape == xd0.shape)
-                if conv is not None:
-                    # x is a convolution's output that has not been launched yet: normalise it on its way
-                    # to memory (nothing is saved: no gradient will flow)
-                    return build_links(conv.absorb_norm(running_mean.data, running_var.data, gamma, beta, eps),
-                                       grad_fn=ctx)
+                # x may be a convolution's output that has not been launched yet: normalise it on its way to memory
+                # (nothing is saved: no gradient will flow)
+                stats = running_mean.data, running_var.data, gamma, beta
+                yd0 = _hip.join_pending(lambda op: op.__class__ is ops.DeferredConv and op.takes_norm()
+                                        and op.out._buf is xd0._buf and op.out.shape == xd0.shape
+                                        and ops.computes_on(*stats), lambda op: op.absorb_norm(*stats, eps))
+                if yd0 is not None:
+                    return build_links(yd0, grad_fn=ctx)
             yd0, mean, var_eps, sd = ops.bn_fwd_eval(xd0, gamma, beta, running_mean.data, running_var.data, eps,
                                                        deferred=no_gradient)
         elif xd0.size == xd0.shape[1]:
@@ -222,35 +223,32 @@ class Relu(Function):
         xt0, = inputs
         xd0 = xt0.data
         inplace = params['inplace']
-        # only a device input can be the output of a parked device operation (a host array has no buffer)
-        parked = None
-        if xd0.__class__ is hiparray:
-            parked = _hip.take_pending_if(lambda op: op.__class__ in _TAKES_RELU and op.out._buf is xd0._buf)
-        if parked is not None:
-            # the input is a BatchNorm output, a residual sum, or a convolution's, that has not been launched
-            # yet: one kernel writes maximum(bn(x), 0) (grad_nn.py:942-959 and :56 in one pass), maximum(a + b, 0) ...
-            if inplace:
-                try:
-                    inplace_precheck(xt0)
-                except RuntimeError:
-                    parked.run()
-                    raise
+        if inplace:
+            inplace_precheck(xt0)
+
+        def join(op):
             out = None if inplace else hiparray.empty(xd0.shape)
-            if parked.__class__ is ops.DeferredBatchNorm:
-                out = parked.run_with_relu(out, keep_coef=ctx.requires_grad and is_grad_enabled())
-                ctx.params['bn_coef'] = parked.coef
-            else:
-                out = parked.run_with_relu(out)
+            if op.__class__ is not ops.DeferredBatchNorm:
+                return op.run_with_relu(out)
+            out = op.run_with_relu(out, keep_coef=ctx.requires_grad and is_grad_enabled())
+            ctx.params['bn_coef'] = op.coef
+            return out
+
+        # only a device input can be the output of a parked device operation (a host array has no buffer)
+        out = None
+        if xd0.__class__ is hiparray:
+            out = _hip.join_pending(lambda op: op.__class__ in _TAKES_RELU and op.out._buf is xd0._buf, join)
+        if out is not None:
+            # the input is a BatchNorm output, a residual sum, or a convolution's, that had not been launched
+            # yet: one kernel writes maximum(bn(x), 0) (grad_nn.py:942-959 and :56 in one pass), maximum(a + b, 0) ...
             yt0 = inplace_update(xt0, ctx) if inplace else build_links(out, grad_fn=ctx)
         elif xd0.__class__ is hiparray:
             if inplace:
-                inplace_precheck(xt0)
                 ops.relu_fwd(xd0, out=xd0)
                 yt0 = inplace_update(xt0, ctx)
             else:
                 yt0 = build_links(ops.relu_fwd(xd0), grad_fn=ctx)
         elif inplace:
-            inplace_precheck(xt0)
             np.maximum(xd0, 0, out=xd0)
             yt0 = inplace_update(xt0, ctx)
         else:

@@ -23,6 +23,11 @@ def _f32(*arrays):
             raise TypeError(f'the device path computes in float32 only, got {a.dtype}')
 
 
+def computes_on(*arrays):
+    """Whether the device path takes all of them (None: not given) as operands."""
+    return all(a is None or (a.__class__ is hiparray and a.dtype == np.float32) for a in arrays)
+
+
 def conv_out_size(size, k, stride, pad, dil):
     """autograd/grad_nn.py:565-566"""
     return math.floor((size + 2 * pad - dil * (k - 1) - 1) / stride + 1)
@@ -85,7 +90,6 @@ class DeferredConv:
         return self.norm is None and self.residual is None
 
     def absorb_norm(self, mean, var, gamma, beta, eps):
-        _f32(mean, var, gamma, beta)
         self._on_demand()
         self.norm = (mean, var, gamma, beta, float(eps))
         self.out = hiparray.lazy(self.out.shape)
@@ -93,7 +97,6 @@ class DeferredConv:
         return self.out
 
     def absorb_add(self, residual):
-        _f32(residual)
         self._on_demand()
         self.residual = residual
         self.out = hiparray.lazy(self.out.shape)
@@ -243,7 +246,6 @@ class DeferredBatchNorm:
         self._launch(self.out, False)
 
     def absorb_add(self, residual):
-        _f32(residual)
         self._on_demand()
         self.residual = residual
         self.out = hiparray.lazy(self.out.shape)

@@ -1,0 +1,127 @@
+"""What happens to an operation that waits for its successor (``_hip.defer``), on the host: the library is a
+stand-in that records the calls and fails them on demand, so nothing here touches a GPU."""
+import gc
+
+import numpy as np
+import pytest
+
+import pytortto_amd as tt
+from pytortto_amd import _hip, ops
+from pytortto_amd.xparray import hiparray
+
+F = tt.nn.functional
+
+
+class _Library:
+    def __init__(self):
+        self.calls, self.fail = [], set()
+
+    def __getattr__(self, name):
+        def function(*args):
+            if name == 'tt_malloc':
+                args[0]._obj.value = 4096 * (1 + len(self.calls))
+            self.calls.append(name)
+            return int(name in self.fail)
+        return function
+
+    def tt_last_error(self):
+        return b'refused by the library'
+
+    def launched(self):
+        """The calls since the last look, but for memory and transfers."""
+        names = [n for n in self.calls if n not in ('tt_malloc', 'tt_free', 'tt_memcpy_h2d')]
+        self.calls.clear()
+        return names
+
+
+@pytest.fixture
+def library(monkeypatch):
+    stand_in = _Library()
+    monkeypatch.setattr(_hip, '_lib', stand_in)
+    monkeypatch.setattr(_hip, '_ready', True)
+    monkeypatch.setattr(_hip, '_pending', None)
+    yield stand_in
+    _hip.take_pending()
+    gc.collect()                # device arrays give their blocks back to the stand-in
+
+
+def _tensor(*shape, dtype=np.float32):
+    return tt.Tensor(hiparray(np.ones(shape, dtype)), dtype=dtype)
+
+
+def _on_device(module):
+    module.cuda()
+    return module
+
+
+CONV, NORM, NORM_EVAL = 'tt_conv2d_fwd_f32', 'tt_bn_act_fwd_train_f32', 'tt_bn_fwd_eval_f32'
+
+
+def test_a_refused_add_leaves_the_batch_norm_in_front_of_it_parked(library):
+    bn = _on_device(tt.nn.BatchNorm2d(4))
+    whole = _tensor(2, 4, 3, 3, dtype=np.int64)
+    y = bn(_tensor(2, 4, 3, 3))
+    library.launched()
+    for operands in ((y, whole), (whole, y)):
+        with pytest.raises(TypeError, match='float32 only'):
+            operands[0] + operands[1]
+    assert _hip.pending().__class__ is ops.DeferredBatchNorm
+    y.data.ptr, bn.running_mean.data.ptr, bn.running_var.data.ptr
+    assert library.launched() == [NORM]
+
+
+def test_a_refused_add_or_batch_norm_leaves_the_convolution_in_front_of_it_parked(library):
+    conv, bn = _on_device(tt.nn.Conv2d(4, 4, 1)), _on_device(tt.nn.BatchNorm2d(4))
+    bn.eval()
+    bn.running_var.data = hiparray(np.ones(4))              # float64
+    whole = _tensor(2, 4, 3, 3, dtype=np.int64)
+    with tt.no_grad():
+        y = conv(_tensor(2, 4, 3, 3))
+        library.launched()
+        with pytest.raises(TypeError, match='float32 only'):
+            y + whole
+        with pytest.raises(TypeError, match='float32 only'):
+            bn(y)
+        assert _hip.pending().__class__ is ops.DeferredConv
+        y.data.ptr
+    assert library.launched() == [CONV]
+
+
+@pytest.mark.parametrize('training', [True, False])
+def test_arrays_of_a_launch_that_fails_after_joining_raise(library, training):
+    conv, bn = _on_device(tt.nn.Conv2d(4, 4, 1)), _on_device(tt.nn.BatchNorm2d(4))
+    bn.train(training)
+    with tt.no_grad():
+        y = bn(conv(_tensor(2, 4, 3, 3)))
+        library.fail = {NORM, 'tt_conv2d_norm_act_fwd_f32'}
+        with pytest.raises(RuntimeError, match='refused by the library'):
+            F.relu(y).data.ptr
+    library.fail = set()
+    for array in (y.data,) + ((bn.running_mean.data, bn.running_var.data) if training else ()):
+        with pytest.raises(RuntimeError, match='refused by the library'):
+            array.ptr
+
+
+def test_an_operation_behind_one_that_fails_is_marked_too(library):
+    bn = _on_device(tt.nn.BatchNorm2d(4))
+    y = bn(_tensor(2, 4, 3, 3))
+    library.fail = {NORM}
+    op = object.__new__(ops.DeferredAdd)
+    op.out = hiparray.lazy((2, 2))
+    with pytest.raises(RuntimeError, match='refused by the library'):
+        _hip.defer(op)
+    assert _hip.pending() is None
+    for array in (y.data, op.out):
+        with pytest.raises(RuntimeError, match='refused by the library'):
+            array.ptr
+
+
+def test_an_in_place_relu_that_is_refused_leaves_its_input_parked(library):
+    x = _tensor(2, 4, 3, 3)
+    t = x + _tensor(2, 4, 3, 3)
+    t.requires_grad = True                                  # a leaf that asks for a gradient
+    library.launched()
+    with pytest.raises(RuntimeError, match='in-place operation'):
+        F.relu(t, inplace=True)
+    t.data.ptr
+    assert library.launched() == ['tt_add_f32']
