@@ -4,6 +4,8 @@ Shape bookkeeping and output allocation happen here; all arithmetic happens in
 ``libtortto_hip.so``.  Each wrapper names the reference lines whose array expressions it
 stands in for (paths relative to the reference's ``src/tortto/``).
 """
+import ctypes
+import functools
 import math
 from math import prod
 
@@ -57,6 +59,9 @@ def conv2d_fwd(x, w, bias, stride, padding, dilation, groups):
     return y
 
 
+_BN_CHANNELS = 65535        # of the BatchNorm entry points
+
+
 class DeferredConv:
     """A convolution whose result needs no gradient, not launched yet (see ``_hip.defer``).  What
     follows it in an evaluation pass -- a BatchNorm with given statistics, a residual add, a ReLU --
@@ -87,7 +92,7 @@ class DeferredConv:
         self.out._buf.fill_on_demand(self._launcher(False), self._operands())
 
     def takes_norm(self):
-        return self.norm is None and self.residual is None
+        return self.norm is None and self.residual is None and self.out.shape[1] <= _BN_CHANNELS
 
     def absorb_norm(self, mean, var, gamma, beta, eps):
         self._on_demand()
@@ -119,15 +124,21 @@ class DeferredConv:
         poison([self.out], exc)
 
 
-# beyond these the C entry point may refuse a geometry or cut the batch into runs: launched at once,
-# so that an error is raised where it belongs
-_DEFER_EXTENT, _DEFER_ELEMENTS = 8192, 1 << 31
+@functools.lru_cache(maxsize=1024, typed=True)
+def _conv2d_fwd_accepts(*dims):
+    """Whether the C entry point takes this geometry, by its own argument checks (the size query runs them and
+    launches nothing); asked once per geometry."""
+    try:
+        return _hip.lib().tt_workspace_size_conv2d_fwd_f32(ctypes.byref(ctypes.c_size_t()), *dims) == 0
+    except ctypes.ArgumentError:
+        return False
 
 
 def conv2d_fwd_deferred(x, w, bias, stride, padding, dilation, groups):
-    """``conv2d_fwd`` with the launch parked for the operations behind it to join."""
+    """``conv2d_fwd`` with the launch parked for the operations behind it to join.  What would be refused is
+    launched at once, so that the error is raised where it belongs, and so is a batch that is cut into runs."""
     shape, dims = _conv2d_geometry(x, w, bias, stride, padding, dilation, groups)
-    if max(x.shape[2:]) >= _DEFER_EXTENT or max(x.size, prod(shape)) >= _DEFER_ELEMENTS or 0 in x.shape:
+    if 0 in x.shape or max(x.size, prod(shape)) >= 1 << 31 or not _conv2d_fwd_accepts(*dims):
         return conv2d_fwd(x, w, bias, stride, padding, dilation, groups)
     op = DeferredConv(x, w, bias, shape, dims)
     _hip.defer(op)
@@ -333,10 +344,12 @@ class DeferredBatchNormEval:
 
 
 def bn_fwd_eval(x, gamma, beta, mean_in, var_in, eps, deferred=False):
-    """(y, mean, var + eps, sd); with ``deferred`` the launch is parked for a ReLU to join."""
+    """(y, mean, var + eps, sd); with ``deferred`` the launch is parked for a ReLU to join, unless it would be
+    refused: that error is raised here."""
     _f32(x, gamma, beta, mean_in, var_in)
     op = DeferredBatchNormEval(x, gamma, beta, mean_in, var_in, eps)
-    if deferred:
+    n, c, hw = op.dims
+    if deferred and computes_on(*op.operands) and 0 < x.size and c <= _BN_CHANNELS and max(n, c) * hw < 1 << 31:
         _hip.defer(op)
     else:
         op.run()

@@ -40,7 +40,9 @@ def library(monkeypatch):
     monkeypatch.setattr(_hip, '_lib', stand_in)
     monkeypatch.setattr(_hip, '_ready', True)
     monkeypatch.setattr(_hip, '_pending', None)
+    ops._conv2d_fwd_accepts.cache_clear()
     yield stand_in
+    ops._conv2d_fwd_accepts.cache_clear()
     _hip.take_pending()
     gc.collect()                # device arrays give their blocks back to the stand-in
 
@@ -125,3 +127,15 @@ def test_an_in_place_relu_that_is_refused_leaves_its_input_parked(library):
         F.relu(t, inplace=True)
     t.data.ptr
     assert library.launched() == ['tt_add_f32']
+
+
+def test_what_the_library_refuses_is_raised_by_the_call(library):
+    conv = _on_device(tt.nn.Conv2d(4, 4, 1))
+    x = _tensor(2, 4, 3, 3)
+    with tt.no_grad():
+        assert conv(x) is not None and _hip.pending() is not None
+        _hip.flush()
+        library.fail = {'tt_workspace_size_conv2d_fwd_f32', CONV}
+        with pytest.raises(RuntimeError, match='refused by the library'):
+            conv(_tensor(2, 4, 3, 5))
+        assert _hip.pending() is None
