@@ -161,11 +161,12 @@ def defer(op):
     never run either, and its arrays are marked."""
     global _pending
     with _lock:
-        try:
-            flush()
-        except Exception as exc:
-            _poison(op, exc)
-            raise
+        if _pending is not None:
+            try:
+                flush()
+            except Exception as exc:
+                _poison(op, exc)
+                raise
         _pending = op
 
 
@@ -198,10 +199,12 @@ def join_pending(wanted, join):
     None.  One step: no other thread finds the slot empty and the arrays not filled yet.  ``wanted`` makes sure that
     ``join`` will not refuse its operands -- an operation that is refused stays parked --, and should ``join`` fail
     all the same, the arrays that will now never be filled are marked as ``flush`` does it."""
+    global _pending
     with _lock:
-        op = take_pending_if(wanted)
-        if op is None:
+        op = _pending
+        if op is None or not wanted(op):
             return None
+        _pending = None
         try:
             return join(op)
         except Exception as exc:
@@ -218,8 +221,9 @@ def _poison(op, exc):
 
 def flush():
     """Run the parked operation, if any.  Should it fail, the arrays it was to fill are marked."""
+    global _pending
     with _lock:
-        op = take_pending()
+        op, _pending = _pending, None
         if op is None:
             return
         try:
@@ -301,10 +305,6 @@ def set_conv_math(mode):
     tolerances as 'f32')."""
     if mode not in CONV_MATH:
         raise ValueError(f"conv math must be one of {sorted(CONV_MATH)}, got {mode!r}")
-    if mode != get_conv_math():
-        # a convolution output that is still to be produced on demand belongs to the mode it was asked for in
-        from .xparray import fill_all
-        fill_all()
     call('tt_set_conv_math', CONV_MATH[mode])
 
 

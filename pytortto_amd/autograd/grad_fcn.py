@@ -75,7 +75,7 @@ class Add(Function):
             takes = (ops.DeferredBatchNorm,)
             if not (ctx.requires_grad and is_grad_enabled()):
                 takes = (ops.DeferredBatchNorm, ops.DeferredConv)
-            y = _hip.join_pending(lambda op: op.__class__ in takes and op.residual is None and ops.computes_on(a, b)
+            y = _hip.join_pending(lambda op: op.__class__ in takes and op.takes_add() and ops.computes_on(a, b)
                                   and (op.out._buf is a._buf) != (op.out._buf is b._buf) and op.out.shape == a.shape,
                                   lambda op: op.absorb_add(b if op.out._buf is a._buf else a))
             if y is None:

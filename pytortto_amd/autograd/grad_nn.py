@@ -227,6 +227,8 @@ class Relu(Function):
             inplace_precheck(xt0)
 
         def join(op):
+            if op.__class__ is ops.DeferredConv:            # waits on: its output is found filled
+                return op.run_with_relu(None if inplace else hiparray.lazy(xd0.shape))
             out = None if inplace else hiparray.empty(xd0.shape)
             if op.__class__ is not ops.DeferredBatchNorm:
                 return op.run_with_relu(out)
@@ -237,7 +239,8 @@ class Relu(Function):
         # only a device input can be the output of a parked device operation (a host array has no buffer)
         out = None
         if xd0.__class__ is hiparray:
-            out = _hip.join_pending(lambda op: op.__class__ in _TAKES_RELU and op.out._buf is xd0._buf, join)
+            out = _hip.join_pending(lambda op: op.__class__ in _TAKES_RELU and op.out._buf is xd0._buf
+                                    and (op.__class__ is not ops.DeferredConv or op.takes_relu()), join)
         if out is not None:
             # the input is a BatchNorm output, a residual sum, or a convolution's, that had not been launched
             # yet: one kernel writes maximum(bn(x), 0) (grad_nn.py:942-959 and :56 in one pass), maximum(a + b, 0) ...

@@ -7,6 +7,7 @@ stands in for (paths relative to the reference's ``src/tortto/``).
 import ctypes
 import functools
 import math
+import weakref
 from math import prod
 
 import numpy as np
@@ -27,7 +28,10 @@ def _f32(*arrays):
 
 def computes_on(*arrays):
     """Whether the device path takes all of them (None: not given) as operands."""
-    return all(a is None or (a.__class__ is hiparray and a.dtype == np.float32) for a in arrays)
+    for a in arrays:
+        if a is not None and (a.__class__ is not hiparray or a._dtype != np.float32):
+            return False
+    return True
 
 
 def conv_out_size(size, k, stride, pad, dil):
@@ -66,62 +70,93 @@ class DeferredConv:
     """A convolution whose result needs no gradient, not launched yet (see ``_hip.defer``).  What
     follows it in an evaluation pass -- a BatchNorm with given statistics, a residual add, a ReLU --
     joins the launch and is applied to the accumulators before they are stored (``absorb_norm``,
-    ``absorb_add``, ``run_with_relu``); anything else finds it launched with what has joined so far.
-    The values in between are never stored: their arrays are produced on demand by the launch up to
-    that point, should anybody ask, and at the latest just before an operand is written in place."""
+    ``absorb_add``, ``run_with_relu``, in this order); anything else finds it launched with what has joined so far.
+
+    A value in between that nobody holds any more when the launch comes is never stored.  One that is still
+    held may be read (a shortcut around the BatchNorm): it is stored where it stands, and what follows it runs
+    in kernels of its own (same bits), so that no convolution is ever computed twice.  The ReLU is parked with the
+    rest for that reason: its caller's names for the values in front of it are gone when the next call comes."""
 
     def __init__(self, x, w, bias, shape, dims):
         self.x, self.w, self.bias, self.dims = x, w, bias, dims
         self.norm = self.residual = None
-        self.out = hiparray.lazy(shape)
+        self.steps = []         # what has joined
+        self.shape = shape
+        self.out = hiparray.lazy(self.shape)
+        self.between = []       # (a weak reference to the buffer of a value in front of ``out``, steps in front of it)
 
-    def _operands(self):
-        return (self.x, self.w, self.bias, *(self.norm[:4] if self.norm else ()), self.residual)
-
-    def _launcher(self, relu):
-        """The launch of what has joined so far, as a function of the array to fill."""
-        x, w, bias, dims, norm, residual = self.x, self.w, self.bias, self.dims, self.norm, self.residual
-        if norm is None and residual is None and not relu:
-            return lambda out: _hip.call('tt_conv2d_fwd_f32', x.ptr, w.ptr, _ptr(bias), out.ptr, *dims)
-        mean, var, gamma, beta, eps = norm or (None, None, None, None, 0.0)
-        return lambda out: _hip.call('tt_conv2d_norm_act_fwd_f32', x.ptr, w.ptr, _ptr(bias), out.ptr, _ptr(mean),
-                                     _ptr(var), _ptr(gamma), _ptr(beta), eps, _ptr(residual), int(relu), *dims)
-
-    def _on_demand(self):
-        """The output so far is about to be absorbed: leave it to be produced on demand."""
-        self.out._buf.fill_on_demand(self._launcher(False), self._operands())
+    def _join(self, step, out):
+        if out is not None:
+            self.between.append((weakref.ref(self.out._buf), len(self.steps)))
+            self.out = out
+        self.steps.append(step)
+        _hip.defer(self)
+        return self.out
 
     def takes_norm(self):
-        return self.norm is None and self.residual is None and self.out.shape[1] <= _BN_CHANNELS
+        return not self.steps and self.shape[1] <= _BN_CHANNELS
+
+    def takes_add(self):
+        return self.residual is None and self.takes_relu()
+
+    def takes_relu(self):
+        return 'relu' not in self.steps
 
     def absorb_norm(self, mean, var, gamma, beta, eps):
-        self._on_demand()
         self.norm = (mean, var, gamma, beta, float(eps))
-        self.out = hiparray.lazy(self.out.shape)
-        _hip.defer(self)
-        return self.out
+        return self._join('norm', hiparray.lazy(self.shape))
 
     def absorb_add(self, residual):
-        self._on_demand()
         self.residual = residual
-        self.out = hiparray.lazy(self.out.shape)
-        _hip.defer(self)
-        return self.out
-
-    def run(self):
-        self._launcher(False)(self.out)
+        return self._join('add', hiparray.lazy(self.shape))
 
     def run_with_relu(self, out=None):
-        launch = self._launcher(True)
-        if out is None:
-            out = self.out
+        """The ReLU's values go to ``out``, or to the operation's own array (an in-place ReLU)."""
+        return self._join('relu', out)
+
+    def _held(self):
+        """(array, steps in front of it) of the values in between that somebody still holds."""
+        buffers = [(ref(), done) for ref, done in self.between]
+        return [(hiparray.on(buf, self.shape, self.out.dtype), done) for buf, done in buffers if buf is not None]
+
+    def run(self):
+        before = None
+        for array, done in (*self._held(), (self.out, len(self.steps))):
+            if before is None:
+                self._launch(array, self.steps[:done])
+            else:
+                self._launch_after(before[0], array, self.steps[before[1]:done])
+            before = array, done
+
+    def _launch(self, out, steps):
+        """The convolution and the ``steps`` behind it, in one launch."""
+        x, w, bias, dims = self.x, self.w, self.bias, self.dims
+        if not steps:
+            _hip.call('tt_conv2d_fwd_f32', x.ptr, w.ptr, _ptr(bias), out.ptr, *dims)
+            return
+        mean, var, gamma, beta, eps = self.norm if 'norm' in steps else (None, None, None, None, 0.0)
+        residual = self.residual if 'add' in steps else None
+        _hip.call('tt_conv2d_norm_act_fwd_f32', x.ptr, w.ptr, _ptr(bias), out.ptr, _ptr(mean), _ptr(var), _ptr(gamma),
+                  _ptr(beta), eps, _ptr(residual), int('relu' in steps), *dims)
+
+    def _launch_after(self, value, out, steps):
+        """``steps`` on a value that has been stored."""
+        relu = 'relu' in steps
+        if 'norm' in steps:
+            mean, var, gamma, beta, eps = self.norm
+            add = 'add' in steps
+            op = DeferredBatchNormEval(value, gamma, beta, mean, var, eps, None if add else out)
+            op.launch(relu and not add)
+            if not add:
+                return
+            value = op.out
+        if 'add' in steps:
+            _hip.call('tt_add_relu_f32' if relu else 'tt_add_f32', value.ptr, self.residual.ptr, out.ptr, out.size)
         else:
-            self._on_demand()
-        launch(out)
-        return out
+            _hip.call('tt_relu_fwd_f32', value.ptr, out.ptr, out.size)
 
     def poison(self, exc):
-        poison([self.out], exc)
+        poison([self.out] + [array for array, _ in self._held()], exc)
 
 
 @functools.lru_cache(maxsize=1024, typed=True)
@@ -256,6 +291,9 @@ class DeferredBatchNorm:
     def run(self):
         self._launch(self.out, False)
 
+    def takes_add(self):
+        return self.residual is None
+
     def absorb_add(self, residual):
         self._on_demand()
         self.residual = residual
@@ -315,10 +353,10 @@ class DeferredBatchNormEval:
     """Normalisation with given statistics (autograd/grad_nn.py:931-959), not launched yet: a ReLU that
     comes next is applied in the same pass, as ``DeferredBatchNorm`` has it for training."""
 
-    def __init__(self, x, gamma, beta, mean_in, var_in, eps):
+    def __init__(self, x, gamma, beta, mean_in, var_in, eps, out=None):
         self.operands = (x, gamma, beta, mean_in, var_in)
         self.eps, self.dims = float(eps), _nchw(x)
-        self.out = hiparray.lazy(x.shape)
+        self.out = hiparray.lazy(x.shape) if out is None else out
         self.stats = [hiparray.empty((self.dims[1],)) for _ in range(3)]     # mean, var + eps, sd
 
     def _launch(self, entry, out, stats):
@@ -326,8 +364,11 @@ class DeferredBatchNormEval:
         _hip.call(entry, x.ptr, _ptr(gamma), _ptr(beta), out.ptr, mean_in.ptr, var_in.ptr, stats[0].ptr, stats[1].ptr,
                   stats[2].ptr, self.eps, *self.dims)
 
+    def launch(self, relu):
+        self._launch('tt_bn_relu_fwd_eval_f32' if relu else 'tt_bn_fwd_eval_f32', self.out, self.stats)
+
     def run(self):
-        self._launch('tt_bn_fwd_eval_f32', self.out, self.stats)
+        self.launch(False)
 
     def run_with_relu(self, out=None):
         if out is None:

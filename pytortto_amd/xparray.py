@@ -127,13 +127,6 @@ def before_write(buf):
                 lazy.ptr
 
 
-def fill_all():
-    """Fill every on-demand buffer now."""
-    with _hip._lock:
-        for lazy in list(_unfilled):
-            lazy.ptr
-
-
 def poison(arrays, exc):
     """Make every later use of ``arrays`` raise ``exc``: the operation that was to fill them failed."""
     def fail(buf):
@@ -180,7 +173,14 @@ class hiparray:
         """An array whose block is allocated when its ``ptr`` is first used."""
         shape = (shape,) if isinstance(shape, int) else tuple(shape)
         dtype = np.dtype(dtype)
-        return cls(_buf=_Buffer(prod(shape) * dtype.itemsize, lazy=True), _shape=shape, dtype=dtype)
+        return cls.on(_Buffer(prod(shape) * dtype.itemsize, lazy=True), shape, dtype)
+
+    @classmethod
+    def on(cls, buf, shape, dtype):
+        """An array with a counter of its own on an existing buffer."""
+        self = object.__new__(cls)
+        self._buf, self._shape, self._dtype, self._version, self._shared = buf, shape, dtype, [0], False
+        return self
 
     @classmethod
     def zeros(cls, shape, dtype=np.float32):

@@ -1,9 +1,12 @@
-"""Operations whose launch waits for a successor, on the device: errors come from the call that is wrong."""
+"""Operations whose launch waits for a successor, on the device: errors come from the call that is wrong, and every
+value that is held has the bits of the separate launches."""
+import itertools
+
 import numpy as np
 import pytest
 
 import pytortto_amd as tt
-from pytortto_amd import _hip
+from pytortto_amd import _hip, ops
 from pytortto_amd.xparray import hiparray
 
 pytestmark = pytest.mark.gpu
@@ -59,3 +62,36 @@ def test_a_refused_evaluation_batch_norm_raises_with_and_without_gradients(behin
             F.batch_norm(wide, flat, flat)
         with pytest.raises(RuntimeError, match='must be positive'):
             F.batch_norm(tt.Tensor(hiparray.zeros((0, 8, 2, 2))), _tensor(8), _tensor(8))
+
+
+@pytest.mark.parametrize('norm,add,relu', [v for v in itertools.product((0, 1), (0, 1), (0, 1, 2)) if any(v)])
+def test_values_held_between_are_those_of_separate_launches(norm, add, relu):
+    """Each set of values in between that a caller can hold; relu 2: in place."""
+    n, c, k = 2, 6, 20
+    x, w, residual, beta, mean, gamma = (_tensor(*s, seed=i) for i, s in
+                                         enumerate(((n, c, 9, 7), (k, c, 3, 3), (n, k, 9, 7), (k,), (k,), (k,))))
+    var = tt.Tensor(hiparray(np.random.default_rng(9).uniform(0.1, 2, k).astype(np.float32)))
+    want = [ops.conv2d_fwd(x.data, w.data, None, (1, 1), (1, 1), (1, 1), 1)]
+    if norm:
+        want.append(ops.bn_fwd_eval(want[-1], gamma.data, beta.data, mean.data, var.data, 1e-5)[0])
+    if add:
+        want.append(ops.add(want[-1], residual.data))
+    if relu == 1:
+        want.append(ops.relu_fwd(want[-1]))
+    elif relu:
+        want[-1] = ops.relu_fwd(want[-1])
+    steps = ([lambda v: F.batch_norm(v, mean, var, gamma, beta)] if norm else []) + ([lambda v: v + residual] if add else []) + \
+        ([lambda v: F.relu(v, inplace=relu == 2)] if relu else [])
+    with tt.no_grad():
+        for held in itertools.product((False, True), repeat=len(steps)):
+            values = []
+            h = F.conv2d(x, w, padding=(1, 1))
+            for step, keep in zip(steps, held):
+                values.append(h if keep else None)
+                h = step(h)
+            values = values[:len(want) - 1] + [h]
+            x_was = x.data.get()            # a call into the library: the launch happens here
+            for got, ref in zip(values, want):
+                if got is not None:
+                    np.testing.assert_array_equal(got.data.get(), ref.get())
+            assert x_was.any()

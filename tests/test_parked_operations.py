@@ -56,7 +56,9 @@ def _on_device(module):
     return module
 
 
-CONV, NORM, NORM_EVAL = 'tt_conv2d_fwd_f32', 'tt_bn_act_fwd_train_f32', 'tt_bn_fwd_eval_f32'
+CONV, NORM = 'tt_conv2d_fwd_f32', 'tt_bn_act_fwd_train_f32'
+CONV_WITH, EVAL, EVAL_RELU = 'tt_conv2d_norm_act_fwd_f32', 'tt_bn_fwd_eval_f32', 'tt_bn_relu_fwd_eval_f32'
+ADD, ADD_RELU, RELU = 'tt_add_f32', 'tt_add_relu_f32', 'tt_relu_fwd_f32'
 
 
 def test_a_refused_add_leaves_the_batch_norm_in_front_of_it_parked(library):
@@ -139,3 +141,74 @@ def test_what_the_library_refuses_is_raised_by_the_call(library):
         with pytest.raises(RuntimeError, match='refused by the library'):
             conv(_tensor(2, 4, 3, 5))
         assert _hip.pending() is None
+
+
+def _nothing_held(conv, bn, x):
+    return F.relu(bn(conv(x)) + x)
+
+
+def _rebound(conv, bn, x):
+    h = conv(x)
+    h = bn(h)
+    h = h + x
+    return F.relu(h)
+
+
+def _rebound_in_place(conv, bn, x):
+    h = conv(x)
+    h = bn(h)
+    return F.relu(h, inplace=True)
+
+
+def _shortcut_around_the_norm(conv, bn, x):
+    a = conv(x)
+    return conv(F.relu(bn(a))) + a
+
+
+def _residual_is_the_input_of_the_norm(conv, bn, x):
+    a = conv(x)
+    return F.relu(bn(a) + a)
+
+
+def _norm_held(conv, bn, x):
+    n = bn(conv(x))
+    return F.relu(n + x) + n
+
+
+def _sum_held(conv, bn, x):
+    s = bn(conv(x)) + x
+    return F.relu(s) + s
+
+
+def _relu_input_held(conv, bn, x):
+    a = conv(x)
+    return F.relu(a) + a
+
+
+def _all_held(conv, bn, x):
+    a = conv(x)
+    n = bn(a)
+    s = n + x
+    return a, n, s, F.relu(s)
+
+
+def _two_relus(conv, bn, x):
+    return F.relu(F.relu(conv(x)))
+
+
+@pytest.mark.parametrize('network,launches', [
+    (_nothing_held, [CONV_WITH]), (_rebound, [CONV_WITH]), (_rebound_in_place, [CONV_WITH]), (_two_relus, [CONV_WITH, RELU]),
+    (_shortcut_around_the_norm, [CONV, EVAL_RELU, CONV_WITH]), (_residual_is_the_input_of_the_norm, [CONV, EVAL, ADD_RELU]),
+    (_norm_held, [CONV_WITH, ADD_RELU, ADD]), (_sum_held, [CONV_WITH, RELU, ADD]), (_relu_input_held, [CONV, RELU, ADD]),
+    (_all_held, [CONV, EVAL, ADD, RELU])], ids=lambda v: getattr(v, '__name__', ''))
+def test_a_convolution_is_launched_once(library, network, launches):
+    """What joined the convolution is one launch with it, unless a value in between is still held when the launch
+    comes: that one is stored, and nothing is computed again to read it."""
+    conv, bn, x = _on_device(tt.nn.Conv2d(4, 4, 1)), _on_device(tt.nn.BatchNorm2d(4)), _tensor(2, 4, 3, 3)
+    bn.eval()
+    with tt.no_grad():
+        conv(x), _hip.flush(), library.launched()
+        y = network(conv, bn, x)
+        for t in y if isinstance(y, tuple) else (y,):
+            t.data.ptr
+    assert library.launched() == launches
