@@ -304,3 +304,41 @@ def test_runs_of_a_long_batch_start_aligned():
         assert 1 <= per < n and per * max(image_a, image_b) < 2 ** 31
         assert (per * image_a) % 4 == 0 and (per * image_b) % 4 == 0, (per, image_a, image_b)
         assert (per + 4) * max(image_a, image_b) >= 2 ** 31 - 1            # not needlessly short
+
+
+@pytest.mark.parametrize('how', ['in place', 'in place, a buffer', 'gradients on inside', 'by hand'])
+def test_functions_that_attach_a_tensor_without_gradients_enabled(how):
+    """A function of the user's own that hangs a tensor on its node under ``no_grad`` -- in place without an
+    ``inplace`` argument, on a tensor that is no input, or otherwise -- keeps the gradients of what lies behind."""
+    from pytortto_amd.autograd.function import Function
+    from pytortto_amd.autograd.grad_mode import enable_grad
+    from pytortto_amd.autograd.helper import build_links, inplace_update
+    buffer = tt.zeros(3)
+
+    class Double(Function):
+        @staticmethod
+        def forward(ctx, *inputs, **params):
+            xt, = inputs
+            if how == 'in place':
+                xt.data *= 2
+                return inplace_update(xt, ctx)
+            if how == 'in place, a buffer':
+                buffer.data[...] = xt.data * 2
+                return inplace_update(buffer, ctx)
+            if how == 'by hand':
+                return tt.Tensor(xt.data * 2, requires_grad=True, grad_fn=ctx, _output_idx=0)
+            with enable_grad():
+                return build_links(xt.data * 2, grad_fn=ctx)
+
+        @staticmethod
+        def backward(ctx, *grad_outputs):
+            return grad_outputs[0] * 2
+
+    x = tt.tensor(np.ones(3, np.float32), requires_grad=True)
+    other = x + tt.tensor(np.ones(3, np.float32))       # a second consumer of x's sum, in the ordinary way
+    h = other + tt.tensor(np.ones(3, np.float32))
+    with tt.no_grad():
+        y = Double.apply(h)
+    z = y + other
+    z.backward(tt.tensor(np.array([1.0, 2.0, 3.0], np.float32)))
+    np.testing.assert_array_equal(x.grad, np.array([3.0, 6.0, 9.0], np.float32))
