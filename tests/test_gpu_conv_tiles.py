@@ -27,3 +27,11 @@ def test_tile_rule(case, tile):
 def test_weight_gradient_rows_that_fill_no_128(k, c, r):
     """Rows and columns on either side of the lines between 64- and 128-wide tiles."""
     _run_conv((3, c, 11, 9, k, r, r, (1, 1), (r // 2, r // 2), (1, 1), 1))
+
+
+@pytest.mark.parametrize('case,sharing', [((1, 16, 9, 9, 336, 1, 1, (1, 1), (0, 0), (1, 1), 1), 5),        # two tiles of 21 steps, eight to a block
+                                          ((8, 128, 28, 28, 128, 3, 3, (1, 1), (1, 1), (1, 1), 1), 441)])  # 49
+def test_blocks_without_a_share_are_not_launched(case, sharing):
+    _run_conv(case)
+    plan = _last_launch()
+    assert plan['whole_tiles'] == 0 and plan['persistent_blocks'] == plan['sharing_blocks'] == sharing
