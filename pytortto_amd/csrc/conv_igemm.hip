@@ -185,8 +185,11 @@ bool wants_stream_k(long long tiles, int chunks, int groups, bool fewest) {
     // dozen steps (16 channels from 32 over 3x3, 128 tiles of 18 steps: 31.7 us split, 14.5 whole; a
     // classifier's 2048 to 10, one tile of 128 steps: 81 us whole, 17.5 split).
     const long long share = std::max(8LL, (tiles * chunks + sk_blocks_f32() - 1) / sk_blocks_f32());
-    if (chunks <= share + 12 && !bf16_math()) return false;   // (those kernels' steps are too short to count)
-    if (fewest) return true;
+    if (chunks <= share + 12 && !bf16_math()) return false;
+    // (bf16 arithmetic: the same line lies at 16 steps, measured on 244 launches of 1 to 150 tiles: below it a
+    // split loses up to a fifth, 100 tiles of 9 steps 11.3 us for 9.0, from it on it gains, 25 tiles of 32 steps
+    // 9.5 us for 14.3, but for 2 % on 42 tiles of 16)
+    if (fewest && (!bf16_math() || chunks >= 16)) return true;
   }
   if (tiles * chunks < 4LL * sk_blocks_f32()) return false;
   const long long rounds = (tiles + cus() - 1) / cus();

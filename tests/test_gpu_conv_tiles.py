@@ -2,6 +2,8 @@
 the device, and few tiles with a long reduction, which is shared between blocks where that shortens it."""
 import pytest
 
+from pytortto_amd import _hip, ops
+from pytortto_amd.xparray import hiparray
 from tests.test_gpu_conv import _last_launch, _run_conv
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +37,18 @@ def test_blocks_without_a_share_are_not_launched(case, sharing):
     _run_conv(case)
     plan = _last_launch()
     assert plan['whole_tiles'] == 0 and plan['persistent_blocks'] == plan['sharing_blocks'] == sharing
+
+
+@pytest.mark.parametrize('case,sharing', [((1, 150, 9, 9, 100, 1, 1, (1, 1), (0, 0), (1, 1), 1), 0),       # 10 steps
+                                          ((1, 241, 9, 9, 100, 1, 1, (1, 1), (0, 0), (1, 1), 1), 8),       # 16, four tiles
+                                          ((8, 138, 20, 20, 128, 1, 1, (1, 1), (0, 0), (1, 1), 1), 0)])    # 9, a hundred tiles
+def test_split_rule_in_bf16_arithmetic(case, sharing):
+    n, c, h, w, k, r, s, stride, pad, dil, groups = case
+    x, wt = hiparray.zeros((n, c, h, w)), hiparray.zeros((k, c, r, s))
+    _hip.set_conv_math('bf16')
+    try:
+        ops.conv2d_fwd(x, wt, None, stride, pad, dil, groups)
+        plan = _last_launch()
+    finally:
+        _hip.set_conv_math('f32')
+    assert plan['persistent_blocks'] == plan['sharing_blocks'] == sharing
