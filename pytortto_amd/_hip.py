@@ -152,18 +152,28 @@ def lib():
 # read by thread B, whose first use of it must find the operation run), so every access goes
 # through one re-entrant lock: parking, the test-and-take of a fusing successor and the flush are
 # each atomic, and a flush started by one thread is finished before another thread's call proceeds.
+#
+# An operation of a kind that ``queues`` waits for one more of its kind to be parked behind it: it never
+# stores a value that nobody holds any more, and in ``h = conv(relu(norm(h)))`` the name has let go of the
+# first convolution's output only once the second has returned.
 _pending = None
+_earlier = None         # parked in front of ``_pending``; never without it
 _lock = threading.RLock()
 
 
 def defer(op):
-    """Park ``op`` (an object with ``run()``); whatever was parked before runs now.  Should that fail, ``op`` will
-    never run either, and its arrays are marked."""
-    global _pending
+    """Park ``op`` (an object with ``run()``); whatever was parked before runs now, but for one that ``queues``
+    in front of another.  Should that fail, ``op`` will never run either, and its arrays are marked."""
+    global _pending, _earlier
     with _lock:
         if _pending is not None:
             try:
-                flush()
+                if getattr(op, 'queues', False) and getattr(_pending, 'queues', False):
+                    if _earlier is not None:
+                        _run_earlier()
+                    _earlier = _pending
+                else:
+                    flush()
             except Exception as exc:
                 _poison(op, exc)
                 raise
@@ -175,22 +185,20 @@ def pending():
 
 
 def take_pending():
-    global _pending
-    with _lock:
-        op, _pending = _pending, None
-    return op
+    return take_pending_if(lambda op: True)
 
 
 def take_pending_if(wanted):
-    """The parked operation, removed from the slot, if ``wanted(op)`` holds for it -- test and take
+    """The operation parked last, removed from the slot, if ``wanted(op)`` holds for it -- test and take
     in one step, so that no other thread can run or steal it in between; otherwise None (and the
     operation stays parked)."""
     global _pending
     with _lock:
-        op = _pending
-        if op is None or not wanted(op):
+        if _pending is None or not wanted(_pending):
             return None
-        _pending = None
+        if _earlier is not None:
+            _run_earlier()
+        op, _pending = _pending, None
     return op
 
 
@@ -209,6 +217,8 @@ def join_pending(wanted, join):
             return join(op)
         except Exception as exc:
             _poison(op, exc)
+            if _earlier is not None:
+                _run_earlier()
             raise
 
 
@@ -219,18 +229,32 @@ def _poison(op, exc):
         poison(exc)
 
 
+def _run(op):
+    try:
+        op.run()
+    except Exception as exc:
+        _poison(op, exc)
+        raise
+
+
+def _run_earlier():
+    global _pending, _earlier
+    op, _earlier, last, _pending = _earlier, None, _pending, None
+    try:
+        _run(op)                # its calls into the library find nothing parked
+    finally:
+        _pending = last
+
+
 def flush():
-    """Run the parked operation, if any.  Should it fail, the arrays it was to fill are marked."""
+    """Run what is parked.  Should an operation fail, the arrays it was to fill are marked."""
     global _pending
     with _lock:
+        if _earlier is not None:
+            _run_earlier()
         op, _pending = _pending, None
-        if op is None:
-            return
-        try:
-            op.run()
-        except Exception as exc:
-            _poison(op, exc)
-            raise
+        if op is not None:
+            _run(op)
 
 
 def call(name, *args):

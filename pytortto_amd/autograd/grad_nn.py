@@ -181,10 +181,10 @@ class BatchNorm(Function):
                 yd0 = _hip.join_pending(lambda op: op.__class__ is ops.DeferredConv and op.takes_norm()
                                         and op.out._buf is xd0._buf and op.out.shape == xd0.shape
                                         and ops.computes_on(*stats), lambda op: op.absorb_norm(*stats, eps))
-                if yd0 is not None:
-                    return build_links(yd0, grad_fn=ctx)
-            yd0, mean, var_eps, sd = ops.bn_fwd_eval(xd0, gamma, beta, running_mean.data, running_var.data, eps,
-                                                       deferred=no_gradient)
+                if yd0 is None:
+                    yd0, = ops.bn_fwd_eval(xd0, gamma, beta, running_mean.data, running_var.data, eps, deferred=True)
+                return build_links(yd0, grad_fn=ctx)
+            yd0, mean, var_eps, sd = ops.bn_fwd_eval(xd0, gamma, beta, running_mean.data, running_var.data, eps)
         elif xd0.size == xd0.shape[1]:
             # eval mode without buffers and one value per channel: the batch statistics are the value
             # itself and zero (grad_nn.py:935-937); only training refuses this shape (:921-922)

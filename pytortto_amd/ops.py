@@ -16,6 +16,9 @@ from . import _hip
 from .xparray import hiparray, poison
 
 
+_F32 = np.dtype(np.float32)
+
+
 def _ptr(a):
     return None if a is None else a.ptr
 
@@ -29,7 +32,7 @@ def _f32(*arrays):
 def computes_on(*arrays):
     """Whether the device path takes all of them (None: not given) as operands."""
     for a in arrays:
-        if a is not None and (a.__class__ is not hiparray or a._dtype != np.float32):
+        if a is not None and (a.__class__ is not hiparray or a._dtype is not _F32 and a._dtype != _F32):
             return False
     return True
 
@@ -75,7 +78,9 @@ class DeferredConv:
     A value in between that nobody holds any more when the launch comes is never stored.  One that is still
     held may be read (a shortcut around the BatchNorm): it is stored where it stands, and what follows it runs
     in kernels of its own (same bits), so that no convolution is ever computed twice.  The ReLU is parked with the
-    rest for that reason: its caller's names for the values in front of it are gone when the next call comes."""
+    rest, and all of it stays parked behind the next convolution until a third, or another call, comes: by then the
+    caller's names for the values in front are mostly gone."""
+    queues = True
 
     def __init__(self, x, w, bias, shape, dims):
         self.x, self.w, self.bias, self.dims = x, w, bias, dims
@@ -160,9 +165,11 @@ class DeferredConv:
 
 
 @functools.lru_cache(maxsize=1024, typed=True)
-def _conv2d_fwd_accepts(*dims):
+def _conv2d_fwd_accepts(elements, *dims):
     """Whether the C entry point takes this geometry, by its own argument checks (the size query runs them and
-    launches nothing); asked once per geometry."""
+    launches nothing), in one run of images (the larger tensor's ``elements`` say so); asked once per geometry."""
+    if 0 in dims[:4] or elements >= 1 << 31:
+        return False
     try:
         return _hip.lib().tt_workspace_size_conv2d_fwd_f32(ctypes.byref(ctypes.c_size_t()), *dims) == 0
     except ctypes.ArgumentError:
@@ -173,7 +180,7 @@ def conv2d_fwd_deferred(x, w, bias, stride, padding, dilation, groups):
     """``conv2d_fwd`` with the launch parked for the operations behind it to join.  What would be refused is
     launched at once, so that the error is raised where it belongs, and so is a batch that is cut into runs."""
     shape, dims = _conv2d_geometry(x, w, bias, stride, padding, dilation, groups)
-    if 0 in x.shape or max(x.size, prod(shape)) >= 1 << 31 or not _conv2d_fwd_accepts(*dims):
+    if not _conv2d_fwd_accepts(max(prod(x.shape), prod(shape)), *dims):
         return conv2d_fwd(x, w, bias, stride, padding, dilation, groups)
     op = DeferredConv(x, w, bias, shape, dims)
     _hip.defer(op)
@@ -353,19 +360,23 @@ class DeferredBatchNormEval:
     """Normalisation with given statistics (autograd/grad_nn.py:931-959), not launched yet: a ReLU that
     comes next is applied in the same pass, as ``DeferredBatchNorm`` has it for training."""
 
-    def __init__(self, x, gamma, beta, mean_in, var_in, eps, out=None):
+    def __init__(self, x, gamma, beta, mean_in, var_in, eps, out=None, keep_stats=False):
         self.operands = (x, gamma, beta, mean_in, var_in)
         self.eps, self.dims = float(eps), _nchw(x)
         self.out = hiparray.lazy(x.shape) if out is None else out
-        self.stats = [hiparray.empty((self.dims[1],)) for _ in range(3)]     # mean, var + eps, sd
+        self.stats = [hiparray.empty((self.dims[1],)) for _ in range(3)] if keep_stats else []   # mean, var + eps, sd
 
-    def _launch(self, entry, out, stats):
+    def _launch(self, entry, out):
         x, gamma, beta, mean_in, var_in = self.operands
-        _hip.call(entry, x.ptr, _ptr(gamma), _ptr(beta), out.ptr, mean_in.ptr, var_in.ptr, stats[0].ptr, stats[1].ptr,
-                  stats[2].ptr, self.eps, *self.dims)
+        if self.stats:
+            stats = [a.ptr for a in self.stats]
+        else:                                               # nobody reads them
+            scratch, step = hiparray.empty((3 * self.dims[1],)), 4 * self.dims[1]
+            stats = [scratch.ptr, scratch.ptr + step, scratch.ptr + 2 * step]
+        _hip.call(entry, x.ptr, _ptr(gamma), _ptr(beta), out.ptr, mean_in.ptr, var_in.ptr, *stats, self.eps, *self.dims)
 
     def launch(self, relu):
-        self._launch('tt_bn_relu_fwd_eval_f32' if relu else 'tt_bn_fwd_eval_f32', self.out, self.stats)
+        self._launch('tt_bn_relu_fwd_eval_f32' if relu else 'tt_bn_fwd_eval_f32', self.out)
 
     def run(self):
         self.launch(False)
@@ -374,10 +385,8 @@ class DeferredBatchNormEval:
         if out is None:
             out = self.out
         else:
-            def recompute(buf):
-                self._launch('tt_bn_fwd_eval_f32', buf, [hiparray.empty((self.dims[1],)) for _ in range(3)])
-            self.out._buf.fill_on_demand(recompute, self.operands)
-        self._launch('tt_bn_relu_fwd_eval_f32', out, self.stats)
+            self.out._buf.fill_on_demand(lambda buf: self._launch('tt_bn_fwd_eval_f32', buf), self.operands)
+        self._launch('tt_bn_relu_fwd_eval_f32', out)
         return out
 
     def poison(self, exc):
@@ -385,16 +394,16 @@ class DeferredBatchNormEval:
 
 
 def bn_fwd_eval(x, gamma, beta, mean_in, var_in, eps, deferred=False):
-    """(y, mean, var + eps, sd); with ``deferred`` the launch is parked for a ReLU to join, unless it would be
-    refused: that error is raised here."""
+    """[y, mean, var + eps, sd]; with ``deferred`` [y], whose launch is parked for a ReLU to join, unless it would
+    be refused: that error is raised here."""
     _f32(x, gamma, beta, mean_in, var_in)
-    op = DeferredBatchNormEval(x, gamma, beta, mean_in, var_in, eps)
+    op = DeferredBatchNormEval(x, gamma, beta, mean_in, var_in, eps, keep_stats=not deferred)
     n, c, hw = op.dims
-    if deferred and computes_on(*op.operands) and 0 < x.size and c <= _BN_CHANNELS and max(n, c) * hw < 1 << 31:
+    if deferred and n and hw and 0 < c <= _BN_CHANNELS and max(n, c) * hw < 1 << 31 and computes_on(*op.operands):
         _hip.defer(op)
     else:
         op.run()
-    return (op.out, *op.stats)
+    return [op.out, *op.stats]
 
 
 def bn_bwd(x, dy, gamma, mean, var_eps, sd, need=(True, True, True), coef=None, add=None):

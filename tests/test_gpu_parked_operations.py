@@ -64,8 +64,19 @@ def test_a_refused_evaluation_batch_norm_raises_with_and_without_gradients(behin
             F.batch_norm(tt.Tensor(hiparray.zeros((0, 8, 2, 2))), _tensor(8), _tensor(8))
 
 
+@pytest.fixture(params=['f32', 'bf16', 'bf16x3', 'channel-last'])
+def math(request):
+    _hip.set_conv_math('bf16' if request.param == 'channel-last' else request.param)
+    _hip.call('tt_conv2d_bf16_first_enable', 2 if request.param == 'channel-last' else 1)
+    try:
+        yield request.param
+    finally:
+        _hip.call('tt_conv2d_bf16_first_enable', 1)
+        _hip.set_conv_math('f32')
+
+
 @pytest.mark.parametrize('norm,add,relu', [v for v in itertools.product((0, 1), (0, 1), (0, 1, 2)) if any(v)])
-def test_values_held_between_are_those_of_separate_launches(norm, add, relu):
+def test_values_held_between_are_those_of_separate_launches(norm, add, relu, math):
     """Each set of values in between that a caller can hold; relu 2: in place."""
     n, c, k = 2, 6, 20
     x, w, residual, beta, mean, gamma = (_tensor(*s, seed=i) for i, s in

@@ -40,6 +40,7 @@ def library(monkeypatch):
     monkeypatch.setattr(_hip, '_lib', stand_in)
     monkeypatch.setattr(_hip, '_ready', True)
     monkeypatch.setattr(_hip, '_pending', None)
+    monkeypatch.setattr(_hip, '_earlier', None)
     ops._conv2d_fwd_accepts.cache_clear()
     yield stand_in
     ops._conv2d_fwd_accepts.cache_clear()
@@ -160,6 +161,16 @@ def _rebound_in_place(conv, bn, x):
     return F.relu(h, inplace=True)
 
 
+def _rebound_late(conv, bn, x):
+    h = conv(x)
+    h = conv(F.relu(bn(h)))             # the name still holds the first value when the second convolution is called
+    return F.relu(bn(h))
+
+
+def _three_in_a_row(conv, bn, x):
+    return conv(F.relu(conv(bn(conv(x)))))
+
+
 def _shortcut_around_the_norm(conv, bn, x):
     a = conv(x)
     return conv(F.relu(bn(a))) + a
@@ -198,6 +209,7 @@ def _two_relus(conv, bn, x):
 
 @pytest.mark.parametrize('network,launches', [
     (_nothing_held, [CONV_WITH]), (_rebound, [CONV_WITH]), (_rebound_in_place, [CONV_WITH]), (_two_relus, [CONV_WITH, RELU]),
+    (_rebound_late, [CONV_WITH, CONV_WITH]), (_three_in_a_row, [CONV_WITH, CONV_WITH, CONV]),
     (_shortcut_around_the_norm, [CONV, EVAL_RELU, CONV_WITH]), (_residual_is_the_input_of_the_norm, [CONV, EVAL, ADD_RELU]),
     (_norm_held, [CONV_WITH, ADD_RELU, ADD]), (_sum_held, [CONV_WITH, RELU, ADD]), (_relu_input_held, [CONV, RELU, ADD]),
     (_all_held, [CONV, EVAL, ADD, RELU])], ids=lambda v: getattr(v, '__name__', ''))
@@ -212,3 +224,30 @@ def test_a_convolution_is_launched_once(library, network, launches):
         for t in y if isinstance(y, tuple) else (y,):
             t.data.ptr
     assert library.launched() == launches
+
+
+def test_a_failing_convolution_leaves_the_one_behind_it_parked(library):
+    """Two convolutions are parked; the first fails when a third comes: its own arrays and the third's raise, the
+    second is launched as it would have been."""
+    conv, x = _on_device(tt.nn.Conv2d(4, 4, 1)), _tensor(2, 4, 3, 3)
+    with tt.no_grad():
+        first, second = conv(x), conv(x)
+        library.launched()
+        library.fail = {CONV}
+        with pytest.raises(RuntimeError, match='refused by the library'):
+            conv(x)
+        library.fail = set()
+    with pytest.raises(RuntimeError, match='refused by the library'):
+        first.data.ptr
+    library.launched()
+    second.data.ptr
+    assert library.launched() == [CONV] and _hip.pending() is None
+
+
+def test_taking_the_last_operation_runs_the_one_in_front_of_it(library):
+    conv, x = _on_device(tt.nn.Conv2d(4, 4, 1)), _tensor(2, 4, 3, 3)
+    with tt.no_grad():
+        first, second = conv(x), conv(x)
+        library.launched()
+        assert _hip.take_pending().out is second.data and library.launched() == [CONV]
+        assert first.data._buf._ptr and not second.data._buf._ptr
