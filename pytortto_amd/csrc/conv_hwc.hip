@@ -118,7 +118,7 @@ struct Hwc {
   int cchunks;         // chunks of one tap
   int chunks;          // taps * cchunks
   int perSplit;
-  int taps, S;         // tap t = (t / S, t % S)
+  int S;               // tap t = (t / S, t % S)
   int rowBytes;        // of wt
   int pixBytes, imgBytes;   // of xt
   int bias;            // bytes added to every pixel offset so that it is never negative
@@ -427,7 +427,7 @@ int hwc_conv(const HwcConv& c, const float* x, const float* w, const float* bias
   q.imgBytes = q.pixBytes * c.H * c.W;
   q.rowBytes = q.pixBytes * taps;
   q.cchunks = pl.chunks / taps; q.chunks = pl.chunks; q.perSplit = pl.perSplit;
-  q.taps = taps; q.R = c.R; q.S = c.S;
+  q.R = c.R; q.S = c.S;
   q.bias = q.pixBytes * (std::max(c.ph, 0) * c.W + std::max(c.pw, 0));
   q.tapRow = q.pixBytes * c.dh * c.W; q.tapCol = q.pixBytes * c.dw;
   q.stepH = c.dh; q.stepW = c.dw;
@@ -443,7 +443,7 @@ int hwc_conv(const HwcConv& c, const float* x, const float* w, const float* bias
     TT_LAUNCH_CHECK();
   }
   const int tiles = (pl.Ipad / (64 * pl.mt)) * ceil_div(p.M, 64 * pl.nt);
-  const int plan[8] = {64 * pl.mt, 64 * pl.nt, tiles, pl.Ipad / (64 * pl.mt), -1, tiles, 0, kModeTapMask | 1 << 8};
+  const int plan[8] = {64 * pl.mt, 64 * pl.nt, tiles, pl.Ipad / (64 * pl.mt), -2, tiles, 0, kModeTapMask | 1 << 8};
   std::copy(plan, plan + 8, plan8);
   tt::ProfScope prof(prof_id);
   const dim3 grid((unsigned)tiles, 1, (unsigned)pl.splits);

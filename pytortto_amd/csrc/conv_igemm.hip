@@ -215,8 +215,9 @@ int sk_launch_blocks() { return bf16_math() ? 3 * cus() : sk_blocks_f32(); }
 
 // 128x128 by default, 64 rows when a group has no more than 64 of them, 32 when it has no more than 32
 // and there are tiles enough (the float32 schedules: an empty row costs as much matrix time as a full
-// one; 8 rows per group, 41 us in 64-row tiles, 30 in these).  When that leaves CUs idle or unevenly loaded the reduction is split stream-K fashion; if it is
-// too short for that, 64x64 tiles raise the block count instead.  `small` asks for 64x64 tiles outright:
+// one; 8 rows per group, 41 us in 64-row tiles, 30 in these).  When that leaves CUs idle or unevenly loaded
+// the reduction is split stream-K fashion; if it is too short for that, 64x64 tiles raise the block count
+// instead.  `small` asks for 64x64 tiles outright:
 // many light blocks (four or five resident per CU) balance better and exchange no partial sums where a
 // tile's reduction is short (plain matrix products with at most 32 chunks) or where several
 // short launches share a grid (the stride-parity classes of an input gradient).
@@ -321,8 +322,9 @@ int g_last_launch[8] = {};
 bool g_bf16_first = true;
 bool g_bf16_first_always = false;   // tests: also where the tile-count rule would keep the other kernels
 
-// Whether the channel-last kernels (conv_hwc.hip) are to be asked; tests switch them with the bf16-first ones.
-bool hwc_math(int groups) { return groups == 1 && bf16_math() && g_bf16_first; }
+// Whether the channel-last kernels (conv_hwc.hip) are to be asked, and whether they take all they support.
+bool g_hwc = true, g_hwc_always = false;
+bool hwc_math(int groups) { return groups == 1 && bf16_math() && g_hwc; }
 
 int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_partial) {
   tt::ProfScope prof(prof_id);
@@ -648,8 +650,10 @@ int tt_conv2d_stream_k_blocks_per_cu(int bf16, int* blocks) {
 
 // Instrumentation (tests): the plan of the last single matrix-product launch of a forward or input
 // gradient call: {tile rows, tile columns (pixels), tiles, row tiles, blocks of the persistent grid
-// (0: one tile per block; -1: one tile per block on the bf16-first kernels), tiles computed whole (the rest share their reduction between blocks),
-// blocks sharing them, addressing mode | bf16 terms per operand element << 8 (0: float32 matrix instructions)}.  Pixel tile t starts at pixel (t / row tiles) * tile columns.
+// (0: one tile per block; -1: one tile per block on the bf16-first kernels, -2: on the channel-last ones), tiles
+// computed whole (the rest share their reduction between blocks), blocks sharing them, addressing mode | bf16
+// terms per operand element << 8 (0: float32 matrix instructions)}.  Pixel tile t starts at pixel
+// (t / row tiles) * tile columns.
 int tt_conv2d_last_launch(int* plan8) {
   TT_API_LOCK();
   TT_REQUIRE(plan8 != nullptr, "tt_conv2d_last_launch: null result pointer");
@@ -657,12 +661,16 @@ int tt_conv2d_last_launch(int* plan8) {
   return 0;
 }
 
-// Instrumentation (tests): with bf16 arithmetic selected, route the launches the bf16-first and the
-// channel-last kernels support to them (1, the default) or keep everything on the float32 kernels' bf16 instantiations (0).
+// Instrumentation (tests): with bf16 arithmetic selected, which kernels are asked.  0: the float32 kernels' bf16
+// instantiations only; 1 (the default): the channel-last and the bf16-first kernels where they are faster; 2: the
+// bf16-first kernels for all they support, whatever its size, and no channel-last ones; 3: the channel-last
+// kernels for all they support, otherwise as 1.
 int tt_conv2d_bf16_first_enable(int on) {
   TT_API_LOCK();
   g_bf16_first = on != 0;
-  g_bf16_first_always = on == 2;   // 2: every supported launch, whatever its tile count (small test shapes)
+  g_bf16_first_always = on == 2;
+  g_hwc = on != 0 && on != 2;
+  g_hwc_always = on == 3;
   return 0;
 }
 
@@ -708,7 +716,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
   const int Cg = C / groups, Kg = K / groups;
   if (hwc_math(groups) && !check_only) {
     const HwcConv hc{N, C, H, W, K, P, Q, R, S, sh, sw, ph, pw, dh, dw, false};
-    if (hwc_supported(hc, g_bf16_first_always)) {
+    if (hwc_supported(hc, g_hwc_always)) {
       if (size_only) {
         *size_only = hwc_workspace(hc);
         return 0;
@@ -773,8 +781,8 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
   TT_API_LOCK();
   if (!check_only) {
     TT_REQUIRE_INIT();
-    TT_REQUIRE(dy && w && dx, "tt_conv2d_dgrad_f32: null tensor pointer");
-    TT_REQUIRE_ALIGNED("tt_conv2d_dgrad_f32", dy, w, dx);
+    TT_REQUIRE(dy && w && dx, "%s: null tensor pointer", fn);
+    TT_REQUIRE_ALIGNED(fn, dy, w, dx);
   }
   if (check_common(fn, N, C, Hx, Wx, K, R, S, sh, sw, ph, pw, dh, dw, groups, P, Q)) return -1;
   const long long dy_elems = (long long)N * K * P * Q;
@@ -790,7 +798,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
   if (hwc_math(groups) && !check_only && sh == 1 && sw == 1) {
     // dx[h] reads dy[h + ph - r*dh]: a convolution of dy with the taps in reverse order
     const HwcConv hc{N, K, P, Q, C, Hx, Wx, R, S, 1, 1, (R - 1) * dh - ph, (S - 1) * dw - pw, dh, dw, true};
-    if (hwc_supported(hc, g_bf16_first_always)) {
+    if (hwc_supported(hc, g_hwc_always)) {
       if (size_only) {
         *size_only = hwc_workspace(hc);
         return 0;
@@ -803,7 +811,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
   const int eh = dh / gh, ew = dw / gw;          // dy row/column step per tap
 
   const int classes = sh * sw;
-  TT_REQUIRE(classes <= 4096, "tt_conv2d_dgrad_f32: stride %d x %d not supported", sh, sw);
+  TT_REQUIRE(classes <= 4096, "%s: stride %d x %d not supported", fn, sh, sw);
   hipStream_t st = check_only ? nullptr : tt::stream();
 
   if (groups == 1 && classes > 1 && classes * Cg <= 64 && Hx >= sh && Wx >= sw) {

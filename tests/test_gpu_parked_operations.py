@@ -67,7 +67,7 @@ def test_a_refused_evaluation_batch_norm_raises_with_and_without_gradients(behin
 @pytest.fixture(params=['f32', 'bf16', 'bf16x3', 'channel-last'])
 def math(request):
     _hip.set_conv_math('bf16' if request.param == 'channel-last' else request.param)
-    _hip.call('tt_conv2d_bf16_first_enable', 2 if request.param == 'channel-last' else 1)
+    _hip.call('tt_conv2d_bf16_first_enable', 3 if request.param == 'channel-last' else 1)
     try:
         yield request.param
     finally:
