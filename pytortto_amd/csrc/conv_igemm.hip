@@ -777,7 +777,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
 static int conv2d_dgrad(const float* dy, const float* w, const float* bias, float* dx, int N, int C, int Hx, int Wx,
                         int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups, int P,
                         int Q, size_t* size_only, bool check_only = false, const Epilogue* epi = nullptr) {
-  const char* fn = "tt_conv2d_dgrad_f32";
+  const char* fn = epi ? "tt_conv2d_dgrad_acc_f32" : "tt_conv2d_dgrad_f32";
   TT_API_LOCK();
   if (!check_only) {
     TT_REQUIRE_INIT();

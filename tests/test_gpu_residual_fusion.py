@@ -166,3 +166,10 @@ def test_values_between_stay_readable():
     _same_bits(t.data, total)
     _same_bits(y.data, ops.relu_fwd(total))
     assert bn.num_batches_tracked.item() == 1.0
+
+
+def test_errors_name_the_entry_point_that_was_called():
+    dy, wt, other = hiparray.zeros((1, 6, 8, 8)), hiparray.zeros((6, 2, 3, 3)), hiparray.zeros((1, 8, 8, 8))
+    for add, name in ((None, 'tt_conv2d_dgrad_f32'), (other, 'tt_conv2d_dgrad_acc_f32')):
+        with pytest.raises(RuntimeError, match=f'^{name}: channels'):
+            ops.conv2d_dgrad(dy, wt, None, (8, 8), (1, 1), (1, 1), (1, 1), 4, add=add)
