@@ -589,6 +589,34 @@ def cpu_baseline_bn(batch_div):
     return nbytes, seconds
 
 
+# keys that the result line carries as they are; the rest of the results is cut to its figures there
+HEADLINE = ('metric', 'value', 'unit', 'n_gpus', 'steps', 'warmup', 'ms_per_step', 'higher_is_better', 'scaling', 'vs_baseline',
+            'dtype', 'data', 'config', 'pct_of_peak', 'wall_ms_per_step', 'wgrad_tflops')
+
+
+def result_line(out):
+    """The results as one short line (some 3 KB): the headline whole, every other section with its numbers and
+    units only, without its tables and explanations, which ``--details`` writes to a file."""
+    def figures(section):
+        kept = {}
+        for key, v in section.items():
+            if isinstance(v, (int, float)) or key in ('unit', 'bound', 'kernel'):
+                kept[key] = v
+            elif isinstance(v, dict) and key not in ('config', 'roofline', 'cpu_baseline', 'kernels_ms_per_step'):
+                inner = {k: u for k, u in v.items() if isinstance(u, (int, float)) or k == 'unit'}
+                if inner:
+                    kept[key] = inner
+        return kept
+    line = {k: out[k] for k in HEADLINE}
+    line['roofline'] = {k: v for k, v in out['roofline'].items() if not isinstance(v, dict)}
+    if out['cpu_baseline']:
+        line['cpu_baseline'] = {k: v for k, v in out['cpu_baseline'].items() if not isinstance(v, dict)}
+    for key, section in out.items():
+        if key not in line and isinstance(section, dict) and key not in ('per_layer', 'kernels_ms_per_step'):
+            line[key] = figures(section)
+    return line
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument('--gpus', type=int, default=1)
@@ -608,6 +636,7 @@ def main():
     ap.add_argument('--stack-only', choices=('preact', 'dcgan'),
                     help='run only the PreAct-ResNet-18 stack or the DCGAN generator stack and print its object '
                          '(for profiling)')
+    ap.add_argument('--details', metavar='FILE', help='write the whole results, with the per-layer tables, to this file')
     args = ap.parse_args()
     if args.gpus != 1:
         print(f'bench.py: this path runs on exactly one GPU (asked for --gpus {args.gpus}); '
@@ -704,11 +733,11 @@ def main():
                      'achieved': round(bf_igemm_tflops, 2), 'peak': PEAK_BF16_MFMA_TFLOPS, 'unit': 'TFLOP/s',
                      'frac': round(bf_igemm_tflops / PEAK_BF16_MFMA_TFLOPS, 4), 'traffic': None,
                      'speedup_over_f32_kernel': round((ms_fwd + ms_dg) / bf_igemm_ms, 2),
-                     'note': 'tensors stay fp32 in HBM.  Forward and stride-1 input gradients run on bf16-first kernels '
-                             '(operands converted on their way into LDS, 32-deep chunks): their 1x1 layers move their bytes at '
-                             'HBM speed, their 3x3 layers are bound by the address unit (one 4-byte gathered element per lane); '
-                             'launches with fewer tiles than compute units and long reductions, strided input gradients and the '
-                             'stem stay on the float32 kernels\' bf16 instantiations'},
+                     'note': 'tensors stay fp32 in HBM.  Forward and stride-1 input gradients from 128 channels on, and those with '
+                             'few tiles and a long reduction, run on channel-last kernels (x rounded and laid out once in front '
+                             'of the product); the other 3x3 layers and the 1x1 layers, which move their bytes at HBM speed, on '
+                             'bf16-first kernels (operands converted on their way into LDS, 32-deep chunks); strided input '
+                             'gradients and the stem on the float32 kernels\' bf16 instantiations'},
         'wgrad_tflops': round(flops_per_pass * args.steps / (bf_prof['conv_wgrad'][1] * 1e-3) / 1e12, 2),
         'kernels_ms_per_step': {k: round(v[1] / args.steps, 4) for k, v in bf_prof.items() if v[0]}}
     progress('convolution step in float32 arithmetic on the bf16 matrix instructions (three terms)')
@@ -775,17 +804,17 @@ def main():
     pool_shape, pool_args = (BATCH, 64, 112, 112), (3, 3, 2, 2, 1, 1, 1, 1)
     px = hiparray(rng.standard_normal(pool_shape, dtype=np.float32))
     py = hiparray.empty((BATCH, 64, 56, 56))
-    ptap = hiparray.empty((BATCH, 64, 56, 56), np.int32)
+    ptap = hiparray.empty((BATCH, 64, 56, 56), np.uint8)      # as MaxPool2d keeps them: windows of up to 256 taps
     pdx = hiparray.empty(pool_shape)
     pool_dims = (BATCH * 64, 112, 112, 56, 56)
 
     def pool_step():
-        call('tt_maxpool2d_fwd_f32', px.ptr, py.ptr, ptap.ptr, *pool_dims, *pool_args)
-        call('tt_maxpool2d_bwd_f32', py.ptr, ptap.ptr, pdx.ptr, *pool_dims, *pool_args)
+        call('tt_maxpool2d_fwd_tap8_f32', px.ptr, py.ptr, ptap.ptr, *pool_dims, *pool_args)
+        call('tt_maxpool2d_bwd_tap8_f32', py.ptr, ptap.ptr, pdx.ptr, *pool_dims, *pool_args)
 
     pool_ms, _ = timed_steps(_hip, pool_step, args.steps, args.warmup)
     pprof = profiled_steps(_hip, pool_step, args.steps)
-    # algorithmic bytes: forward reads x, writes y and the int32 taps; backward reads dy and taps, writes dx
+    # algorithmic bytes: forward reads x, writes y and a byte per tap index; backward reads dy and taps, writes dx
     pool_fwd_bytes = px.nbytes + py.nbytes + ptap.nbytes
     pool_bytes = 2 * pool_fwd_bytes
     n_pb, ms_pb = pprof['maxpool_bwd']
@@ -957,7 +986,7 @@ def main():
                     'unit': 'GB/s', 'ms_per_step': round(pool_ms, 4),
                     'pct_of_peak': round(100 * pool_bytes / (pool_ms * 1e-3) / 1e9 / PEAK_HBM_GBS, 1),
                     'config': {'workload': 'MaxPool2d(3, stride 2, padding 1) fwd+bwd fp32 NCHW at [64,64,112,112] '
-                                           '(ResNet-50 stem pooling); bytes: x + y + int32 taps, both ways'},
+                                           '(ResNet-50 stem pooling); bytes: x + y + byte taps, both ways'},
                     'roofline': {'bound': 'hbm', 'kernel': 'maxpool_bwd_scatter (reads dy, taps; writes dx)',
                                  'achieved': round(pool_bwd_gbs, 1), 'peak': PEAK_HBM_GBS, 'unit': 'GB/s',
                                  'frac': round(pool_bwd_gbs / PEAK_HBM_GBS, 4),
@@ -970,7 +999,10 @@ def main():
         'resnet50_step': model,
         'stacks': stacks,
     }
-    print(json.dumps(out))
+    if args.details:
+        with open(args.details, 'w') as f:
+            json.dump(out, f, indent=1)
+    print(json.dumps(result_line(out)))
 
 
 if __name__ == '__main__':
