@@ -958,26 +958,48 @@ static int conv2d_wgrad(const float* x, const float* dy, float* dw, int N, int C
   // (measured on the ResNet-50 shapes: 4-7 % faster there, slower for 3x3 layers).
   if (J % 128 != 0 && J % 128 <= 64) bn = 64;
   if (R == 1 && S == 1 && Kg >= 128) bn = 64;
-  // 64 rows where they pad less: matrix time goes with the padded area, and a smaller tile takes longer for
-  // its share of it (float32 schedules: 128 x 64 and 64 x 128 about 7 %, 64 x 64 about 20 %).  192 rows x
-  // 1440 columns, 24 images of 45 x 37: 303 us in 128 x 64 tiles, 244 in 64 x 128.
-  if (tt::conv_math() != TT_CONV_MATH_BF16 && Kg > 64 && Kg % 128 != 0 && Kg % 128 <= 64) {
-    auto cost = [&](int m, int n) {
-      return (double)ceil_div(Kg, m) * m * ceil_div(J, n) * n * (m * n == 16384 ? 1.0 : m * n == 8192 ? 1.07 : 1.25);
-    };
-    const double now = cost(bm, bn);
-    for (int n : {128, 64})
-      if (cost(64, n) < 0.95 * now && cost(64, n) < cost(bm, bn)) {
-        bm = 64;
-        bn = n;
-      }
-  }
-  const int tilesI = ceil_div(Kg, bm), tilesJ = ceil_div(J, bn);
-  const long long tiles = (long long)tilesI * tilesJ * groups;
   // Two blocks fit a CU (LDS), so 2 x CUs (512 on an MI355X) run at a time and all take equally
   // long: fill one such round as well as possible, or two rounds if that fills them clearly better;
   // at least 8 chunks (256 pixels) of work per split.
   const int kSlots = 2 * tt::compute_units();
+  auto splits_of = [&](long long tiles, int chunks) {
+    int splits = (int)(kSlots / tiles);
+    const int two = (int)(2 * kSlots / tiles);
+    if ((double)tiles * two / (2.0 * kSlots) > (double)tiles * splits / kSlots + 0.08) splits = two;
+    if (splits > chunks / 8) splits = chunks / 8;
+    return splits < 1 ? 1 : splits > 4096 ? 4096 : splits;
+  };
+  // 64 rows where they pad less: matrix time goes with the padded area, and a smaller tile takes longer for
+  // its share of it (float32 schedules: 128 x 64 and 64 x 128 about 7 %, 64 x 64 about 20 %).  192 rows x
+  // 1440 columns, 24 images of 45 x 37: 303 us in 128 x 64 tiles, 244 in 64 x 128.
+  // Only where the longest chain of a block gets clearly shorter, too, chunks times the time of one (64 x 128
+  // gathers twice the columns of 128 x 64): with few chunks, or many row tiles of few columns, it does not (134 x
+  // 576 of 5092 pixels 27.1 us in 128 x 64 tiles, 28.9 in 64 x 128; 541 x 101 in four groups, 1x1 stride 2, 67.8 and
+  // 82.1).  Over 90 layers of such rows: 13 % less time than in 128 rows, none slower; without this 14 % and five.
+  if (tt::conv_math() != TT_CONV_MATH_BF16 && Kg > 64 && Kg % 128 != 0 && Kg % 128 <= 64) {
+    auto area = [&](int m, int n) {
+      return (double)ceil_div(Kg, m) * m * ceil_div(J, n) * n * (m * n == 16384 ? 1.0 : m * n == 8192 ? 1.07 : 1.25);
+    };
+    const long long pixels = (long long)N * P * Q;
+    auto chain = [&](int m, int n) {
+      const long long t = (long long)ceil_div(Kg, m) * ceil_div(J, n) * groups;
+      const int chunks = ceil_div(pixels, kBK), cps = ceil_div(chunks, splits_of(t, chunks));
+      const double chunk = m * n == 16384 ? 1.0 : m == 128 ? 0.535 : n == 128 ? 0.6 : 0.3125;
+      return (double)ceil_div(t * ceil_div(chunks, cps), kSlots) * cps * chunk;
+    };
+    int m64 = bm, n64 = bn;
+    for (int n : {128, 64})
+      if (area(64, n) < 0.95 * area(bm, bn) && area(64, n) < area(m64, n64)) {
+        m64 = 64;
+        n64 = n;
+      }
+    if (chain(m64, n64) < 0.9 * chain(bm, bn)) {
+      bm = m64;
+      bn = n64;
+    }
+  }
+  const int tilesI = ceil_div(Kg, bm), tilesJ = ceil_div(J, bn);
+  const long long tiles = (long long)tilesI * tilesJ * groups;
   struct Run { int n0, n, chunks, cps, splits, slot0; };
   std::vector<Run> runs;
   int slots = 0;
@@ -986,13 +1008,7 @@ static int conv2d_wgrad(const float* x, const float* dy, float* dw, int N, int C
     r.n0 = n0;
     r.n = std::min(per_run, N - n0);
     r.chunks = ceil_div((long long)r.n * P * Q, kBK);
-    int splits = (int)(kSlots / tiles);
-    const int two = (int)(2 * kSlots / tiles);
-    if ((double)tiles * two / (2.0 * kSlots) > (double)tiles * splits / kSlots + 0.08) splits = two;
-    if (splits > r.chunks / 8) splits = r.chunks / 8;
-    if (splits < 1) splits = 1;
-    if (splits > 4096) splits = 4096;
-    r.cps = ceil_div(r.chunks, splits);
+    r.cps = ceil_div(r.chunks, splits_of(tiles, r.chunks));
     r.splits = ceil_div(r.chunks, r.cps);
     r.slot0 = slots;
     slots += r.splits;

@@ -1,5 +1,7 @@
 """The tile rule of the float32 forward and input gradient at its lines: up to 32 rows with tiles enough for
 the device, and few tiles with a long reduction, which is shared between blocks where that shortens it."""
+import ctypes
+
 import pytest
 
 from pytortto_amd import _hip, ops
@@ -52,3 +54,16 @@ def test_split_rule_in_bf16_arithmetic(case, sharing):
     finally:
         _hip.set_conv_math('f32')
     assert plan['persistent_blocks'] == plan['sharing_blocks'] == sharing
+
+
+@pytest.mark.parametrize('dims,tiles', [((24, 160, 45, 37, 192, 3, 3, 1, 1, 1, 1, 1, 1, 1), 3 * 12),      # 64 x 128
+                                        ((67, 64, 38, 8, 134, 3, 3, 2, 2, 1, 1, 1, 1, 1), 2 * 9),         # few chunks: 128 x 64
+                                        ((130, 404, 17, 12, 2164, 1, 1, 2, 2, 0, 0, 1, 1, 4), 4 * 5 * 2)])
+def test_weight_gradient_tile_rule(dims, tiles):
+    n, c, h, w, k, r, s, sh, sw, ph, pw, dh, dw, g = dims
+    p, q = ((h + 2 * ph - r) // sh + 1, (w + 2 * pw - s) // sw + 1)
+    x, dy = hiparray.zeros((n, c, h, w)), hiparray.zeros((n, k, p, q))
+    ops.conv2d_wgrad(x, dy, (k, c // g, r, s), (sh, sw), (ph, pw), (dh, dw), g)
+    plan = (ctypes.c_int * 4)()
+    _hip.call('tt_conv2d_last_wgrad_launch', plan)
+    assert plan[0] == tiles
