@@ -375,6 +375,7 @@ bool hwc_supported(const HwcConv& c, bool always) {
   const bool pointwise = taps == 1;
   if (pointwise && (c.sh != 1 || c.sw != 1 || c.ph != 0 || c.pw != 0 || (c.P * c.Q) % 4 == 0)) return false;
   const Plan pl = make_plan(c);
+  if (pl.Cp / kBK > 65535) return false;                                   // the grid of channels_last
   // 32-bit offsets inside a tile's images, the weights and the whole batch's pixels
   const long long pix = 2LL * pl.Cp, img = pix * c.H * c.W;
   const long long images = 127 / ((long long)c.P * c.Q) + 2;

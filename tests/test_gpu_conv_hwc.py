@@ -197,3 +197,13 @@ def test_accumulation_and_mask_in_the_input_gradient(case, math):
     for add, relu_y, want in ((other, None, total), (None, y, ops.relu_bwd(dx, y)), (other, y, ops.relu_bwd(total, y))):
         _same_bits(ops.conv2d_dgrad(dy, wt, None, *geometry, add=add, relu_y=relu_y), want)
         assert _plan()[4] == CHANNEL_LAST
+
+
+@pytest.mark.parametrize('c,taken', [(65535 * 64, True), (65535 * 64 + 1, False)])
+def test_more_channels_than_a_grid_has_rows(c, taken, math):
+    """The layout pass has a row of blocks for every 64 channels.  (Only the plan is asked, through the workspace.)"""
+    _hip.call('tt_conv2d_bf16_first_enable', 1)
+    nbytes = ctypes.c_size_t()
+    _hip.call('tt_workspace_size_conv2d_fwd_f32', ctypes.byref(nbytes), 2, c, 1, 1, 64, 1, 1, 1, 1, 0, 0, 1, 1, 1)
+    padded = -(-c // 64) * 64
+    assert (nbytes.value - 2 * (2 + 64) * padded < 8 * 4 * 64 * 2 + 3 * 256) == taken
