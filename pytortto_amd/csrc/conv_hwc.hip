@@ -9,11 +9,13 @@
 // out contiguously; the product then fetches 16 bytes (eight channels) per lane, for any tap, and writes
 // them to LDS as they are.  The pass costs one read of x and one write of its 2 bytes per element; the
 // layouts live in the library's workspace for the length of a call.
-// Measured with the passes around the product, batch 64, forward: 512 channels 7x7 86 us with the other
-// kernels, 55 with these (340 of 477 TFLOP/s of the product alone); 256 channels 14x14 75, 53; the same at
-// stride 2 86, 62; 64 channels 56x56 51, 73: the rule in hwc_supported.
-// The product is bound by the path into and out of LDS: a chunk of a 128 x 128 tile moves 32 KB into it
-// and 64 KB out of it, 768 cycles at 128 bytes each, for 512 cycles of matrix instructions.
+// Measured, batch 64, forward, random operands, 14.8 GFLOP each; the whole call in the other kernels, here, and
+// of that the product: 512 channels 7x7 80.5 us, 49.1, 27.9 (530 TFLOP/s); 256 channels 14x14 72.9, 49.1,
+// 30.6 (484), the same at stride 2 80.6, 57.0, 30.2; 128 channels 28x28 43.8, 42.5, 30.4; 64 channels 56x56
+// 50.2, 63.6, 44.9 (330): the rule in hwc_supported.
+// No unit bounds the product: the matrix pipe and the LDS are each busy for a fifth of its cycles (0.17 to
+// 0.19, no bank conflicts).  It is a chain of fetch, LDS and matrix instructions per chunk, with a barrier, in two
+// blocks per compute unit.
 // (In three bfloat16 terms per element the same kernels were no faster than the gathering ones: six
 // products read three times the bytes, and 6 bytes per element are written and read around them.)
 //

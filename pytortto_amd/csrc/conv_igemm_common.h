@@ -29,13 +29,12 @@ typedef const intx2 __attribute__((address_space(4))) * ConstKTab;   // constant
 // -- forward, the evaluation-mode BatchNorm, residual add and ReLU behind a convolution; backward, the
 // gradient that has already arrived for x added to this one (res) and the backward of the ReLU that
 // made x (mask) -- in the order and with the roundings of the kernels they stand in for.  `on` == 0:
-// none of it.  Bound by memory: the three
-// separate launches read and wrote y up to seven times over (a ResNet-50 evaluation pass at batch 64
-// in bf16 arithmetic spent half its time in them: 5.50 ms, 3.37 ms with this; 184 launches become 60,
-// which at batch 2 takes 3.37 ms to 2.66).  Backward, the accumulation and the mask behind a residual
-// block's input gradient were seven tensor passes and are three: with the residual add and the masks of
-// batchnorm.hip, a ResNet-50 training step at batch 64 takes 20.53 ms for 21.97, at batch 32 in bf16
-// arithmetic 9.64 for 10.27.
+// none of it.  Bound by memory: the three separate launches read and wrote y up to seven times over (a
+// ResNet-50 evaluation pass at batch 64 in bf16 arithmetic spent half its time in them: 5.50 ms, 3.37 ms with
+// this; 184 launches become 60, which at batch 2 takes 3.37 ms to 2.66).  Backward, the accumulation and
+// the mask behind a residual block's input gradient were seven tensor passes and are three: with the residual
+// add and the masks of batchnorm.hip, a ResNet-50 training step at batch 64 takes 20.53 ms for 21.97, at
+// batch 32 in bf16 arithmetic 9.64 for 10.27.
 struct Epilogue {
   const float *mean, *var, *gamma, *beta;   // [G*I] each; gamma / beta may be null
   const float* res;                         // laid out as `out`, or null
@@ -212,9 +211,9 @@ bool bf16_first_supported(const Igemm& p, int groups, int bm);
 void bf16_first_launch(const Igemm& p, int groups, int bm, hipStream_t st);
 
 
-// The channel-last kernels (conv_hwc.hip): one group, operands rounded to bfloat16.  x is [N][C][H][W], the result [N][I][P][Q]; output pixel (u, v) reads
-// input rows u*sh - ph + r*dh (ph, pw may be negative).  dgrad: w is [C][I][R][S] with its taps reversed
-// instead of [I][C][R][S].
+// The channel-last kernels (conv_hwc.hip): one group, operands rounded to bfloat16.  x is [N][C][H][W], the
+// result [N][I][P][Q]; output pixel (u, v) reads input rows u*sh - ph + r*dh (ph, pw may be negative).
+// dgrad: w is [C][I][R][S] with its taps reversed instead of [I][C][R][S].
 struct HwcConv {
   int N, C, H, W, I, P, Q, R, S, sh, sw, ph, pw, dh, dw;
   bool dgrad;
