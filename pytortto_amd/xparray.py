@@ -102,6 +102,10 @@ class _Buffer:
                     self.deps = ()
         return self._ptr
 
+    def settle(self):
+        """Have the contents now: something they come from is about to change."""
+        self.ptr
+
     def __del__(self):
         try:
             if self._ptr:
@@ -111,20 +115,45 @@ class _Buffer:
             pass
 
 
-# buffers whose contents are still to be produced on demand (normally none or a handful: the
+class _Loan(_Buffer):
+    """The contents of another buffer, for holders that only read them: the same block, until somebody is about
+    to overwrite it (``before_write``); then a copy."""
+    __slots__ = ('source',)
+
+    def __init__(self, source):
+        super().__init__(source.nbytes, lazy=True)
+        self.source = source
+        with _hip._lock:
+            self.deps = (source,)
+            _unfilled.add(self)
+
+    @property
+    def ptr(self):
+        source = self.source
+        return _Buffer.ptr.fget(self) if source is None else source.ptr
+
+    def settle(self):
+        source, self.source = self.source, None
+        self.deps = ()
+        _unfilled.discard(self)
+        if self.nbytes:
+            _hip.call('tt_memcpy_d2d', self.ptr, source.ptr, self.nbytes)
+
+
+# buffers whose contents are still to be produced on demand, or lent by another (normally none or a handful: the
 # array of an absorbed BatchNorm or Add output lives only as long as somebody holds its tensor)
 _unfilled = weakref.WeakSet()
 
 
 def before_write(buf):
     """Called before ``buf`` is overwritten in place: every on-demand buffer that would read it
-    is filled now, from the values the reference's eager evaluation saw."""
+    is filled now, from the values the reference's eager evaluation saw, and every loan of it becomes a copy."""
     if not _unfilled:
         return
     with _hip._lock:
         for lazy in list(_unfilled):
             if any(d is buf for d in lazy.deps):
-                lazy.ptr
+                lazy.settle()
 
 
 def poison(arrays, exc):
@@ -259,6 +288,13 @@ class hiparray:
         copies give it, and the copy is made only for a holder that writes."""
         self._shared = True
         other = hiparray(_buf=self._buf, _shape=self._shape, dtype=self._dtype)
+        other._shared = True
+        return other
+
+    def lent(self):
+        """This array's values as they are now, without a copy: one is made if this block is about to be
+        overwritten while a holder still has them, or if a holder is about to write them."""
+        other = hiparray.on(_Loan(self._buf), self._shape, self._dtype)
         other._shared = True
         return other
 
