@@ -262,8 +262,8 @@ int tt_conv2d_images_per_run(int N, long long image_a, long long image_b, int* p
 int tt_conv2d_last_launch(int* plan8);
 /* The same for the weight gradient, whose blocks add each other's partial sums inside the kernel
  * when the device holds the whole grid at once and leave them to a second kernel otherwise:
- *   tt_conv2d_last_wgrad_launch: {tiles, reduction splits, 1 if added inside the kernel, partial-sum
- *     slots} of the last launch (host pointer to 4 ints);
+ *   tt_conv2d_last_wgrad_launch: {tiles, reduction splits, 1 if added inside the kernel (-3: a launch of the
+ *     kernels for few rows), partial-sum slots} of the last launch (host pointer to 4 ints);
  *   tt_conv2d_wgrad_force_occupancy: pretend the device holds `blocks` blocks per compute unit
  *     (-1: ask the device). */
 /* tt_conv2d_bf16_first_enable: with TT_CONV_MATH_BF16 selected, which kernels forward and stride-1
@@ -280,6 +280,9 @@ int tt_conv2d_last_launch(int* plan8);
 int tt_conv2d_bf16_first_enable(int on);
 int tt_conv2d_last_wgrad_launch(int* plan4);
 int tt_conv2d_wgrad_force_occupancy(int blocks);
+/* Which launches go to the kernels for few rows (tt_conv2d_last_launch reports -3 blocks for them): 1 (the
+ * default): where they are faster; 0: none; 2: all that they support. */
+int tt_conv2d_narrow_enable(int on);
 
 /* out[K] = sum over n and the HW plane of t[N,K,HW]: the bias gradient gd0.sum((0,2,3)),
  * autograd/grad_nn.py:728, :774. */

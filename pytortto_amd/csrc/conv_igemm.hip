@@ -40,6 +40,7 @@
 #include <vector>
 
 #include "conv_igemm_common.h"
+#include "conv_narrow.h"
 
 namespace {
 
@@ -724,6 +725,20 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
       return hwc_conv(hc, x, w, bias, y, epi, TT_PROF_CONV_IGEMM_FWD, g_last_launch);
     }
   }
+  if (!check_only) {
+    NarrowConv nc{x, w, bias, y, Kg, Cg, groups, tt::make_fastdiv((uint32_t)Cg), {}, Cg * R * S, R * S, Kg * Cg * R * S, 1, 1, S,
+                  sh, sw, dh, dw, H, W, C * H * W, Cg * H * W, H * W, K * P * Q, Kg * P * Q, P * Q, Q, 1, 1, false, 1, {}, {}};
+    if (epi) nc.epi = *epi;
+    nc.c[0] = NarrowClass{P, Q, N * P * Q, tt::make_fastdiv((uint32_t)(P * Q)), tt::make_fastdiv((uint32_t)Q),
+                          tt::make_fastdiv((uint32_t)S), {}, -ph, -pw, R, S, 0, 0, 0, 0, 0};
+    if (narrow_conv_takes(nc, bf16_math())) {
+      if (size_only) {
+        *size_only = 0;
+        return 0;
+      }
+      return narrow_conv_launch(nc, bf16_math(), TT_PROF_CONV_IGEMM_FWD, g_last_launch);
+    }
+  }
   const int Kred = Cg * R * S;
   const int M = N * P * Q;
   const int KQ = ceil_div(Kred, 4 * kBKQ) * kBKQ;
@@ -813,6 +828,34 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
   const int classes = sh * sw;
   TT_REQUIRE(classes <= 4096, "%s: stride %d x %d not supported", fn, sh, sw);
   hipStream_t st = check_only ? nullptr : tt::stream();
+
+  if (!check_only && std::min(sh, Hx) * std::min(sw, Wx) <= kNarrowClasses) {
+    NarrowConv nc{dy, w, bias, dx, Cg, Kg, groups, tt::make_fastdiv((uint32_t)Kg), {}, R * S, Cg * R * S, Kg * Cg * R * S, rstep, sstep, S,
+                  1, 1, -eh, -ew, P, Q, K * P * Q, Kg * P * Q, P * Q, C * Hx * Wx, Cg * Hx * Wx, Hx * Wx, Wx, sh, sw, true, 0, {}, {}};
+    if (epi) nc.epi = *epi;
+    for (int ch = 0; ch < sh && ch < Hx; ++ch)
+      for (int cw = 0; cw < sw && cw < Wx; ++cw) {
+        // the first tap of the class in either direction, then every rstep-th, sstep-th
+        int r0 = -1, s0 = -1;
+        for (int r = 0; r < R && r < rstep && r0 < 0; ++r)
+          if (((ch + ph - r * dh) % sh + sh) % sh == 0) r0 = r;
+        for (int s = 0; s < S && s < sstep && s0 < 0; ++s)
+          if (((cw + pw - s * dw) % sw + sw) % sw == 0) s0 = s;
+        const int U = ceil_div(Hx - ch, sh), V = ceil_div(Wx - cw, sw);
+        const bool any = r0 >= 0 && s0 >= 0;   // a class without taps holds the bias, or zeros
+        const int TB = any ? ceil_div(R - r0, rstep) : 0, TC = any ? ceil_div(S - s0, sstep) : 1;
+        nc.c[nc.n++] = NarrowClass{U, V, N * U * V, tt::make_fastdiv((uint32_t)(U * V)), tt::make_fastdiv((uint32_t)V),
+                                   tt::make_fastdiv((uint32_t)TC), {}, any ? (ch + ph - r0 * dh) / sh : 0,
+                                   any ? (cw + pw - s0 * dw) / sw : 0, TB, TC, any ? r0 : 0, any ? s0 : 0, ch, cw, 0};
+      }
+    if (narrow_conv_takes(nc, bf16_math())) {
+      if (size_only) {
+        *size_only = 0;
+        return 0;
+      }
+      return narrow_conv_launch(nc, bf16_math(), TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
+    }
+  }
 
   if (groups == 1 && classes > 1 && classes * Cg <= 64 && Hx >= sh && Wx >= sw) {
     // tiny Cg: per-class GEMMs would fill 3 of 32 MFMA rows; stack all classes as rows instead

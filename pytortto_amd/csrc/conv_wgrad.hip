@@ -30,7 +30,7 @@
 #include <type_traits>
 #include <vector>
 
-#include "tt_common.h"
+#include "conv_narrow.h"
 
 namespace {
 
@@ -897,7 +897,7 @@ int fuse_flags(unsigned** out) {
   *out = g_fuse_flags;
   return 0;
 }
-int g_last_wgrad[4] = {};   // instrumentation: {tiles * groups, splits, partial sums added in the kernel, slots}
+int g_last_wgrad[4] = {};   // instrumentation: {tiles * groups, splits, partial sums added in the kernel (-3: conv_narrow.hip), slots}
 
 }  // namespace
 
@@ -949,6 +949,22 @@ static int conv2d_wgrad(const float* x, const float* dy, float* dw, int N, int C
   if (per_run < N && per_run >= 4) per_run -= per_run % 4;   // later runs start 16-byte aligned: vector fetches stay on
   const int Cg = C / groups, Kg = K / groups;
   const int J = Cg * R * S;
+
+  if (per_run >= N && !check_only) {
+    const bool bf16 = tt::conv_math() == TT_CONV_MATH_BF16;
+    ttc::NarrowWgrad nw{x, dy, dw, nullptr, Kg, J, N * P * Q, groups, tt::make_fastdiv((uint32_t)(P * Q)), tt::make_fastdiv((uint32_t)Q),
+                        tt::make_fastdiv((uint32_t)(R * S)), tt::make_fastdiv((uint32_t)S), H, W, H * W, P * Q, R, S, sh, sw, ph, pw,
+                        dh, dw_, C * H * W, Cg * H * W, K * P * Q, Kg * P * Q, ph * W + pw, 0, 0, 0, 0, 0, 0};
+    if (ttc::narrow_wgrad_takes(nw)) {
+      if (size_only) {
+        *size_only = ttc::narrow_wgrad_workspace(nw);
+        return 0;
+      }
+      const int plan[4] = {nw.tilesI * nw.tilesJ * groups, nw.splits, -3, nw.splits};   // -3: the kernels for few rows
+      std::copy(plan, plan + 4, g_last_wgrad);
+      return ttc::narrow_wgrad_launch(nw, bf16);
+    }
+  }
 
   int bm = 128, bn = 128;
   if (Kg <= 64) bm = 64;
