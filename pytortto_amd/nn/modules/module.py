@@ -80,9 +80,16 @@ class Module:
         self._modules[name] = module
 
     def __getattr__(self, name):
-        for registry in ('_parameters', '_buffers', '_modules'):
-            table = self.__dict__.get(registry)
-            if table is not None and name in table:
+        own = self.__dict__
+        if '_buffers' in own:           # set up; every layer of a forward pass looks two to six names up here
+            table = own['_parameters']
+            if name in table:
+                return table[name]
+            table = own['_buffers']
+            if name in table:
+                return table[name]
+            table = own['_modules']
+            if name in table:
                 return table[name]
         raise AttributeError("'{}' object has no attribute '{}'".format(type(self).__name__, name))
 

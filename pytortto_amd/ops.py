@@ -25,7 +25,7 @@ def _ptr(a):
 
 def _f32(*arrays):
     for a in arrays:
-        if a is not None and a.dtype != np.float32:
+        if a is not None and a.dtype is not _F32 and a.dtype != _F32:
             raise TypeError(f'the device path computes in float32 only, got {a.dtype}')
 
 
@@ -42,20 +42,27 @@ def conv_out_size(size, k, stride, pad, dil):
     return math.floor((size + 2 * pad - dil * (k - 1) - 1) / stride + 1)
 
 
+@functools.lru_cache(maxsize=1024, typed=True)
+def _conv2d_shapes(n, c, h, wd, k, cg, r, s, sh, sw, ph, pw, dh, dw, groups):
+    """(shape of y, the C entry points' integer arguments); p or q may be empty."""
+    p, q = conv_out_size(h, r, sh, ph, dh), conv_out_size(wd, s, sw, pw, dw)
+    return (n, k, p, q), (n, c, h, wd, k, r, s, sh, sw, ph, pw, dh, dw, groups)
+
+
 # ---- convolution -------------------------------------------------------------------------------
 
 def _conv2d_geometry(x, w, bias, stride, padding, dilation, groups):
     """(shape of y, the C entry points' integer arguments); raises for an empty output."""
     _f32(x, w, bias)
     n, c, h, wd = x.shape
-    k, _, r, s = w.shape
-    p = conv_out_size(h, r, stride[0], padding[0], dilation[0])
-    q = conv_out_size(wd, s, stride[1], padding[1], dilation[1])
+    k, cg, r, s = w.shape
+    shape, dims = _conv2d_shapes(n, c, h, wd, k, cg, r, s, stride[0], stride[1], padding[0], padding[1], dilation[0],
+                                 dilation[1], groups)
+    p, q = shape[2:]
     if p <= 0 or q <= 0:
         raise RuntimeError(f'Calculated output size ({k} x {p} x {q}) is too small for input {x.shape} '
                            f'and kernel {(r, s)}')
-    return (n, k, p, q), (n, c, h, wd, k, r, s, stride[0], stride[1], padding[0], padding[1], dilation[0], dilation[1],
-                          groups)
+    return shape, dims
 
 
 def conv2d_fwd(x, w, bias, stride, padding, dilation, groups):

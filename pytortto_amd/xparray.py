@@ -11,6 +11,7 @@
 import ctypes
 import weakref
 from math import prod
+from operator import attrgetter
 
 import numpy as np
 
@@ -53,6 +54,9 @@ class Device:
 
     def __hash__(self):
         return hash(('hip', self.id))
+
+
+_F32 = np.dtype(np.float32)
 
 
 class _Buffer:
@@ -193,16 +197,18 @@ class hiparray:
     # ---- construction helpers -------------------------------------------------------------
     @classmethod
     def empty(cls, shape, dtype=np.float32):
-        shape = (shape,) if isinstance(shape, int) else tuple(shape)
-        dtype = np.dtype(dtype)
-        return cls(_buf=_Buffer(prod(shape) * dtype.itemsize), _shape=shape, dtype=dtype)
+        if shape.__class__ is not tuple:
+            shape = (shape,) if isinstance(shape, int) else tuple(shape)
+        dtype = _F32 if dtype is np.float32 else np.dtype(dtype)
+        return cls.on(_Buffer(prod(shape) * dtype.itemsize), shape, dtype)
 
     @classmethod
     def lazy(cls, shape, dtype=np.float32):
         """An array whose block is allocated when its ``ptr`` is first used."""
-        shape = (shape,) if isinstance(shape, int) else tuple(shape)
-        dtype = np.dtype(dtype)
-        return cls.on(_Buffer(prod(shape) * dtype.itemsize, lazy=True), shape, dtype)
+        if shape.__class__ is not tuple:
+            shape = (shape,) if isinstance(shape, int) else tuple(shape)
+        dtype = _F32 if dtype is np.float32 else np.dtype(dtype)
+        return cls.on(_Buffer(prod(shape) * dtype.itemsize, True), shape, dtype)
 
     @classmethod
     def on(cls, buf, shape, dtype):
@@ -225,15 +231,13 @@ class hiparray:
     # ---- ndarray-like attributes ----------------------------------------------------------
     @property
     def ptr(self):
-        return self._buf.ptr
+        buf = self._buf
+        block = buf._ptr
+        return block if block and buf.on_demand is None else buf.ptr
 
-    @property
-    def shape(self):
-        return self._shape
-
-    @property
-    def dtype(self):
-        return self._dtype
+    # (looked at dozens of times per layer: getters without a Python frame)
+    shape = property(attrgetter('_shape'))
+    dtype = property(attrgetter('_dtype'))
 
     @property
     def ndim(self):
