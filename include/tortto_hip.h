@@ -283,6 +283,8 @@ int tt_conv2d_wgrad_force_occupancy(int blocks);
 /* Which launches go to the kernels for few rows (tt_conv2d_last_launch reports -3 blocks for them): 1 (the
  * default): where they are faster; 0: none; 2: all that they support. */
 int tt_conv2d_narrow_enable(int on);
+/* The same for the kernels that keep a patch of the source in LDS (TT_CONV_MATH_BF16X3; reported as -4). */
+int tt_conv2d_patch_enable(int on);
 
 /* out[K] = sum over n and the HW plane of t[N,K,HW]: the bias gradient gd0.sum((0,2,3)),
  * autograd/grad_nn.py:728, :774. */

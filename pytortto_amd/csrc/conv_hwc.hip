@@ -453,12 +453,14 @@ int hwc_conv(const HwcConv& c, const float* x, const float* w, const float* bias
   if (pl.mt == 2) hwc_product<2, 2><<<grid, kThreads, 0, st>>>(p, q);
   else hwc_product<1, 2><<<grid, kThreads, 0, st>>>(p, q);
   TT_LAUNCH_CHECK();
-  if (pl.splits > 1) {
-    const uint32_t total = (uint32_t)q.outElems;
-    const int blocks = std::min(ceil_div(total, kThreads), 8 * tt::compute_units());
-    hwc_finish<<<blocks, kThreads, 0, st>>>(p, q.partial, pl.splits, total, p.divUV, tt::make_fastdiv((uint32_t)c.I));
-    TT_LAUNCH_CHECK();
-  }
+  return pl.splits > 1 ? add_partials(p, q.partial, pl.splits) : 0;
+}
+
+int add_partials(const Igemm& p, const float* partial, int splits) {
+  const uint32_t total = (uint32_t)p.I * (uint32_t)p.M;
+  const int blocks = std::min(ceil_div(total, kThreads), 8 * tt::compute_units());
+  hwc_finish<<<blocks, kThreads, 0, tt::stream()>>>(p, partial, splits, total, p.divUV, tt::make_fastdiv((uint32_t)p.I));
+  TT_LAUNCH_CHECK();
   return 0;
 }
 

@@ -41,6 +41,7 @@
 
 #include "conv_igemm_common.h"
 #include "conv_narrow.h"
+#include "conv_patch.h"
 
 namespace {
 
@@ -725,6 +726,16 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
       return hwc_conv(hc, x, w, bias, y, epi, TT_PROF_CONV_IGEMM_FWD, g_last_launch);
     }
   }
+  if (split_math() && groups == 1 && !check_only && sh == 1 && sw == 1) {
+    const PatchConv pc{N, C, H, W, K, P, Q, R, S, ph, pw, dh, dw, false};
+    if (patch_conv_takes(pc)) {
+      if (size_only) {
+        *size_only = patch_workspace(pc);
+        return 0;
+      }
+      return patch_conv_launch(pc, x, w, bias, y, epi, TT_PROF_CONV_IGEMM_FWD, g_last_launch);
+    }
+  }
   if (!check_only) {
     NarrowConv nc{x, w, bias, y, Kg, Cg, groups, tt::make_fastdiv((uint32_t)Cg), {}, Cg * R * S, R * S, Kg * Cg * R * S, 1, 1, S,
                   sh, sw, dh, dw, H, W, C * H * W, Cg * H * W, H * W, K * P * Q, Kg * P * Q, P * Q, Q, 1, 1, false, 1, {}, {}};
@@ -819,6 +830,16 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
         return 0;
       }
       return hwc_conv(hc, dy, w, bias, dx, epi, TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
+    }
+  }
+  if (split_math() && groups == 1 && !check_only && sh == 1 && sw == 1) {
+    const PatchConv pc{N, K, P, Q, C, Hx, Wx, R, S, (R - 1) * dh - ph, (S - 1) * dw - pw, dh, dw, true};
+    if (patch_conv_takes(pc)) {
+      if (size_only) {
+        *size_only = patch_workspace(pc);
+        return 0;
+      }
+      return patch_conv_launch(pc, dy, w, bias, dx, epi, TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
     }
   }
   const int gh = gcd(sh, dh), gw = gcd(sw, dw);

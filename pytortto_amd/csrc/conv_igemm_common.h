@@ -224,6 +224,9 @@ size_t hwc_workspace(const HwcConv& c);
 // Enqueues the call; `plan8` as tt_conv2d_last_launch reports it.
 int hwc_conv(const HwcConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi, int prof_id,
              int* plan8);
+// Enqueues the sum of `splits` partial results in order, each laid out as p.out (one group), and the launch's
+// bias and epilogue.
+int add_partials(const Igemm& p, const float* partial, int splits);
 
 // The kernel body of conv_igemm_kernel.h in one arithmetic (conv_igemm_launch.h).  launch: `bm` x `bn` is
 // the tile the caller planned; `sk_blocks` > 0 asks for the persistent (stream-K) grid, which is launched

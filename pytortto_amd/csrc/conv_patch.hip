@@ -1,0 +1,493 @@
+// Convolutions of unit stride whose operands travel as three bfloat16 terms: Conv2d forward and the input
+// gradient.
+//
+//   D[i, m] = sum over channels c and taps t of  W[i][c][t] * X[pixel(m, t)][c]      (+ epilogue)
+//
+// The kernels that gather in place (conv_igemm_kernel.h) fetch a source element, write it to LDS and split
+// it into its terms once per tap, and do so between barriers 24 matrix instructions apart: nothing overlaps
+// with anything, and the matrix pipe is busy for a third of the time.  Here a block fetches the patch of the
+// source that its pixels reach -- all taps of it -- once per sixteen channels, splits it once, and runs the
+// taps out of LDS: a tap is a constant added to the address of a lane's pixel.  Between two barriers lie 24
+// matrix instructions per wave for every tap (216 for a 3x3 kernel), and a source element is fetched 1.3 to
+// 1.7 times instead of nine.  The weights are split and laid out once per call, in the order in which a
+// wave's lanes hold them, and go from memory to registers without passing LDS.
+//
+// Measured, 3x3, forward: 160 to 192 channels 45x37 at batch 24 117 us (189 TFLOP/s of the product: its six matrix
+// instructions run at 1.13 PFLOP/s, what a large bf16 product reaches here), 184 in the kernels that gather; 64
+// channels 32x32 at batch 128 63 us (50 of them the product), 72; 128 channels 16x16 67, 98.  With two blocks on a
+// compute unit the device's power bounds it; with one, what a wave does between two chunks (the matrix pipes
+// are busy 40 % of the time then) and, where a reduction is shared, the sums' way through memory.
+//
+// The pixels of a tile are consecutive pixels of the batch, whatever the image's shape.  Their source lies in
+// a virtual image that holds the images of the batch below each other, each framed by what the taps reach
+// outside it: virtual pixel (n*VR + j)*PW + k is row j + bh, column k + bw of image n, zero outside.  A
+// pixel's taps are at fixed distances there, so the patch is one range of it.  Where two images' frames (or
+// two rows') meet, they are zeros from either side, and share them.
+#include <algorithm>
+#include <initializer_list>
+#include <utility>
+
+#include "conv_igemm_common.h"
+#include "conv_patch.h"
+
+namespace {
+
+using namespace ttc;
+
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef unsigned uintx4 __attribute__((ext_vector_type(4)));
+
+constexpr int kBK = 16;              // channels of a chunk: the depth of one matrix step
+constexpr int kTerms = 3;
+constexpr int kUnit = 16 * kTerms;   // bytes of a patch pixel's eight channels.  48 bytes from lane to lane
+                                     // spread eight lanes' 16-byte accesses over all banks
+constexpr int kMaxTaps = 31;
+
+// Eight float32 values as three vectors of bfloat16 terms that add up to them exactly: term i of a value is
+// the bf16 nearest to what the terms before it leave.
+__device__ __forceinline__ void split8(const float (&v)[8], uintx4 (&out)[kTerms]) {
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float e = v[2 * q], o = v[2 * q + 1];
+#pragma unroll
+    for (int i = 0; i < kTerms; ++i) {
+      const bf16x2 pair = {(__bf16)e, (__bf16)o};
+      unsigned t = __builtin_bit_cast(unsigned, pair);
+      asm("" : "+v"(t));   // or the compiler rounds the even value a second time, by itself
+      out[i][q] = t;
+      if (i < kTerms - 1) {
+        e -= as_float(t << 16);
+        o -= as_float(t & 0xffff0000u);
+      }
+    }
+  }
+}
+
+// ---- weights -> wt[32 rows][chunk][tap][term][lane], 16 bytes each: lane 32*h + l holds row l, channels 8h.. --
+// forward: row k, w[k][c][tap];  input gradient: row c, channel k, taps in reverse order.  A block lays out
+// one strip of 32 rows and sixteen channels: reads runs of w, turns them in LDS, writes runs of wt.
+template <bool DGRAD>
+__global__ __launch_bounds__(kThreads) void patch_weights(const float* __restrict__ w, uintx4* __restrict__ wt, int rows, int chans,
+                                                         int taps, tt::FastDiv divRun, int chunks) {
+  extern __shared__ float strip[];   // [outer][run + 1]: forward 32 rows x 16 channels' taps, gradient 16 x 32 rows' taps
+  const int chunk = blockIdx.x, r0 = blockIdx.y * 32, c0 = chunk * kBK;
+  const int run = divRun.d;          // (DGRAD ? 32 : 16) * taps
+  const int outer = DGRAD ? kBK : 32;
+  for (int u = threadIdx.x; u < outer * run; u += kThreads) {
+    const int a = (int)tt::fd_div((uint32_t)u, divRun), b = u - a * run;
+    bool ok;
+    size_t at;
+    if constexpr (DGRAD) {
+      ok = c0 + a < chans && r0 * taps + b < rows * taps;
+      at = ((size_t)(c0 + a) * rows + r0) * taps + b;
+    } else {
+      ok = r0 + a < rows && c0 * taps + b < chans * taps;
+      at = ((size_t)(r0 + a) * chans + c0) * taps + b;
+    }
+    strip[a * (run + 1) + b] = ok ? w[at] : 0.f;
+  }
+  __syncthreads();
+  uintx4* __restrict__ dst = wt + ((size_t)blockIdx.y * chunks + chunk) * taps * (kTerms * 64);
+  for (int u = threadIdx.x; u < taps * 64; u += kThreads) {
+    const int tap = u >> 6, lane = u & 63, row = lane & 31, c = 8 * (lane >> 5);
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = DGRAD ? strip[(c + e) * (run + 1) + row * taps + (taps - 1 - tap)] : strip[row * (run + 1) + (c + e) * taps + tap];
+    uintx4 t[kTerms];
+    split8(v, t);
+#pragma unroll
+    for (int i = 0; i < kTerms; ++i) dst[(tap * kTerms + i) * 64 + lane] = t[i];
+  }
+}
+
+// ---- the product -------------------------------------------------------------------------------------
+struct Patch {
+  const float* src;
+  const uintx4* wt;
+  float* partial;      // splits > 1: [splits][elements of out] sums over a part of the chunks each
+  long long outElems;
+  int C, chunks, perSplit, taps, S;
+  int plane, image;    // bytes of a source plane, an image
+  int PW, VR;          // the virtual image's pitch and rows per image
+  int tapRow, tapCol;  // steps of a tap row / column in the patch, in bytes
+  int px;              // pixels of the patch held in LDS
+  int images;
+  tt::FastDiv divPW, divVR;
+};
+
+// Tile 32*WM rows x 32*NT*(4/WM) pixels; every wave has 32 rows and NT x 32 pixels.  The patch has at most 128*IT
+// pixels: a thread fetches and splits eight channels of IT of them.
+template <int WM, int NT, int IT, bool EPI>
+__global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, const Patch q) {
+  constexpr int WN = 4 / WM, BM = 32 * WM, BN = 32 * NT * WN;
+  extern __shared__ __align__(16) char lds[];   // [half][px] units; then the epilogue's constants
+  float* const epi_lds = reinterpret_cast<float*>(lds + 2 * q.px * kUnit);
+
+  const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  const int tile = tt::xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const int tilesI = p.Ipad / BM;
+  const int i0 = (tile % tilesI) * BM;
+  const int m0 = (tile / tilesI) * BN;
+  const int q0 = (int)blockIdx.z * q.perSplit, q1 = min(q.chunks, q0 + q.perSplit);
+
+  auto virtual_pixel = [&](const uint32_t m, uint32_t& n) __attribute__((always_inline)) {
+    n = tt::fd_div(m, p.divUV);
+    const uint32_t rem = m - n * p.divUV.d;
+    const uint32_t u = tt::fd_div(rem, p.divV);
+    return (n * (uint32_t)q.VR + u) * (uint32_t)q.PW + (rem - u * p.divV.d);
+  };
+  uint32_t n0;
+  const uint32_t first = virtual_pixel((uint32_t)__builtin_amdgcn_readfirstlane(m0), n0);
+  const __amdgpu_buffer_rsrc_t srd =
+      __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)q.src + (long long)n0 * q.image), 0, kSrdRecords, kSrdFlags);
+
+  // what this thread fetches: half `wave / 2` of the patch pixels it*128 + tid % 128
+  const int half = wave >> 1, pp0 = tid & 127;
+  const int at = (half * q.px + pp0) * kUnit;
+  int voff[IT];
+#pragma unroll
+  for (int it = 0; it < IT; ++it) {
+    const int pp = it * 128 + pp0;
+    const uint32_t v = first + (uint32_t)pp;
+    const uint32_t row = tt::fd_div(v, q.divPW), n = tt::fd_div(row, q.divVR);
+    const int ih = (int)(row - n * (uint32_t)q.VR) + p.bh, iw = (int)(v - row * (uint32_t)q.PW) + p.bw;
+    const bool inside = pp < q.px && (unsigned)ih < (unsigned)p.Hlim && (unsigned)iw < (unsigned)p.Wlim && n < (uint32_t)q.images;
+    voff[it] = inside ? (int)(n - n0) * q.image + (ih * p.Wlim + iw) * 4 : (int)0x80000000;
+  }
+  float reg[IT][8];
+  auto fetch = [&](const int chunk) __attribute__((always_inline)) {
+    const int c0 = chunk * kBK + 8 * half;
+#pragma unroll
+    for (int it = 0; it < IT; ++it)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const int vo = c0 + e < q.C ? voff[it] : (int)0x80000000;
+        reg[it][e] = as_float(__builtin_amdgcn_raw_buffer_load_b32(srd, vo, (c0 + e) * q.plane, 0));
+      }
+  };
+  auto stage = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int it = 0; it < IT; ++it) {
+      uintx4 t[kTerms];
+      split8(reg[it], t);
+      if (it * 128 + pp0 < q.px) {
+#pragma unroll
+        for (int i = 0; i < kTerms; ++i) *reinterpret_cast<uintx4*>(lds + at + it * 128 * kUnit + 16 * i) = t[i];
+      }
+    }
+  };
+
+  // Products of the first terms in `acc`, all others, 2^-8 of them and less, in `small`: the long chain has one
+  // rounding per sixteen channels and tap where a single one would have six.
+  floatx16 acc[1][NT], small[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[0][y][r] = small[y][r] = 0.f;
+
+  int base[NT];   // the lane's pixels in the patch
+#pragma unroll
+  for (int y = 0; y < NT; ++y) {
+    const int m = m0 + (wn * NT + y) * 32 + l32;
+    uint32_t n;
+    base[y] = (int)(virtual_pixel((uint32_t)(m < p.M ? m : m0), n) - first + (uint32_t)(h * q.px)) * kUnit;
+  }
+
+  // the wave's weights: one run of 3 KB per tap, fetched two taps ahead into the registers that a tap is done with
+  const uintx4* wptr = q.wt + ((size_t)(i0 / 32 + wm) * q.chunks + q0) * (size_t)(q.taps * kTerms * 64);
+  uintx4 w1[kTerms], w2[kTerms];
+  auto load_weights = [&](uintx4 (&to)[kTerms]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kTerms; ++i) to[i] = wptr[i * 64 + lane];
+    wptr += kTerms * 64;
+  };
+  uintx4 b[2][2][kTerms];   // two 32-pixel tiles at a time, and the two behind them
+  auto load_pixels = [&](const int y, const int offset, uintx4 (&to)[2][kTerms]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < kTerms; ++i) to[j][i] = *reinterpret_cast<const uintx4*>(lds + base[y + j] + offset + 16 * i);
+  };
+  // One tap: 6*NT matrix instructions.  b[first_buf] holds its first pixels; a step's pixels are read while the step
+  // before it multiplies, and two tiles' products alternate, since each waits for the one before it on the same
+  // accumulator.  The weights that are read past a wave's last tap are not used.
+  auto tap = [&](uintx4 (&w)[kTerms], const int first_buf, const int off, const int next) __attribute__((always_inline)) {
+    bf16x8 a[kTerms];
+#pragma unroll
+    for (int i = 0; i < kTerms; ++i) a[i] = __builtin_bit_cast(bf16x8, w[i]);
+#pragma unroll
+    for (int y = 0; y < NT; y += 2) {
+      auto& x = b[(first_buf + y / 2) & 1];
+      auto& behind = b[(first_buf + y / 2 + 1) & 1];
+      if (y + 2 < NT) load_pixels(y + 2, off, behind);
+      else load_pixels(0, next, behind);
+      __builtin_amdgcn_sched_barrier(0);
+      auto product = [&](const int i, const int k, floatx16 (&to)[NT]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          to[y + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], __builtin_bit_cast(bf16x8, x[j][k]), to[y + j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      product(0, 2, small);
+      product(0, 0, acc[0]);
+      product(2, 0, small);
+      product(1, 1, small);
+      product(0, 1, small);
+      product(1, 0, small);
+    }
+    load_weights(w);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  const bool whole = q.partial == nullptr;
+  if constexpr (EPI) {
+    if (whole && p.epi.on) epilogue_constants<BM>(p, 0, i0, tid, epi_lds);   // published by the barrier below
+  }
+  fetch(q0);
+  load_weights(w1);
+  load_weights(w2);
+  stage();
+  __syncthreads();
+  load_pixels(0, 0, b[0]);
+  if (q0 + 1 < q1) fetch(q0 + 1);   // in flight across this chunk's matrix instructions
+  // The taps of all chunks in pairs, whatever their number.  One too many has zero weights.
+  int c = q0, t = 0, ts = 0, row = 0, off = 0, next = 0;   // tap t of chunk c, column ts of its kernel row
+  auto look = [&]() __attribute__((always_inline)) {   // where the tap behind this one lies
+    next = off + q.tapCol;
+    if (++ts == q.S) {
+      ts = 0;
+      next = row += q.tapRow;
+    }
+    if (t + 1 == q.taps) next = 0;
+  };
+  auto advance = [&](const int next_buf) __attribute__((always_inline)) {
+    off = next;
+    if (++t == q.taps) {
+      t = ts = row = 0;
+      if (++c < q1) {
+        __syncthreads();   // the patch has been read by every wave
+        stage();
+        __syncthreads();
+        load_pixels(0, 0, b[next_buf]);
+        if (c + 1 < q1) fetch(c + 1);
+      }
+    }
+    look();
+  };
+  look();
+  const int total = (q1 - q0) * q.taps;
+  constexpr int kOdd = (NT / 2) & 1;   // the buffer that a pair's second tap begins with
+  for (int k = 0; k < total; k += 2) {
+    tap(w1, 0, off, next);
+    advance(kOdd);
+    if (k + 1 == total)
+#pragma unroll
+      for (int i = 0; i < kTerms; ++i) w2[i] = uintx4{0, 0, 0, 0};
+    tap(w2, kOdd, off, next);
+    advance(0);
+  }
+  uint32_t obase[NT];
+  bool mok[NT];
+#pragma unroll
+  for (int y = 0; y < NT; ++y) {
+    const int m = m0 + (wn * NT + y) * 32 + l32;
+    mok[y] = m < p.M;
+    const uint32_t mm = mok[y] ? (uint32_t)m : 0u, n = tt::fd_div(mm, p.divUV);
+    obase[y] = (uint32_t)((int)n * p.outStrideN + (int)(mm - n * p.divUV.d));
+  }
+#pragma unroll
+  for (int y = 0; y < NT; ++y) acc[0][y] += small[y];
+
+  if constexpr (EPI) {
+    if (whole && p.epi.on) {
+      store_through_epilogue<BM, 1, NT>(p, acc, obase, mok, i0, wm * 32, h, epi_lds);
+      return;
+    }
+  }
+  // accumulator register r of a 32x32 tile holds row 8*(r/4) + 4*h + r%4, column l32
+  float* __restrict__ out = whole ? p.out : q.partial + (size_t)blockIdx.z * (size_t)q.outElems;
+  const bool biased = whole && p.bias != nullptr;
+  const uint32_t hoff = (uint32_t)(4 * h * p.outStrideI);
+  const int srow = __builtin_amdgcn_readfirstlane(i0 + wm * 32);
+  float bz[16];
+#pragma unroll
+  for (int r = 0; r < 16; ++r) bz[r] = biased ? p.bias[min(srow + 8 * (r >> 2) + 4 * h + (r & 3), p.I - 1)] : 0.f;
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0f70);   // every load done before the first store: they share one counter
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int r = 0; r < 16; ++r) {
+    const int row = srow + 8 * (r >> 2) + (r & 3);
+    float* __restrict__ rowp = out + (size_t)row * (size_t)p.outStrideI;
+    if (row + 4 * h < p.I) {
+#pragma unroll
+      for (int y = 0; y < NT; ++y)
+        if (mok[y]) rowp[obase[y] + hoff] = biased ? acc[0][y][r] + bz[r] : acc[0][y][r];
+    }
+  }
+}
+
+int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
+size_t align_up(size_t v) { return (v + 255) / 256 * 256; }
+
+struct Plan {
+  int WM, NT, IT, Ipad, px, PW, VR, chunks, perSplit, splits, tiles;
+  size_t wt, partial;   // bytes of workspace
+  double cost;
+};
+
+int g_patch = 1;   // tests: 0 = never, 2 = wherever they can
+
+// The virtual image's rows per image, or its pitch: what the taps reach, less the zeros that two frames share.
+int framed(int pixels, int taps, int dil, int pad, int limit) {
+  const int reach = (taps - 1) * dil, behind = pixels - 1 + reach - pad - (limit - 1);
+  return pixels + reach - std::max(0, std::min({pad, behind, reach}));
+}
+
+bool make_plan(const PatchConv& c, Plan* best) {
+  const int taps = c.R * c.S;
+  const long long M = (long long)c.N * c.P * c.Q;
+  best->cost = -1;
+  for (const auto& shape : {std::pair{4, 4}, {2, 4}, {2, 2}}) {
+    Plan pl{};
+    pl.WM = shape.first; pl.NT = shape.second;
+    const int BM = 32 * pl.WM, BN = 128 * pl.NT / pl.WM;
+    pl.VR = framed(c.P, c.R, c.dh, c.ph, c.H);
+    pl.PW = framed(c.Q, c.S, c.dw, c.pw, c.W);
+    // the longest range of the virtual image that BN consecutive pixels and their taps cover
+    const long long rows = (BN + c.Q - 2) / c.Q, images = (BN + (long long)c.P * c.Q - 2) / ((long long)c.P * c.Q);
+    const long long px = BN + rows * (pl.PW - c.Q) + images * (long long)(pl.VR - c.P) * pl.PW +
+                         (long long)(c.R - 1) * c.dh * pl.PW + (long long)(c.S - 1) * c.dw;
+    if (px > 512) continue;
+    pl.px = (int)px;
+    pl.IT = px <= 384 ? 3 : 4;
+    pl.Ipad = ceil_div(c.I, BM) * BM;
+    pl.chunks = ceil_div(c.C, kBK);
+    pl.tiles = (pl.Ipad / BM) * ceil_div(M, BN);
+    // two taps' weights more: the product reads ahead of its last
+    pl.wt = align_up(((size_t)pl.Ipad / 32 * pl.chunks * taps + 2) * kTerms * 1024);
+    // Microseconds, fitted to 75 launches of 4 to 2000 blocks (10 % root mean square): a chunk of a block that
+    // shares its compute unit, a block's start and end; a block that has the unit for itself takes a sixth longer.
+    // Shares of a reduction are written, read and added.  (The weights' layout costs the same for all.)
+    const double chunk = pl.NT == 4 ? 0.55 * taps + 1.0 : 0.29 * taps + 0.9;
+    for (int s = 1; s <= 8 && s <= pl.chunks; ++s) {
+      const int per = ceil_div(pl.chunks, s);
+      if (ceil_div(pl.chunks, per) != s) continue;
+      const double blocks = (double)pl.tiles * s / tt::compute_units();   // of a compute unit
+      const double cost = std::max(1.17, blocks + 0.1) * (per * chunk + 4) + (s > 1 ? 5 + (2 * s + 1) * 4e-6 / 7 * (double)c.I * M : 0);
+      if (best->cost < 0 || cost < best->cost) {
+        pl.perSplit = per;
+        pl.splits = s;
+        pl.cost = cost;
+        pl.partial = s > 1 ? align_up(sizeof(float) * (size_t)s * c.I * M) : 0;
+        *best = pl;
+      }
+    }
+  }
+  return best->cost >= 0;
+}
+
+}  // namespace
+
+namespace ttc {
+
+size_t patch_workspace(const PatchConv& c) {
+  Plan pl;
+  return make_plan(c, &pl) ? pl.wt + pl.partial : 0;
+}
+
+bool patch_conv_takes(const PatchConv& c) {
+  if (g_patch == 0) return false;
+  const int taps = c.R * c.S;
+  if (taps > kMaxTaps) return false;
+  if ((c.R - 1LL) * c.dh > 512 || (c.S - 1LL) * c.dw > 512) return false;   // wider than a patch
+  Plan pl;
+  if (!make_plan(c, &pl)) return false;
+  // 32-bit offsets: virtual pixels of the batch, source bytes of the images that a patch touches
+  const long long frame = (long long)pl.VR * pl.PW, image = 4LL * c.C * c.H * c.W;
+  if ((c.N + 1) * frame + 1024 >= (1LL << 31) || (pl.px / frame + 2) * image >= (1LL << 31)) return false;
+  if (pl.Ipad / 32 > 65535) return false;   // the grid of patch_weights
+  if (g_patch == 2) return true;
+  if (pl.wt + pl.partial > ((size_t)1 << 30)) return false;   // workspace stays with the library
+  // Against the kernels that gather in place, whose time is about 16 us and 7 us per 1e9 products and sums (53
+  // launches of 0.5 to 25e9; they take less where a long reduction is shared between many blocks, and more, up to
+  // twice, where it is not).  So it is taken for 28 of 75 launches, 1.12 times as fast on average: 64 channels
+  // 32x32 at batch 128 72.1 us, 62.7 here; 128 channels 16x16 98.0, 67.2; 256 channels 8x8 77.0, 70.4; 160 to 192
+  // channels 45x37 at batch 24 183.9, 117.0; and not for 128 channels 28x28 at batch 8 (29.3, 32.9) or 3 channels
+  // (23.4, 56.8), whose rows and channels are mostly padding.
+  const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
+  const double gigas = 2e-9 * c.I * c.C * taps * c.N * c.P * c.Q;
+  return taps >= 4 && padding <= 1.5 && gigas >= 1.5 && pl.cost + 3 + 4e-6 * c.I * c.C * taps < 16 + 7 * gigas;
+}
+
+int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi,
+                      int prof_id, int* plan8) {
+  const int taps = c.R * c.S;
+  Plan pl;
+  if (!make_plan(c, &pl)) return tt::fail(-1, "patch convolution: no plan");
+  void* ws = nullptr;
+  if (tt::workspace(pl.wt + pl.partial, &ws)) return -1;
+  hipStream_t st = tt::stream();
+  Igemm p{};
+  p.bias = bias; p.out = out;
+  if (epi) p.epi = *epi;
+  p.I = c.I; p.Ipad = pl.Ipad; p.M = c.N * c.P * c.Q;
+  p.divUV = tt::make_fastdiv((uint32_t)(c.P * c.Q));
+  p.divV = tt::make_fastdiv((uint32_t)c.Q);
+  p.bh = -c.ph; p.bw = -c.pw;
+  p.Hlim = c.H; p.Wlim = c.W;
+  p.outStrideN = c.I * c.P * c.Q; p.outStrideI = c.P * c.Q;
+  Patch q{};
+  q.src = x; q.wt = (const uintx4*)ws;
+  q.partial = pl.splits > 1 ? (float*)((char*)ws + pl.wt) : nullptr;
+  q.outElems = (long long)p.I * p.M;
+  q.C = c.C; q.chunks = pl.chunks; q.perSplit = pl.perSplit; q.taps = taps; q.S = c.S;
+  q.plane = 4 * c.H * c.W; q.image = q.plane * c.C;
+  q.PW = pl.PW; q.VR = pl.VR;
+  q.tapRow = c.dh * pl.PW * kUnit; q.tapCol = c.dw * kUnit;
+  q.px = pl.px; q.images = c.N;
+  q.divPW = tt::make_fastdiv((uint32_t)pl.PW); q.divVR = tt::make_fastdiv((uint32_t)pl.VR);
+  {
+    tt::ProfScope prof(TT_PROF_CONV_PREP);
+    const int run = (c.dgrad ? 32 : kBK) * taps, outer = c.dgrad ? kBK : 32;
+    const dim3 grid((unsigned)pl.chunks, (unsigned)(pl.Ipad / 32));
+    const size_t lds = sizeof(float) * (size_t)outer * (run + 1);
+    const tt::FastDiv divRun = tt::make_fastdiv((uint32_t)run);
+    if (c.dgrad) patch_weights<true><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, taps, divRun, pl.chunks);
+    else patch_weights<false><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, taps, divRun, pl.chunks);
+    TT_LAUNCH_CHECK();
+  }
+  const int BM = 32 * pl.WM, BN = 128 * pl.NT / pl.WM;
+  const int plan[8] = {BM, BN, pl.tiles, pl.Ipad / BM, -4, pl.tiles, pl.splits, kModeTapMask | 3 << 8};
+  std::copy(plan, plan + 8, plan8);
+  tt::ProfScope prof(prof_id);
+  const dim3 grid((unsigned)pl.tiles, 1, (unsigned)pl.splits);
+  const size_t lds = 2 * (size_t)pl.px * kUnit + 4 * sizeof(float) * BM;
+  const bool epilogue = p.epi.on && pl.splits == 1;
+#define TT_PATCH(WM, NT, IT)                                                                  \
+  (epilogue ? patch_product<WM, NT, IT, true><<<grid, kThreads, lds, st>>>(p, q) \
+            : patch_product<WM, NT, IT, false><<<grid, kThreads, lds, st>>>(p, q))
+  if (pl.WM == 4) {
+    if (pl.IT == 3) TT_PATCH(4, 4, 3); else TT_PATCH(4, 4, 4);
+  } else if (pl.NT == 4) {
+    if (pl.IT == 3) TT_PATCH(2, 4, 3); else TT_PATCH(2, 4, 4);
+  } else {
+    if (pl.IT == 3) TT_PATCH(2, 2, 3); else TT_PATCH(2, 2, 4);
+  }
+#undef TT_PATCH
+  TT_LAUNCH_CHECK();
+  if (pl.splits > 1) return add_partials(p, q.partial, pl.splits);
+  return 0;
+}
+
+}  // namespace ttc
+
+extern "C" int tt_conv2d_patch_enable(int on) {
+  TT_API_LOCK();
+  TT_REQUIRE(on >= 0 && on <= 2, "tt_conv2d_patch_enable: %d is out of range (0..2)", on);
+  g_patch = on;
+  return 0;
+}

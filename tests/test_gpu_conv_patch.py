@@ -1,0 +1,106 @@
+"""The kernels that keep a patch of the source in LDS (three bfloat16 terms, unit stride), over every geometry they
+take: the float32 bar of tests/test_gpu_conv.py, and sums no further from float64 ones than those of the kernels
+that gather in place."""
+import numpy as np
+import pytest
+
+from pytortto_amd import _hip, ops
+from pytortto_amd.xparray import hiparray
+from tests.cases import CONV_CASES, random_conv_cases, random_large_kernel_cases
+from tests.test_gpu_conv import TILE_CASES, _last_launch, _run_conv
+
+pytestmark = pytest.mark.gpu
+
+ALWAYS, WHERE_FASTER, NEVER = 2, 1, 0
+
+
+@pytest.fixture
+def patch():
+    def choose(which):
+        _hip.call('tt_conv2d_patch_enable', which)
+    _hip.set_conv_math('bf16x3')
+    yield choose
+    choose(WHERE_FASTER)
+    _hip.set_conv_math('f32')
+
+
+# n, c, h, w, k, r, s, stride, pad, dilation, groups: one pixel; images smaller than a tile, many in it, framed by more
+# zeros than the taps reach, by fewer, by none; rows wider than a tile; channels and rows on either side of 16, 32, 64,
+# 128; one tap; as many as there may be; a single tile with its reduction shared
+EDGES = [
+    (1, 1, 1, 1, 1, 1, 1, (1, 1), (0, 0), (1, 1), 1), (70, 16, 2, 4, 32, 3, 3, (1, 1), (1, 1), (1, 1), 1),
+    (300, 17, 2, 3, 33, 3, 3, (1, 1), (1, 1), (1, 1), 1), (31, 15, 5, 4, 31, 3, 3, (1, 1), (0, 0), (1, 1), 1),
+    (9, 24, 7, 7, 64, 3, 3, (1, 1), (4, 3), (1, 1), 1), (3, 40, 9, 13, 65, 5, 5, (1, 1), (2, 2), (1, 1), 1),
+    (5, 33, 14, 14, 128, 3, 3, (1, 1), (2, 2), (2, 2), 1), (2, 16, 28, 28, 129, 3, 2, (1, 1), (1, 0), (1, 3), 1),
+    (1, 20, 3, 140, 70, 2, 3, (1, 1), (0, 1), (1, 1), 1), (2, 16, 40, 300, 32, 1, 3, (1, 1), (0, 1), (1, 1), 1),
+    (4, 64, 12, 11, 96, 1, 1, (1, 1), (0, 0), (1, 1), 1), (2, 8, 12, 40, 8, 1, 31, (1, 1), (0, 15), (1, 1), 1),
+    (2, 18, 16, 15, 34, 5, 6, (1, 1), (2, 2), (1, 1), 1), (1, 512, 7, 7, 64, 3, 3, (1, 1), (1, 1), (1, 1), 1),
+    (40, 130, 14, 14, 200, 3, 3, (1, 1), (1, 1), (1, 1), 1), (6, 48, 61, 43, 160, 3, 3, (1, 1), (1, 1), (1, 1), 1),
+]
+
+
+@pytest.mark.parametrize('case', EDGES + [c for c in CONV_CASES + TILE_CASES if c[7] == (1, 1) and c[10] == 1])
+@pytest.mark.parametrize('bias', [True, False])
+def test_meets_the_float32_bar(case, bias, patch):
+    patch(ALWAYS)
+    _run_conv(case, seed=5, bias=bias)
+    if case in EDGES:
+        assert _last_launch()['persistent_blocks'] == -4
+
+
+@pytest.mark.parametrize('case', random_conv_cases(60, 91) + random_large_kernel_cases(8, 92))
+def test_random_geometries(case, patch):
+    patch(ALWAYS)
+    _run_conv(case, seed=6)
+
+
+@pytest.mark.parametrize('n,c,hw,k', [(9, 64, 14, 96), (2, 256, 7, 70), (40, 32, 28, 64)])   # the second shares its reduction
+def test_epilogues(n, c, hw, k, patch):
+    """The same bits as the entry points they stand in for."""
+    patch(ALWAYS)
+    rng = np.random.default_rng(3)
+    x, w, res, mask = (hiparray(rng.standard_normal(s).astype(np.float32))
+                       for s in ((n, c, hw, hw), (k, c, 3, 3), (n, k, hw, hw), (n, c, hw, hw)))
+    mean, gamma, beta = (hiparray(rng.standard_normal(k).astype(np.float32)) for _ in range(3))
+    var = hiparray(rng.random(k).astype(np.float32) + np.float32(.5))
+    y = ops.conv2d_fwd(x, w, None, (1, 1), (1, 1), (1, 1), 1)
+    out = hiparray.empty(y.shape)
+    _hip.call('tt_conv2d_norm_act_fwd_f32', x.ptr, w.ptr, None, out.ptr, mean.ptr, var.ptr, gamma.ptr, beta.ptr, 1e-5,
+              res.ptr, 1, n, c, hw, hw, k, 3, 3, 1, 1, 1, 1, 1, 1, 1)
+    assert _last_launch()['persistent_blocks'] == -4
+    want = np.maximum(ops.bn_fwd_eval(y, gamma, beta, mean, var, 1e-5)[0].get() + res.get(), 0)
+    assert np.array_equal(out.get(), want)
+    dx = ops.conv2d_dgrad(res, w, None, (hw, hw), (1, 1), (1, 1), (1, 1), 1).get()
+    fused = ops.conv2d_dgrad(res, w, None, (hw, hw), (1, 1), (1, 1), (1, 1), 1, add=x, relu_y=mask).get()
+    assert _last_launch()['persistent_blocks'] == -4
+    assert np.array_equal(fused, (dx + x.get()) * (mask.get() > 0))
+
+
+@pytest.mark.parametrize('dims', [(4, 64, 28, 28, 64, 3), (2, 512, 7, 7, 512, 3), (4, 128, 16, 16, 256, 3), (3, 96, 20, 17, 48, 5),
+                                  (8, 64, 56, 56, 64, 3)])
+def test_sums_are_as_accurate_as_in_the_other_kernels(dims, patch):
+    """Against the exact sums of both arithmetics' kernels that gather in place."""
+    import torch
+    n, c, h, w, k, r = dims
+    rng = np.random.default_rng(11)
+    xh, wh = rng.standard_normal((n, c, h, w)).astype(np.float32), rng.standard_normal((k, c, r, r)).astype(np.float32)
+    dyh = rng.standard_normal((n, k, h, w)).astype(np.float32)
+    x64, w64 = torch.tensor(xh, dtype=torch.float64, requires_grad=True), torch.tensor(wh, dtype=torch.float64)
+    y64 = torch.nn.functional.conv2d(x64, w64, padding=r // 2)
+    y64.backward(torch.tensor(dyh, dtype=torch.float64))
+    want = {'y': y64.detach().numpy(), 'dx': x64.grad.numpy()}
+    x, wt, dy = hiparray(xh), hiparray(wh), hiparray(dyh)
+    geometry = ((1, 1), (r // 2, r // 2), (1, 1), 1)
+
+    def errors():
+        got = {'y': ops.conv2d_fwd(x, wt, None, *geometry).get(), 'dx': ops.conv2d_dgrad(dy, wt, None, (h, w), *geometry).get()}
+        return {key: np.linalg.norm(got[key] - want[key]) / np.linalg.norm(want[key]) for key in got}
+    patch(ALWAYS)
+    new = errors()
+    patch(NEVER)
+    old = errors()
+    _hip.set_conv_math('f32')
+    f32 = errors()
+    for key in want:
+        print(dims, key, 'patch %.2e, gathered %.2e, float32 %.2e' % (new[key], old[key], f32[key]))
+        assert new[key] <= old[key] and new[key] <= f32[key], key
