@@ -98,8 +98,11 @@ int tt_probe_hbm_f32(size_t bytes, double* read_gbs, double* copy_gbs);
 /* ---- convolution ------------------------------------------------------------------------- */
 
 /* Matrix arithmetic of the three convolution passes (no counterpart in the reference,
- * whose path is float32 throughout).  TT_CONV_MATH_F32 (the default) multiplies in float32 on
- * v_mfma_f32_32x32x2_f32 and is the mode that meets the reference's tolerances.
+ * whose path is float32 throughout).  TT_CONV_MATH_F32 (the default) computes in float32 and is the mode that
+ * meets the reference's tolerances: on v_mfma_f32_32x32x2_f32 -- and in large forward passes and input gradients of
+ * unit stride with four taps or more, where it is faster and its error against float64 sums half as large, by the
+ * three exact terms of TT_CONV_MATH_BF16X3; sums that these do not hold (operands that are not finite or round
+ * to a bf16 infinity, results below 2^-96) are formed again without them.
  * TT_CONV_MATH_BF16 is the optional reduced-precision variant: tensors stay float32 in memory,
  * both operands are rounded to bfloat16 (nearest even) on their way into
  * v_mfma_f32_32x32x16_bf16 and products are accumulated in float32 (the weight gradient's
@@ -283,7 +286,7 @@ int tt_conv2d_wgrad_force_occupancy(int blocks);
 /* Which launches go to the kernels for few rows (tt_conv2d_last_launch reports -3 blocks for them): 1 (the
  * default): where they are faster; 0: none; 2: all that they support. */
 int tt_conv2d_narrow_enable(int on);
-/* The same for the kernels that keep a patch of the source in LDS (TT_CONV_MATH_BF16X3; reported as -4). */
+/* The same for the kernels that keep a patch of the source in LDS (TT_CONV_MATH_BF16X3 and _F32; reported as -4). */
 int tt_conv2d_patch_enable(int on);
 
 /* out[K] = sum over n and the HW plane of t[N,K,HW]: the bias gradient gd0.sum((0,2,3)),

@@ -327,6 +327,11 @@ bool g_bf16_first_always = false;   // tests: also where the tile-count rule wou
 // Whether the channel-last kernels (conv_hwc.hip) are to be asked, and whether they take all they support.
 bool g_hwc = true, g_hwc_always = false;
 bool hwc_math(int groups) { return groups == 1 && bf16_math() && g_hwc; }
+// Whether the patch kernels (conv_patch.hip) are to be asked.  In float32 arithmetic they may store a value twice:
+// an epilogue must not read what it writes.
+bool patch_math(int groups, const Epilogue* epi, const float* out) {
+  return groups == 1 && !bf16_math() && (epi == nullptr || split_math() || (epi->res != out && epi->mask != out));
+}
 
 int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_partial) {
   tt::ProfScope prof(prof_id);
@@ -726,14 +731,14 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
       return hwc_conv(hc, x, w, bias, y, epi, TT_PROF_CONV_IGEMM_FWD, g_last_launch);
     }
   }
-  if (split_math() && groups == 1 && !check_only && sh == 1 && sw == 1) {
+  if (patch_math(groups, epi, y) && !check_only && sh == 1 && sw == 1) {
     const PatchConv pc{N, C, H, W, K, P, Q, R, S, ph, pw, dh, dw, false};
-    if (patch_conv_takes(pc)) {
+    if (patch_conv_takes(pc, !split_math())) {
       if (size_only) {
         *size_only = patch_workspace(pc);
         return 0;
       }
-      return patch_conv_launch(pc, x, w, bias, y, epi, TT_PROF_CONV_IGEMM_FWD, g_last_launch);
+      return patch_conv_launch(pc, x, w, bias, y, epi, !split_math(), TT_PROF_CONV_IGEMM_FWD, g_last_launch);
     }
   }
   if (!check_only) {
@@ -832,14 +837,14 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
       return hwc_conv(hc, dy, w, bias, dx, epi, TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
     }
   }
-  if (split_math() && groups == 1 && !check_only && sh == 1 && sw == 1) {
+  if (patch_math(groups, epi, dx) && !check_only && sh == 1 && sw == 1) {
     const PatchConv pc{N, K, P, Q, C, Hx, Wx, R, S, (R - 1) * dh - ph, (S - 1) * dw - pw, dh, dw, true};
-    if (patch_conv_takes(pc)) {
+    if (patch_conv_takes(pc, !split_math())) {
       if (size_only) {
         *size_only = patch_workspace(pc);
         return 0;
       }
-      return patch_conv_launch(pc, dy, w, bias, dx, epi, TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
+      return patch_conv_launch(pc, dy, w, bias, dx, epi, !split_math(), TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
     }
   }
   const int gh = gcd(sh, dh), gw = gcd(sw, dw);

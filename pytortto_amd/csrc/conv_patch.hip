@@ -18,6 +18,12 @@
 // compute unit the device's power bounds it; with one, what a wave does between two chunks (the matrix pipes
 // are busy 40 % of the time then) and, where a reduction is shared, the sums' way through memory.
 //
+// Float32 arithmetic uses them too, where a call is large: the terms add up to the operands exactly, what is left out
+// of a product is below half an ulp of it, and the error against float64 sums is 0.33 to 0.66 times that of the
+// float32 instructions, which round twice as often (42 launches).  A ResNet-50 training step at batch 64 takes
+// 19.43 ms for 20.27, a PreAct-ResNet-18 one at batch 128 4.81 for 5.35.  What three terms do not hold is summed
+// again (terms_fail).
+//
 // The pixels of a tile are consecutive pixels of the batch, whatever the image's shape.  Their source lies in
 // a virtual image that holds the images of the batch below each other, each framed by what the taps reach
 // outside it: virtual pixel (n*VR + j)*PW + k is row j + bh, column k + bw of image n, zero outside.  A
@@ -114,7 +120,57 @@ struct Patch {
   int px;              // pixels of the patch held in LDS
   int images;
   tt::FastDiv divPW, divVR;
+  // float32 launches: the weights as they came, strides of a row and a channel; null otherwise
+  const float* w;
+  int wRow, wChan, dgrad, dh, dw;
 };
+
+// What the launch does to a sum on its way to memory, for one value: the steps of store_through_epilogue.
+__device__ __forceinline__ float finish_value(const Igemm& p, const int i, const uint32_t e, float v) {
+  if (p.bias) v += p.bias[i];
+  if (p.epi.on) {
+    if (p.epi.norm) {
+      const float sd = __fsqrt_rn(__fadd_rn(p.epi.var[i], p.epi.eps));
+      v = fmaf(v - p.epi.mean[i], __fdiv_rn(p.epi.gamma ? p.epi.gamma[i] : 1.0f, sd), p.epi.beta ? p.epi.beta[i] : 0.0f);
+    }
+    if (p.epi.res) v += p.epi.res[e];
+    if (p.epi.relu) v = (v > 0.f || v != v) ? v : 0.f;
+    if (p.epi.mask) v *= p.epi.mask[e] > 0.f ? 1.f : 0.f;
+  }
+  return v;
+}
+
+// Values for which the terms do not stand for the operands: a sum with an operand that is not finite, or whose
+// first term is not, comes out as NaN; one that overflows may have done so by its terms' roundings; and operands
+// below 2^-110 lose bits of their last term to the least bfloat16, which only sums of such operands notice.
+__device__ __forceinline__ bool terms_fail(const float v) {
+  const float a = __builtin_fabsf(v);
+  return !(a <= 3.402823466e38f) || (a < 0x1p-96f && a > 0.f);
+}
+
+// One sum in float64, over the channels [c0, c1): the rare path behind terms_fail.  A NaN stays one, so that data
+// full of them cost a product each.
+__device__ __forceinline__ float exact_sum(const Igemm& p, const Patch& q, const int i, const uint32_t m, const int c0, const int c1) {
+  const uint32_t n = tt::fd_div(m, p.divUV), rem = m - n * p.divUV.d;
+  const uint32_t u = tt::fd_div(rem, p.divV);
+  const int ih = (int)u + p.bh, iw = (int)(rem - u * p.divV.d) + p.bw;
+  const int R = q.taps / q.S;
+  const char* image = (const char*)q.src + (long long)n * q.image;
+  double sum = 0.0;
+  for (int c = c0; c < c1 && sum == sum; ++c) {
+    const float* x = (const float*)(image + (long long)c * q.plane);
+    const float* w = q.w + (long long)i * q.wRow + (long long)c * q.wChan;
+    for (int r = 0; r < R; ++r) {
+      const int h = ih + r * q.dh;
+      for (int s = 0; s < q.S; ++s) {   // a tap outside the image multiplies a zero, as everywhere
+        const int v = iw + s * q.dw, t = r * q.S + s;
+        const bool inside = (unsigned)h < (unsigned)p.Hlim && (unsigned)v < (unsigned)p.Wlim;
+        sum = fma(inside ? (double)x[h * p.Wlim + v] : 0.0, (double)w[q.dgrad ? q.taps - 1 - t : t], sum);
+      }
+    }
+  }
+  return (float)sum;
+}
 
 // Tile 32*WM rows x 32*NT*(4/WM) pixels; every wave has 32 rows and NT x 32 pixels.  The patch has at most 128*IT
 // pixels: a thread fetches and splits eight channels of IT of them.
@@ -301,32 +357,55 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
 #pragma unroll
   for (int y = 0; y < NT; ++y) acc[0][y] += small[y];
 
+  unsigned long long again = 0;   // values to be summed once more (bit 16*y + r)
+  if (q.w) {
+#pragma unroll
+    for (int y = 0; y < NT; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) again |= (unsigned long long)terms_fail(acc[0][y][r]) << (16 * y + r);
+  }
   if constexpr (EPI) {
     if (whole && p.epi.on) {
-      store_through_epilogue<BM, 1, NT>(p, acc, obase, mok, i0, wm * 32, h, epi_lds);
-      return;
+#pragma unroll
+      for (int y = 0; y < NT; y += 2) {   // two tiles at a time: their residuals and masks are as many registers again
+        const floatx16 two[1][2] = {{acc[0][y], acc[0][y + 1]}};
+        const uint32_t ob[2] = {obase[y], obase[y + 1]};
+        const bool ok[2] = {mok[y], mok[y + 1]};
+        store_through_epilogue<BM, 1, 2>(p, two, ob, ok, i0, wm * 32, h, epi_lds);
+      }
     }
   }
   // accumulator register r of a 32x32 tile holds row 8*(r/4) + 4*h + r%4, column l32
-  float* __restrict__ out = whole ? p.out : q.partial + (size_t)blockIdx.z * (size_t)q.outElems;
-  const bool biased = whole && p.bias != nullptr;
-  const uint32_t hoff = (uint32_t)(4 * h * p.outStrideI);
-  const int srow = __builtin_amdgcn_readfirstlane(i0 + wm * 32);
-  float bz[16];
+  float* out = whole ? p.out : q.partial + (size_t)blockIdx.z * (size_t)q.outElems;
+  if (!EPI || !whole || !p.epi.on) {
+    const bool biased = whole && p.bias != nullptr;
+    const uint32_t hoff = (uint32_t)(4 * h * p.outStrideI);
+    const int srow = __builtin_amdgcn_readfirstlane(i0 + wm * 32);
+    float bz[16];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) bz[r] = biased ? p.bias[min(srow + 8 * (r >> 2) + 4 * h + (r & 3), p.I - 1)] : 0.f;
-  __builtin_amdgcn_sched_barrier(0);
-  __builtin_amdgcn_s_waitcnt(0x0f70);   // every load done before the first store: they share one counter
-  __builtin_amdgcn_sched_barrier(0);
+    for (int r = 0; r < 16; ++r) bz[r] = biased ? p.bias[min(srow + 8 * (r >> 2) + 4 * h + (r & 3), p.I - 1)] : 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0x0f70);   // every load done before the first store: they share one counter
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int row = srow + 8 * (r >> 2) + (r & 3);
-    float* __restrict__ rowp = out + (size_t)row * (size_t)p.outStrideI;
-    if (row + 4 * h < p.I) {
+    for (int r = 0; r < 16; ++r) {
+      const int row = srow + 8 * (r >> 2) + (r & 3);
+      float* __restrict__ rowp = out + (size_t)row * (size_t)p.outStrideI;
+      if (row + 4 * h < p.I) {
 #pragma unroll
-      for (int y = 0; y < NT; ++y)
-        if (mok[y]) rowp[obase[y] + hoff] = biased ? acc[0][y][r] + bz[r] : acc[0][y][r];
+        for (int y = 0; y < NT; ++y)
+          if (mok[y]) rowp[obase[y] + hoff] = biased ? acc[0][y][r] + bz[r] : acc[0][y][r];
+      }
     }
+  }
+  for (; again; again &= again - 1) {
+    const int bit = __builtin_ctzll(again), r = bit & 15;
+    const int i = i0 + wm * 32 + 8 * (r >> 2) + 4 * h + (r & 3), m = m0 + (wn * NT + (bit >> 4)) * 32 + l32;
+    if (i >= p.I || m >= p.M) continue;
+    const float v = exact_sum(p, q, i, (uint32_t)m, q0 * kBK, min(q.C, q1 * kBK));
+    const uint32_t n = tt::fd_div((uint32_t)m, p.divUV);
+    const uint32_t e = n * (uint32_t)p.outStrideN + ((uint32_t)m - n * p.divUV.d) + (uint32_t)i * (uint32_t)p.outStrideI;
+    out[e] = whole ? finish_value(p, i, e, v) : v;
   }
 }
 
@@ -399,7 +478,7 @@ size_t patch_workspace(const PatchConv& c) {
   return make_plan(c, &pl) ? pl.wt + pl.partial : 0;
 }
 
-bool patch_conv_takes(const PatchConv& c) {
+bool patch_conv_takes(const PatchConv& c, bool f32) {
   if (g_patch == 0) return false;
   const int taps = c.R * c.S;
   if (taps > kMaxTaps) return false;
@@ -420,11 +499,14 @@ bool patch_conv_takes(const PatchConv& c) {
   // (23.4, 56.8), whose rows and channels are mostly padding.
   const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
   const double gigas = 2e-9 * c.I * c.C * taps * c.N * c.P * c.Q;
-  return taps >= 4 && padding <= 1.5 && gigas >= 1.5 && pl.cost + 3 + 4e-6 * c.I * c.C * taps < 16 + 7 * gigas;
+  // In float32 arithmetic the kernels that gather take 7.5 us and more (94 for 9.7e9 and 119 to 138 for 14.8e9, where
+  // these take 63 to 68 and 90 to 102); small calls, which gain a few microseconds at most, stay with them.
+  return taps >= 4 && padding <= 1.5 && gigas >= (f32 ? 4.0 : 1.5) &&
+         pl.cost + 3 + 4e-6 * c.I * c.C * taps < 16 + (f32 ? 7.5 : 7.0) * gigas;
 }
 
 int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi,
-                      int prof_id, int* plan8) {
+                      bool f32, int prof_id, int* plan8) {
   const int taps = c.R * c.S;
   Plan pl;
   if (!make_plan(c, &pl)) return tt::fail(-1, "patch convolution: no plan");
@@ -449,6 +531,11 @@ int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const 
   q.PW = pl.PW; q.VR = pl.VR;
   q.tapRow = c.dh * pl.PW * kUnit; q.tapCol = c.dw * kUnit;
   q.px = pl.px; q.images = c.N;
+  if (f32) {
+    q.w = w;
+    q.wRow = c.dgrad ? taps : c.C * taps; q.wChan = c.dgrad ? c.I * taps : taps;
+    q.dgrad = c.dgrad; q.dh = c.dh; q.dw = c.dw;
+  }
   q.divPW = tt::make_fastdiv((uint32_t)pl.PW); q.divVR = tt::make_fastdiv((uint32_t)pl.VR);
   {
     tt::ProfScope prof(TT_PROF_CONV_PREP);

@@ -16,9 +16,9 @@ ALWAYS, WHERE_FASTER, NEVER = 2, 1, 0
 
 @pytest.fixture
 def patch():
-    def choose(which):
+    def choose(which, math='bf16x3'):
         _hip.call('tt_conv2d_patch_enable', which)
-    _hip.set_conv_math('bf16x3')
+        _hip.set_conv_math(math)
     yield choose
     choose(WHERE_FASTER)
     _hip.set_conv_math('f32')
@@ -40,9 +40,9 @@ EDGES = [
 
 
 @pytest.mark.parametrize('case', EDGES + [c for c in CONV_CASES + TILE_CASES if c[7] == (1, 1) and c[10] == 1])
-@pytest.mark.parametrize('bias', [True, False])
-def test_meets_the_float32_bar(case, bias, patch):
-    patch(ALWAYS)
+@pytest.mark.parametrize('bias,math', [(True, 'bf16x3'), (False, 'f32')])
+def test_meets_the_float32_bar(case, bias, math, patch):
+    patch(ALWAYS, math)
     _run_conv(case, seed=5, bias=bias)
     if case in EDGES:
         assert _last_launch()['persistent_blocks'] == -4
@@ -50,14 +50,15 @@ def test_meets_the_float32_bar(case, bias, patch):
 
 @pytest.mark.parametrize('case', random_conv_cases(60, 91) + random_large_kernel_cases(8, 92))
 def test_random_geometries(case, patch):
-    patch(ALWAYS)
+    patch(ALWAYS, 'f32')
     _run_conv(case, seed=6)
 
 
+@pytest.mark.parametrize('math', ['bf16x3', 'f32'])
 @pytest.mark.parametrize('n,c,hw,k', [(9, 64, 14, 96), (2, 256, 7, 70), (40, 32, 28, 64)])   # the second shares its reduction
-def test_epilogues(n, c, hw, k, patch):
+def test_epilogues(n, c, hw, k, math, patch):
     """The same bits as the entry points they stand in for."""
-    patch(ALWAYS)
+    patch(ALWAYS, math)
     rng = np.random.default_rng(3)
     x, w, res, mask = (hiparray(rng.standard_normal(s).astype(np.float32))
                        for s in ((n, c, hw, hw), (k, c, 3, 3), (n, k, hw, hw), (n, c, hw, hw)))
@@ -74,6 +75,41 @@ def test_epilogues(n, c, hw, k, patch):
     fused = ops.conv2d_dgrad(res, w, None, (hw, hw), (1, 1), (1, 1), (1, 1), 1, add=x, relu_y=mask).get()
     assert _last_launch()['persistent_blocks'] == -4
     assert np.array_equal(fused, (dx + x.get()) * (mask.get() > 0))
+
+
+@pytest.mark.parametrize('n,c,hw,k', [(9, 64, 14, 96), (2, 256, 7, 70), (3, 17, 28, 33)])
+@pytest.mark.parametrize('scale', [1.0, 2.0 ** 120, 2.0 ** -126, 2.0 ** -140])
+def test_operands_the_terms_do_not_hold(n, c, hw, k, scale, patch):
+    """float32 arithmetic: infinities, NaN, magnitudes that round to a bfloat16 infinity and operands whose last terms
+    it cannot hold give what the other kernels give, behind an epilogue as well."""
+    rng = np.random.default_rng(4)
+    xh, wh = rng.standard_normal((n, c, hw, hw)).astype(np.float32), rng.standard_normal((k, c, 3, 3)).astype(np.float32)
+    xh, wh = np.ldexp(xh, int(np.log2(scale))), wh / np.float32(4)
+    if scale == 1.0:
+        xh[0, 0, 2, 3], xh[0, 1, 2, 5], xh[1, c - 1, 0, 0], xh[1, 3, 5, 5] = np.inf, -np.inf, np.nan, np.float32(3.4e38)
+        wh[5, 2, 1, 1] = -np.inf
+    x, w = hiparray(xh), hiparray(wh)
+    bias = hiparray(rng.standard_normal(k).astype(np.float32) * np.float32(scale))
+    add = hiparray((rng.standard_normal((n, c, hw, hw)) * scale).astype(np.float32))
+    dy = hiparray(np.resize(xh, (n, k, hw, hw)))
+    geometry = ((1, 1), (1, 1), (1, 1), 1)
+
+    def results():
+        return (ops.conv2d_fwd(x, w, None, *geometry).get(), ops.conv2d_fwd(x, w, bias, *geometry).get(),
+                ops.conv2d_dgrad(dy, w, None, (hw, hw), *geometry).get(),
+                ops.conv2d_dgrad(dy, w, None, (hw, hw), *geometry, add=add, relu_y=add).get())
+    patch(ALWAYS, 'f32')
+    got = results()
+    assert _last_launch()['persistent_blocks'] == -4
+    patch(NEVER, 'f32')
+    for a, b in zip(got, results()):
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert np.array_equal(np.isinf(a), np.isinf(b))
+        finite = np.isfinite(a) & np.isfinite(b)
+        assert finite.mean() > .5
+        size = float(np.abs(b[finite], dtype=np.float64).max())
+        # the least bfloat16 is 2^-133: what rounds to no term at all is missing from a sum of nothing else
+        np.testing.assert_allclose(a[finite], b[finite], rtol=1e-5, atol=max(1e-6 * min(size, 1e3 * scale), 2.0 ** -133 * 9 * max(c, k)))
 
 
 @pytest.mark.parametrize('dims', [(4, 64, 28, 28, 64, 3), (2, 512, 7, 7, 512, 3), (4, 128, 16, 16, 256, 3), (3, 96, 20, 17, 48, 5),
@@ -99,7 +135,7 @@ def test_sums_are_as_accurate_as_in_the_other_kernels(dims, patch):
     new = errors()
     patch(NEVER)
     old = errors()
-    _hip.set_conv_math('f32')
+    patch(NEVER, 'f32')
     f32 = errors()
     for key in want:
         print(dims, key, 'patch %.2e, gathered %.2e, float32 %.2e' % (new[key], old[key], f32[key]))
