@@ -79,18 +79,21 @@ __global__ __launch_bounds__(kThreads) void patch_weights(const float* __restric
   const int chunk = blockIdx.x, r0 = blockIdx.y * 32, c0 = chunk * kBK;
   const int run = divRun.d;          // (DGRAD ? 32 : 16) * taps
   const int outer = DGRAD ? kBK : 32;
-  for (int u = threadIdx.x; u < outer * run; u += kThreads) {
-    const int a = (int)tt::fd_div((uint32_t)u, divRun), b = u - a * run;
-    bool ok;
-    size_t at;
-    if constexpr (DGRAD) {
-      ok = c0 + a < chans && r0 * taps + b < rows * taps;
-      at = ((size_t)(c0 + a) * rows + r0) * taps + b;
-    } else {
-      ok = r0 + a < rows && c0 * taps + b < chans * taps;
-      at = ((size_t)(r0 + a) * chans + c0) * taps + b;
+  for (int u0 = threadIdx.x; u0 < outer * run; u0 += 8 * kThreads) {   // eight loads in flight: small layers have few blocks
+    float v[8];
+    int at[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int u = u0 + e * kThreads;
+      const int a = (int)tt::fd_div((uint32_t)u, divRun), b = u - a * run;
+      const bool ok = a < outer && (DGRAD ? c0 + a < chans && r0 * taps + b < rows * taps : r0 + a < rows && c0 * taps + b < chans * taps);
+      const size_t from = DGRAD ? ((size_t)(c0 + a) * rows + r0) * taps + b : ((size_t)(r0 + a) * chans + c0) * taps + b;
+      at[e] = a < outer ? a * (run + 1) + b : -1;
+      v[e] = ok ? w[from] : 0.f;
     }
-    strip[a * (run + 1) + b] = ok ? w[at] : 0.f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (at[e] >= 0) strip[at[e]] = v[e];
   }
   __syncthreads();
   uintx4* __restrict__ dst = wt + ((size_t)blockIdx.y * chunks + chunk) * taps * (kTerms * 64);
@@ -451,7 +454,7 @@ bool make_plan(const PatchConv& c, Plan* best) {
     // Microseconds, fitted to 75 launches of 4 to 2000 blocks (10 % root mean square): a chunk of a block that
     // shares its compute unit, a block's start and end; a block that has the unit for itself takes a sixth longer.
     // Shares of a reduction are written, read and added.  (The weights' layout costs the same for all.)
-    const double chunk = pl.NT == 4 ? 0.55 * taps + 1.0 : 0.29 * taps + 0.9;
+    const double chunk = pl.NT == 4 ? 0.55 * taps + 1.0 : 0.32 * taps + 1.0;
     for (int s = 1; s <= 8 && s <= pl.chunks; ++s) {
       const int per = ceil_div(pl.chunks, s);
       if (ceil_div(pl.chunks, per) != s) continue;
