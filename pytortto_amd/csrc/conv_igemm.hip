@@ -732,7 +732,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
     }
   }
   if (patch_math(groups, epi, y) && !check_only && sh == 1 && sw == 1) {
-    const PatchConv pc{N, C, H, W, K, P, Q, R, S, ph, pw, dh, dw, false};
+    const PatchConv pc{N, C, H, W, K, P * Q, Q, 1, 1, R * S, false, 1, {{P, Q, R, S, ph, pw, dh, dw, 0, 0, 0, S, 1}}};
     if (patch_conv_takes(pc, !split_math())) {
       if (size_only) {
         *size_only = patch_workspace(pc);
@@ -805,6 +805,13 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
   return launch_igemm(p, groups, t, TT_PROF_CONV_IGEMM_FWD, (floatx4*)((char*)ws + wp_bytes));
 }
 
+// The first tap that reaches dx rows (columns) of residue `cls` modulo the stride; the others follow `step` apart.
+static int first_tap(int cls, int stride, int pad, int dil, int taps, int step) {
+  for (int r = 0; r < taps && r < step; ++r)
+    if (((cls + pad - r * dil) % stride + stride) % stride == 0) return r;
+  return -1;
+}
+
 static int conv2d_dgrad(const float* dy, const float* w, const float* bias, float* dx, int N, int C, int Hx, int Wx,
                         int K, int R, int S, int sh, int sw, int ph, int pw, int dh, int dw, int groups, int P,
                         int Q, size_t* size_only, bool check_only = false, const Epilogue* epi = nullptr) {
@@ -837,16 +844,6 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
       return hwc_conv(hc, dy, w, bias, dx, epi, TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
     }
   }
-  if (patch_math(groups, epi, dx) && !check_only && sh == 1 && sw == 1) {
-    const PatchConv pc{N, K, P, Q, C, Hx, Wx, R, S, (R - 1) * dh - ph, (S - 1) * dw - pw, dh, dw, true};
-    if (patch_conv_takes(pc, !split_math())) {
-      if (size_only) {
-        *size_only = patch_workspace(pc);
-        return 0;
-      }
-      return patch_conv_launch(pc, dy, w, bias, dx, epi, !split_math(), TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
-    }
-  }
   const int gh = gcd(sh, dh), gw = gcd(sw, dw);
   const int rstep = sh / gh, sstep = sw / gw;   // valid taps of a class: r0, r0+rstep, ...
   const int eh = dh / gh, ew = dw / gw;          // dy row/column step per tap
@@ -855,6 +852,29 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
   TT_REQUIRE(classes <= 4096, "%s: stride %d x %d not supported", fn, sh, sw);
   hipStream_t st = check_only ? nullptr : tt::stream();
 
+  if (patch_math(groups, epi, dx) && !check_only && classes <= kPatchClasses && sh <= Hx && sw <= Wx) {
+    PatchConv pc{N, K, P, Q, C, Hx * Wx, Wx, sh, sw, R * S, true, 0, {}};
+    bool every = true;   // class has a tap
+    for (int ch = 0; ch < sh; ++ch)
+      for (int cw = 0; cw < sw; ++cw) {
+        const int r0 = first_tap(ch, sh, ph, dh, R, rstep), s0 = first_tap(cw, sw, pw, dw, S, sstep);
+        every = every && r0 >= 0 && s0 >= 0;
+        if (!every) continue;
+        // dx[h] reads dy[(h + ph - r*dh) / sh]: with the taps in reverse order, ascending rows
+        const int TB = ceil_div(R - r0, rstep), TC = ceil_div(S - s0, sstep);
+        pc.c[pc.n++] = PatchConvClass{ceil_div(Hx - ch, sh), ceil_div(Wx - cw, sw), TB, TC, (TB - 1) * eh - (ch + ph - r0 * dh) / sh,
+                                      (TC - 1) * ew - (cw + pw - s0 * dw) / sw, eh, ew, ch, cw,
+                                      (r0 + (TB - 1) * rstep) * S + s0 + (TC - 1) * sstep, -rstep * S, -sstep};
+      }
+    if (every && patch_conv_takes(pc, !split_math())) {
+      if (size_only) {
+        *size_only = patch_workspace(pc);
+        return 0;
+      }
+      return patch_conv_launch(pc, dy, w, bias, dx, epi, !split_math(), TT_PROF_CONV_IGEMM_DGRAD, g_last_launch);
+    }
+  }
+
   if (!check_only && std::min(sh, Hx) * std::min(sw, Wx) <= kNarrowClasses) {
     NarrowConv nc{dy, w, bias, dx, Cg, Kg, groups, tt::make_fastdiv((uint32_t)Kg), {}, R * S, Cg * R * S, Kg * Cg * R * S, rstep, sstep, S,
                   1, 1, -eh, -ew, P, Q, K * P * Q, Kg * P * Q, P * Q, C * Hx * Wx, Cg * Hx * Wx, Hx * Wx, Wx, sh, sw, true, 0, {}, {}};
@@ -862,11 +882,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
     for (int ch = 0; ch < sh && ch < Hx; ++ch)
       for (int cw = 0; cw < sw && cw < Wx; ++cw) {
         // the first tap of the class in either direction, then every rstep-th, sstep-th
-        int r0 = -1, s0 = -1;
-        for (int r = 0; r < R && r < rstep && r0 < 0; ++r)
-          if (((ch + ph - r * dh) % sh + sh) % sh == 0) r0 = r;
-        for (int s = 0; s < S && s < sstep && s0 < 0; ++s)
-          if (((cw + pw - s * dw) % sw + sw) % sw == 0) s0 = s;
+        const int r0 = first_tap(ch, sh, ph, dh, R, rstep), s0 = first_tap(cw, sw, pw, dw, S, sstep);
         const int U = ceil_div(Hx - ch, sh), V = ceil_div(Wx - cw, sw);
         const bool any = r0 >= 0 && s0 >= 0;   // a class without taps holds the bias, or zeros
         const int TB = any ? ceil_div(R - r0, rstep) : 0, TC = any ? ceil_div(S - s0, sstep) : 1;

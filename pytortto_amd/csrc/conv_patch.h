@@ -4,11 +4,20 @@
 
 namespace ttc {
 
-// x is [N][C][H][W], the result [N][I][P][Q]; output pixel (u, v) reads input rows u - ph + r*dh (ph, pw may be
-// negative).  dgrad: w is [C][I][R][S] with its taps reversed instead of [I][C][R][S].
+// A forward pass is one class of pixels, an input gradient one for each parity of its stride.  Pixel (n, u, v) of
+// U x V reads source rows u - ph + r*dh, columns v - pw + s*dw for its R x S taps (ph, pw may be negative), tap (r, s)
+// being element w0 + r*wRow + s*wCol of the kernel, and lands in row u*ou + ouh, column v*ov + ovw of its plane.
+constexpr int kPatchClasses = 4;
+struct PatchConvClass {
+  int U, V, R, S, ph, pw, dh, dw, ouh, ovw, w0, wRow, wCol;
+};
+// The source is [N][C][H][W], the result [N][I][outPlane], its rows outRow long.  dgrad: w is [C][I][taps] instead of
+// [I][C][taps].
 struct PatchConv {
-  int N, C, H, W, I, P, Q, R, S, ph, pw, dh, dw;
+  int N, C, H, W, I, outPlane, outRow, ou, ov, taps;
   bool dgrad;
+  int n;
+  PatchConvClass c[kPatchClasses];
 };
 // f32: the call is one of float32 arithmetic (TT_CONV_MATH_F32), not of bf16x3: operands of any magnitude, infinities
 // and NaN give what they give there.

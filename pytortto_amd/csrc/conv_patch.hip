@@ -69,12 +69,20 @@ __device__ __forceinline__ void split8(const float (&v)[8], uintx4 (&out)[kTerms
   }
 }
 
+// Which taps of the kernel the classes of a call run, for the layout of their weights: tap (r, s) of class k is
+// element w0 + r*wRow + s*wCol of the kernel, its weights begin at wt (units of 16 bytes).
+struct PatchTaps {
+  int n;
+  int taps[kPatchClasses], S[kPatchClasses], w0[kPatchClasses], wRow[kPatchClasses], wCol[kPatchClasses];
+  size_t wt[kPatchClasses];
+};
+
 // ---- weights -> wt[32 rows][chunk][tap][term][lane], 16 bytes each: lane 32*h + l holds row l, channels 8h.. --
-// forward: row k, w[k][c][tap];  input gradient: row c, channel k, taps in reverse order.  A block lays out
-// one strip of 32 rows and sixteen channels: reads runs of w, turns them in LDS, writes runs of wt.
+// forward: row k, w[k][c][tap];  input gradient: row c, channel k.  A block lays out one strip of 32 rows and
+// sixteen channels for every class: reads runs of w, turns them in LDS, writes runs of wt.
 template <bool DGRAD>
 __global__ __launch_bounds__(kThreads) void patch_weights(const float* __restrict__ w, uintx4* __restrict__ wt, int rows, int chans,
-                                                         int taps, tt::FastDiv divRun, int chunks) {
+                                                         int taps, tt::FastDiv divRun, int chunks, const PatchTaps classes) {
   extern __shared__ float strip[];   // [outer][run + 1]: forward 32 rows x 16 channels' taps, gradient 16 x 32 rows' taps
   const int chunk = blockIdx.x, r0 = blockIdx.y * 32, c0 = chunk * kBK;
   const int run = divRun.d;          // (DGRAD ? 32 : 16) * taps
@@ -96,36 +104,52 @@ __global__ __launch_bounds__(kThreads) void patch_weights(const float* __restric
       if (at[e] >= 0) strip[at[e]] = v[e];
   }
   __syncthreads();
-  uintx4* __restrict__ dst = wt + ((size_t)blockIdx.y * chunks + chunk) * taps * (kTerms * 64);
-  for (int u = threadIdx.x; u < taps * 64; u += kThreads) {
-    const int tap = u >> 6, lane = u & 63, row = lane & 31, c = 8 * (lane >> 5);
-    float v[8];
+  for (int k = 0; k < classes.n; ++k) {
+    const int mine = classes.taps[k], S = classes.S[k];
+    uintx4* __restrict__ dst = wt + classes.wt[k] + ((size_t)blockIdx.y * chunks + chunk) * mine * (kTerms * 64);
+    for (int u = threadIdx.x; u < mine * 64; u += kThreads) {
+      const int tap = u >> 6, lane = u & 63, row = lane & 31, c = 8 * (lane >> 5);
+      const int from = classes.w0[k] + tap / S * classes.wRow[k] + tap % S * classes.wCol[k];
+      float v[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      v[e] = DGRAD ? strip[(c + e) * (run + 1) + row * taps + (taps - 1 - tap)] : strip[row * (run + 1) + (c + e) * taps + tap];
-    uintx4 t[kTerms];
-    split8(v, t);
+      for (int e = 0; e < 8; ++e) v[e] = DGRAD ? strip[(c + e) * (run + 1) + row * taps + from] : strip[row * (run + 1) + (c + e) * taps + from];
+      uintx4 t[kTerms];
+      split8(v, t);
 #pragma unroll
-    for (int i = 0; i < kTerms; ++i) dst[(tap * kTerms + i) * 64 + lane] = t[i];
+      for (int i = 0; i < kTerms; ++i) dst[(tap * kTerms + i) * 64 + lane] = t[i];
+    }
   }
 }
 
 // ---- the product -------------------------------------------------------------------------------------
+struct PatchClass {
+  int M;                     // pixels (n, u, v)
+  tt::FastDiv divUV, divV;
+  int bh, bw, ouh, ovw;      // tap 0 reads row u + bh, column v + bw; the result is row u*ou + ouh, column v*ov + ovw
+  int taps, S;
+  int PW, VR;                // the virtual image's pitch and rows per image
+  tt::FastDiv divPW, divVR;
+  int px;                    // pixels of the patch held in LDS
+  int tapRow, tapCol;        // steps of a tap row / column in the patch, in bytes
+  int dh, dw;                // the same in pixels of the source
+  int w0, wRow, wCol;        // tap (r, s) is element w0 + r*wRow + s*wCol of the kernel
+  int block0;                // its first tile
+  size_t wt;                 // where its weights begin, units of 16 bytes
+};
 struct Patch {
   const float* src;
   const uintx4* wt;
   float* partial;      // splits > 1: [splits][elements of out] sums over a part of the chunks each
   long long outElems;
-  int C, chunks, perSplit, taps, S;
+  int C, chunks, perSplit;
   int plane, image;    // bytes of a source plane, an image
-  int PW, VR;          // the virtual image's pitch and rows per image
-  int tapRow, tapCol;  // steps of a tap row / column in the patch, in bytes
-  int px;              // pixels of the patch held in LDS
+  int maxPx;           // of the classes' patches
   int images;
-  tt::FastDiv divPW, divVR;
   // float32 launches: the weights as they came, strides of a row and a channel; null otherwise
   const float* w;
-  int wRow, wChan, dgrad, dh, dw;
+  int wI, wC;
+  int classes;
+  PatchClass c[kPatchClasses];
 };
 
 // What the launch does to a sum on its way to memory, for one value: the steps of store_through_epilogue.
@@ -153,22 +177,20 @@ __device__ __forceinline__ bool terms_fail(const float v) {
 
 // One sum in float64, over the channels [c0, c1): the rare path behind terms_fail.  A NaN stays one, so that data
 // full of them cost a product each.
-__device__ __forceinline__ float exact_sum(const Igemm& p, const Patch& q, const int i, const uint32_t m, const int c0, const int c1) {
-  const uint32_t n = tt::fd_div(m, p.divUV), rem = m - n * p.divUV.d;
-  const uint32_t u = tt::fd_div(rem, p.divV);
-  const int ih = (int)u + p.bh, iw = (int)(rem - u * p.divV.d) + p.bw;
-  const int R = q.taps / q.S;
+__device__ __forceinline__ float exact_sum(const Igemm& p, const Patch& q, const PatchClass& k, const int i, const uint32_t n, const int u, const int v,
+                                          const int c0, const int c1) {
+  const int R = k.taps / k.S;
   const char* image = (const char*)q.src + (long long)n * q.image;
   double sum = 0.0;
   for (int c = c0; c < c1 && sum == sum; ++c) {
     const float* x = (const float*)(image + (long long)c * q.plane);
-    const float* w = q.w + (long long)i * q.wRow + (long long)c * q.wChan;
+    const float* w = q.w + (long long)i * q.wI + (long long)c * q.wC + k.w0;
     for (int r = 0; r < R; ++r) {
-      const int h = ih + r * q.dh;
-      for (int s = 0; s < q.S; ++s) {   // a tap outside the image multiplies a zero, as everywhere
-        const int v = iw + s * q.dw, t = r * q.S + s;
-        const bool inside = (unsigned)h < (unsigned)p.Hlim && (unsigned)v < (unsigned)p.Wlim;
-        sum = fma(inside ? (double)x[h * p.Wlim + v] : 0.0, (double)w[q.dgrad ? q.taps - 1 - t : t], sum);
+      const int h = u + k.bh + r * k.dh;
+      for (int s = 0; s < k.S; ++s) {   // a tap outside the image multiplies a zero, as everywhere
+        const int j = v + k.bw + s * k.dw;
+        const bool inside = (unsigned)h < (unsigned)p.Hlim && (unsigned)j < (unsigned)p.Wlim;
+        sum = fma(inside ? (double)x[h * p.Wlim + j] : 0.0, (double)w[r * k.wRow + s * k.wCol], sum);
       }
     }
   }
@@ -181,22 +203,31 @@ template <int WM, int NT, int IT, bool EPI>
 __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, const Patch q) {
   constexpr int WN = 4 / WM, BM = 32 * WM, BN = 32 * NT * WN;
   extern __shared__ __align__(16) char lds[];   // [half][px] units; then the epilogue's constants
-  float* const epi_lds = reinterpret_cast<float*>(lds + 2 * q.px * kUnit);
+  float* const epi_lds = reinterpret_cast<float*>(lds + 2 * q.maxPx * kUnit);
 
   const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, h = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WN, wn = wave % WN;
-  const int tile = tt::xcd_remap((int)blockIdx.x, (int)gridDim.x);
-  const int tilesI = p.Ipad / BM;
+  const int all = tt::xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  int ci = 0;
+  while (ci + 1 < q.classes && all >= q.c[ci + 1].block0) ++ci;
+  const PatchClass& k = q.c[ci];
+  const int tile = all - k.block0, tilesI = p.Ipad / BM;
   const int i0 = (tile % tilesI) * BM;
   const int m0 = (tile / tilesI) * BN;
   const int q0 = (int)blockIdx.z * q.perSplit, q1 = min(q.chunks, q0 + q.perSplit);
 
+  // pixel m is (n, u, v)
+  auto split_pixel = [&](const uint32_t m, uint32_t& n, uint32_t& u, uint32_t& v) __attribute__((always_inline)) {
+    n = tt::fd_div(m, k.divUV);
+    v = m - n * k.divUV.d;
+    u = tt::fd_div(v, k.divV);
+    v -= u * k.divV.d;
+  };
   auto virtual_pixel = [&](const uint32_t m, uint32_t& n) __attribute__((always_inline)) {
-    n = tt::fd_div(m, p.divUV);
-    const uint32_t rem = m - n * p.divUV.d;
-    const uint32_t u = tt::fd_div(rem, p.divV);
-    return (n * (uint32_t)q.VR + u) * (uint32_t)q.PW + (rem - u * p.divV.d);
+    uint32_t u, v;
+    split_pixel(m, n, u, v);
+    return (n * (uint32_t)k.VR + u) * (uint32_t)k.PW + v;
   };
   uint32_t n0;
   const uint32_t first = virtual_pixel((uint32_t)__builtin_amdgcn_readfirstlane(m0), n0);
@@ -205,15 +236,15 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
 
   // what this thread fetches: half `wave / 2` of the patch pixels it*128 + tid % 128
   const int half = wave >> 1, pp0 = tid & 127;
-  const int at = (half * q.px + pp0) * kUnit;
+  const int at = (half * k.px + pp0) * kUnit;
   int voff[IT];
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
     const int pp = it * 128 + pp0;
     const uint32_t v = first + (uint32_t)pp;
-    const uint32_t row = tt::fd_div(v, q.divPW), n = tt::fd_div(row, q.divVR);
-    const int ih = (int)(row - n * (uint32_t)q.VR) + p.bh, iw = (int)(v - row * (uint32_t)q.PW) + p.bw;
-    const bool inside = pp < q.px && (unsigned)ih < (unsigned)p.Hlim && (unsigned)iw < (unsigned)p.Wlim && n < (uint32_t)q.images;
+    const uint32_t row = tt::fd_div(v, k.divPW), n = tt::fd_div(row, k.divVR);
+    const int ih = (int)(row - n * (uint32_t)k.VR) + k.bh, iw = (int)(v - row * (uint32_t)k.PW) + k.bw;
+    const bool inside = pp < k.px && (unsigned)ih < (unsigned)p.Hlim && (unsigned)iw < (unsigned)p.Wlim && n < (uint32_t)q.images;
     voff[it] = inside ? (int)(n - n0) * q.image + (ih * p.Wlim + iw) * 4 : (int)0x80000000;
   }
   float reg[IT][8];
@@ -232,7 +263,7 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
     for (int it = 0; it < IT; ++it) {
       uintx4 t[kTerms];
       split8(reg[it], t);
-      if (it * 128 + pp0 < q.px) {
+      if (it * 128 + pp0 < k.px) {
 #pragma unroll
         for (int i = 0; i < kTerms; ++i) *reinterpret_cast<uintx4*>(lds + at + it * 128 * kUnit + 16 * i) = t[i];
       }
@@ -252,11 +283,11 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
   for (int y = 0; y < NT; ++y) {
     const int m = m0 + (wn * NT + y) * 32 + l32;
     uint32_t n;
-    base[y] = (int)(virtual_pixel((uint32_t)(m < p.M ? m : m0), n) - first + (uint32_t)(h * q.px)) * kUnit;
+    base[y] = (int)(virtual_pixel((uint32_t)(m < k.M ? m : m0), n) - first + (uint32_t)(h * k.px)) * kUnit;
   }
 
   // the wave's weights: one run of 3 KB per tap, fetched two taps ahead into the registers that a tap is done with
-  const uintx4* wptr = q.wt + ((size_t)(i0 / 32 + wm) * q.chunks + q0) * (size_t)(q.taps * kTerms * 64);
+  const uintx4* wptr = q.wt + k.wt + ((size_t)(i0 / 32 + wm) * q.chunks + q0) * (size_t)(k.taps * kTerms * 64);
   uintx4 w1[kTerms], w2[kTerms];
   auto load_weights = [&](uintx4 (&to)[kTerms]) __attribute__((always_inline)) {
 #pragma unroll
@@ -284,10 +315,10 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
       if (y + 2 < NT) load_pixels(y + 2, off, behind);
       else load_pixels(0, next, behind);
       __builtin_amdgcn_sched_barrier(0);
-      auto product = [&](const int i, const int k, floatx16 (&to)[NT]) __attribute__((always_inline)) {
+      auto product = [&](const int i, const int term, floatx16 (&to)[NT]) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < 2; ++j)
-          to[y + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], __builtin_bit_cast(bf16x8, x[j][k]), to[y + j], 0, 0, 0);
+          to[y + j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i], __builtin_bit_cast(bf16x8, x[j][term]), to[y + j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
       };
       product(0, 2, small);
@@ -315,16 +346,16 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
   // The taps of all chunks in pairs, whatever their number.  One too many has zero weights.
   int c = q0, t = 0, ts = 0, row = 0, off = 0, next = 0;   // tap t of chunk c, column ts of its kernel row
   auto look = [&]() __attribute__((always_inline)) {   // where the tap behind this one lies
-    next = off + q.tapCol;
-    if (++ts == q.S) {
+    next = off + k.tapCol;
+    if (++ts == k.S) {
       ts = 0;
-      next = row += q.tapRow;
+      next = row += k.tapRow;
     }
-    if (t + 1 == q.taps) next = 0;
+    if (t + 1 == k.taps) next = 0;
   };
   auto advance = [&](const int next_buf) __attribute__((always_inline)) {
     off = next;
-    if (++t == q.taps) {
+    if (++t == k.taps) {
       t = ts = row = 0;
       if (++c < q1) {
         __syncthreads();   // the patch has been read by every wave
@@ -337,14 +368,14 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
     look();
   };
   look();
-  const int total = (q1 - q0) * q.taps;
+  const int total = (q1 - q0) * k.taps;
   constexpr int kOdd = (NT / 2) & 1;   // the buffer that a pair's second tap begins with
-  for (int k = 0; k < total; k += 2) {
+  for (int i = 0; i < total; i += 2) {
     tap(w1, 0, off, next);
     advance(kOdd);
-    if (k + 1 == total)
+    if (i + 1 == total)
 #pragma unroll
-      for (int i = 0; i < kTerms; ++i) w2[i] = uintx4{0, 0, 0, 0};
+      for (int j = 0; j < kTerms; ++j) w2[j] = uintx4{0, 0, 0, 0};
     tap(w2, kOdd, off, next);
     advance(0);
   }
@@ -353,9 +384,10 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
 #pragma unroll
   for (int y = 0; y < NT; ++y) {
     const int m = m0 + (wn * NT + y) * 32 + l32;
-    mok[y] = m < p.M;
-    const uint32_t mm = mok[y] ? (uint32_t)m : 0u, n = tt::fd_div(mm, p.divUV);
-    obase[y] = (uint32_t)((int)n * p.outStrideN + (int)(mm - n * p.divUV.d));
+    mok[y] = m < k.M;
+    uint32_t n, u, v;
+    split_pixel(mok[y] ? (uint32_t)m : 0u, n, u, v);
+    obase[y] = n * (uint32_t)p.outStrideN + (u * (uint32_t)p.ou + (uint32_t)k.ouh) * (uint32_t)p.outRow + v * (uint32_t)p.ov + (uint32_t)k.ovw;
   }
 #pragma unroll
   for (int y = 0; y < NT; ++y) acc[0][y] += small[y];
@@ -404,11 +436,13 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
   for (; again; again &= again - 1) {
     const int bit = __builtin_ctzll(again), r = bit & 15;
     const int i = i0 + wm * 32 + 8 * (r >> 2) + 4 * h + (r & 3), m = m0 + (wn * NT + (bit >> 4)) * 32 + l32;
-    if (i >= p.I || m >= p.M) continue;
-    const float v = exact_sum(p, q, i, (uint32_t)m, q0 * kBK, min(q.C, q1 * kBK));
-    const uint32_t n = tt::fd_div((uint32_t)m, p.divUV);
-    const uint32_t e = n * (uint32_t)p.outStrideN + ((uint32_t)m - n * p.divUV.d) + (uint32_t)i * (uint32_t)p.outStrideI;
-    out[e] = whole ? finish_value(p, i, e, v) : v;
+    if (i >= p.I || m >= k.M) continue;
+    uint32_t n, u, v;
+    split_pixel((uint32_t)m, n, u, v);
+    const float sum = exact_sum(p, q, k, i, n, (int)u, (int)v, q0 * kBK, min(q.C, q1 * kBK));
+    const uint32_t e = n * (uint32_t)p.outStrideN + (u * (uint32_t)p.ou + (uint32_t)k.ouh) * (uint32_t)p.outRow + v * (uint32_t)p.ov +
+                       (uint32_t)k.ovw + (uint32_t)i * (uint32_t)p.outStrideI;
+    out[e] = whole ? finish_value(p, i, e, sum) : sum;
   }
 }
 
@@ -416,8 +450,9 @@ int ceil_div(long long a, long long b) { return (int)((a + b - 1) / b); }
 size_t align_up(size_t v) { return (v + 255) / 256 * 256; }
 
 struct Plan {
-  int WM, NT, IT, Ipad, px, PW, VR, chunks, perSplit, splits, tiles;
-  size_t wt, partial;   // bytes of workspace
+  int WM, NT, IT, Ipad, maxPx, chunks, perSplit, splits, tiles;
+  int px[kPatchClasses], PW[kPatchClasses], VR[kPatchClasses], block0[kPatchClasses];
+  size_t at[kPatchClasses], wt, partial;   // the classes' weights (units of 16 bytes); bytes of workspace
   double cost;
 };
 
@@ -430,41 +465,55 @@ int framed(int pixels, int taps, int dil, int pad, int limit) {
 }
 
 bool make_plan(const PatchConv& c, Plan* best) {
-  const int taps = c.R * c.S;
-  const long long M = (long long)c.N * c.P * c.Q;
   best->cost = -1;
   for (const auto& shape : {std::pair{4, 4}, {2, 4}, {2, 2}}) {
     Plan pl{};
     pl.WM = shape.first; pl.NT = shape.second;
     const int BM = 32 * pl.WM, BN = 128 * pl.NT / pl.WM;
-    pl.VR = framed(c.P, c.R, c.dh, c.ph, c.H);
-    pl.PW = framed(c.Q, c.S, c.dw, c.pw, c.W);
-    // the longest range of the virtual image that BN consecutive pixels and their taps cover
-    const long long rows = (BN + c.Q - 2) / c.Q, images = (BN + (long long)c.P * c.Q - 2) / ((long long)c.P * c.Q);
-    const long long px = BN + rows * (pl.PW - c.Q) + images * (long long)(pl.VR - c.P) * pl.PW +
-                         (long long)(c.R - 1) * c.dh * pl.PW + (long long)(c.S - 1) * c.dw;
-    if (px > 512) continue;
-    pl.px = (int)px;
-    pl.IT = px <= 384 ? 3 : 4;
     pl.Ipad = ceil_div(c.I, BM) * BM;
     pl.chunks = ceil_div(c.C, kBK);
-    pl.tiles = (pl.Ipad / BM) * ceil_div(M, BN);
-    // two taps' weights more: the product reads ahead of its last
-    pl.wt = align_up(((size_t)pl.Ipad / 32 * pl.chunks * taps + 2) * kTerms * 1024);
+    size_t wt = 0;
+    bool fits = true;
+    for (int k = 0; k < c.n && fits; ++k) {
+      const PatchConvClass& g = c.c[k];
+      const long long M = (long long)c.N * g.U * g.V;
+      pl.VR[k] = framed(g.U, g.R, g.dh, g.ph, c.H);
+      pl.PW[k] = framed(g.V, g.S, g.dw, g.pw, c.W);
+      // the longest range of the virtual image that BN consecutive pixels and their taps cover
+      const long long rows = (BN + g.V - 2) / g.V, images = (BN + (long long)g.U * g.V - 2) / ((long long)g.U * g.V);
+      const long long px = BN + rows * (pl.PW[k] - g.V) + images * (long long)(pl.VR[k] - g.U) * pl.PW[k] +
+                           (long long)(g.R - 1) * g.dh * pl.PW[k] + (long long)(g.S - 1) * g.dw;
+      fits = px <= 512;
+      pl.px[k] = (int)px;
+      pl.maxPx = std::max(pl.maxPx, pl.px[k]);
+      pl.block0[k] = pl.tiles;
+      pl.tiles += (pl.Ipad / BM) * ceil_div(M, BN);
+      pl.at[k] = wt;
+      wt += (size_t)pl.Ipad / 32 * pl.chunks * g.R * g.S * kTerms * 64;
+    }
+    if (!fits) continue;
+    pl.IT = pl.maxPx <= 384 ? 3 : 4;
+    pl.wt = align_up((wt + 2 * kTerms * 64) * 16);   // two taps' weights more: the product reads ahead of its last
     // Microseconds, fitted to 75 launches of 4 to 2000 blocks (10 % root mean square): a chunk of a block that
     // shares its compute unit, a block's start and end; a block that has the unit for itself takes a sixth longer.
     // Shares of a reduction are written, read and added.  (The weights' layout costs the same for all.)
-    const double chunk = pl.NT == 4 ? 0.55 * taps + 1.0 : 0.32 * taps + 1.0;
     for (int s = 1; s <= 8 && s <= pl.chunks; ++s) {
       const int per = ceil_div(pl.chunks, s);
       if (ceil_div(pl.chunks, per) != s) continue;
-      const double blocks = (double)pl.tiles * s / tt::compute_units();   // of a compute unit
-      const double cost = std::max(1.17, blocks + 0.1) * (per * chunk + 4) + (s > 1 ? 5 + (2 * s + 1) * 4e-6 / 7 * (double)c.I * M : 0);
+      double work = 0, longest = 0, outputs = 0;
+      for (int k = 0; k < c.n; ++k) {
+        const int taps = c.c[k].R * c.c[k].S;
+        const double block = per * (pl.NT == 4 ? 0.55 * taps + 1.0 : 0.32 * taps + 1.0) + 4;
+        work += block * s * ((k + 1 < c.n ? pl.block0[k + 1] : pl.tiles) - pl.block0[k]);
+        longest = std::max(longest, block);
+        outputs += (double)c.I * c.N * c.c[k].U * c.c[k].V;
+      }
+      const double cost = std::max(1.17 * longest, work / tt::compute_units() + 0.1 * longest) + (s > 1 ? 5 + (2 * s + 1) * 4e-6 / 7 * outputs : 0);
       if (best->cost < 0 || cost < best->cost) {
         pl.perSplit = per;
         pl.splits = s;
         pl.cost = cost;
-        pl.partial = s > 1 ? align_up(sizeof(float) * (size_t)s * c.I * M) : 0;
+        pl.partial = s > 1 ? align_up(sizeof(float) * (size_t)s * (size_t)outputs) : 0;
         *best = pl;
       }
     }
@@ -482,15 +531,21 @@ size_t patch_workspace(const PatchConv& c) {
 }
 
 bool patch_conv_takes(const PatchConv& c, bool f32) {
-  if (g_patch == 0) return false;
-  const int taps = c.R * c.S;
-  if (taps > kMaxTaps) return false;
-  if ((c.R - 1LL) * c.dh > 512 || (c.S - 1LL) * c.dw > 512) return false;   // wider than a patch
+  if (g_patch == 0 || c.n < 1 || c.taps > kMaxTaps) return false;
+  double sums = 0;
+  for (int k = 0; k < c.n; ++k) {
+    const PatchConvClass& g = c.c[k];
+    if ((g.R - 1LL) * g.dh > 512 || (g.S - 1LL) * g.dw > 512) return false;   // wider than a patch
+    sums += (double)g.R * g.S * g.U * g.V;
+  }
   Plan pl;
   if (!make_plan(c, &pl)) return false;
   // 32-bit offsets: virtual pixels of the batch, source bytes of the images that a patch touches
-  const long long frame = (long long)pl.VR * pl.PW, image = 4LL * c.C * c.H * c.W;
-  if ((c.N + 1) * frame + 1024 >= (1LL << 31) || (pl.px / frame + 2) * image >= (1LL << 31)) return false;
+  const long long image = 4LL * c.C * c.H * c.W;
+  for (int k = 0; k < c.n; ++k) {
+    const long long frame = (long long)pl.VR[k] * pl.PW[k];
+    if ((c.N + 1) * frame + 1024 >= (1LL << 31) || (pl.px[k] / frame + 2) * image >= (1LL << 31)) return false;
+  }
   if (pl.Ipad / 32 > 65535) return false;   // the grid of patch_weights
   if (g_patch == 2) return true;
   if (pl.wt + pl.partial > ((size_t)1 << 30)) return false;   // workspace stays with the library
@@ -500,17 +555,16 @@ bool patch_conv_takes(const PatchConv& c, bool f32) {
   // 32x32 at batch 128 72.1 us, 62.7 here; 128 channels 16x16 98.0, 67.2; 256 channels 8x8 77.0, 70.4; 160 to 192
   // channels 45x37 at batch 24 183.9, 117.0; and not for 128 channels 28x28 at batch 8 (29.3, 32.9) or 3 channels
   // (23.4, 56.8), whose rows and channels are mostly padding.
-  const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
-  const double gigas = 2e-9 * c.I * c.C * taps * c.N * c.P * c.Q;
   // In float32 arithmetic the kernels that gather take 7.5 us and more (94 for 9.7e9 and 119 to 138 for 14.8e9, where
   // these take 63 to 68 and 90 to 102); small calls, which gain a few microseconds at most, stay with them.
-  return taps >= 4 && padding <= 1.5 && gigas >= (f32 ? 4.0 : 1.5) &&
-         pl.cost + 3 + 4e-6 * c.I * c.C * taps < 16 + (f32 ? 7.5 : 7.0) * gigas;
+  const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
+  const double gigas = 2e-9 * c.I * c.C * c.N * sums;
+  return c.taps >= 4 && padding <= 1.5 && gigas >= (f32 ? 4.0 : 1.5) &&
+         pl.cost + 3 + 4e-6 * c.I * c.C * c.taps < 16 + (f32 ? 7.5 : 7.0) * gigas;
 }
 
 int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi,
                       bool f32, int prof_id, int* plan8) {
-  const int taps = c.R * c.S;
   Plan pl;
   if (!make_plan(c, &pl)) return tt::fail(-1, "patch convolution: no plan");
   void* ws = nullptr;
@@ -519,35 +573,42 @@ int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const 
   Igemm p{};
   p.bias = bias; p.out = out;
   if (epi) p.epi = *epi;
-  p.I = c.I; p.Ipad = pl.Ipad; p.M = c.N * c.P * c.Q;
-  p.divUV = tt::make_fastdiv((uint32_t)(c.P * c.Q));
-  p.divV = tt::make_fastdiv((uint32_t)c.Q);
-  p.bh = -c.ph; p.bw = -c.pw;
+  p.I = c.I; p.Ipad = pl.Ipad; p.M = c.N * c.outPlane;
+  p.divUV = tt::make_fastdiv((uint32_t)c.outPlane);
   p.Hlim = c.H; p.Wlim = c.W;
-  p.outStrideN = c.I * c.P * c.Q; p.outStrideI = c.P * c.Q;
+  p.outStrideN = c.I * c.outPlane; p.outStrideI = c.outPlane; p.outRow = c.outRow;
+  p.ou = c.ou; p.ov = c.ov;
   Patch q{};
   q.src = x; q.wt = (const uintx4*)ws;
   q.partial = pl.splits > 1 ? (float*)((char*)ws + pl.wt) : nullptr;
   q.outElems = (long long)p.I * p.M;
-  q.C = c.C; q.chunks = pl.chunks; q.perSplit = pl.perSplit; q.taps = taps; q.S = c.S;
+  q.C = c.C; q.chunks = pl.chunks; q.perSplit = pl.perSplit;
   q.plane = 4 * c.H * c.W; q.image = q.plane * c.C;
-  q.PW = pl.PW; q.VR = pl.VR;
-  q.tapRow = c.dh * pl.PW * kUnit; q.tapCol = c.dw * kUnit;
-  q.px = pl.px; q.images = c.N;
+  q.maxPx = pl.maxPx; q.images = c.N;
   if (f32) {
     q.w = w;
-    q.wRow = c.dgrad ? taps : c.C * taps; q.wChan = c.dgrad ? c.I * taps : taps;
-    q.dgrad = c.dgrad; q.dh = c.dh; q.dw = c.dw;
+    q.wI = c.dgrad ? c.taps : c.C * c.taps;
+    q.wC = c.dgrad ? c.I * c.taps : c.taps;
   }
-  q.divPW = tt::make_fastdiv((uint32_t)pl.PW); q.divVR = tt::make_fastdiv((uint32_t)pl.VR);
+  q.classes = c.n;
+  PatchTaps taps{};
+  taps.n = c.n;
+  for (int k = 0; k < c.n; ++k) {
+    const PatchConvClass& g = c.c[k];
+    q.c[k] = PatchClass{c.N * g.U * g.V, tt::make_fastdiv((uint32_t)(g.U * g.V)), tt::make_fastdiv((uint32_t)g.V), -g.ph, -g.pw, g.ouh, g.ovw,
+                        g.R * g.S, g.S, pl.PW[k], pl.VR[k], tt::make_fastdiv((uint32_t)pl.PW[k]), tt::make_fastdiv((uint32_t)pl.VR[k]),
+                        pl.px[k], g.dh * pl.PW[k] * kUnit, g.dw * kUnit, g.dh, g.dw, g.w0, g.wRow, g.wCol, pl.block0[k], pl.at[k]};
+    taps.taps[k] = g.R * g.S; taps.S[k] = g.S;
+    taps.w0[k] = g.w0; taps.wRow[k] = g.wRow; taps.wCol[k] = g.wCol; taps.wt[k] = pl.at[k];
+  }
   {
     tt::ProfScope prof(TT_PROF_CONV_PREP);
-    const int run = (c.dgrad ? 32 : kBK) * taps, outer = c.dgrad ? kBK : 32;
+    const int run = (c.dgrad ? 32 : kBK) * c.taps, outer = c.dgrad ? kBK : 32;
     const dim3 grid((unsigned)pl.chunks, (unsigned)(pl.Ipad / 32));
     const size_t lds = sizeof(float) * (size_t)outer * (run + 1);
     const tt::FastDiv divRun = tt::make_fastdiv((uint32_t)run);
-    if (c.dgrad) patch_weights<true><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, taps, divRun, pl.chunks);
-    else patch_weights<false><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, taps, divRun, pl.chunks);
+    if (c.dgrad) patch_weights<true><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, c.taps, divRun, pl.chunks, taps);
+    else patch_weights<false><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, c.taps, divRun, pl.chunks, taps);
     TT_LAUNCH_CHECK();
   }
   const int BM = 32 * pl.WM, BN = 128 * pl.NT / pl.WM;
@@ -555,9 +616,9 @@ int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const 
   std::copy(plan, plan + 8, plan8);
   tt::ProfScope prof(prof_id);
   const dim3 grid((unsigned)pl.tiles, 1, (unsigned)pl.splits);
-  const size_t lds = 2 * (size_t)pl.px * kUnit + 4 * sizeof(float) * BM;
+  const size_t lds = 2 * (size_t)pl.maxPx * kUnit + 4 * sizeof(float) * BM;
   const bool epilogue = p.epi.on && pl.splits == 1;
-#define TT_PATCH(WM, NT, IT)                                                                  \
+#define TT_PATCH(WM, NT, IT)                                                     \
   (epilogue ? patch_product<WM, NT, IT, true><<<grid, kThreads, lds, st>>>(p, q) \
             : patch_product<WM, NT, IT, false><<<grid, kThreads, lds, st>>>(p, q))
   if (pl.WM == 4) {

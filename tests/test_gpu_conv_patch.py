@@ -1,4 +1,4 @@
-"""The kernels that keep a patch of the source in LDS (three bfloat16 terms, unit stride), over every geometry they
+"""The kernels that keep a patch of the source in LDS (three bfloat16 terms), over every geometry they
 take: the float32 bar of tests/test_gpu_conv.py, and sums no further from float64 ones than those of the kernels
 that gather in place."""
 import numpy as np
@@ -6,8 +6,9 @@ import pytest
 
 from pytortto_amd import _hip, ops
 from pytortto_amd.xparray import hiparray
-from tests.cases import CONV_CASES, random_conv_cases, random_large_kernel_cases
+from tests.cases import CONV_CASES, CONVT_CASES, random_conv_cases, random_convt_cases, random_large_kernel_cases
 from tests.test_gpu_conv import TILE_CASES, _last_launch, _run_conv
+from tests.test_gpu_conv import test_conv_transpose_forward_backward as _conv_transpose_checks
 
 pytestmark = pytest.mark.gpu
 
@@ -38,13 +39,22 @@ EDGES = [
     (40, 130, 14, 14, 200, 3, 3, (1, 1), (1, 1), (1, 1), 1), (6, 48, 61, 43, 160, 3, 3, (1, 1), (1, 1), (1, 1), 1),
 ]
 
+# input gradients of two and four classes: of equal and unequal sizes and taps, one tap each, with dilation, rows of dx
+# that no tap reaches
+STRIDED = [
+    (4, 33, 16, 16, 40, 4, 4, (2, 2), (1, 1), (1, 1), 1), (3, 20, 15, 13, 48, 3, 3, (2, 2), (1, 1), (1, 1), 1),
+    (2, 64, 9, 8, 30, 2, 2, (2, 2), (0, 0), (1, 1), 1), (5, 24, 11, 20, 65, 3, 4, (1, 2), (1, 1), (1, 1), 1),
+    (2, 40, 21, 17, 24, 5, 3, (2, 1), (3, 0), (1, 2), 1), (2, 36, 20, 19, 130, 3, 5, (2, 2), (0, 2), (3, 1), 1),
+    (1, 200, 14, 14, 64, 3, 3, (2, 2), (1, 1), (1, 1), 1), (2, 17, 12, 31, 33, 2, 4, (1, 4), (0, 1), (1, 1), 1),
+]
 
-@pytest.mark.parametrize('case', EDGES + [c for c in CONV_CASES + TILE_CASES if c[7] == (1, 1) and c[10] == 1])
+
+@pytest.mark.parametrize('case', EDGES + STRIDED + [c for c in CONV_CASES + TILE_CASES if c[10] == 1])
 @pytest.mark.parametrize('bias,math', [(True, 'bf16x3'), (False, 'f32')])
 def test_meets_the_float32_bar(case, bias, math, patch):
     patch(ALWAYS, math)
     _run_conv(case, seed=5, bias=bias)
-    if case in EDGES:
+    if case in EDGES + STRIDED:   # the input gradient
         assert _last_launch()['persistent_blocks'] == -4
 
 
@@ -52,6 +62,13 @@ def test_meets_the_float32_bar(case, bias, math, patch):
 def test_random_geometries(case, patch):
     patch(ALWAYS, 'f32')
     _run_conv(case, seed=6)
+
+
+@pytest.mark.parametrize('case', CONVT_CASES + random_convt_cases(20, 93))
+@pytest.mark.parametrize('math', ['bf16x3', 'f32'])
+def test_transposed(case, math, patch):
+    patch(ALWAYS, math)
+    _conv_transpose_checks(case)
 
 
 @pytest.mark.parametrize('math', ['bf16x3', 'f32'])
@@ -112,21 +129,23 @@ def test_operands_the_terms_do_not_hold(n, c, hw, k, scale, patch):
         np.testing.assert_allclose(a[finite], b[finite], rtol=1e-5, atol=max(1e-6 * min(size, 1e3 * scale), 2.0 ** -133 * 9 * max(c, k)))
 
 
-@pytest.mark.parametrize('dims', [(4, 64, 28, 28, 64, 3), (2, 512, 7, 7, 512, 3), (4, 128, 16, 16, 256, 3), (3, 96, 20, 17, 48, 5),
-                                  (8, 64, 56, 56, 64, 3)])
+@pytest.mark.parametrize('dims', [(4, 64, 28, 28, 64, 3, 1), (2, 512, 7, 7, 512, 3, 1), (4, 128, 16, 16, 256, 3, 1), (3, 96, 20, 17, 48, 5, 1),
+                                  (8, 64, 56, 56, 64, 3, 1), (4, 64, 32, 32, 128, 4, 2), (4, 128, 28, 28, 256, 3, 2)])
 def test_sums_are_as_accurate_as_in_the_other_kernels(dims, patch):
     """Against the exact sums of both arithmetics' kernels that gather in place."""
     import torch
-    n, c, h, w, k, r = dims
+    n, c, h, w, k, r, stride = dims
+    pad = (r - 1) // 2
+    p, q = ((x + 2 * pad - r) // stride + 1 for x in (h, w))
     rng = np.random.default_rng(11)
     xh, wh = rng.standard_normal((n, c, h, w)).astype(np.float32), rng.standard_normal((k, c, r, r)).astype(np.float32)
-    dyh = rng.standard_normal((n, k, h, w)).astype(np.float32)
+    dyh = rng.standard_normal((n, k, p, q)).astype(np.float32)
     x64, w64 = torch.tensor(xh, dtype=torch.float64, requires_grad=True), torch.tensor(wh, dtype=torch.float64)
-    y64 = torch.nn.functional.conv2d(x64, w64, padding=r // 2)
+    y64 = torch.nn.functional.conv2d(x64, w64, padding=pad, stride=stride)
     y64.backward(torch.tensor(dyh, dtype=torch.float64))
     want = {'y': y64.detach().numpy(), 'dx': x64.grad.numpy()}
     x, wt, dy = hiparray(xh), hiparray(wh), hiparray(dyh)
-    geometry = ((1, 1), (r // 2, r // 2), (1, 1), 1)
+    geometry = ((stride, stride), (pad, pad), (1, 1), 1)
 
     def errors():
         got = {'y': ops.conv2d_fwd(x, wt, None, *geometry).get(), 'dx': ops.conv2d_dgrad(dy, wt, None, (h, w), *geometry).get()}
