@@ -99,8 +99,8 @@ int tt_probe_hbm_f32(size_t bytes, double* read_gbs, double* copy_gbs);
 
 /* Matrix arithmetic of the three convolution passes (no counterpart in the reference,
  * whose path is float32 throughout).  TT_CONV_MATH_F32 (the default) computes in float32 and is the mode that
- * meets the reference's tolerances: on v_mfma_f32_32x32x2_f32 -- and in large forward passes and input gradients of
- * unit stride with four taps or more, where it is faster and its error against float64 sums half as large, by the
+ * meets the reference's tolerances: on v_mfma_f32_32x32x2_f32 -- and in large forward passes and input gradients,
+ * where it is faster and its error against float64 sums smaller, by the
  * three exact terms of TT_CONV_MATH_BF16X3; sums that these do not hold (operands that are not finite or round
  * to a bf16 infinity, results below 2^-96) are formed again without them.
  * TT_CONV_MATH_BF16 is the optional reduced-precision variant: tensors stay float32 in memory,
@@ -288,6 +288,9 @@ int tt_conv2d_wgrad_force_occupancy(int blocks);
 int tt_conv2d_narrow_enable(int on);
 /* The same for the kernels that keep a patch of the source in LDS (TT_CONV_MATH_BF16X3 and _F32; reported as -4). */
 int tt_conv2d_patch_enable(int on);
+/* The same for float32 launches (TT_CONV_MATH_F32) of the kernels that gather in place: on three exact bf16 terms
+ * (tt_conv2d_last_launch reports 3 in bits 8.. of its last word) or on the float32 instructions. */
+int tt_conv2d_f32_terms_enable(int on);
 
 /* out[K] = sum over n and the HW plane of t[N,K,HW]: the bias gradient gd0.sum((0,2,3)),
  * autograd/grad_nn.py:728, :774. */

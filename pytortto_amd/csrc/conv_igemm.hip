@@ -206,6 +206,25 @@ bool bf16_math() { return tt::conv_math() == TT_CONV_MATH_BF16; }
 bool split_math() { return tt::conv_math() == TT_CONV_MATH_BF16X3; }
 // bf16 terms per operand element of the matrix instructions in use (0: float32 instructions)
 int math_terms() { return bf16_math() ? 1 : split_math() ? 3 : 0; }
+
+int g_f32_terms = 1;   // tests: 0 = never, 2 = wherever they can
+
+// Whether a float32 launch of I rows runs on the three-term kernels: `gigas` 1e9 products and sums, `taps` of them a
+// channel.
+// Their matrix step takes 192 cycles for 256 and halves the weights' and pixels' way through LDS, but not a launch's
+// start, its stores and the exchange of shared sums, and theirs are 128-row tiles where the float32 kernels take 64:
+// below 3e9 the two trade places (460 to 158 channels 27x27 at batch 13, 1.4e9: 26.9 us in float32, 31.3; 128 to 512
+// 28x28 at batch 16, 1.6e9: 22.9, 18.6), as they do where rows are padding (228 to 279 channels, 3.3e9: 49.9, 55.8)
+// or few and the call bound by its pixels (256 to 64 channels 56x56 at batch 64: 67, 68).  Above it 75 of 76 launches
+// gain, 1.2 times on average: 512 to 256 channels 28x28 at batch 64 119 us, 89; 64 to 256 56x56 87, 63; 1024 to 256
+// 14x14 65, 50; 3x3 stride 2 128 channels 56x56 123, 103; the stem 170, 130.  Errors against float64 sums are 0.44 to
+// 0.86 times those of the float32 instructions in all 150 launches measured.
+bool f32_terms(int I, int groups, int taps, double gigas, const Epilogue* epi, const float* out) {
+  if (math_terms() != 0 || groups != 1 || g_f32_terms == 0) return false;
+  if (epi && (epi->res == out || epi->mask == out)) return false;   // a value may be stored twice
+  if (g_f32_terms == 2) return true;
+  return I > (taps > 1 ? 32 : 64) && gigas * I >= 2.7 * (I <= 64 ? 64 : ceil_div(I, 128) * 128);
+}
 const IgemmUnit& unit(int terms, bool epilogue) {
   if (epilogue) return terms == 3 ? igemm_epi_bf16x3_unit() : terms == 1 ? igemm_epi_bf16_unit() : igemm_epi_f32_unit();
   return terms == 3 ? igemm_bf16x3_unit() : terms == 1 ? igemm_bf16_unit() : igemm_f32_unit();
@@ -359,6 +378,7 @@ int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_pa
       p.skEpoch = g_sk_epoch;
     }
   }
+  const int terms = p.w ? 3 : math_terms();
   hipStream_t st = tt::stream();
   // The reduced-precision mode's own kernels: 128-pixel tiles, one tile per block, nothing shared.
   // They share no reduction between blocks, so launches with fewer tiles than compute units and a
@@ -379,9 +399,9 @@ int launch_igemm(Igemm& p, int groups, TileChoice t, int prof_id, floatx4* sk_pa
     return 0;
   }
   const int plan[8] = {t.bm, t.bn, p.tiles, p.tilesI, t.sk_blocks, t.sk_blocks > 0 ? p.skDpTiles : p.tiles,
-                       t.sk_blocks > 0 ? p.skBlocks : 0, p.mode | math_terms() << 8};
+                       t.sk_blocks > 0 ? p.skBlocks : 0, p.mode | terms << 8};
   std::copy(plan, plan + 8, g_last_launch);
-  const bool persistent = unit(math_terms(), p.epi.on).launch(p, groups, t.sk_blocks, t.bm, t.bn, g_sk_forced_occupancy, st);
+  const bool persistent = unit(terms, p.epi.on).launch(p, groups, t.sk_blocks, t.bm, t.bn, g_sk_forced_occupancy, st);
   if (!persistent) {   // also when the device could not hold the persistent grid: one tile per block
     g_last_launch[4] = 0;
     g_last_launch[5] = p.tiles;
@@ -681,6 +701,13 @@ int tt_conv2d_bf16_first_enable(int on) {
   return 0;
 }
 
+int tt_conv2d_f32_terms_enable(int on) {
+  TT_API_LOCK();
+  TT_REQUIRE(on >= 0 && on <= 2, "tt_conv2d_f32_terms_enable: %d is out of range (0..2)", on);
+  g_f32_terms = on;
+  return 0;
+}
+
 // Instrumentation (tests): pretend that every stream-K instantiation holds `blocks` blocks per
 // compute unit (-1: ask the device again), so that the data-parallel fallback can be exercised.
 int tt_conv2d_stream_k_force_occupancy(int blocks) {
@@ -759,7 +786,8 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
   const int M = N * P * Q;
   const int KQ = ceil_div(Kred, 4 * kBKQ) * kBKQ;
   const bool plain = R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-  const TileChoice t = choose_tile(Kg, M, groups, KQ / kBKQ, true, plain && KQ / kBKQ <= 32 && !bf16_math() && !split_math());
+  const bool in_terms = f32_terms(Kg, groups, R * S, 2e-9 * M * Kg * Kred, epi, y);
+  const TileChoice t = choose_tile(Kg, M, groups, KQ / kBKQ, true, plain && KQ / kBKQ <= 32 && math_terms() == 0 && !in_terms);
   const int Ipad = ceil_div(Kg, t.bm) * t.bm;
 
   const size_t wp_bytes = align_up(sizeof(floatx4) * (size_t)groups * KQ * Ipad, 256);
@@ -781,6 +809,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
     p.wRowStride = Kred;
   }
   p.wbuf = in_place ? (const void*)w : (const void*)wp;
+  if (in_terms) { p.w = w; p.wI = Kred; p.wC = R * S; p.wRow = S; p.wCol = 1; }
   p.I = Kg; p.Ipad = Ipad; p.KQ = KQ; p.M = M;
   p.divUV = tt::make_fastdiv((uint32_t)(P * Q));
   p.divV = tt::make_fastdiv((uint32_t)Q);
@@ -1079,8 +1108,9 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
       const int M = N * U * V;
       const int KQ = ceil_div(Kred, 4 * kBKQ) * kBKQ;
       const bool plain = R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
+      const bool in_terms = allow_stream_k && Kred > 0 && f32_terms(Cg, groups, nTr * nTs, 2e-9 * M * Cg * Kred, epi, dx);
       const TileChoice t = choose_tile(Cg, M, groups, KQ / kBKQ, allow_stream_k,
-                                       (plain && KQ / kBKQ <= 32 && !bf16_math() && !split_math()) || !allow_stream_k);
+                                       (plain && KQ / kBKQ <= 32 && math_terms() == 0 && !in_terms) || !allow_stream_k);
       const int Ipad = ceil_div(Cg, t.bm) * t.bm;
       floatx4* wp = (floatx4*)((char*)ws + wp_bytes * slot);
       Igemm p{};
@@ -1097,6 +1127,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
       p.cellFill = cell_fill;
       if (epi) p.epi = *epi;   // stride 1: this is the only class, and its launch writes every element of dx
       p.Kred = Kred;
+      if (in_terms) { p.w = w; p.wI = R * S; p.wC = Cg * R * S; p.w0 = r0 * S + s0; p.wRow = rstep * S; p.wCol = sstep; }
       if (KQ > 0) {
         // h = u*sh + ch reads dy row (h + ph - r0*dh)/sh = u + (ch + ph - r0*dh)/sh  (exact)
         p.bh = (ch + ph - r0 * dh) / sh;   // numerator is a multiple of sh by choice of r0

@@ -98,6 +98,10 @@ struct Igemm {
   unsigned skEpoch;          // differs from launch to launch, so the flags never need clearing
   unsigned* skError;         // one word in pinned host memory: set when a wait for a flag ran out
   Epilogue epi;
+  // float32 launches of the three-term kernels: the weights as they came, element i*wI + c*wC + w0 + b*wRow + t*wCol
+  // for row i, channel c and tap (b, t); null otherwise
+  const float* w;
+  int wI, wC, w0, wRow, wCol;
 };
 
 
@@ -203,6 +207,50 @@ __device__ __forceinline__ void store_through_epilogue(const Igemm& p, const flo
       }
     }
   }
+}
+
+// What the launch does to a sum on its way to memory, for one value: the steps of store_through_epilogue.
+__device__ __forceinline__ float finish_value(const Igemm& p, const int i, const uint32_t e, float v) {
+  if (p.bias) v += p.bias[i];
+  if (p.epi.on) {
+    if (p.epi.norm) {
+      const float sd = __fsqrt_rn(__fadd_rn(p.epi.var[i], p.epi.eps));
+      v = fmaf(v - p.epi.mean[i], __fdiv_rn(p.epi.gamma ? p.epi.gamma[i] : 1.0f, sd), p.epi.beta ? p.epi.beta[i] : 0.0f);
+    }
+    if (p.epi.res) v += p.epi.res[e];
+    if (p.epi.relu) v = (v > 0.f || v != v) ? v : 0.f;
+    if (p.epi.mask) v *= p.epi.mask[e] > 0.f ? 1.f : 0.f;
+  }
+  return v;
+}
+
+// Values for which the terms do not stand for the operands: a sum with an operand that is not finite, or whose
+// first term is not, comes out as NaN; one that overflows may have done so by its terms' roundings; and operands
+// below 2^-110 lose bits of their last term to the least bfloat16, which only sums of such operands notice.
+__device__ __forceinline__ bool terms_fail(const float v) {
+  const float a = __builtin_fabsf(v);
+  return !(a <= 3.402823466e38f) || (a < 0x1p-96f && a > 0.f);
+}
+
+// Whether one of them may be among a lane's sums (zeros raise it too), in one instruction and a half for each: twice a
+// value's bits, less twice those of 2^-96, is at least the constant below for what terms_fail finds, and for a zero.
+template <int MT, int NT>
+__device__ __forceinline__ bool terms_may_fail(const floatx16 (&acc)[MT][NT]) {
+  constexpr unsigned kLeast = 2u * 0x0f800000u;   // bits of 2^-96
+  unsigned most[2] = {0, 0};
+#pragma unroll
+  for (int x = 0; x < MT; ++x)
+#pragma unroll
+    for (int y = 0; y < NT; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        unsigned t[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) t[j] = (__builtin_bit_cast(unsigned, (float)acc[x][y][r + j]) << 1) - kLeast;
+        unsigned& to = most[(r >> 1) & 1];
+        to = max(max(t[0], t[1]), to);
+      }
+  return max(most[0], most[1]) >= 0xff000000u - kLeast;
 }
 
 // The bf16-first kernels (conv_igemm_bf16.hip).  `supported` tells whether they take launch `p`

@@ -592,6 +592,54 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
     }
   };
 
+  // One sum in float64: the rare path behind terms_fail.  A NaN stays one, so that data full of them cost a product each.
+  auto exact_sum = [&](const int i, const uint32_t n, const int u, const int v) __attribute__((always_inline)) {
+    const int channels = p.Kred / (p.TB * p.TC);
+    double sum = 0.0;
+    for (int c = 0; c < channels && sum == sum; ++c) {
+      const float* x = p.src + (long long)n * p.srcStrideN + (long long)c * p.kStride;
+      const float* w = p.w + (long long)i * p.wI + (long long)c * p.wC + p.w0;
+      for (int b = 0; b < p.TB; ++b) {
+        const int ih = u * p.su + p.bh + b * p.stepH;
+        for (int t = 0; t < p.TC; ++t) {   // a tap outside the image multiplies a zero, as everywhere
+          const int iw = v * p.sv + p.bw + t * p.stepW;
+          const bool inside = (unsigned)ih < (unsigned)p.Hlim && (unsigned)iw < (unsigned)p.Wlim;
+          sum = fma(inside ? (double)x[(long long)ih * p.srcRow + iw] : 0.0, (double)w[b * p.wRow + t * p.wCol], sum);
+        }
+      }
+    }
+    return (float)sum;
+  };
+
+  // Stores the tile; float32 sums that three terms do not hold are formed and stored again.
+  auto finish = [&]() __attribute__((always_inline)) {
+    if constexpr (BF != 3) {
+      epilogue();
+    } else {
+      unsigned long long again = 0;   // bit 16*(x*NT + y) + r
+      if (p.w && terms_may_fail<MT, NT>(acc)) {
+#pragma unroll
+        for (int x = 0; x < MT; ++x)
+#pragma unroll
+          for (int y = 0; y < NT; ++y)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) again |= (unsigned long long)terms_fail(acc[x][y][r]) << (16 * (x * NT + y) + r);
+      }
+      epilogue();
+      for (; again; again &= again - 1) {
+        const int bit = __builtin_ctzll(again), r = bit & 15, x = (bit >> 4) / NT, y = (bit >> 4) % NT;
+        const int i = i0 + (wm * MT + x) * 32 + 8 * (r >> 2) + 4 * h + (r & 3), m = m0 + (wn * NT + y) * 32 + l32;
+        if (i >= p.I || m >= p.M) continue;
+        const uint32_t n = tt::fd_div((uint32_t)m, p.divUV);
+        const uint32_t rem = (uint32_t)m - n * p.divUV.d;
+        const uint32_t u = tt::fd_div(rem, p.divV);
+        const uint32_t v = rem - u * p.divV.d;
+        const uint32_t e = (uint32_t)((int)n * p.outStrideN + ((int)u * p.ou + p.ouh) * p.outRow + (int)v * p.ov + p.ovw + i * p.outStrideI);
+        p.out[e] = finish_value(p, i, e, exact_sum(i, n, (int)u, (int)v));
+      }
+    }
+  };
+
   const int chunks = p.KQ / kBKQ;
   // (published by the barriers of the reduction that follows; the epilogue of the tile before has
   // ended with one)
@@ -605,7 +653,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
     set_tile(xcd_remap(block_x, p.tiles));
     epi_constants();
     run_segment(0, chunks);
-    epilogue();
+    finish();
   } else {
     // Whole rounds of tiles are computed one tile per block as usual.  The tiles left over would
     // load the CUs unevenly, so their reduction steps (tile-major sequence of T = tiles*chunks
@@ -663,7 +711,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
         set_tile(tile);
         epi_constants();
         run_segment(0, chunks);
-        epilogue();
+        finish();
         __syncthreads();
       }
       for (int t = t_first; t <= t_last; ++t) {
@@ -672,7 +720,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
         set_tile(p.skDpTiles + t);
         epi_constants();
         run_segment(0, chunks);
-        epilogue();
+        finish();
         __syncthreads();
       }
       if (has_closing) {
@@ -715,7 +763,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
                 for (int e = 0; e < 4; ++e) acc[x][y][4 * q + e] += v[q][e];
             }
         }
-        epilogue();
+        finish();
       }
     }
   }

@@ -152,29 +152,6 @@ struct Patch {
   PatchClass c[kPatchClasses];
 };
 
-// What the launch does to a sum on its way to memory, for one value: the steps of store_through_epilogue.
-__device__ __forceinline__ float finish_value(const Igemm& p, const int i, const uint32_t e, float v) {
-  if (p.bias) v += p.bias[i];
-  if (p.epi.on) {
-    if (p.epi.norm) {
-      const float sd = __fsqrt_rn(__fadd_rn(p.epi.var[i], p.epi.eps));
-      v = fmaf(v - p.epi.mean[i], __fdiv_rn(p.epi.gamma ? p.epi.gamma[i] : 1.0f, sd), p.epi.beta ? p.epi.beta[i] : 0.0f);
-    }
-    if (p.epi.res) v += p.epi.res[e];
-    if (p.epi.relu) v = (v > 0.f || v != v) ? v : 0.f;
-    if (p.epi.mask) v *= p.epi.mask[e] > 0.f ? 1.f : 0.f;
-  }
-  return v;
-}
-
-// Values for which the terms do not stand for the operands: a sum with an operand that is not finite, or whose
-// first term is not, comes out as NaN; one that overflows may have done so by its terms' roundings; and operands
-// below 2^-110 lose bits of their last term to the least bfloat16, which only sums of such operands notice.
-__device__ __forceinline__ bool terms_fail(const float v) {
-  const float a = __builtin_fabsf(v);
-  return !(a <= 3.402823466e38f) || (a < 0x1p-96f && a > 0.f);
-}
-
 // One sum in float64, over the channels [c0, c1): the rare path behind terms_fail.  A NaN stays one, so that data
 // full of them cost a product each.
 __device__ __forceinline__ float exact_sum(const Igemm& p, const Patch& q, const PatchClass& k, const int i, const uint32_t n, const int u, const int v,
@@ -393,7 +370,7 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
   for (int y = 0; y < NT; ++y) acc[0][y] += small[y];
 
   unsigned long long again = 0;   // values to be summed once more (bit 16*y + r)
-  if (q.w) {
+  if (q.w && terms_may_fail<1, NT>(acc)) {
 #pragma unroll
     for (int y = 0; y < NT; ++y)
 #pragma unroll

@@ -1,0 +1,152 @@
+"""Float32 launches of the kernels that gather in place on three exact bf16 terms: every addressing mode, tile and way
+of storing, the float32 bar of tests/test_gpu_conv.py, sums no further from float64 ones than those of the float32
+instructions, and operands that the terms do not hold."""
+import numpy as np
+import pytest
+
+from pytortto_amd import _hip, ops
+from pytortto_amd.xparray import hiparray
+from tests.cases import CONV_CASES, random_conv_cases
+from tests.test_gpu_conv import TILE_CASES, _last_launch, _run_conv
+
+pytestmark = pytest.mark.gpu
+
+ALWAYS, WHERE_FASTER, NEVER = 2, 1, 0
+
+
+@pytest.fixture
+def terms():
+    def choose(which):
+        _hip.call('tt_conv2d_f32_terms_enable', which)
+        _hip.call('tt_conv2d_patch_enable', which if which == WHERE_FASTER else NEVER)
+        _hip.call('tt_conv2d_narrow_enable', which if which == WHERE_FASTER else NEVER)
+    yield choose
+    choose(WHERE_FASTER)
+
+
+def in_terms():
+    return _last_launch()['mode'] >> 8 == 3
+
+
+# n, c, h, w, k, r, s, stride, pad, dilation, groups: whole matrix products; pixels in no whole quads; channels in no
+# whole chunks; rows and pixels around a tile's edge; a shared reduction; strided with cells, without; masks of 31, 49
+# and more taps; one pixel
+EDGES = [
+    (4, 64, 12, 12, 96, 1, 1, (1, 1), (0, 0), (1, 1), 1), (3, 48, 7, 7, 129, 1, 1, (1, 1), (0, 0), (1, 1), 1),
+    (5, 33, 9, 11, 65, 1, 1, (1, 1), (0, 0), (1, 1), 1), (2, 2048, 7, 7, 64, 1, 1, (1, 1), (0, 0), (1, 1), 1),
+    (2, 32, 14, 12, 40, 1, 1, (2, 2), (0, 0), (1, 1), 1), (3, 32, 15, 13, 130, 1, 1, (2, 2), (0, 0), (1, 1), 1),
+    (1, 16, 9, 9, 70, 1, 1, (1, 3), (1, 1), (1, 1), 1), (2, 17, 15, 14, 72, 3, 3, (2, 2), (1, 1), (1, 1), 1),
+    (2, 3, 30, 30, 64, 7, 7, (2, 2), (3, 3), (1, 1), 1), (1, 5, 20, 20, 66, 9, 8, (1, 1), (4, 4), (1, 1), 1),
+    (3, 96, 28, 28, 127, 3, 3, (1, 1), (1, 1), (1, 1), 1), (1, 1, 1, 1, 1, 1, 1, (1, 1), (0, 0), (1, 1), 1),
+    (64, 8, 8, 8, 32, 3, 3, (1, 1), (2, 2), (2, 2), 1),
+]
+
+
+@pytest.mark.parametrize('case', EDGES + [c for c in CONV_CASES + TILE_CASES if c[10] == 1] + random_conv_cases(40, 17))
+def test_meets_the_float32_bar(case, terms):
+    terms(ALWAYS)
+    _run_conv(case, seed=5, bias=case in EDGES[::2])
+
+
+def _arrays(n, c, hw, k, r, stride, rng):
+    p = (hw + 2 * (r // 2) - r) // stride + 1
+    return (rng.standard_normal(s).astype(np.float32) for s in ((n, c, hw, hw), (k, c, r, r), (n, k, p, p)))
+
+
+GEOMETRIES = [(9, 64, 14, 96, 1, 1), (2, 512, 7, 70, 1, 1), (8, 256, 28, 256, 1, 1), (3, 64, 28, 128, 1, 2), (3, 17, 28, 33, 3, 2),
+              (4, 48, 28, 130, 3, 1)]
+
+
+@pytest.mark.parametrize('dims', GEOMETRIES)
+def test_sums_are_as_accurate_as_in_float32_instructions(dims, terms):
+    import torch
+    n, c, hw, k, r, stride = dims
+    xh, wh, dyh = _arrays(*dims, np.random.default_rng(11))
+    x64, w64 = torch.tensor(xh, dtype=torch.float64, requires_grad=True), torch.tensor(wh, dtype=torch.float64)
+    y64 = torch.nn.functional.conv2d(x64, w64, padding=r // 2, stride=stride)
+    y64.backward(torch.tensor(dyh, dtype=torch.float64))
+    x, w, dy = hiparray(xh), hiparray(wh), hiparray(dyh)
+    geometry = ((stride, stride), (r // 2, r // 2), (1, 1), 1)
+    one_launch = stride == 1 or r == 1   # the classes of other strided gradients share a grid of float32 instructions
+
+    def errors(expected):
+        y = ops.conv2d_fwd(x, w, None, *geometry)
+        assert in_terms() == expected
+        dx = ops.conv2d_dgrad(dy, w, None, (hw, hw), *geometry)
+        assert in_terms() == (expected and one_launch)
+        return [np.linalg.norm(a.get() - b) / np.linalg.norm(b) for a, b in ((y, y64.detach().numpy()), (dx, x64.grad.numpy()))]
+    terms(ALWAYS)
+    new = errors(True)
+    terms(NEVER)
+    old = errors(False)
+    print(dims, new, old)
+    assert new[0] <= old[0] and new[1] <= old[1]
+
+
+@pytest.mark.parametrize('dims', GEOMETRIES[:2] + GEOMETRIES[3:])
+@pytest.mark.parametrize('scale', [1.0, 2.0 ** 120, 2.0 ** -126, 2.0 ** -140])
+def test_operands_the_terms_do_not_hold(dims, scale, terms):
+    """Infinities, NaN, magnitudes that round to a bfloat16 infinity and operands whose last terms it cannot hold give
+    what the float32 instructions give, behind an epilogue as well."""
+    n, c, hw, k, r, stride = dims
+    rng = np.random.default_rng(4)
+    xh, wh, dyh = _arrays(*dims, rng)
+    xh, dyh, wh = np.ldexp(xh, int(np.log2(scale))), np.ldexp(dyh, int(np.log2(scale))), wh / np.float32(4)
+    if scale == 1.0:
+        for a in (xh, dyh):
+            a[0, 0, 2, 2], a[0, 1, 2, 4], a[1, -1, 0, 0], a[1, 3, 4, 4] = np.inf, -np.inf, np.nan, np.float32(3.4e38)
+        wh[5, 2, 0, 0] = -np.inf
+    x, w, dy = hiparray(xh), hiparray(wh), hiparray(dyh)
+    bias = hiparray(rng.standard_normal(k).astype(np.float32) * np.float32(scale))
+    add = hiparray((rng.standard_normal((n, c, hw, hw)) * scale).astype(np.float32))
+    geometry = ((stride, stride), (r // 2, r // 2), (1, 1), 1)
+
+    def results():
+        out = [ops.conv2d_fwd(x, w, None, *geometry).get(), ops.conv2d_fwd(x, w, bias, *geometry).get(),
+               ops.conv2d_dgrad(dy, w, None, (hw, hw), *geometry).get()]
+        if stride == 1:
+            out.append(ops.conv2d_dgrad(dy, w, None, (hw, hw), *geometry, add=add, relu_y=add).get())
+        return out
+    terms(ALWAYS)
+    got = results()
+    terms(NEVER)
+    for a, b in zip(got, results()):
+        assert np.array_equal(np.isnan(a), np.isnan(b))
+        assert np.array_equal(np.isinf(a), np.isinf(b))
+        finite = np.isfinite(a) & np.isfinite(b)
+        assert finite.mean() > .5
+        size = float(np.abs(b[finite], dtype=np.float64).max())
+        # the least bfloat16 is 2^-133: what rounds to no term at all is missing from a sum of nothing else
+        np.testing.assert_allclose(a[finite], b[finite], rtol=1e-5,
+                                   atol=max(1e-6 * min(size, 1e3 * scale), 2.0 ** -133 * r * r * max(c, k)))
+
+
+@pytest.mark.parametrize('dims', [d for d in GEOMETRIES if d[5] == 1])
+def test_epilogues(dims, terms):
+    """The same bits as the entry points they stand in for; an epilogue that writes what it reads keeps the float32
+    instructions, which store a value once."""
+    n, c, hw, k, r, _ = dims
+    terms(ALWAYS)
+    rng = np.random.default_rng(3)
+    x, w, res = (hiparray(a) for a in _arrays(*dims, rng))
+    mask = hiparray(rng.standard_normal(x.shape).astype(np.float32))
+    mean, gamma, beta = (hiparray(rng.standard_normal(k).astype(np.float32)) for _ in range(3))
+    var = hiparray(rng.random(k).astype(np.float32) + np.float32(.5))
+    geometry = ((1, 1), (r // 2, r // 2), (1, 1), 1)
+    y = ops.conv2d_fwd(x, w, None, *geometry)
+    want = np.maximum(ops.bn_fwd_eval(y, gamma, beta, mean, var, 1e-5)[0].get() + res.get(), 0)
+
+    def fused(out, residual):
+        _hip.call('tt_conv2d_norm_act_fwd_f32', x.ptr, w.ptr, None, out.ptr, mean.ptr, var.ptr, gamma.ptr, beta.ptr, 1e-5,
+                  residual.ptr, 1, n, c, hw, hw, k, r, r, 1, 1, r // 2, r // 2, 1, 1, 1)
+        return out.get()
+    assert np.array_equal(fused(hiparray.empty(y.shape), res), want) and in_terms()
+    dx = ops.conv2d_dgrad(res, w, None, (hw, hw), *geometry).get()
+    both = ops.conv2d_dgrad(res, w, None, (hw, hw), *geometry, add=x, relu_y=mask).get()
+    assert in_terms() and np.array_equal(both, (dx + x.get()) * (mask.get() > 0))
+    try:
+        got = fused(res, res)
+    except _hip.HipError:
+        return
+    assert not in_terms()
+    np.testing.assert_allclose(got, want, rtol=1e-4, atol=1e-4 * float(np.abs(want).max()))
