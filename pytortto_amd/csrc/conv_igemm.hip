@@ -217,13 +217,14 @@ int g_f32_terms = 1;   // tests: 0 = never, 2 = wherever they can
 // 28x28 at batch 16, 1.6e9: 22.9, 18.6), as they do where rows are padding (228 to 279 channels, 3.3e9: 49.9, 55.8)
 // or few and the call bound by its pixels (256 to 64 channels 56x56 at batch 64: 67, 68).  Above it 75 of 76 launches
 // gain, 1.2 times on average: 512 to 256 channels 28x28 at batch 64 119 us, 89; 64 to 256 56x56 87, 63; 1024 to 256
-// 14x14 65, 50; 3x3 stride 2 128 channels 56x56 123, 103; the stem 170, 130.  Errors against float64 sums are 0.44 to
+// 14x14 65, 50; 3x3 stride 2 128 channels 56x56 123, 103; the stem 170, 130.  Calls of several taps start where those
+// that keep a patch in LDS do.  Errors against float64 sums are 0.44 to
 // 0.86 times those of the float32 instructions in all 150 launches measured.
 bool f32_terms(int I, int groups, int taps, double gigas, const Epilogue* epi, const float* out) {
   if (math_terms() != 0 || groups != 1 || g_f32_terms == 0) return false;
   if (epi && (epi->res == out || epi->mask == out)) return false;   // a value may be stored twice
   if (g_f32_terms == 2) return true;
-  return I > (taps > 1 ? 32 : 64) && gigas * I >= 2.7 * (I <= 64 ? 64 : ceil_div(I, 128) * 128);
+  return I > (taps > 1 ? 32 : 64) && gigas * I >= (taps > 1 ? 4.0 : 2.7) * (I <= 64 ? 64 : ceil_div(I, 128) * 128);
 }
 const IgemmUnit& unit(int terms, bool epilogue) {
   if (epilogue) return terms == 3 ? igemm_epi_bf16x3_unit() : terms == 1 ? igemm_epi_bf16_unit() : igemm_epi_f32_unit();
