@@ -944,7 +944,7 @@ def main():
                    'global_batch': BATCH, 'device': info['name'].strip(), 'compute_units': info['compute_units']},
         'pct_of_peak': round(100 * conv_tflops / PEAK_FP32_MFMA_TFLOPS, 1),
         'wall_ms_per_step': round(conv_wall_ms, 3),
-        'roofline': {'bound': 'mfma', 'kernel': 'igemm_f32 (Conv2d forward + input gradient)',
+        'roofline': {'bound': 'mfma', 'kernel': 'igemm_f32, and igemm_bf16x3 / patch_product for large launches (Conv2d forward + input gradient)',
                      'achieved': round(igemm_tflops, 2), 'peak': PEAK_FP32_MFMA_TFLOPS, 'unit': 'TFLOP/s',
                      'frac': round(igemm_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
                      'traffic': igemm_traffic, 'traffic_note': igemm_traffic_why,
