@@ -534,8 +534,8 @@ bool patch_conv_takes(const PatchConv& c, bool f32) {
   // (23.4, 56.8), whose rows and channels are mostly padding.
   // In float32 arithmetic small calls, which gain a few microseconds at most, stay with them, and the line lies a little
   // higher: it was fitted to float32 instructions (94 us for 9.7e9 and 119 to 138 for 14.8e9, where these take 63 to 68
-  // and 90 to 102).  From 4e9 on the kernels that gather run on three terms too (f32_terms); 7.0 here then moves one
-  // launch of a PreAct-ResNet-18 step and its time by less than runs differ (4.70 ms, 4.73).
+  // and 90 to 102).  From 4e9 on the kernels that gather run on three terms too (f32_terms); 7.0 here moves some
+  // launches of a PreAct-ResNet-18 step and its time by less than runs differ (4.70 ms, 4.73).
   const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
   const double gigas = 2e-9 * c.I * c.C * c.N * sums;
   return c.taps >= 4 && padding <= 1.5 && gigas >= (f32 ? 4.0 : 1.5) &&
