@@ -137,11 +137,20 @@ class _Loan(_Buffer):
         return _Buffer.ptr.fget(self) if source is None else source.ptr
 
     def settle(self):
-        source, self.source = self.source, None
-        self.deps = ()
-        _unfilled.discard(self)
-        if self.nbytes:
-            _hip.call('tt_memcpy_d2d', self.ptr, source.ptr, self.nbytes)
+        # What is parked may read this loan: it runs while there is a source to read, and it may settle the loan itself.
+        # The block is published, and the source let go of, once the copy into it is on its way.
+        with _hip._lock:
+            _hip.flush()
+            source = self.source
+            if source is None:
+                return
+            if self.nbytes:
+                fresh = _Buffer(self.nbytes)
+                _hip.call('tt_memcpy_d2d', fresh._ptr, source.ptr, self.nbytes)
+                self._ptr, fresh._ptr = fresh._ptr, 0
+            self.source = None
+            self.deps = ()
+            _unfilled.discard(self)
 
 
 # buffers whose contents are still to be produced on demand, or lent by another (normally none or a handful: the
