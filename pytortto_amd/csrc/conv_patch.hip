@@ -48,6 +48,9 @@ constexpr int kTerms = 3;
 constexpr int kUnit = 16 * kTerms;   // bytes of a patch pixel's eight channels.  48 bytes from lane to lane
                                      // spread eight lanes' 16-byte accesses over all banks
 constexpr int kMaxTaps = 31;
+// Taps of weights that a wave of the product reads past its own: two ahead of the one it multiplies, and an odd
+// number of taps is rounded up to a pair, whose second tap fetches one more.
+constexpr int kReadPast = 3;
 
 // Eight float32 values as three vectors of bfloat16 terms that add up to them exactly: term i of a value is
 // the bf16 nearest to what the terms before it leave.
@@ -470,7 +473,7 @@ bool make_plan(const PatchConv& c, Plan* best) {
     }
     if (!fits) continue;
     pl.IT = pl.maxPx <= 384 ? 3 : 4;
-    pl.wt = align_up((wt + 2 * kTerms * 64) * 16);   // two taps' weights more: the product reads ahead of its last
+    pl.wt = align_up((wt + kReadPast * kTerms * 64) * 16);
     // Microseconds, fitted to 75 launches of 4 to 2000 blocks (10 % root mean square): a chunk of a block that
     // shares its compute unit, a block's start and end; a block that has the unit for itself takes a sixth longer.
     // Shares of a reduction are written, read and added.  (The weights' layout costs the same for all.)

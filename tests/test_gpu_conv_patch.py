@@ -71,6 +71,18 @@ def test_transposed(case, math, patch):
     _conv_transpose_checks(case)
 
 
+@pytest.mark.parametrize('c,r', [(48, 3), (32, 3), (80, 5), (16, 1)])
+def test_the_workspace_holds_what_is_read_ahead(c, r, patch):
+    """The product fetches weights two taps ahead and runs an odd number of taps as if it were one more: a 128-row
+    layer's waves read up to three taps of 3 KB past their last.  (A size query: nothing is launched.)"""
+    import ctypes
+    patch(ALWAYS, 'f32')
+    taps = -(-c // 16) * r * r
+    size = ctypes.c_size_t()
+    _hip.call('tt_workspace_size_conv2d_fwd_f32', ctypes.byref(size), 64, c, 28, 28, 128, r, r, 1, 1, r // 2, r // 2, 1, 1, 1)
+    assert size.value >= 3072 * (4 * taps + 2 + taps % 2)
+
+
 @pytest.mark.parametrize('math', ['bf16x3', 'f32'])
 @pytest.mark.parametrize('n,c,hw,k', [(9, 64, 14, 96), (2, 256, 7, 70), (40, 32, 28, 64)])   # the second shares its reduction
 def test_epilogues(n, c, hw, k, math, patch):
