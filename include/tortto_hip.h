@@ -101,8 +101,9 @@ int tt_probe_hbm_f32(size_t bytes, double* read_gbs, double* copy_gbs);
  * whose path is float32 throughout).  TT_CONV_MATH_F32 (the default) computes in float32 and is the mode that
  * meets the reference's tolerances: on v_mfma_f32_32x32x2_f32 -- and in large forward passes and input gradients,
  * where it is faster and its error against float64 sums smaller, by the
- * three exact terms of TT_CONV_MATH_BF16X3; sums that these do not hold (operands that are not finite or round
- * to a bf16 infinity, results below 2^-96) are formed again without them.
+ * three exact terms of TT_CONV_MATH_BF16X3, which hold float32 values of any magnitude there (both operands are scaled by
+ * a power of two on the way); sums that come out as an infinity or NaN all the same (operands that are not finite or from
+ * 2^104, results from 2^80 on) are formed again without them.
  * TT_CONV_MATH_BF16 is the optional reduced-precision variant: tensors stay float32 in memory,
  * both operands are rounded to bfloat16 (nearest even) on their way into
  * v_mfma_f32_32x32x16_bf16 and products are accumulated in float32 (the weight gradient's

@@ -171,6 +171,15 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
     }
   };
 
+  const float lift = BF == 3 && p.w ? kLift : 1.f;   // on the way into LDS
+  auto lifted = [&](floatx4 v) __attribute__((always_inline)) {
+    if constexpr (BF == 3) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] *= lift;
+    }
+    return v;
+  };
+
   // plain-GEMM mode: thread (gpq, gkr) loads rows gkr .. gkr+GR-1 of the chunk's 16 k rows for
   // pixel quad gpq with one 16-byte load per row; no bounds tests, no table (the reduction is a
   // whole number of chunks in this mode), and only the scalar offset moves with k
@@ -186,7 +195,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   auto store_g = [&](int buf) __attribute__((always_inline)) {
     float* tile = reinterpret_cast<float*>(&Bs[buf][0][0]);
 #pragma unroll
-    for (int j = 0; j < GR; ++j) *reinterpret_cast<floatx4*>(tile + (gkr + j) * BN + 4 * gpq) = greg[j];
+    for (int j = 0; j < GR; ++j) *reinterpret_cast<floatx4*>(tile + (gkr + j) * BN + 4 * gpq) = lifted(greg[j]);
   };
 
   floatx4 areg[A_ITEMS];
@@ -242,7 +251,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
   };
   auto store_a_item = [&](int buf, int it) __attribute__((always_inline)) {
     const int q = aq0 + it * (kThreads / BM);
-    if (BM >= 64 || q < kBKQ) As[buf][q][arow] = areg[it];
+    if (BM >= 64 || q < kBKQ) As[buf][q][arow] = lifted(areg[it]);
   };
   auto store_b_item = [&](int buf, int it) __attribute__((always_inline)) {
     floatx4 v = breg[it];
@@ -250,7 +259,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) v[j] = bok[it][j] ? breg[it][j] : 0.f;
     }
-    Bs[buf][bq0 + it * (kThreads / BN)][pix] = v;
+    Bs[buf][bq0 + it * (kThreads / BN)][pix] = lifted(v);
   };
 
   // MFMA operands of one chunk: [kk][tile] float4 = four k-steps each.  Lanes 0-31 take quad
@@ -592,7 +601,7 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
     }
   };
 
-  // One sum in float64: the rare path behind terms_fail.  A NaN stays one, so that data full of them cost a product each.
+  // One sum in float64: the rare path behind not_finite.  A NaN stays one, so that data full of them cost a product each.
   auto exact_sum = [&](const int i, const uint32_t n, const int u, const int v) __attribute__((always_inline)) {
     const int channels = p.Kred / (p.TB * p.TC);
     double sum = 0.0;
@@ -617,13 +626,17 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
       epilogue();
     } else {
       unsigned long long again = 0;   // bit 16*(x*NT + y) + r
-      if (p.w && terms_may_fail<MT, NT>(acc)) {
+      if (p.w) {
+        const bool any = not_finite<MT, NT>(acc);
 #pragma unroll
         for (int x = 0; x < MT; ++x)
 #pragma unroll
           for (int y = 0; y < NT; ++y)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) again |= (unsigned long long)terms_fail(acc[x][y][r]) << (16 * (x * NT + y) + r);
+            for (int r = 0; r < 16; ++r) {
+              if (any) again |= (unsigned long long)!(__builtin_fabsf(acc[x][y][r]) <= 3.402823466e38f) << (16 * (x * NT + y) + r);
+              acc[x][y][r] *= kLower;
+            }
       }
       epilogue();
       for (; again; again &= again - 1) {

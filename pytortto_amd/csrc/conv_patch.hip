@@ -22,7 +22,7 @@
 // of a product is below half an ulp of it, and the error against float64 sums is 0.33 to 0.66 times that of the
 // float32 instructions, which round twice as often (42 launches).  A ResNet-50 training step at batch 64 takes
 // 19.43 ms for 20.27, a PreAct-ResNet-18 one at batch 128 4.81 for 5.35.  What three terms do not hold is summed
-// again (terms_fail).
+// again (not_finite).
 //
 // The pixels of a tile are consecutive pixels of the batch, whatever the image's shape.  Their source lies in
 // a virtual image that holds the images of the batch below each other, each framed by what the taps reach
@@ -85,7 +85,7 @@ struct PatchTaps {
 // sixteen channels for every class: reads runs of w, turns them in LDS, writes runs of wt.
 template <bool DGRAD>
 __global__ __launch_bounds__(kThreads) void patch_weights(const float* __restrict__ w, uintx4* __restrict__ wt, int rows, int chans,
-                                                         int taps, tt::FastDiv divRun, int chunks, const PatchTaps classes) {
+                                                         int taps, tt::FastDiv divRun, int chunks, float lift, const PatchTaps classes) {
   extern __shared__ float strip[];   // [outer][run + 1]: forward 32 rows x 16 channels' taps, gradient 16 x 32 rows' taps
   const int chunk = blockIdx.x, r0 = blockIdx.y * 32, c0 = chunk * kBK;
   const int run = divRun.d;          // (DGRAD ? 32 : 16) * taps
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(kThreads) void patch_weights(const float* __restric
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-      if (at[e] >= 0) strip[at[e]] = v[e];
+      if (at[e] >= 0) strip[at[e]] = v[e] * lift;
   }
   __syncthreads();
   for (int k = 0; k < classes.n; ++k) {
@@ -155,7 +155,7 @@ struct Patch {
   PatchClass c[kPatchClasses];
 };
 
-// One sum in float64, over the channels [c0, c1): the rare path behind terms_fail.  A NaN stays one, so that data
+// One sum in float64, over the channels [c0, c1): the rare path behind not_finite.  A NaN stays one, so that data
 // full of them cost a product each.
 __device__ __forceinline__ float exact_sum(const Igemm& p, const Patch& q, const PatchClass& k, const int i, const uint32_t n, const int u, const int v,
                                           const int c0, const int c1) {
@@ -238,9 +238,12 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
         reg[it][e] = as_float(__builtin_amdgcn_raw_buffer_load_b32(srd, vo, (c0 + e) * q.plane, 0));
       }
   };
+  const float lift = q.w ? kLift : 1.f;
   auto stage = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int it = 0; it < IT; ++it) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) reg[it][e] *= lift;
       uintx4 t[kTerms];
       split8(reg[it], t);
       if (it * 128 + pp0 < k.px) {
@@ -373,11 +376,15 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
   for (int y = 0; y < NT; ++y) acc[0][y] += small[y];
 
   unsigned long long again = 0;   // values to be summed once more (bit 16*y + r)
-  if (q.w && terms_may_fail<1, NT>(acc)) {
+  if (q.w) {
+    const bool any = not_finite<1, NT>(acc);
 #pragma unroll
     for (int y = 0; y < NT; ++y)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) again |= (unsigned long long)terms_fail(acc[0][y][r]) << (16 * y + r);
+      for (int r = 0; r < 16; ++r) {
+        if (any) again |= (unsigned long long)!(__builtin_fabsf(acc[0][y][r]) <= 3.402823466e38f) << (16 * y + r);
+        acc[0][y][r] *= kLower;
+      }
   }
   if constexpr (EPI) {
     if (whole && p.epi.on) {
@@ -589,8 +596,8 @@ int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const 
     const dim3 grid((unsigned)pl.chunks, (unsigned)(pl.Ipad / 32));
     const size_t lds = sizeof(float) * (size_t)outer * (run + 1);
     const tt::FastDiv divRun = tt::make_fastdiv((uint32_t)run);
-    if (c.dgrad) patch_weights<true><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, c.taps, divRun, pl.chunks, taps);
-    else patch_weights<false><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, c.taps, divRun, pl.chunks, taps);
+    if (c.dgrad) patch_weights<true><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, c.taps, divRun, pl.chunks, f32 ? kLift : 1.f, taps);
+    else patch_weights<false><<<grid, kThreads, lds, st>>>(w, (uintx4*)ws, c.I, c.C, c.taps, divRun, pl.chunks, f32 ? kLift : 1.f, taps);
     TT_LAUNCH_CHECK();
   }
   const int BM = 32 * pl.WM, BN = 128 * pl.NT / pl.WM;

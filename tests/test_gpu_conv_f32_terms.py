@@ -116,9 +116,49 @@ def test_operands_the_terms_do_not_hold(dims, scale, terms):
         finite = np.isfinite(a) & np.isfinite(b)
         assert finite.mean() > .5
         size = float(np.abs(b[finite], dtype=np.float64).max())
-        # the least bfloat16 is 2^-133: what rounds to no term at all is missing from a sum of nothing else
+        # float32 instructions round every product and sum to a multiple of 2^-149
         np.testing.assert_allclose(a[finite], b[finite], rtol=1e-5,
-                                   atol=max(1e-6 * min(size, 1e3 * scale), 2.0 ** -133 * r * r * max(c, k)))
+                                   atol=max(1e-6 * min(size, 1e3 * scale), 2.0 ** -150 * r * r * max(c, k)))
+
+
+def _distance(got, want, size):
+    """2-norm of the error, beyond the rounding of a result, in units of the sums of magnitudes."""
+    return float(np.linalg.norm(np.maximum(np.abs(got - want) - 2.0 ** -150, 0) / size))
+
+
+@pytest.mark.parametrize('kernels', ['gather', 'patch'])
+@pytest.mark.parametrize('dims', [(9, 64, 14, 96, 1, 1), (3, 17, 28, 33, 3, 1), (3, 64, 28, 128, 3, 2)])
+@pytest.mark.parametrize('ex,ew', [(-120, 40), (-124, 60), (-126, 60), (-133, 60), (-135, 30), (-140, 100), (60, -126),
+                                   (100, -140), (-126, 0), (-140, 0), (-70, -70), (-90, 30), (60, 15), (90, 20)])
+def test_operands_of_any_magnitude(dims, ex, ew, kernels, terms):
+    """Sums as near to float64 ones as those of the float32 instructions, where the last terms of one operand lie
+    below the least bfloat16, where all of them do, and where lifted sums overflow."""
+    import torch
+    n, c, hw, k, r, stride = dims
+    xh, wh, dyh = (np.ldexp(a, e) for a, e in zip(_arrays(*dims, np.random.default_rng(8)), (ex, ew, ex)))
+    geometry = ((stride, stride), (r // 2, r // 2), (1, 1), 1)
+
+    def sums(x, w, dy):
+        x, w, dy = (torch.tensor(a, dtype=torch.float64) for a in (x, w, dy))
+        x.requires_grad = True
+        y = torch.nn.functional.conv2d(x, w, padding=r // 2, stride=stride)
+        y.backward(dy)
+        return y.detach().numpy(), x.grad.numpy()
+    want, size = sums(xh, wh, dyh), sums(np.abs(xh), np.abs(wh), np.abs(dyh))
+    x, w, dy = hiparray(xh), hiparray(wh), hiparray(dyh)
+
+    def errors():
+        got = (ops.conv2d_fwd(x, w, None, *geometry).get(), ops.conv2d_dgrad(dy, w, None, (hw, hw), *geometry).get())
+        return [_distance(a.astype(np.float64), b, np.where(s > 0, s, 1)) for a, b, s in zip(got, want, size)]
+    terms(NEVER)
+    old = errors()
+    terms(ALWAYS)
+    if kernels == 'patch':
+        _hip.call('tt_conv2d_patch_enable', ALWAYS)
+    new = errors()
+    assert _last_launch()['persistent_blocks'] == -4 or kernels == 'gather'
+    print(dims, ex, ew, kernels, new, old)
+    assert all(a <= b for a, b in zip(new, old)), (new, old)
 
 
 @pytest.mark.parametrize('dims', [d for d in GEOMETRIES if d[5] == 1])
