@@ -222,7 +222,7 @@ int g_f32_terms = 1;   // tests: 0 = never, 2 = wherever they can
 // 0.86 times those of the float32 instructions in all 150 launches measured.
 bool f32_terms(int I, int groups, int taps, double gigas, const Epilogue* epi, const float* out) {
   if (math_terms() != 0 || groups != 1 || g_f32_terms == 0) return false;
-  if (epi && (epi->res == out || epi->mask == out)) return false;   // a value may be stored twice
+  if (epi && (epi->res == out || epi->mask == out)) return false;   // in place: as they always ran (nobody here asks for it)
   if (g_f32_terms == 2) return true;
   return I > (taps > 1 ? 32 : 64) && gigas * I >= (taps > 1 ? 4.0 : 2.7) * (I <= 64 ? 64 : ceil_div(I, 128) * 128);
 }
@@ -347,8 +347,8 @@ bool g_bf16_first_always = false;   // tests: also where the tile-count rule wou
 // Whether the channel-last kernels (conv_hwc.hip) are to be asked, and whether they take all they support.
 bool g_hwc = true, g_hwc_always = false;
 bool hwc_math(int groups) { return groups == 1 && bf16_math() && g_hwc; }
-// Whether the patch kernels (conv_patch.hip) are to be asked.  In float32 arithmetic they may store a value twice:
-// an epilogue must not read what it writes.
+// Whether the patch kernels (conv_patch.hip) are to be asked: in float32 arithmetic not for an epilogue that reads what it
+// writes (f32_terms).
 bool patch_math(int groups, const Epilogue* epi, const float* out) {
   return groups == 1 && !bf16_math() && (epi == nullptr || split_math() || (epi->res != out && epi->mask != out));
 }

@@ -209,28 +209,13 @@ __device__ __forceinline__ void store_through_epilogue(const Igemm& p, const flo
   }
 }
 
-// What the launch does to a sum on its way to memory, for one value: the steps of store_through_epilogue.
-__device__ __forceinline__ float finish_value(const Igemm& p, const int i, const uint32_t e, float v) {
-  if (p.bias) v += p.bias[i];
-  if (p.epi.on) {
-    if (p.epi.norm) {
-      const float sd = __fsqrt_rn(__fadd_rn(p.epi.var[i], p.epi.eps));
-      v = fmaf(v - p.epi.mean[i], __fdiv_rn(p.epi.gamma ? p.epi.gamma[i] : 1.0f, sd), p.epi.beta ? p.epi.beta[i] : 0.0f);
-    }
-    if (p.epi.res) v += p.epi.res[e];
-    if (p.epi.relu) v = (v > 0.f || v != v) ? v : 0.f;
-    if (p.epi.mask) v *= p.epi.mask[e] > 0.f ? 1.f : 0.f;
-  }
-  return v;
-}
-
 // Float32 launches on three bfloat16 terms multiply both operands by kLift on their way in and the sums by kLower
 // on their way out: exact, and what a term holds then reaches down to the least float32, 2^-149 (a bfloat16 has no bit
 // below 2^-133, so that without it operands under 2^-110 lost bits and those under 2^-134 all of them: 64 products
 // of 2^-126 and 2^60 were off by 7e-4, of 2^-135 and 2^60 they were zero).  One vector instruction per value:
 // 512 to 256 channels 1x1, 28x28 at batch 64, 95 us without, 98 with; 128 channels 3x3, 16x16 at batch 128, 69 and 69.
 // What it takes from the other end -- operands from 2^104, sums from 2^80 on -- comes out as an infinity or NaN, like
-// everything that is not finite itself, and such sums are formed again (exact_sum).
+// everything that is not finite itself, and such sums are formed again (float32_sums).
 constexpr float kLift = 0x1p24f, kLower = 0x1p-48f;
 
 // Whether a lane's sums hold an infinity or NaN.  Two values an instruction (v_maximum3_f32, which keeps NaN).
@@ -245,6 +230,75 @@ __device__ __forceinline__ bool not_finite(const floatx16 (&acc)[MT][NT]) {
       for (int r = 0; r < 16; r += 2)
         most = __builtin_elementwise_maximum(__builtin_elementwise_maximum(__builtin_fabsf(acc[x][y][r]), __builtin_fabsf(acc[x][y][r + 1])), most);
   return !(most <= 3.402823466e38f);
+}
+
+// The operands of a wave's tiles as they lie in memory: lane l32 + 32*h holds row l32 of every row tile and pixel l32
+// of every pixel tile.  Tap (r, s) of channel c is w[x][c*wC + r*wRow + s*wCol] and pixel row ih[y] + r*dh, column
+// iw[y] + s*dw of the plane src[y] + c*plane, zero outside it.
+template <int MT, int NT>
+struct WaveOperands {
+  const float* w[MT];
+  const float* src[NT];
+  int ih[NT], iw[NT];
+  int R, S, wC, wRow, wCol, dh, dw, H, W, srcRow;
+  long long plane;
+};
+
+// Their sums over the channels [c0, c1) on the float32 matrix instructions, what launches without terms compute: for
+// the few waves of a launch in three terms that not_finite stops.  Operands come straight from memory, four
+// steps' loads in flight: launches whose every sum is infinite or NaN take 368 us for 128 on the float32 instructions alone
+// (512 to 256 channels 1x1, 28x28 at batch 64) and 224 for 93 (128 channels 3x3, 16x16 at batch 128); summed
+// one by one, in float64, they took 26.8 and 13.3 ms.  One infinite pixel in every image costs 230 and 214 us, then 9.9
+// and 7.4 ms.
+template <int MT, int NT>
+__device__ __forceinline__ void float32_sums(floatx16 (&acc)[MT][NT], const WaveOperands<MT, NT>& o, const int c0, const int c1, const int h) {
+#pragma unroll
+  for (int x = 0; x < MT; ++x)
+#pragma unroll
+    for (int y = 0; y < NT; ++y)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[x][y][r] = 0.f;
+  constexpr int kSteps = 4;
+  for (int r = 0; r < o.R; ++r)
+    for (int s = 0; s < o.S; ++s) {
+      const float* w[MT];
+      const float* src[NT];
+      bool inside[NT];
+#pragma unroll
+      for (int x = 0; x < MT; ++x) w[x] = o.w[x] + r * o.wRow + s * o.wCol;
+#pragma unroll
+      for (int y = 0; y < NT; ++y) {
+        const int ih = o.ih[y] + r * o.dh, iw = o.iw[y] + s * o.dw;
+        inside[y] = (unsigned)ih < (unsigned)o.H && (unsigned)iw < (unsigned)o.W;
+        src[y] = o.src[y] + (inside[y] ? (long long)ih * o.srcRow + iw : 0);
+      }
+      for (int c = c0; c < c1; c += 2 * kSteps) {   // lanes 0-31 hold a step's first channel, lanes 32-63 its second
+        float a[kSteps][MT], b[kSteps][NT];
+#pragma unroll
+        for (int k = 0; k < kSteps; ++k) {
+          const int ch = c + 2 * k + h;
+          const long long at = min(ch, c1 - 1);
+#pragma unroll
+          for (int x = 0; x < MT; ++x) a[k][x] = w[x][at * o.wC];
+#pragma unroll
+          for (int y = 0; y < NT; ++y) b[k][y] = src[y][at * o.plane];
+#pragma unroll
+          for (int x = 0; x < MT; ++x) a[k][x] = ch < c1 ? a[k][x] : 0.f;
+#pragma unroll
+          for (int y = 0; y < NT; ++y) b[k][y] = ch < c1 && inside[y] ? b[k][y] : 0.f;
+        }
+        // eight products add up on their own first: shorter chains, and smaller errors, than one over the whole reduction
+#pragma unroll
+        for (int x = 0; x < MT; ++x)
+#pragma unroll
+          for (int y = 0; y < NT; ++y) {
+            floatx16 part = {};
+#pragma unroll
+            for (int k = 0; k < kSteps; ++k) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[k][x], b[k][y], part, 0, 0, 0);
+            acc[x][y] += part;
+          }
+      }
+    }
 }
 
 // The bf16-first kernels (conv_igemm_bf16.hip).  `supported` tells whether they take launch `p`

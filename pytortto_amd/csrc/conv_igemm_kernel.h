@@ -601,56 +601,38 @@ __device__ __forceinline__ void igemm_body(const Igemm& p, const int block_x) {
     }
   };
 
-  // One sum in float64: the rare path behind not_finite.  A NaN stays one, so that data full of them cost a product each.
-  auto exact_sum = [&](const int i, const uint32_t n, const int u, const int v) __attribute__((always_inline)) {
-    const int channels = p.Kred / (p.TB * p.TC);
-    double sum = 0.0;
-    for (int c = 0; c < channels && sum == sum; ++c) {
-      const float* x = p.src + (long long)n * p.srcStrideN + (long long)c * p.kStride;
-      const float* w = p.w + (long long)i * p.wI + (long long)c * p.wC + p.w0;
-      for (int b = 0; b < p.TB; ++b) {
-        const int ih = u * p.su + p.bh + b * p.stepH;
-        for (int t = 0; t < p.TC; ++t) {   // a tap outside the image multiplies a zero, as everywhere
-          const int iw = v * p.sv + p.bw + t * p.stepW;
-          const bool inside = (unsigned)ih < (unsigned)p.Hlim && (unsigned)iw < (unsigned)p.Wlim;
-          sum = fma(inside ? (double)x[(long long)ih * p.srcRow + iw] : 0.0, (double)w[b * p.wRow + t * p.wCol], sum);
+  // Stores the tile; float32 sums that three terms do not hold are formed again.
+  auto finish = [&]() __attribute__((always_inline)) {
+    if constexpr (BF == 3) {
+      if (p.w) {
+        if (__builtin_amdgcn_ballot_w64(not_finite<MT, NT>(acc))) {
+          WaveOperands<MT, NT> o;
+          o.R = p.TB; o.S = p.TC; o.wC = p.wC; o.wRow = p.wRow; o.wCol = p.wCol; o.dh = p.stepH; o.dw = p.stepW;
+          o.H = p.Hlim; o.W = p.Wlim; o.srcRow = p.srcRow; o.plane = p.kStride;
+#pragma unroll
+          for (int x = 0; x < MT; ++x) o.w[x] = p.w + (long long)min(i0 + (wm * MT + x) * 32 + l32, p.I - 1) * p.wI + p.w0;
+#pragma unroll
+          for (int y = 0; y < NT; ++y) {
+            const uint32_t m = (uint32_t)min(m0 + (wn * NT + y) * 32 + l32, p.M - 1);
+            const uint32_t n = tt::fd_div(m, p.divUV);
+            const uint32_t rem = m - n * p.divUV.d;
+            const uint32_t u = tt::fd_div(rem, p.divV);
+            o.src[y] = p.src + (long long)n * p.srcStrideN;
+            o.ih[y] = (int)u * p.su + p.bh;
+            o.iw[y] = (int)(rem - u * p.divV.d) * p.sv + p.bw;
+          }
+          float32_sums<MT, NT>(acc, o, 0, p.Kred / (p.TB * p.TC), h);
+        } else {
+#pragma unroll
+          for (int x = 0; x < MT; ++x)
+#pragma unroll
+            for (int y = 0; y < NT; ++y)
+#pragma unroll
+              for (int r = 0; r < 16; ++r) acc[x][y][r] *= kLower;
         }
       }
     }
-    return (float)sum;
-  };
-
-  // Stores the tile; float32 sums that three terms do not hold are formed and stored again.
-  auto finish = [&]() __attribute__((always_inline)) {
-    if constexpr (BF != 3) {
-      epilogue();
-    } else {
-      unsigned long long again = 0;   // bit 16*(x*NT + y) + r
-      if (p.w) {
-        const bool any = not_finite<MT, NT>(acc);
-#pragma unroll
-        for (int x = 0; x < MT; ++x)
-#pragma unroll
-          for (int y = 0; y < NT; ++y)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-              if (any) again |= (unsigned long long)!(__builtin_fabsf(acc[x][y][r]) <= 3.402823466e38f) << (16 * (x * NT + y) + r);
-              acc[x][y][r] *= kLower;
-            }
-      }
-      epilogue();
-      for (; again; again &= again - 1) {
-        const int bit = __builtin_ctzll(again), r = bit & 15, x = (bit >> 4) / NT, y = (bit >> 4) % NT;
-        const int i = i0 + (wm * MT + x) * 32 + 8 * (r >> 2) + 4 * h + (r & 3), m = m0 + (wn * NT + y) * 32 + l32;
-        if (i >= p.I || m >= p.M) continue;
-        const uint32_t n = tt::fd_div((uint32_t)m, p.divUV);
-        const uint32_t rem = (uint32_t)m - n * p.divUV.d;
-        const uint32_t u = tt::fd_div(rem, p.divV);
-        const uint32_t v = rem - u * p.divV.d;
-        const uint32_t e = (uint32_t)((int)n * p.outStrideN + ((int)u * p.ou + p.ouh) * p.outRow + (int)v * p.ov + p.ovw + i * p.outStrideI);
-        p.out[e] = finish_value(p, i, e, exact_sum(i, n, (int)u, (int)v));
-      }
-    }
+    epilogue();
   };
 
   const int chunks = p.KQ / kBKQ;

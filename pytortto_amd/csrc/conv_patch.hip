@@ -22,7 +22,7 @@
 // of a product is below half an ulp of it, and the error against float64 sums is 0.33 to 0.66 times that of the
 // float32 instructions, which round twice as often (42 launches).  A ResNet-50 training step at batch 64 takes
 // 19.43 ms for 20.27, a PreAct-ResNet-18 one at batch 128 4.81 for 5.35.  What three terms do not hold is summed
-// again (not_finite).
+// again on the float32 instructions (not_finite).
 //
 // The pixels of a tile are consecutive pixels of the batch, whatever the image's shape.  Their source lies in
 // a virtual image that holds the images of the batch below each other, each framed by what the taps reach
@@ -154,28 +154,6 @@ struct Patch {
   int classes;
   PatchClass c[kPatchClasses];
 };
-
-// One sum in float64, over the channels [c0, c1): the rare path behind not_finite.  A NaN stays one, so that data
-// full of them cost a product each.
-__device__ __forceinline__ float exact_sum(const Igemm& p, const Patch& q, const PatchClass& k, const int i, const uint32_t n, const int u, const int v,
-                                          const int c0, const int c1) {
-  const int R = k.taps / k.S;
-  const char* image = (const char*)q.src + (long long)n * q.image;
-  double sum = 0.0;
-  for (int c = c0; c < c1 && sum == sum; ++c) {
-    const float* x = (const float*)(image + (long long)c * q.plane);
-    const float* w = q.w + (long long)i * q.wI + (long long)c * q.wC + k.w0;
-    for (int r = 0; r < R; ++r) {
-      const int h = u + k.bh + r * k.dh;
-      for (int s = 0; s < k.S; ++s) {   // a tap outside the image multiplies a zero, as everywhere
-        const int j = v + k.bw + s * k.dw;
-        const bool inside = (unsigned)h < (unsigned)p.Hlim && (unsigned)j < (unsigned)p.Wlim;
-        sum = fma(inside ? (double)x[h * p.Wlim + j] : 0.0, (double)w[r * k.wRow + s * k.wCol], sum);
-      }
-    }
-  }
-  return (float)sum;
-}
 
 // Tile 32*WM rows x 32*NT*(4/WM) pixels; every wave has 32 rows and NT x 32 pixels.  The patch has at most 128*IT
 // pixels: a thread fetches and splits eight channels of IT of them.
@@ -362,11 +340,14 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
     tap(w2, kOdd, off, next);
     advance(0);
   }
+  int again = lane;
+  asm("" : "+v"(again));   // where a lane's values lie is worked out again: kept over the loop it would take registers there
+  const int col = again & 31, hh = again >> 5;
   uint32_t obase[NT];
   bool mok[NT];
 #pragma unroll
   for (int y = 0; y < NT; ++y) {
-    const int m = m0 + (wn * NT + y) * 32 + l32;
+    const int m = m0 + (wn * NT + y) * 32 + col;
     mok[y] = m < k.M;
     uint32_t n, u, v;
     split_pixel(mok[y] ? (uint32_t)m : 0u, n, u, v);
@@ -375,16 +356,27 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
 #pragma unroll
   for (int y = 0; y < NT; ++y) acc[0][y] += small[y];
 
-  unsigned long long again = 0;   // values to be summed once more (bit 16*y + r)
   if (q.w) {
-    const bool any = not_finite<1, NT>(acc);
+    if (__builtin_amdgcn_ballot_w64(not_finite<1, NT>(acc))) {   // sums that three terms do not hold
+      WaveOperands<1, NT> o;
+      o.R = k.taps / k.S; o.S = k.S; o.wC = q.wC; o.wRow = k.wRow; o.wCol = k.wCol; o.dh = k.dh; o.dw = k.dw;
+      o.H = p.Hlim; o.W = p.Wlim; o.srcRow = p.Wlim; o.plane = q.plane / 4;
+      o.w[0] = q.w + (long long)min(i0 + wm * 32 + col, p.I - 1) * q.wI + k.w0;
 #pragma unroll
-    for (int y = 0; y < NT; ++y)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        if (any) again |= (unsigned long long)!(__builtin_fabsf(acc[0][y][r]) <= 3.402823466e38f) << (16 * y + r);
-        acc[0][y][r] *= kLower;
+      for (int y = 0; y < NT; ++y) {
+        uint32_t n, u, v;
+        split_pixel((uint32_t)min(m0 + (wn * NT + y) * 32 + col, k.M - 1), n, u, v);
+        o.src[y] = (const float*)((const char*)q.src + (long long)n * q.image);
+        o.ih[y] = (int)u + k.bh;
+        o.iw[y] = (int)v + k.bw;
       }
+      float32_sums<1, NT>(acc, o, q0 * kBK, min(q.C, q1 * kBK), hh);
+    } else {
+#pragma unroll
+      for (int y = 0; y < NT; ++y)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][y][r] *= kLower;
+    }
   }
   if constexpr (EPI) {
     if (whole && p.epi.on) {
@@ -393,7 +385,7 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
         const floatx16 two[1][2] = {{acc[0][y], acc[0][y + 1]}};
         const uint32_t ob[2] = {obase[y], obase[y + 1]};
         const bool ok[2] = {mok[y], mok[y + 1]};
-        store_through_epilogue<BM, 1, 2>(p, two, ob, ok, i0, wm * 32, h, epi_lds);
+        store_through_epilogue<BM, 1, 2>(p, two, ob, ok, i0, wm * 32, hh, epi_lds);
       }
     }
   }
@@ -401,11 +393,11 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
   float* out = whole ? p.out : q.partial + (size_t)blockIdx.z * (size_t)q.outElems;
   if (!EPI || !whole || !p.epi.on) {
     const bool biased = whole && p.bias != nullptr;
-    const uint32_t hoff = (uint32_t)(4 * h * p.outStrideI);
+    const uint32_t hoff = (uint32_t)(4 * hh * p.outStrideI);
     const int srow = __builtin_amdgcn_readfirstlane(i0 + wm * 32);
     float bz[16];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) bz[r] = biased ? p.bias[min(srow + 8 * (r >> 2) + 4 * h + (r & 3), p.I - 1)] : 0.f;
+    for (int r = 0; r < 16; ++r) bz[r] = biased ? p.bias[min(srow + 8 * (r >> 2) + 4 * hh + (r & 3), p.I - 1)] : 0.f;
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_waitcnt(0x0f70);   // every load done before the first store: they share one counter
     __builtin_amdgcn_sched_barrier(0);
@@ -413,23 +405,12 @@ __global__ __launch_bounds__(kThreads, 2) void patch_product(const Igemm p, cons
     for (int r = 0; r < 16; ++r) {
       const int row = srow + 8 * (r >> 2) + (r & 3);
       float* __restrict__ rowp = out + (size_t)row * (size_t)p.outStrideI;
-      if (row + 4 * h < p.I) {
+      if (row + 4 * hh < p.I) {
 #pragma unroll
         for (int y = 0; y < NT; ++y)
           if (mok[y]) rowp[obase[y] + hoff] = biased ? acc[0][y][r] + bz[r] : acc[0][y][r];
       }
     }
-  }
-  for (; again; again &= again - 1) {
-    const int bit = __builtin_ctzll(again), r = bit & 15;
-    const int i = i0 + wm * 32 + 8 * (r >> 2) + 4 * h + (r & 3), m = m0 + (wn * NT + (bit >> 4)) * 32 + l32;
-    if (i >= p.I || m >= k.M) continue;
-    uint32_t n, u, v;
-    split_pixel((uint32_t)m, n, u, v);
-    const float sum = exact_sum(p, q, k, i, n, (int)u, (int)v, q0 * kBK, min(q.C, q1 * kBK));
-    const uint32_t e = n * (uint32_t)p.outStrideN + (u * (uint32_t)p.ou + (uint32_t)k.ouh) * (uint32_t)p.outRow + v * (uint32_t)p.ov +
-                       (uint32_t)k.ovw + (uint32_t)i * (uint32_t)p.outStrideI;
-    out[e] = whole ? finish_value(p, i, e, sum) : sum;
   }
 }
 
