@@ -220,11 +220,14 @@ int g_f32_terms = 1;   // tests: 0 = never, 2 = wherever they can
 // 14x14 65, 50; 3x3 stride 2 128 channels 56x56 123, 103; the stem 170, 130.  Calls of several taps start where those
 // that keep a patch in LDS do.  Errors against float64 sums are 0.44 to
 // 0.86 times those of the float32 instructions in all 150 launches measured.
-bool f32_terms(int I, int groups, int taps, double gigas, const Epilogue* epi, const float* out) {
+// Sums of fewer than four products stay with those: of one, what the terms leave out and the second rounding make the
+// error 1.4 times theirs, of two 1.1, of three 0.9 to 1.04; of four 0.8 to 0.95, of sixteen 0.5 to 0.7 (relative to a
+// sum's magnitudes; the larger figures where operands spread over e^12).
+bool f32_terms(int I, int groups, int taps, int length, double gigas, const Epilogue* epi, const float* out) {
   if (math_terms() != 0 || groups != 1 || g_f32_terms == 0) return false;
   if (epi && (epi->res == out || epi->mask == out)) return false;   // in place: as they always ran (nobody here asks for it)
   if (g_f32_terms == 2) return true;
-  return I > (taps > 1 ? 32 : 64) && gigas * I >= (taps > 1 ? 4.0 : 2.7) * (I <= 64 ? 64 : ceil_div(I, 128) * 128);
+  return length >= 4 && I > (taps > 1 ? 32 : 64) && gigas * I >= (taps > 1 ? 4.0 : 2.7) * (I <= 64 ? 64 : ceil_div(I, 128) * 128);
 }
 const IgemmUnit& unit(int terms, bool epilogue) {
   if (epilogue) return terms == 3 ? igemm_epi_bf16x3_unit() : terms == 1 ? igemm_epi_bf16_unit() : igemm_epi_f32_unit();
@@ -787,7 +790,7 @@ static int conv2d_fwd(const float* x, const float* w, const float* bias, float* 
   const int M = N * P * Q;
   const int KQ = ceil_div(Kred, 4 * kBKQ) * kBKQ;
   const bool plain = R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-  const bool in_terms = f32_terms(Kg, groups, R * S, 2e-9 * M * Kg * Kred, epi, y);
+  const bool in_terms = f32_terms(Kg, groups, R * S, Kred, 2e-9 * M * Kg * Kred, epi, y);
   const TileChoice t = choose_tile(Kg, M, groups, KQ / kBKQ, true, plain && KQ / kBKQ <= 32 && math_terms() == 0 && !in_terms);
   const int Ipad = ceil_div(Kg, t.bm) * t.bm;
 
@@ -1109,7 +1112,7 @@ static int conv2d_dgrad(const float* dy, const float* w, const float* bias, floa
       const int M = N * U * V;
       const int KQ = ceil_div(Kred, 4 * kBKQ) * kBKQ;
       const bool plain = R == 1 && S == 1 && sh == 1 && sw == 1 && ph == 0 && pw == 0;
-      const bool in_terms = allow_stream_k && Kred > 0 && f32_terms(Cg, groups, nTr * nTs, 2e-9 * M * Cg * Kred, epi, dx);
+      const bool in_terms = allow_stream_k && Kred > 0 && f32_terms(Cg, groups, nTr * nTs, Kred, 2e-9 * M * Cg * Kred, epi, dx);
       const TileChoice t = choose_tile(Cg, M, groups, KQ / kBKQ, allow_stream_k,
                                        (plain && KQ / kBKQ <= 32 && math_terms() == 0 && !in_terms) || !allow_stream_k);
       const int Ipad = ceil_div(Cg, t.bm) * t.bm;

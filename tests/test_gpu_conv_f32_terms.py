@@ -218,6 +218,25 @@ def test_sums_formed_again_keep_pace(dims, kernels, terms):
     assert again < 10 * alone
 
 
+@pytest.mark.parametrize('c', [1, 3, 4])
+def test_short_sums_stay_on_the_more_accurate_instructions(c, terms):
+    """However large the launch: three products and fewer are nearer to their float64 sum in float32 instructions."""
+    rng = np.random.default_rng(12)
+    x, w = hiparray.zeros((550 // c, c, 112, 112)), hiparray.zeros((256, c, 1, 1))      # 3.5e9 products and sums
+    terms(WHERE_FASTER)
+    ops.conv2d_fwd(x, w, None, (1, 1), (0, 0), (1, 1), 1)
+    assert in_terms() == (c >= 4)
+    xh, wh = rng.standard_normal((8, c, 56, 56)).astype(np.float32), rng.standard_normal((96, c, 1, 1)).astype(np.float32)
+    want = np.einsum('nchw,kc->nkhw', xh.astype(np.float64), wh[:, :, 0, 0].astype(np.float64))
+    size = np.einsum('nchw,kc->nkhw', np.abs(xh).astype(np.float64), np.abs(wh[:, :, 0, 0]).astype(np.float64))
+
+    def error(which):
+        terms(which)
+        return _distance(ops.conv2d_fwd(hiparray(xh), hiparray(wh), None, (1, 1), (0, 0), (1, 1), 1).get().astype(np.float64), want, size)
+    if c >= 4:
+        assert error(ALWAYS) <= error(NEVER)
+
+
 @pytest.mark.parametrize('dims', [d for d in GEOMETRIES if d[5] == 1])
 def test_epilogues(dims, terms):
     """The same bits as the entry points they stand in for; an epilogue that writes what it reads keeps the float32
