@@ -506,6 +506,9 @@ bool patch_conv_takes(const PatchConv& c, bool f32) {
     if ((g.R - 1LL) * g.dh > 512 || (g.S - 1LL) * g.dw > 512) return false;   // wider than a patch
     sums += (double)g.R * g.S * g.U * g.V;
   }
+  // most calls are too small: no plan for them (0.1 to 0.2 us of host time each)
+  const double gigas = 2e-9 * c.I * c.C * c.N * sums;
+  if (g_patch != 2 && (c.taps < 4 || gigas < (f32 ? 4.0 : 1.5))) return false;
   Plan pl;
   if (!make_plan(c, &pl)) return false;
   // 32-bit offsets: virtual pixels of the batch, source bytes of the images that a patch touches
@@ -528,9 +531,7 @@ bool patch_conv_takes(const PatchConv& c, bool f32) {
   // and 90 to 102).  From 4e9 on the kernels that gather run on three terms too (f32_terms); 7.0 here moves some
   // launches of a PreAct-ResNet-18 step and its time by less than runs differ (4.70 ms, 4.73).
   const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
-  const double gigas = 2e-9 * c.I * c.C * c.N * sums;
-  return c.taps >= 4 && padding <= 1.5 && gigas >= (f32 ? 4.0 : 1.5) &&
-         pl.cost + 3 + 4e-6 * c.I * c.C * c.taps < 16 + (f32 ? 7.5 : 7.0) * gigas;
+  return padding <= 1.5 && pl.cost + 3 + 4e-6 * c.I * c.C * c.taps < 16 + (f32 ? 7.5 : 7.0) * gigas;
 }
 
 int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi,
