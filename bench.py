@@ -29,6 +29,7 @@ sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3
 PEAK_BF16_MFMA_TFLOPS = 2500.0   # dense, published
+PEAK_TERMS_TFLOPS = PEAK_BF16_MFMA_TFLOPS / 6   # of float32 products in three bf16 terms: six matrix instructions for one
 PEAK_HBM_GBS = 8000.0
 
 # ResNet-50 convolutions at 224x224: (C_in, H_in, C_out, kernel, stride, pad, occurrences)
@@ -281,6 +282,20 @@ def timed_steps(hip, step, steps, warmup):
     return ms / steps, wall / steps
 
 
+def share_in_terms(call, layers):
+    """Share of the forward and input-gradient work that runs on three bf16 terms, by the library's own launch plans."""
+    import ctypes
+    plan, total, terms = (ctypes.c_int * 8)(), 0.0, 0.0
+    for l in layers:
+        passes = l.passes(call)
+        for name in ('fwd', 'dgrad'):
+            passes[name]()
+            call('tt_conv2d_last_launch', plan)
+            total += l.count * l.flops
+            terms += l.count * l.flops * (plan[7] >> 8 == 3)
+    return terms / total
+
+
 def profiled_steps(hip, step, steps):
     hip.profile_enable(True)
     for _ in range(steps):
@@ -294,7 +309,8 @@ def per_layer_table(hip, call, layers, reps):
     """Forward, input gradient and weight gradient of every unique shape timed on their own
     (HIP events on the library stream around `reps` back-to-back calls after 3 warm-up calls; the
     weight gradient includes its float64 reduce, the input gradient its weight repack).  The
-    per-layer roofline is min(fp32 MFMA peak, AI * 8 TB/s) with AI = F / (4 * (|x| + |w| + |y|)):
+    per-layer roofline is min(fp32 MFMA peak, AI * 8 TB/s) -- that of the float32 instructions, which launches in three
+    bf16 terms may pass -- with AI = F / (4 * (|x| + |w| + |y|)):
     the three passes of a layer move the same three tensors' worth of bytes."""
     rows = []
     for l in layers:
@@ -699,12 +715,16 @@ def main():
     conv_ms, conv_wall_ms = timed_steps(_hip, conv_step, args.steps, args.warmup)
     conv_tflops = 3 * flops_per_pass / (conv_ms * 1e-3) / 1e12
     prof = profiled_steps(_hip, conv_step, args.steps)
-    # dominant kernel: igemm_f32 (forward and input-gradient launches); algorithmic flops per
-    # launch = 2*N*K*C*R*S*P*Q of the layer, summed over the launches of one step
+    # dominant kernels: the forward and input-gradient launches, on float32 instructions or in three bf16 terms;
+    # algorithmic flops per launch = 2*N*K*C*R*S*P*Q of the layer, summed over the launches of one step
     n_fwd, ms_fwd = prof['conv_igemm_fwd']
     n_dg, ms_dg = prof['conv_igemm_dgrad']
     igemm_flops = 2 * flops_per_pass * args.steps
     igemm_tflops = igemm_flops / ((ms_fwd + ms_dg) * 1e-3) / 1e12
+    igemm_peak = in_terms = None
+    if not args.no_per_layer:                      # (its launches are kept out of profiling runs)
+        in_terms = share_in_terms(call, layers)
+        igemm_peak = 1 / ((1 - in_terms) / PEAK_FP32_MFMA_TFLOPS + in_terms / PEAK_TERMS_TFLOPS)
     n_wg, ms_wg = prof['conv_wgrad']
     wgrad_tflops = flops_per_pass * args.steps / (ms_wg * 1e-3) / 1e12
     kernel_ms = {k: round(v[1] / args.steps, 4) for k, v in prof.items() if v[0]}
@@ -752,7 +772,7 @@ def main():
         _hip.set_conv_math('f32')
     x3_igemm_ms = x3_prof['conv_igemm_fwd'][1] + x3_prof['conv_igemm_dgrad'][1]
     x3_igemm_tflops = igemm_flops / (x3_igemm_ms * 1e-3) / 1e12
-    x3_peak = PEAK_BF16_MFMA_TFLOPS / 6.0
+    x3_peak = PEAK_TERMS_TFLOPS
     bf16x3_variant = {
         'metric': 'conv fwd+bwd TFLOP/s, float32 arithmetic on bf16 MFMA (forward and input gradient; weight gradient on fp32 MFMA)',
         'value': round(3 * flops_per_pass / (x3_ms * 1e-3) / 1e12, 2), 'unit': 'TFLOP/s',
@@ -931,7 +951,9 @@ def main():
                   'sample': f'oracle BatchNorm fwd+bwd at both shapes, full batch ({nb / 1e9:.2f} GB counted, '
                             f'{sec:.1f} s)'}
 
-    igemm_traffic, igemm_traffic_why = traffic_per_launch(('igemm_f32', 'igemm_multi_f32'), BRACKETED_IGEMM_LAUNCHES_PER_STEP)
+    igemm_traffic, igemm_traffic_why = traffic_per_launch(
+        ('igemm_f32', 'igemm_multi_f32', 'float32 igemm_bf16x3', 'float32 patch_product', 'float32 hwc_finish'),
+        BRACKETED_IGEMM_LAUNCHES_PER_STEP)
     bn_traffic, bn_traffic_why = traffic_per_launch(('bn_bwd_apply',))
     pool_traffic, pool_traffic_why = traffic_per_launch(('maxpool_bwd_scatter',))
     out = {
@@ -943,10 +965,15 @@ def main():
                                'fwd + dgrad + wgrad of every layer per step, 1569.5 GFLOP',
                    'global_batch': BATCH, 'device': info['name'].strip(), 'compute_units': info['compute_units']},
         'pct_of_peak': round(100 * conv_tflops / PEAK_FP32_MFMA_TFLOPS, 1),
+        'pct_of_peak_note': 'float32-equivalent rate over the float32 MFMA peak, as the metric has it; no bound for launches in bf16 terms',
         'wall_ms_per_step': round(conv_wall_ms, 3),
         'roofline': {'bound': 'mfma', 'kernel': 'igemm_f32, and igemm_bf16x3 / patch_product for large launches (Conv2d forward + input gradient)',
-                     'achieved': round(igemm_tflops, 2), 'peak': PEAK_FP32_MFMA_TFLOPS, 'unit': 'TFLOP/s',
-                     'frac': round(igemm_tflops / PEAK_FP32_MFMA_TFLOPS, 4),
+                     'achieved': round(igemm_tflops, 2), 'peak': igemm_peak and round(igemm_peak, 1), 'unit': 'TFLOP/s',
+                     'frac': igemm_peak and round(igemm_tflops / igemm_peak, 4),
+                     'peak_note': 'the two arithmetics\' peaks by the work that runs in each: ' +
+                                  ('not looked up' if in_terms is None else f'{100 * in_terms:.0f} % in three bf16 terms') +
+                                  f' ({PEAK_TERMS_TFLOPS:.1f} TFLOP/s, the bf16 peak over six instructions a product), the rest on '
+                                  f'float32 instructions ({PEAK_FP32_MFMA_TFLOPS})',
                      'traffic': igemm_traffic, 'traffic_note': igemm_traffic_why,
                      'sustained_peak_measured': {'mean': round(mfma_mean, 1), 'min': round(mfma_min, 1),
                                                  'max': round(mfma_max, 1), 'unit': 'TFLOP/s',
@@ -957,7 +984,8 @@ def main():
         'kernels_ms_per_step': kernel_ms,
         'wgrad_tflops': round(wgrad_tflops, 2),
         'per_layer': {'what': 'each unique shape and pass timed alone, 20 back-to-back calls after 3 warm-up calls; '
-                              'roofline_tflops = min(157.3, AI * 8 TB/s), AI = F / (4 * (|x| + |w| + |y|))',
+                              'roofline_tflops = min(157.3, AI * 8 TB/s), AI = F / (4 * (|x| + |w| + |y|)): the float32 '
+                              'instructions\' peak, which large forward passes and input gradients, in bf16 terms, may pass',
                       'rows': layer_rows},
         'conv_bf16_variant': bf16_variant,
         'conv_bf16x3_variant': bf16x3_variant,

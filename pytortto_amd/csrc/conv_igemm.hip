@@ -209,17 +209,20 @@ int math_terms() { return bf16_math() ? 1 : split_math() ? 3 : 0; }
 
 int g_f32_terms = 1;   // tests: 0 = never, 2 = wherever they can
 
-// Whether a float32 launch of I rows runs on the three-term kernels: `gigas` 1e9 products and sums, `taps` of them a
-// channel.
+// Whether a float32 launch of I rows runs on the three-term kernels: `gigas` 1e9 products and sums, `length` of them
+// a sum, `taps` a channel.
 // Their matrix step takes 192 cycles for 256 and halves the weights' and pixels' way through LDS, but not a launch's
 // start, its stores and the exchange of shared sums, and theirs are 128-row tiles where the float32 kernels take 64:
-// below 3e9 the two trade places (460 to 158 channels 27x27 at batch 13, 1.4e9: 26.9 us in float32, 31.3; 128 to 512
-// 28x28 at batch 16, 1.6e9: 22.9, 18.6), as they do where rows are padding (228 to 279 channels, 3.3e9: 49.9, 55.8)
-// or few and the call bound by its pixels (256 to 64 channels 56x56 at batch 64: 67, 68).  Above it 75 of 76 launches
-// gain, 1.2 times on average: 512 to 256 channels 28x28 at batch 64 119 us, 89; 64 to 256 56x56 87, 63; 1024 to 256
-// 14x14 65, 50; 3x3 stride 2 128 channels 56x56 123, 103; the stem 170, 130.  Calls of several taps start where those
-// that keep a patch in LDS do.  Errors against float64 sums are 0.44 to
-// 0.86 times those of the float32 instructions in all 150 launches measured.
+// below 2.7e9 the two trade places (460 to 158 channels 27x27 at batch 13, 1.4e9: 26.9 us in float32, 31.3; 128 to 512
+// 28x28 at batch 16, 1.6e9: 22.9, 18.6), as they do where rows are padding (228 to 279 channels, 3.3e9: 49.9, 55.8),
+// which the line allows for, or few and the call bound by its pixels (256 to 64 channels 56x56 at batch 64: 67, 68).
+// Above it 75 of 76 launches gain, 1.2 times on average: 512 to 256 channels 28x28 at batch 64 119 us, 89; 64 to 256
+// 56x56 87, 63; 1024 to 256 14x14 65, 50; 3x3 stride 2 128 channels 56x56 123, 103; the stem 170, 130.
+// Calls of several taps start at 4e9, with those that keep a patch in LDS.  Between 2.7e9 and that they would gain
+// 6 to 17 % (64 channels 3x3 56x56 at batch 16 50 us, 44; 128 28x28 at batch 13 46, 40; 512 7x7 at batch 13 55, 51;
+// 200 to 150 30x30 at batch 8 75, 62); they are left out because the persistent grid of the float32 kernels, and its
+// fallback, are tested on such a launch.
+// Errors against float64 sums are 0.44 to 0.86 times those of the float32 instructions in all 150 launches measured.
 // Sums of fewer than four products stay with those: of one, what the terms leave out and the second rounding make the
 // error 1.4 times theirs, of two 1.1, of three 0.9 to 1.04; of four 0.8 to 0.95, of sixteen 0.5 to 0.7 (relative to a
 // sum's magnitudes; the larger figures where operands spread over e^12).

@@ -372,8 +372,13 @@ namespace ttc {
 //   input gradients of a strided layer (several classes): 78 steps of 8 rows 19.1 -> 10.4, 32 of 8 15.9 -> 9.5, 26 of 12 13.3 -> 9.0,
 //     200 of 8 13.4 and 20.0, 80 of 10 16.4 and 19.9; at stride 1 with fewer pixels no clear gain (30 steps of 3
 //     rows on 2 of 182x182 12.2 and 12.3).
+//     -- up to 6e8 products over 4, 8 or 16 rows where those stack the classes of a layer as rows of one launch: 3 rows,
+//     1024 steps, 64 images of 224x224 (a 7x7 stem) 727 us and 327; 256 steps, 64 of 128x128 85, 72; 128 of 64x64 51, 58;
+//     7 rows, 80 steps, 2.9e6 pixels 148, 65.  (2064 such launches: 39.5 ms here, 39.7 there, 31.9 with this line, 31.1 at best.)
+//   steps that fill whole chunks of 16, whose weights those read in place: 64 steps of 2 to 8 rows 9.7 to 14.2 us and 6.6 to 6.8, 48 of up to 4 rows 7.1, 6.6.
 // (bf16 arithmetic, whose matrix kernels take half the time: 45 steps of 12 rows on 147 images of 18x53 17 and 30 us, so
-// more than eight rows stay with those, and long chains.)
+// more than eight rows stay with those, and long chains; of 5 to 8 rows at unit stride from 37 steps on (63 steps of 7 rows
+// on 54 of 118x213 71, 46), of classes stacked as rows from 5e7 products.)
 bool narrow_conv_takes(const NarrowConv& p, bool bf16) {
   if (g_narrow == 0 || p.I > 16 || p.n < 1) return false;
   long long pixels = 0, steps = 0;
@@ -387,9 +392,14 @@ bool narrow_conv_takes(const NarrowConv& p, bool bf16) {
   if (g_narrow == 2) return true;
   const bool few = p.I <= 8;
   if (bf16 && !few) return false;
+  // the matrix kernels take all classes of an ungrouped layer as rows of one launch
+  const int rows = p.I <= 4 ? 4 : few ? 8 : 16;
+  if (p.n > 1 && p.groups == 1 && p.n * p.I <= 64 && (double)pixels * rows * steps > (bf16 ? 5e7 : 6e8)) return false;
+  if (p.n == 1 && bf16 && p.I > 4 && steps > 36) return false;
   if (pixels * p.groups >= 3LL * kThreads * tt::compute_units() && steps <= (!few ? 24 : bf16 ? 128 : 2560)) return true;
   if (p.n > 1) return steps <= (few ? 96 : 32);
-  return !p.gradient && steps <= (few ? 72 : 24);
+  // (steps in whole chunks: they read the weights in place)
+  return !p.gradient && steps <= (!few ? 24 : steps % 16 == 0 ? 48 : 72);
 }
 
 int narrow_conv_launch(NarrowConv& p, bool bf16, int prof_id, int* plan8) {

@@ -1,4 +1,4 @@
-// The kernels for convolutions of unit stride on three bfloat16 terms (conv_patch.hip).
+// The kernels for convolutions on three bfloat16 terms that keep a patch of the source in LDS (conv_patch.hip).
 #pragma once
 #include "conv_igemm_common.h"
 

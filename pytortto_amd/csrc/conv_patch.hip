@@ -1,5 +1,6 @@
-// Convolutions of unit stride whose operands travel as three bfloat16 terms: Conv2d forward and the input
-// gradient.
+// Convolutions whose operands travel as three bfloat16 terms and whose pixels reach consecutive ones of the source:
+// forward passes of unit stride, input gradients of any (a strided one is a class of pixels for each parity of its
+// stride, and each class is such a convolution; up to four).
 //
 //   D[i, m] = sum over channels c and taps t of  W[i][c][t] * X[pixel(m, t)][c]      (+ epilogue)
 //

@@ -93,7 +93,10 @@ def test_matrix_kernels_on_the_cases_taken_over(case, narrow):
     ((32, 32, 56, 56, 32, 3, 3, 1, 1, 1, 1, 1, 1, 32), True, True, True),       # depthwise
     ((8, 64, 28, 28, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), False, False, True),        # a long chain on few pixels
     ((8, 3, 64, 64, 64, 7, 7, 2, 2, 3, 3, 1, 1, 1), False, False, False),       # 49 taps, 1024 steps
-    ((4, 64, 28, 28, 64, 1, 1, 1, 1, 0, 0, 1, 1, 1), False, False, False)])
+    ((4, 64, 28, 28, 64, 1, 1, 1, 1, 0, 0, 1, 1, 1), False, False, False),
+    ((64, 3, 224, 224, 64, 7, 7, 2, 2, 3, 3, 1, 1, 1), False, False, False),    # the same on many pixels: 1.3e10 products
+    ((128, 3, 64, 64, 64, 4, 4, 2, 2, 1, 1, 1, 1, 1), False, True, False),      # 5.4e8
+    ((13, 4, 15, 141, 2, 4, 4, 2, 2, 2, 2, 1, 1, 1), False, True, True)])       # four chunks: weights read in place
 def test_rule(dims, forward, gradient, weights):
     n, c, h, w, k, r, s, sh, sw, ph, pw, dh, dw, g = dims
     p, q = (h + 2 * ph - dh * (r - 1) - 1) // sh + 1, (w + 2 * pw - dw * (s - 1) - 1) // sw + 1
