@@ -40,7 +40,7 @@ struct NarrowWgrad {
   int xN, xG, dyN, dyG, xBias;   // xBias = ph*W + pw
   int KT, JT, tilesI, tilesJ, splits, perSplit;   // set by narrow_wgrad_takes
 };
-bool narrow_wgrad_takes(NarrowWgrad& p);
+bool narrow_wgrad_takes(NarrowWgrad& p, bool bf16);
 size_t narrow_wgrad_workspace(const NarrowWgrad& p);
 int narrow_wgrad_launch(NarrowWgrad& p, bool bf16);
 

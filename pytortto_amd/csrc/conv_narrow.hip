@@ -424,7 +424,7 @@ int narrow_conv_launch(NarrowConv& p, bool bf16, int prof_id, int* plan8) {
   return 0;
 }
 
-bool narrow_wgrad_takes(NarrowWgrad& p) {
+bool narrow_wgrad_takes(NarrowWgrad& p, bool bf16) {
   if (g_narrow == 0 || p.R * p.S > 31) return false;
   const long long span = 255 / (long long)p.PQ + 2;
   const long long reach = 4 * ((span + 1) * std::max(p.xN, p.dyN) + 2LL * p.xBias + ((long long)p.H + p.ph + (long long)p.R * p.dh + 2) * p.W +
@@ -448,7 +448,18 @@ bool narrow_wgrad_takes(NarrowWgrad& p) {
   // those kernels add their partial sums themselves (1x1, 1 x 64, 8 of 28x28: 11.6 and 12.6; 8 x 657 of 1309 pixels 12.7
   // and 15.8).
   const bool fits = p.Kg <= 8 || p.J <= 8 || (p.Kg <= 16 && p.J <= 96);
-  return fits && (p.R * p.S > 1 ? p.M >= 4096 || p.J <= 128 : p.M >= 16384);
+  const bool taps = p.R * p.S > 1;
+  if (!fits || (taps ? p.M < 4096 && p.J > 128 : p.M < 16384)) return false;
+  // Over 6780 launches that are left (144.2 ms here, 214.6 on the matrix kernels) one in seventeen was more than 8 % slower
+  // here; most of them are among these, which go back (142.8 ms, and one in a hundred):
+  //   sums that take the second launch, of up to 64 columns: one tile there, added in place (1103 launches 14.2 -> 13.4 ms);
+  if (taps && p.J <= 64 && p.splits > 1 && p.M < (bf16 && p.J > 16 ? 16384 : 8192)) return false;
+  //   a chain or two of steps, where one block's start is all of it (166 launches 7.8 -> 7.0 us each);
+  if (taps && p.M <= 128 && p.J > 8 && p.J <= 128) return false;
+  //   and in bf16 arithmetic many products a fetched value: the matrix kernels take half the time (41 of more than eight
+  //   rows 33 -> 29 us each, 65 of five to eight 90 -> 85).
+  if (bf16 && (p.Kg > 8 ? p.J > 32 && p.M > 32768 : p.Kg > 4 && p.J > 1024)) return false;
+  return true;
 }
 size_t narrow_wgrad_workspace(const NarrowWgrad& p) {
   return p.splits > 1 ? sizeof(float) * 64 * (size_t)p.tilesI * p.tilesJ * p.groups * p.splits : 0;

@@ -955,7 +955,7 @@ static int conv2d_wgrad(const float* x, const float* dy, float* dw, int N, int C
     ttc::NarrowWgrad nw{x, dy, dw, nullptr, Kg, J, N * P * Q, groups, tt::make_fastdiv((uint32_t)(P * Q)), tt::make_fastdiv((uint32_t)Q),
                         tt::make_fastdiv((uint32_t)(R * S)), tt::make_fastdiv((uint32_t)S), H, W, H * W, P * Q, R, S, sh, sw, ph, pw,
                         dh, dw_, C * H * W, Cg * H * W, K * P * Q, Kg * P * Q, ph * W + pw, 0, 0, 0, 0, 0, 0};
-    if (ttc::narrow_wgrad_takes(nw)) {
+    if (ttc::narrow_wgrad_takes(nw, bf16)) {
       if (size_only) {
         *size_only = ttc::narrow_wgrad_workspace(nw);
         return 0;

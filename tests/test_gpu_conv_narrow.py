@@ -8,6 +8,7 @@ import pytest
 import oracle
 from pytortto_amd import _hip, ops
 from pytortto_amd.xparray import hiparray
+from tests.brute import bf16_round
 from tests.cases import CONV_CASES, CONVT_CASES, random_conv_cases, random_convt_cases, random_large_kernel_cases
 from tests.test_gpu_conv import TILE_CASES, _check, _last_launch, _run_conv
 from tests.test_gpu_conv_bf16 import _forward_and_input_gradient
@@ -96,7 +97,7 @@ def test_matrix_kernels_on_the_cases_taken_over(case, narrow):
     ((4, 64, 28, 28, 64, 1, 1, 1, 1, 0, 0, 1, 1, 1), False, False, False),
     ((64, 3, 224, 224, 64, 7, 7, 2, 2, 3, 3, 1, 1, 1), False, False, False),    # the same on many pixels: 1.3e10 products
     ((128, 3, 64, 64, 64, 4, 4, 2, 2, 1, 1, 1, 1, 1), False, True, False),      # 5.4e8
-    ((13, 4, 15, 141, 2, 4, 4, 2, 2, 2, 2, 1, 1, 1), False, True, True)])       # four chunks: weights read in place
+    ((13, 4, 15, 141, 2, 4, 4, 2, 2, 2, 2, 1, 1, 1), False, True, False)])      # four chunks: weights read in place
 def test_rule(dims, forward, gradient, weights):
     n, c, h, w, k, r, s, sh, sw, ph, pw, dh, dw, g = dims
     p, q = (h + 2 * ph - dh * (r - 1) - 1) // sh + 1, (w + 2 * pw - dw * (s - 1) - 1) // sw + 1
@@ -110,3 +111,38 @@ def test_rule(dims, forward, gradient, weights):
     plan = (ctypes.c_int * 4)()
     _hip.call('tt_conv2d_last_wgrad_launch', plan)
     assert (plan[2] == -3) == weights
+
+
+@pytest.mark.parametrize('dims,f32,bf16', [
+    ((2, 4, 32, 16, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, True),         # 36 columns, 1024 pixels: one launch
+    ((2, 4, 33, 16, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), False, False),       # 1056
+    ((2, 8, 33, 16, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, True),         # 72 columns
+    ((8, 4, 32, 32, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, False),        # 8192
+    ((16, 4, 32, 32, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, True),        # 16384
+    ((1, 4, 8, 16, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), False, False),        # 128
+    ((1, 4, 8, 17, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, True),
+    ((33, 33, 32, 32, 9, 1, 1, 1, 1, 0, 0, 1, 1, 1), True, False),      # nine rows, 33 columns, 33792
+    ((33, 32, 32, 32, 9, 1, 1, 1, 1, 0, 0, 1, 1, 1), True, True),
+    ((8, 114, 32, 32, 5, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, False),      # five rows, 1026 columns
+    ((8, 114, 32, 32, 4, 3, 3, 1, 1, 1, 1, 1, 1, 1), True, True)])
+def test_rule_of_the_weight_gradient(dims, f32, bf16):
+    import torch
+    n, c, h, w, k, r, s, sh, sw, ph, pw, dh, dw, g = dims
+    p, q = (h + 2 * ph - dh * (r - 1) - 1) // sh + 1, (w + 2 * pw - dw * (s - 1) - 1) // sw + 1
+    rng = np.random.default_rng(2)
+    x, dy = (rng.standard_normal(a).astype(np.float32) for a in ((n, c, h, w), (n, k, p, q)))
+    plan = (ctypes.c_int * 4)()
+    try:
+        for math, narrow_ones in (('f32', f32), ('bf16', bf16)):
+            _hip.set_conv_math(math)
+            got = ops.conv2d_wgrad(hiparray(x), hiparray(dy), (k, c // g, r, s), (sh, sw), (ph, pw), (dh, dw), g).get()
+            _hip.call('tt_conv2d_last_wgrad_launch', plan)
+            assert (plan[2] == -3) == narrow_ones
+            a, b = (torch.tensor(v if math == 'f32' else bf16_round(v), dtype=torch.float64) for v in (x, dy))
+
+            def sums(a, b):
+                return torch.nn.grad.conv2d_weight(a, (k, c // g, r, s), b, (sh, sw), (ph, pw), (dh, dw), g).numpy()
+            # a sum of m rounded products is off by about sqrt(m) roundings of its magnitudes' sum, in whatever order
+            assert (np.abs(got - sums(a, b)) <= 2.0 ** -24 * (n * p * q) ** .5 * sums(a.abs(), b.abs())).all()
+    finally:
+        _hip.set_conv_math('f32')
