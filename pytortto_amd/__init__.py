@@ -42,8 +42,9 @@ class cuda:
         convolution passes with operands rounded to bfloat16 inside the kernels and float32
         accumulation; tensors stay float32, results then differ from the float32 path by a few 1e-3
         of their magnitude -- or ``'bf16x3'``: float32 arithmetic carried out on the bf16 matrix
-        instructions (three exact bf16 terms per operand element), which meets the float32 path's
-        tolerances and is faster on layers with at least one tile per compute unit."""
+        instructions (three exact bf16 terms per operand element) in every forward pass and input
+        gradient, which meets the float32 path's tolerances.  ``'f32'`` carries its large calls out
+        that way too, with operands of any magnitude, so this mode gains on smaller ones only."""
         _hip.set_conv_math(mode)
 
     @staticmethod

@@ -329,7 +329,7 @@ def set_conv_math(mode):
     instructions), 'bf16' (operands rounded to bfloat16 inside the kernel, float32 accumulation;
     tensors stay float32) or 'bf16x3' (float32 arithmetic on the bf16 matrix pipe: every operand
     element as three bf16 terms that add up to it exactly, six products per step; meets the same
-    tolerances as 'f32')."""
+    tolerances as 'f32', which takes that path for large calls by itself)."""
     if mode not in CONV_MATH:
         raise ValueError(f"conv math must be one of {sorted(CONV_MATH)}, got {mode!r}")
     call('tt_set_conv_math', CONV_MATH[mode])
