@@ -425,7 +425,7 @@ struct Plan {
   int WM, NT, IT, Ipad, maxPx, chunks, perSplit, splits, tiles;
   int px[kPatchClasses], PW[kPatchClasses], VR[kPatchClasses], block0[kPatchClasses];
   size_t at[kPatchClasses], wt, partial;   // the classes' weights (units of 16 bytes); bytes of workspace
-  double cost;
+  double cost, longest;   // microseconds: of the launch, of its longest block
 };
 
 int g_patch = 1;   // tests: 0 = never, 2 = wherever they can
@@ -485,6 +485,7 @@ bool make_plan(const PatchConv& c, Plan* best) {
         pl.perSplit = per;
         pl.splits = s;
         pl.cost = cost;
+        pl.longest = longest;
         pl.partial = s > 1 ? align_up(sizeof(float) * (size_t)s * (size_t)outputs) : 0;
         *best = pl;
       }
@@ -535,7 +536,19 @@ bool patch_conv_takes(const PatchConv& c, bool f32) {
   // and 90 to 102).  From 4e9 on the kernels that gather run on three terms too (f32_terms); 7.0 here moves some
   // launches of a PreAct-ResNet-18 step and its time by less than runs differ (4.70 ms, 4.73).
   const double padding = (double)pl.chunks * kBK * pl.Ipad / ((double)c.C * c.I);
-  return padding <= 1.5 && pl.cost + 3 + 4e-6 * c.I * c.C * c.taps < 16 + (f32 ? 7.5 : 7.0) * gigas;
+  const double weights = 4e-6 * c.I * c.C * c.taps;
+  if (padding > 1.5 || pl.cost + 3 + weights >= 16 + (f32 ? 7.5 : 7.0) * gigas) return false;
+  if (f32) return true;
+  // Outside float32 arithmetic, where the other side is the same product, one in eight of 1339 launches that are left was
+  // more than 8 % slower here (194.9 ms here, 223.7 there, 191.6 at best).  Most had between one and two blocks to a compute
+  // unit, of which some run two while the others wait, or several classes; and the others' time grows with the padding of
+  // their rows.  With these three in the line 1045 stay (193.4 ms, 32 slower by more than 8 %; of another draw 3424, 3.6 %
+  // of them slower, 1.18 times as fast in all): 36 to 363 channels 4x4 7x28 at batch 24 41.9 us and 31.7 go back, 96 to 62
+  // 5x5 7x42 at batch 58 65.4 and 54.7.
+  const int blocks = pl.tiles * pl.splits, cus = tt::compute_units();
+  const double here = blocks > cus && blocks <= 2 * cus ? std::max(pl.cost, 1.75 * pl.longest) : pl.cost;
+  const int rows = c.I > 64 ? 128 : 32;
+  return here + weights + (c.n > 1 ? 6 : 0) < 14 + (2.3 + 4.7 * (ceil_div(c.I, rows) * rows) / c.I) * gigas;
 }
 
 int patch_conv_launch(const PatchConv& c, const float* x, const float* w, const float* bias, float* out, const Epilogue* epi,

@@ -83,6 +83,21 @@ def test_the_workspace_holds_what_is_read_ahead(c, r, patch):
     assert size.value >= 3072 * (4 * taps + 2 + taps % 2)
 
 
+@pytest.mark.parametrize('dims,bf16x3,f32', [
+    ((128, 128, 16, 16, 128, 3, 1), True, True),      # 256 blocks
+    ((136, 128, 16, 16, 128, 3, 1), False, True),     # 272: some compute units have two to run
+    ((264, 128, 16, 16, 128, 3, 1), True, True),      # 528
+    ((24, 36, 7, 28, 363, 4, 2), False, False),       # 264, and below what float32 arithmetic sends here
+    ((58, 96, 7, 42, 62, 5, 2), False, True)])        # 268 that share their reductions
+def test_rule(dims, bf16x3, f32, patch):
+    n, c, h, w, k, r, pad = dims
+    x, wt = hiparray.zeros((n, c, h, w)), hiparray.zeros((k, c, r, r))
+    for math, expected in (('bf16x3', bf16x3), ('f32', f32)):
+        patch(WHERE_FASTER, math)
+        ops.conv2d_fwd(x, wt, None, (1, 1), (pad, pad), (1, 1), 1)
+        assert (_last_launch()['persistent_blocks'] == -4) == expected, math
+
+
 @pytest.mark.parametrize('math', ['bf16x3', 'f32'])
 @pytest.mark.parametrize('n,c,hw,k', [(9, 64, 14, 96), (2, 256, 7, 70), (40, 32, 28, 64)])   # the second shares its reduction
 def test_epilogues(n, c, hw, k, math, patch):
